@@ -12,6 +12,7 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
@@ -64,6 +65,21 @@ def build_library(verbose=False, jobs=8, defines=(), output=None):
     return lib_path
 
 
+NATIVE_PATH = os.path.join(HERE, "_native.so")
+
+
+def build_native():
+    """Compiles the CPython module behind ops.py (host code only; it calls
+    libsnn_hip.so by address, so it links to nothing of it)."""
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared",
+           "-fvisibility=hidden", "-Wall", "-Wextra",
+           "-I" + sysconfig.get_paths()["include"],
+           "-I" + os.path.join(ROOT, "include"),
+           os.path.join(CSRC, "py_native.cpp"), "-o", NATIVE_PATH]
+    subprocess.check_call(cmd)
+    return NATIVE_PATH
+
+
 CPP_TEST_DIR = os.path.join(ROOT, "tests", "cpp")
 
 
@@ -104,4 +120,5 @@ if __name__ == "__main__":
     a = ap.parse_args()
     print(build_library(verbose=a.v, defines=a.define, output=a.output))
     if a.output is None:
+        print(build_native())
         print(build_cpp_tests())
