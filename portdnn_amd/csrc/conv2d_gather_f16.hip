@@ -1,0 +1,991 @@
+// Half-precision forward convolution and input gradient for every window,
+// stride and channel count, as an implicit GEMM on MFMA (gfx950): binary16
+// operands, fp32 accumulation, binary16 result.
+//
+//   forward         Y[pixel][f]  = sum over (tap, c) X[pixel o tap][c] * W[tap][c][f]
+//   input gradient  dX[pixel][c] = sum over (tap, f) dY[pixel o tap][f] * W[tap'][c][f]
+//
+// (the Forward and InputBackprop directions of sycldnn::conv2d::launch,
+// include/portdnn/conv2d/launch.h:59-118.)  The gradient of a strided
+// convolution is split by classes: the dX pixels whose padded row and column
+// have one remainder modulo the strides are reached by the same sub-window of
+// taps, and form a dense stride-1 convolution of dY with that sub-filter.  All
+// classes run in one launch, the one with the most taps first, and store their
+// pixels straight into dX; a class that no tap reaches stores zeros.
+//
+// The reduction runs over 16-byte pieces -- eight channels of one tap -- of a
+// pixel, flattened over (tap, piece): chunks of 32 channels are four pieces,
+// which may belong to different taps, so channel counts that are no multiple
+// of 32 waste nothing but the last chunk's tail.  Source tensors whose channel
+// count is no multiple of 8 are copied once with the count rounded up.
+//
+//   * A work-group owns BM pixels x BN features.  Per chunk both tiles, [row][4
+//     pieces], arrive in one of three LDS buffers by loads that write LDS
+//     directly (1 KB = 16 rows per instruction), two chunks ahead: one barrier
+//     per chunk, and no wave waits for more than the loads of the chunk it is
+//     about to multiply.  Padding pixels, ragged tails and rows past the last
+//     pixel load from out of range, which stores zeros.
+//   * Which of its four positions in an LDS row a piece takes is XORed with
+//     bits of the row, so that the ds_read_b128 of 8 or 16 consecutive rows
+//     touch different banks.
+//   * A forward filter (and a gradient's whose feature count is no multiple of
+//     8) is packed first, [32 features][chunk][row][4 pieces] in the same
+//     swizzled order (2-5 us), zeros where channels or features end.  The
+//     gradient's is read in place: its reduction index is the contiguous one.
+//   * Features are the MFMA rows and pixels the columns, with the features of
+//     a block permuted in the packed filter so that a lane ends with 16
+//     consecutive features of one pixel (two 16-byte stores).
+#include <algorithm>
+#include <climits>
+#include <cmath>
+#include <cstdlib>
+#include <cstring>
+
+#include "gemm_tile.h"
+#include "snn_kernels.h"
+
+namespace snn {
+namespace {
+
+using gemm::float16v;
+using gemm::xcd_remap;
+
+typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+typedef unsigned int uint2v __attribute__((ext_vector_type(2)));
+typedef unsigned int uint4v __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) void* lds_ptr;
+constexpr unsigned kOob = 0x7FFFFFF0u;
+constexpr size_t kMaxBufferBytes = 0x7FFFFFF0u;
+constexpr int kRowBytes = 64;     // one chunk (32 halves) of one row
+constexpr int kMaxClasses = 16;
+constexpr int kMaxWindow = 12;    // the two tap masks of a pixel share a word
+
+// n / d for 0 <= n < 2^31 by one multiplication: (2 n * magic) >> (32 + shift)
+// with magic = ceil(2^(31 + shift) / d), 2^shift >= d.  (Divisions by values
+// known at launch only are 35 instructions; a lane has a dozen of them, as long
+// as the multiplications of a short reduction.)
+struct Divisor {
+  unsigned magic, shift;
+};
+Divisor divisor(int d) {
+  unsigned shift = 0;
+  while ((1u << shift) < static_cast<unsigned>(d)) ++shift;
+  const unsigned long long top = 1ull << (31 + shift);
+  return {static_cast<unsigned>((top + d - 1) / d), shift};
+}
+__device__ __forceinline__ int divide(int n, Divisor d) {
+  return static_cast<int>(
+      __umulhi(static_cast<unsigned>(n) << 1, d.magic) >> d.shift);
+}
+
+struct GatherClass {
+  int rows, cols;        // pixels of the class per image
+  Divisor by_rows, by_cols;
+  int pixels;            // ... and over the batch
+  int off_r, off_c;      // source row / column of tap (0, 0) for pixel (0, 0)
+  int win_r, win_c;      // taps
+  int out_r0, out_c0;    // output row / column of pixel (0, 0)
+  int n_chunks;
+  unsigned pack_block;   // first 2 KB block of its packed filter
+  Divisor by_win_c;
+  int tap_r0, tap_rs;    // filter row of tap row t: tap_r0 + t * tap_rs
+  int tap_c0, tap_cs;
+};
+
+struct Gather {
+  int src_rows, src_cols;
+  int cp;                // pieces per source pixel
+  Divisor by_cp;
+  int step_r, step_c;    // source step per class pixel
+  int out_rows, out_cols, out_step_r, out_step_c;
+  int channels, features;
+  int win_cols;          // columns of the whole filter
+  int n_tiles_n;
+  int n_splits;          // work-groups that share a tile's reduction
+  unsigned n_tiles;      // tiles of all classes
+  int n_classes;
+  int mirrored;          // input gradient: w[tap][feature][channel]
+  GatherClass cls[kMaxClasses];
+};
+
+__device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* p,
+                                                   unsigned bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes,
+                                           0x00020000);
+}
+
+// Position of piece c in LDS row r: c ^ swz(r % 16).
+__host__ __device__ constexpr unsigned swz(unsigned r16) {
+  return ((r16 >> 1) ^ (r16 >> 3)) & 3u;
+}
+
+// Image, row and column of pixel m of a class.
+struct Pixel { int n, y, x; };
+__device__ __forceinline__ Pixel pixel_of(int m, const GatherClass& cls) {
+  const int t = divide(m, cls.by_cols);
+  const int n = divide(t, cls.by_rows);
+  return {n, t - n * cls.rows, m - t * cls.cols};
+}
+
+// Which feature of its block of 32 an MFMA row holds.  A lane's accumulators are
+// rows 8 g + 4 h + i (h = lane / 32): g = 0, 1 become features 8 h ... + 7 and
+// g = 2, 3 features 16 + 8 h ... + 7, so that one 16-byte store of the two lanes
+// of a pixel covers 32 consecutive bytes.
+__host__ __device__ constexpr int feature_of_row(unsigned row) {
+  return static_cast<int>(16 * (row >> 4) + 8 * ((row >> 2) & 1) +
+                          4 * ((row >> 3) & 1) + (row & 3));
+}
+
+// (a function of its own: the compiler drops the host side of a kernel template
+// whose body names the LDS-direct load)
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t rsrc,
+                                            char* lds, unsigned offset) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr)lds, 16, offset, 0, 0,
+                                           0);
+}
+
+constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
+
+// Tiles run over feature tiles, then classes, then pixels: the classes of one
+// piece of dX are written side by side.  (Class after class, every work-group
+// in flight wrote the same half of the rows and columns, which are the same
+// half of the memory channels: 56x56x256 <- 512, 1x1 stride 2, at batch 128,
+// 168 -> 110 us;
+// 56x56x128 <- 128, 3x3, 73 -> 61.)
+struct TileOf { int m, cls, n; };
+__device__ __forceinline__ TileOf tile_of(unsigned tile, const Gather& g) {
+  const unsigned n = tile % g.n_tiles_n, t = tile / g.n_tiles_n;
+  return {static_cast<int>(t / g.n_classes), static_cast<int>(t % g.n_classes),
+          static_cast<int>(n)};
+}
+
+// Filter pack (the first n_pack_groups work-groups, one lane per 16-byte
+// piece) and, behind it, the copy of a source tensor to whole pieces.
+__global__ void __launch_bounds__(256)
+    gather_prepare_kernel(const _Float16* __restrict__ w,
+                          _Float16* __restrict__ wpk, Gather g,
+                          unsigned n_pack_lanes, unsigned n_pack_groups,
+                          const _Float16* __restrict__ src,
+                          _Float16* __restrict__ wide, unsigned n_pieces) {
+  half8 v;
+  if (blockIdx.x < n_pack_groups) {
+    const unsigned idx = blockIdx.x * 256 + threadIdx.x;
+    if (idx >= n_pack_lanes) return;
+    const unsigned block = idx >> 7, row = (idx >> 2) & 31, slot = idx & 3;
+    int k = 0;
+    while (k + 1 < g.n_classes && block >= g.cls[k + 1].pack_block) ++k;
+    const GatherClass& cls = g.cls[k];
+    const unsigned local = block - cls.pack_block;
+    const unsigned nb = local / cls.n_chunks, chunk = local % cls.n_chunks;
+    const int q = static_cast<int>(chunk * 4 + (slot ^ swz(row & 15)));
+    const int tap = divide(q, g.by_cp);
+    const int c = (q - tap * g.cp) * 8;
+    const int tr = divide(tap, cls.by_win_c), ts = tap - tr * cls.win_c;
+    const int f = nb * 32 + feature_of_row(row);
+    const bool ok = tr < cls.win_r && f < g.features;
+    const int valid = ok ? min(8, g.channels - c) : 0;
+    const size_t at_tap =
+        static_cast<size_t>((cls.tap_r0 + tr * cls.tap_rs) * g.win_cols +
+                            cls.tap_c0 + ts * cls.tap_cs);
+    const _Float16* from =
+        g.mirrored ? w + (at_tap * g.features + f) * g.channels + c
+                   : w + (at_tap * g.channels + c) * g.features + f;
+    const size_t stride = g.mirrored ? 1 : static_cast<size_t>(g.features);
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      v[e] = e < valid ? from[e * stride] : static_cast<_Float16>(0.f);
+    *reinterpret_cast<half8*>(wpk + static_cast<size_t>(idx) * 8) = v;
+    return;
+  }
+  const unsigned idx = (blockIdx.x - n_pack_groups) * 256 + threadIdx.x;
+  if (idx >= n_pieces) return;
+  const unsigned pixel = divide(idx, g.by_cp);
+  const int c = static_cast<int>(idx - pixel * g.cp) * 8;
+  const _Float16* from = src + static_cast<size_t>(pixel) * g.channels + c;
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    v[e] = c + e < g.channels ? from[e] : static_cast<_Float16>(0.f);
+  *reinterpret_cast<half8*>(wide + static_cast<size_t>(idx) * 8) = v;
+}
+
+// WM x WN waves of TM x TN blocks of 32 pixels x 32 features.  UNIFORM: whole
+// chunks per tap (channels in multiples of 32), tap bookkeeping in scalar
+// registers; otherwise every lane works out the tap of its own piece.  IN_PLACE:
+// `wpk` is the gradient's filter itself, w[tap][feature][channel].
+template <int WM, int WN, int TM, int TN, bool UNIFORM, bool IN_PLACE>
+__global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
+    conv_gather_f16_kernel(const _Float16* __restrict__ src,
+                           const _Float16* __restrict__ wpk,
+                           _Float16* __restrict__ dst,
+                           float* __restrict__ part, Gather g,
+                           unsigned src_bytes, unsigned wpk_bytes,
+                           unsigned dst_bytes, unsigned n_groups) {
+  constexpr int NW = WM * WN;
+  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
+  constexpr int LA = BM / 16 / NW;                      // loads per wave, chunk
+  constexpr int B_BLOCKS = BN / 16;
+  constexpr int LB = B_BLOCKS >= NW ? B_BLOCKS / NW : 1;
+  static_assert(LA * NW * 16 == BM && (B_BLOCKS % NW == 0 || NW % B_BLOCKS == 0),
+                "whole load instructions per wave");
+  constexpr int STAGE = (BM + BN) * kRowBytes;
+  // three objects, so that the compiler ties an LDS read to the loads of its
+  // own buffer only
+  __shared__ __align__(1024) char buf0[STAGE];
+  __shared__ __align__(1024) char buf1[STAGE];
+  __shared__ __align__(1024) char buf2[STAGE];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = threadIdx.x >> 6;
+  const int wm = wave / WN, wn = wave % WN;
+  const unsigned group = xcd_remap(blockIdx.x, n_groups);
+  const unsigned tile = group / g.n_splits, split = group % g.n_splits;
+  const TileOf at = tile_of(tile, g);
+  const GatherClass cls = g.cls[at.cls];
+  const int m0 = at.m * BM, n0 = at.n * BN;
+  if (m0 >= cls.pixels) return;
+  const int per_split = (cls.n_chunks + g.n_splits - 1) / g.n_splits;
+  const int chunk0 = min(cls.n_chunks, static_cast<int>(split) * per_split);
+  const int n_chunks = min(cls.n_chunks - chunk0, per_split);
+
+  // A class that no tap reaches: zeros, whole runs of features per pixel.
+  if (cls.n_chunks == 0 && (g.features & 7) == 0) {
+    if (split != 0) return;
+    const __amdgpu_buffer_rsrc_t out = make_rsrc(dst, dst_bytes);
+    for (int i = threadIdx.x; i < BM * (BN / 8); i += 64 * NW) {
+      const int m = m0 + i / (BN / 8), f = n0 + i % (BN / 8) * 8;
+      const Pixel px = pixel_of(m, cls);
+      const unsigned pixel =
+          (px.n * g.out_rows + px.y * g.out_step_r + cls.out_r0) * g.out_cols +
+          px.x * g.out_step_c + cls.out_c0;
+      const uint4v zero = {0u, 0u, 0u, 0u};
+      __builtin_amdgcn_raw_buffer_store_b128(
+          zero, out, m < cls.pixels && f < g.features
+                         ? (pixel * g.features + f) * 2u : kOob, 0, 0);
+    }
+    return;
+  }
+
+  const __amdgpu_buffer_rsrc_t src_rsrc = make_rsrc(src, src_bytes);
+  const __amdgpu_buffer_rsrc_t wpk_rsrc = make_rsrc(wpk, wpk_bytes);
+
+  // Rows this lane loads: byte offset of tap (0, 0), the lane's piece included
+  // where it is the same for every chunk, and the taps inside the image (rows
+  // in the low half of the word, columns in the high half).
+  const unsigned piece = (lane & 3u) ^ swz((lane >> 2) & 15u);
+  unsigned a_off[LA], a_mask[LA];
+#pragma unroll
+  for (int i = 0; i < LA; ++i) {
+    const int m = m0 + 16 * (wave + NW * i) + (lane >> 2);
+    const Pixel px = pixel_of(m, cls);
+    const int iy = px.y * g.step_r + cls.off_r;
+    const int ix = px.x * g.step_c + cls.off_c;
+    // taps r with 0 <= iy + r < src_rows, bits low .. high - 1
+    auto bits = [](int low, int high) {
+      low = max(low, 0);
+      return high > low ? (1u << high) - (1u << low) : 0u;
+    };
+    const unsigned rows = bits(-iy, min(cls.win_r, g.src_rows - iy));
+    const unsigned cols = bits(-ix, min(cls.win_c, g.src_cols - ix));
+    a_mask[i] = m < cls.pixels ? rows | cols << 16 : 0u;
+    a_off[i] = (static_cast<unsigned>((px.n * g.src_rows + iy) * g.src_cols + ix) *
+                    g.cp + (UNIFORM ? piece : 0u)) * 16u;
+  }
+  unsigned b_off[LB];  // of chunk 0
+  int b_block[LB];
+#pragma unroll
+  for (int i = 0; i < LB; ++i) {
+    b_block[i] = (wave + NW * i) % B_BLOCKS;
+    if constexpr (IN_PLACE) {
+      const int f = n0 + b_block[i] / 2 * 32 +
+                    feature_of_row((b_block[i] & 1) * 16 + (lane >> 2));
+      // (2^31 stays out of range whatever is added)
+      b_off[i] = f < g.features ? static_cast<unsigned>(f * g.channels) * 2u +
+                                      (UNIFORM ? piece * 16u : 0u)
+                                : 0x80000000u;
+    } else {
+      b_off[i] = ((cls.pack_block + static_cast<unsigned>(n0 / 32 + b_block[i] / 2) *
+                                        cls.n_chunks) * 2 +
+                  (b_block[i] & 1)) * 1024u + lane * 16u;
+    }
+  }
+
+  const int cp = g.cp, src_cols = g.src_cols, win_c = cls.win_c;
+  const Divisor by_cp = g.by_cp, by_win_c = cls.by_win_c;
+  int tap_r = 0, tap_c = 0, c4 = 0;  // UNIFORM: of the next chunk to load
+  int q = chunk0 * 4 + piece;        // otherwise: the lane's next piece
+  if (UNIFORM && chunk0 > 0) {
+    const int tap = chunk0 * 4 / cp;
+    c4 = chunk0 * 4 - tap * cp;
+    tap_r = tap / win_c;
+    tap_c = tap - tap_r * win_c;
+  }
+  unsigned b_chunk = IN_PLACE ? 0u : chunk0 * 2048u;
+  // IN_PLACE: bytes from a tap to the next column's, the next row's
+  const int filter_row = cp * 8 * 2, filter_tap = g.features * filter_row;
+  const int tap_at = (cls.tap_r0 * g.win_cols + cls.tap_c0) * filter_tap;
+  const int tap_dr = cls.tap_rs * g.win_cols * filter_tap;
+  const int tap_dc = cls.tap_cs * filter_tap;
+  const int win_r = cls.win_r;
+  auto issue = [&](char* buf) {
+    int tr = tap_r, ts = tap_c;
+    unsigned tap_off;
+    if constexpr (UNIFORM) {
+      if constexpr (IN_PLACE)
+        b_chunk = static_cast<unsigned>(tap_at + tr * tap_dr + ts * tap_dc +
+                                        c4 * 16);
+      tap_off = static_cast<unsigned>((tr * src_cols + ts) * cp + c4) * 16u;
+      c4 += 4;
+      if (c4 == cp) {
+        c4 = 0;
+        if (++tap_c == win_c) { tap_c = 0; ++tap_r; }
+      }
+    } else {
+      const int tap = divide(q, by_cp);
+      tr = divide(tap, by_win_c);
+      ts = tap - tr * win_c;
+      tap_off = (static_cast<unsigned>(tr * src_cols + ts) * cp +
+                 (q - tap * cp)) * 16u;
+      if constexpr (IN_PLACE)
+        b_chunk = tr < win_r ? static_cast<unsigned>(tap_at + tr * tap_dr +
+                                                     ts * tap_dc +
+                                                     (q - tap * cp) * 16)
+                             : 0x80000000u;
+      q += 4;
+    }
+#pragma unroll
+    for (int i = 0; i < LA; ++i) {
+      const unsigned ok = (a_mask[i] >> tr) & (a_mask[i] >> (16 + ts)) & 1u;
+      load_to_lds(src_rsrc, buf + (wave + NW * i) * 1024,
+                  ok != 0 ? a_off[i] + tap_off : kOob);
+    }
+#pragma unroll
+    for (int i = 0; i < LB; ++i)
+      load_to_lds(wpk_rsrc, buf + BM * kRowBytes + b_block[i] * 1024,
+                  IN_PLACE && !UNIFORM ? (b_off[i] | b_chunk) >= 0x80000000u
+                                             ? kOob : b_off[i] + b_chunk
+                                       : b_off[i] + b_chunk);
+    if constexpr (!IN_PLACE) b_chunk += 2048;
+  };
+
+  float16v acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+
+  const int l32 = lane & 31, khalf = lane >> 5;
+  const int in_row =
+      static_cast<int>((static_cast<unsigned>(khalf) ^ swz(lane & 15u)) * 16u);
+  const int px_at = (wm * TM * 32 + l32) * kRowBytes + in_row;
+  const int ft_at = (BM + wn * TN * 32 + l32) * kRowBytes + in_row;
+  // Operands of reduction step S (16 channels) of a chunk.  (Step 1 reads
+  // pieces 2 and 3: bit 1 of the swizzled position flips.)
+  struct Operands { half8 a[TN], b[TM]; };
+  auto fetch = [&](const char* buf, int s, Operands& o) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+      o.a[i] = *reinterpret_cast<const half8*>(
+          buf + (ft_at ^ (32 * s)) + i * 32 * kRowBytes);
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+      o.b[j] = *reinterpret_cast<const half8*>(
+          buf + (px_at ^ (32 * s)) + j * 32 * kRowBytes);
+  };
+  auto multiply = [&](const Operands& o) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+            o.a[i], o.b[j], acc[i][j], 0, 0, 0);
+  };
+
+  // One chunk: its step 0 operands are in `even`, the next two chunks are
+  // arriving.  Step 1 is read while step 0 multiplies; then every wave is done
+  // with the buffer, the load of the chunk after next-but-one goes into it,
+  // and the next chunk's step 0 is read while step 1 multiplies.
+  Operands even, odd;
+  int done = 0;
+  auto step = [&](char* cur, const char* next, bool more1, bool more2,
+                  bool more3) {
+    fetch(cur, 1, odd);
+    __builtin_amdgcn_sched_barrier(0);
+    multiply(even);
+    __builtin_amdgcn_sched_barrier(0);
+    if (more1) {
+      if (more2)
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(LA + LB) & ~0x0F00);  // and LDS
+      else
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0) & ~0x0F00);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if (more3) issue(cur);
+      fetch(next, 0, even);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    multiply(odd);
+    __builtin_amdgcn_sched_barrier(0);
+    ++done;
+  };
+  if (n_chunks > 0) {
+    issue(buf0);
+    if (n_chunks > 1) issue(buf1);
+    if (n_chunks > 2) issue(buf2);
+    // (all three: a wait for the first alone makes the compiler put a full
+    // wait into every turn of the loop)
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(buf0, 0, even);
+    while (done + 5 < n_chunks) {
+      step(buf0, buf1, true, true, true);
+      step(buf1, buf2, true, true, true);
+      step(buf2, buf0, true, true, true);
+    }
+    // at most five chunks are left
+    auto last = [&](char* cur, const char* next) {
+      if (done < n_chunks)
+        step(cur, next, done + 1 < n_chunks, done + 2 < n_chunks,
+             done + 3 < n_chunks);
+    };
+    last(buf0, buf1);
+    last(buf1, buf2);
+    last(buf2, buf0);
+    last(buf0, buf1);
+    last(buf1, buf2);
+  }
+
+  // A shared reduction: the fp32 tile in accumulator order, 1 KB per store.
+  if (g.n_splits > 1) {
+    float4v* const out =
+        reinterpret_cast<float4v*>(part) +
+        (static_cast<size_t>(split) * g.n_tiles + tile) * (BM * BN / 4) +
+        wave * (TN * TM * 256) + lane;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float4v four = {acc[i][j][4 * v], acc[i][j][4 * v + 1],
+                                acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]};
+          out[((i * TM + j) * 4 + v) * 64] = four;
+        }
+    return;
+  }
+
+  // A lane holds features f0 .. f0 + 7 and f0 + 16 .. f0 + 23 of one pixel per
+  // block.
+  const __amdgpu_buffer_rsrc_t dst_rsrc = make_rsrc(dst, dst_bytes);
+#pragma unroll
+  for (int j = 0; j < TM; ++j) {
+    const int m = m0 + (wm * TM + j) * 32 + l32;
+    const Pixel px = pixel_of(m, cls);
+    const int out_y = px.y * g.out_step_r + cls.out_r0;
+    const int out_x = px.x * g.out_step_c + cls.out_c0;
+    const unsigned at =
+        static_cast<unsigned>(((px.n * g.out_rows + out_y) * g.out_cols + out_x) *
+                              g.features) * 2u;
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+      const int f0 = n0 + (wn * TN + i) * 32 + 8 * khalf;
+      const int count = m < cls.pixels ? g.features - f0 : 0;
+      const unsigned off = at + static_cast<unsigned>(f0) * 2u;
+      half8 lo, hi;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        lo[v] = static_cast<_Float16>(acc[i][j][v]);
+        hi[v] = static_cast<_Float16>(acc[i][j][8 + v]);
+      }
+      const uint4v w0 = __builtin_bit_cast(uint4v, lo);
+      const uint4v w1 = __builtin_bit_cast(uint4v, hi);
+      if ((g.features & 7) == 0) {
+        __builtin_amdgcn_raw_buffer_store_b128(w0, dst_rsrc,
+                                               count > 0 ? off : kOob, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b128(
+            w1, dst_rsrc, count > 16 ? off + 32u : kOob, 0, 0);
+      } else if ((g.features & 3) == 0) {
+        const unsigned words[8] = {w0[0], w0[1], w0[2], w0[3],
+                                   w1[0], w1[1], w1[2], w1[3]};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const uint2v two = {words[2 * v], words[2 * v + 1]};
+          __builtin_amdgcn_raw_buffer_store_b64(
+              two, dst_rsrc,
+              count > 4 * v + v / 2 * 8 ? off + 8u * v + v / 2 * 16u : kOob, 0,
+              0);
+        }
+      } else {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const _Float16 h = v < 8 ? lo[v] : hi[v - 8];
+          __builtin_amdgcn_raw_buffer_store_b16(
+              __builtin_bit_cast(unsigned short, h), dst_rsrc,
+              count > v + v / 8 * 8 ? off + 2u * v + v / 8 * 16u : kOob, 0, 0);
+        }
+      }
+    }
+  }
+}
+
+// Sums the splits of every tile in order and rounds: one float4 -- four
+// consecutive features of a pixel -- per lane.
+template <int WM, int WN, int TM, int TN>
+__global__ void __launch_bounds__(256)
+    gather_reduce_kernel(const float4v* __restrict__ part,
+                         _Float16* __restrict__ dst, Gather g) {
+  constexpr unsigned BM = 32 * WM * TM, BN = 32 * WN * TN;
+  constexpr unsigned kTileVecs = BM * BN / 4;
+  const unsigned at = blockIdx.x * 256 + threadIdx.x;
+  const unsigned tile = at / kTileVecs, in = at % kTileVecs;
+  if (tile >= g.n_tiles) return;
+  const TileOf where = tile_of(tile, g);
+  const GatherClass& cls = g.cls[where.cls];
+  const unsigned lane = in % 64, v = in / 64 % 4, block = in / 256 % (TN * TM);
+  const unsigned wave = in / (256 * TN * TM);
+  const unsigned i = block / TM, j = block % TM;
+  const int m = where.m * static_cast<int>(BM) +
+                static_cast<int>((wave / WN * TM + j) * 32 + lane % 32);
+  const int f = where.n * static_cast<int>(BN) +
+                static_cast<int>((wave % WN * TN + i) * 32) +
+                feature_of_row(8 * v + 4 * (lane / 32));
+  if (m >= cls.pixels || f >= g.features) return;
+  if (cls.n_chunks == 0 && (g.features & 7) == 0) return;  // stored already
+  float4v sum = {0.f, 0.f, 0.f, 0.f};
+  const float4v* from = part + at;
+#pragma unroll 4
+  for (int s = 0; s < g.n_splits; ++s)
+    sum += from[static_cast<size_t>(s) * g.n_tiles * kTileVecs];
+  const Pixel px = pixel_of(m, cls);
+  _Float16* const out =
+      dst + (static_cast<size_t>(px.n * g.out_rows + px.y * g.out_step_r +
+                                 cls.out_r0) * g.out_cols +
+             px.x * g.out_step_c + cls.out_c0) * g.features + f;
+  typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+  half4 r;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) r[e] = static_cast<_Float16>(sum[e]);
+  if ((g.features & 3) == 0) {
+    *reinterpret_cast<half4*>(out) = r;
+  } else {
+    for (int e = 0; e < 4 && f + e < g.features; ++e) out[e] = r[e];
+  }
+}
+
+struct GatherPlan {
+  Gather g;
+  bool ok = false;
+  int batch = 0;
+  size_t src_pixels = 0;
+  bool widen = false;       // source channels are no multiple of 8
+  size_t out_elems = 0;
+  size_t pack_blocks = 0;   // 2 KB blocks of packed filter
+  size_t wide_halves = 0;   // of the widened source
+  size_t part_floats = 0;   // of the tiles whose reduction is shared
+  int tile = 0;             // index into kTiles
+  int n_splits = 1;
+  size_t filter_elems = 0;
+  bool in_place = false;    // the filter may be read as it is
+  size_t workspace_halves(bool packs) const {
+    return (packs ? pack_blocks * 1024 : 0) + wide_halves + 2 * part_floats;
+  }
+};
+
+// Tile shapes, with what one work-group needs per chunk: alone on its CU
+// (bound by the time a load takes) and its share of a CU that is full.
+struct TileShape {
+  int pixels, features;
+  double alone_us, share_us;
+};
+constexpr TileShape kTiles[] = {
+    {256, 128, 0.57, 0.46}, {256, 64, 0.34, 0.376}, {128, 128, 0.27, 0.24},
+    {128, 64, 0.245, 0.17},  {128, 32, 0.23, 0.135}, {64, 64, 0.22, 0.103}};
+constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+constexpr int kNumCus = 256;
+constexpr int kMaxSplits = 16;
+
+int tuned(const char* name, int otherwise) {
+#ifdef SNN_HIP_TUNING
+  const char* const env = std::getenv(name);
+  if (env != nullptr) return std::atoi(env);
+#endif
+  return otherwise;
+}
+
+// Tile shape and splits of the reduction: the least time by a model of the
+// launch, chunks x the fuller of "one chunk after the other" and "every
+// work-group's share of its CU", plus what a split reduction adds -- its
+// second launch and the partial tiles written and read.  The constants were
+// measured; against forced choices the model's was within about 10 % of the
+// best on forty shapes from 1x7x7x512 to 16x224x224x64.
+void choose_tile(GatherPlan* plan) {
+  const Gather& g = plan->g;
+  int pixels = 0;
+  double chunks = 0;
+  for (int k = 0; k < g.n_classes; ++k) {
+    pixels = std::max(pixels, g.cls[k].pixels);
+    chunks += g.cls[k].n_chunks;
+  }
+  chunks /= g.n_classes;
+  auto tiles_of = [&](const TileShape& t) {
+    return static_cast<double>(ceil_div(pixels, t.pixels)) * g.n_classes *
+           ceil_div(g.features, t.features);
+  };
+  double best = 1e30;
+  for (int i = 0; i < kNumTiles; ++i) {
+    const TileShape& t = kTiles[i];
+    const double tiles = tiles_of(t);
+    for (int splits = 1; splits <= kMaxSplits; splits *= 2) {
+      if (splits > 1 && chunks / splits < 4) break;
+      const double rounds = std::ceil(tiles * splits / kNumCus);
+      double us = std::ceil(chunks / splits) *
+                      std::max(t.alone_us, rounds * t.share_us) +
+                  0.5 * rounds;
+      if (splits > 1)
+        us += 3.0 + splits * tiles * t.pixels * t.features * 8 / 3e6;
+      if (us < best) {
+        best = us;
+        plan->tile = i;
+        plan->n_splits = splits;
+      }
+    }
+  }
+  plan->tile = tuned("SNN_HIP_GATHER_TILE", plan->tile);
+  plan->n_splits = tuned("SNN_HIP_GATHER_SPLITS", plan->n_splits);
+  const TileShape& t = kTiles[plan->tile];
+  plan->part_floats =
+      plan->n_splits > 1 ? static_cast<size_t>(plan->n_splits * tiles_of(t)) *
+                               t.pixels * t.features
+                         : 0;
+}
+
+GatherPlan compute_plan(int direction, const snn_hip_conv2d_params& p) {
+  GatherPlan plan;
+  if (direction != SNN_HIP_FORWARD && direction != SNN_HIP_INPUT_BACKPROP)
+    return plan;
+  const bool grad = direction == SNN_HIP_INPUT_BACKPROP;
+  if (p.window_rows > kMaxWindow || p.window_cols > kMaxWindow) return plan;
+  if (grad && p.stride_rows * p.stride_cols > kMaxClasses) return plan;
+  Gather& g = plan.g;
+  g.src_rows = grad ? p.out_rows : p.in_rows;
+  g.src_cols = grad ? p.out_cols : p.in_cols;
+  g.out_rows = grad ? p.in_rows : p.out_rows;
+  g.out_cols = grad ? p.in_cols : p.out_cols;
+  g.channels = grad ? p.features : p.channels;
+  g.features = grad ? p.channels : p.features;
+  g.cp = (g.channels + 7) / 8;
+  g.by_cp = divisor(g.cp);
+  g.step_r = grad ? 1 : p.stride_rows;
+  g.step_c = grad ? 1 : p.stride_cols;
+  g.out_step_r = grad ? p.stride_rows : 1;
+  g.out_step_c = grad ? p.stride_cols : 1;
+  g.win_cols = p.window_cols;
+  g.mirrored = grad;
+  plan.batch = p.batch;
+  plan.src_pixels = static_cast<size_t>(p.batch) * g.src_rows * g.src_cols;
+  plan.widen = g.channels % 8 != 0;
+  if (plan.widen) plan.wide_halves = plan.src_pixels * g.cp * 8;
+  if (plan.src_pixels * g.cp * 16 > kMaxBufferBytes ||
+      static_cast<size_t>(p.batch) * g.out_rows * g.out_cols * g.features * 2 >
+          kMaxBufferBytes)
+    return plan;
+  g.n_classes = 0;
+  if (!grad) {
+    GatherClass& c = g.cls[g.n_classes++];
+    c.rows = p.out_rows; c.cols = p.out_cols;
+    c.off_r = -p.pad_rows; c.off_c = -p.pad_cols;
+    c.win_r = p.window_rows; c.win_c = p.window_cols;
+    c.out_r0 = 0; c.out_c0 = 0;
+    c.tap_r0 = 0; c.tap_rs = 1; c.tap_c0 = 0; c.tap_cs = 1;
+  } else {
+    // One axis of a class: input positions first, first + stride, ... are
+    // reached by taps a, a + stride, ... at source position
+    // i + off + (taps - 1 - j) for tap a + stride * j.
+    auto axis = [](int a, int in, int window, int stride, int pad, int* count,
+                   int* first, int* taps, int* off, int* tap0) {
+      *first = ((a - pad) % stride + stride) % stride;
+      *count = in > *first ? (in - *first + stride - 1) / stride : 0;
+      *taps = window > a ? (window - a + stride - 1) / stride : 0;
+      *off = (*first + pad - a) / stride - (*taps - 1);
+      *tap0 = a + stride * (*taps - 1);
+    };
+    for (int a = 0; a < p.stride_rows; ++a)
+      for (int b = 0; b < p.stride_cols; ++b) {
+        GatherClass c;
+        axis(a, p.in_rows, p.window_rows, p.stride_rows, p.pad_rows, &c.rows,
+             &c.out_r0, &c.win_r, &c.off_r, &c.tap_r0);
+        axis(b, p.in_cols, p.window_cols, p.stride_cols, p.pad_cols, &c.cols,
+             &c.out_c0, &c.win_c, &c.off_c, &c.tap_c0);
+        c.tap_rs = -p.stride_rows;
+        c.tap_cs = -p.stride_cols;
+        if (c.rows <= 0 || c.cols <= 0) continue;
+        if (c.win_r == 0 || c.win_c == 0) c.win_r = c.win_c = 0;
+        g.cls[g.n_classes++] = c;
+      }
+  }
+  const int n_nb = ceil_div(g.features, 32);
+  for (int k = 0; k < g.n_classes; ++k) {
+    GatherClass& c = g.cls[k];
+    c.pixels = p.batch * c.rows * c.cols;
+    c.n_chunks = ceil_div(c.win_r * c.win_c * g.cp, 4);
+    c.by_win_c = divisor(std::max(c.win_c, 1));
+    c.by_rows = divisor(c.rows);
+    c.by_cols = divisor(c.cols);
+    c.pack_block = static_cast<unsigned>(plan.pack_blocks);
+    plan.pack_blocks += static_cast<size_t>(n_nb) * c.n_chunks;
+  }
+  plan.filter_elems = static_cast<size_t>(p.window_rows) * p.window_cols *
+                      p.channels * p.features;
+  plan.in_place = grad && !plan.widen && plan.filter_elems * 2 <= kMaxBufferBytes / 2;
+  plan.out_elems =
+      static_cast<size_t>(p.batch) * g.out_rows * g.out_cols * g.features;
+  choose_tile(&plan);
+  plan.ok = plan.pack_blocks * 2048 <= kMaxBufferBytes / 2 && g.n_classes > 0;
+  return plan;
+}
+
+// The plan of the most recent shape is kept per thread: layers are usually
+// launched many times with the same parameters.
+const GatherPlan& make_plan(int direction, const snn_hip_conv2d_params& p) {
+  struct Cached {
+    int direction = -1;
+    snn_hip_conv2d_params params;
+    GatherPlan plan;
+  };
+  thread_local Cached cached[2];
+  Cached& c = cached[direction == SNN_HIP_INPUT_BACKPROP ? 1 : 0];
+#ifdef SNN_HIP_TUNING
+  c.direction = -1;
+#endif
+  if (c.direction != direction || std::memcmp(&c.params, &p, sizeof(p)) != 0) {
+    c.plan = compute_plan(direction, p);
+    c.params = p;
+    c.direction = direction;
+  }
+  return c.plan;
+}
+
+template <int WM, int WN, int TM, int TN>
+void launch_tile(const _Float16* src, const _Float16* wpk, _Float16* dst,
+                 float* part, const GatherPlan& plan, bool in_place,
+                 hipStream_t stream) {
+  constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
+  Gather g = plan.g;
+  g.n_tiles_n = ceil_div(g.features, BN);
+  int pixels = 0;
+  for (int k = 0; k < g.n_classes; ++k)
+    pixels = std::max(pixels, g.cls[k].pixels);
+  const unsigned n_tiles = static_cast<unsigned>(ceil_div(pixels, BM)) *
+                           static_cast<unsigned>(g.n_classes * g.n_tiles_n);
+  g.n_tiles = n_tiles;
+  g.n_splits = plan.n_splits;
+  const unsigned n_groups = n_tiles * static_cast<unsigned>(g.n_splits);
+  const unsigned src_bytes = static_cast<unsigned>(plan.src_pixels * g.cp * 16);
+  const unsigned wpk_bytes = static_cast<unsigned>(
+      in_place ? plan.filter_elems * 2 : plan.pack_blocks * 2048);
+  const unsigned dst_bytes = static_cast<unsigned>(plan.out_elems * 2);
+  {
+    KernelTimer timer(stream);
+    if (in_place && g.cp % 4 == 0)
+      hipLaunchKernelGGL((conv_gather_f16_kernel<WM, WN, TM, TN, true, true>),
+                         dim3(n_groups), dim3(64 * WM * WN), 0, stream, src,
+                         wpk, dst, part, g, src_bytes, wpk_bytes, dst_bytes,
+                         n_groups);
+    else if (in_place)
+      hipLaunchKernelGGL((conv_gather_f16_kernel<WM, WN, TM, TN, false, true>),
+                         dim3(n_groups), dim3(64 * WM * WN), 0, stream, src,
+                         wpk, dst, part, g, src_bytes, wpk_bytes, dst_bytes,
+                         n_groups);
+    else if (g.cp % 4 == 0)
+      hipLaunchKernelGGL((conv_gather_f16_kernel<WM, WN, TM, TN, true, false>),
+                         dim3(n_groups), dim3(64 * WM * WN), 0, stream, src,
+                         wpk, dst, part, g, src_bytes, wpk_bytes, dst_bytes,
+                         n_groups);
+    else
+      hipLaunchKernelGGL((conv_gather_f16_kernel<WM, WN, TM, TN, false, false>),
+                         dim3(n_groups), dim3(64 * WM * WN), 0, stream, src,
+                         wpk, dst, part, g, src_bytes, wpk_bytes, dst_bytes,
+                         n_groups);
+  }
+  if (g.n_splits > 1)
+    hipLaunchKernelGGL((gather_reduce_kernel<WM, WN, TM, TN>),
+                       dim3(n_tiles * (BM * BN / 1024)), dim3(256), 0, stream,
+                       reinterpret_cast<const float4v*>(part), dst, g);
+}
+
+// Returns -1 when there is no room for its temporaries.
+int launch_gather(const GatherPlan& plan, const _Float16* input,
+                  const _Float16* filter, _Float16* output,
+                  _Float16* workspace, size_t workspace_elems,
+                  hipStream_t stream) {
+  const Gather& g = plan.g;
+  const bool in_place =
+      plan.in_place && (reinterpret_cast<uintptr_t>(filter) & 15u) == 0;
+  const size_t need = plan.workspace_halves(!in_place);
+  _Float16* packed = workspace;
+  const bool temporary =
+      need != 0 && (workspace == nullptr || workspace_elems < need ||
+                    (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0);
+  if (temporary) {
+    void* ptr = nullptr;
+    if (temp_malloc_async(&ptr, need * sizeof(_Float16), stream) !=
+        hipSuccess) {
+      (void)hipGetLastError();
+      return -1;
+    }
+    packed = static_cast<_Float16*>(ptr);
+  }
+  // (every part is a multiple of 16 bytes)
+  const size_t pack_blocks = in_place ? 0 : plan.pack_blocks;
+  _Float16* const wide = packed + pack_blocks * 1024;
+  float* const part = reinterpret_cast<float*>(wide + plan.wide_halves);
+  const unsigned pack_lanes = static_cast<unsigned>(pack_blocks * 128);
+  const unsigned pack_groups = ceil_div(pack_lanes, 256u);
+  const unsigned pieces =
+      plan.widen ? static_cast<unsigned>(plan.src_pixels * g.cp) : 0u;
+  const unsigned groups = pack_groups + ceil_div(pieces, 256u);
+  if (groups > 0)
+    hipLaunchKernelGGL(gather_prepare_kernel, dim3(groups), dim3(256), 0,
+                       stream, filter, packed, g, pack_lanes, pack_groups,
+                       input, wide, pieces);
+  const _Float16* const src = plan.widen ? wide : input;
+  const _Float16* const weights = in_place ? filter : packed;
+  switch (plan.tile) {
+    case 0: launch_tile<2, 2, 4, 2>(src, weights, output, part, plan, in_place, stream); break;
+    case 1: launch_tile<4, 1, 2, 2>(src, weights, output, part, plan, in_place, stream); break;
+    case 2: launch_tile<2, 2, 2, 2>(src, weights, output, part, plan, in_place, stream); break;
+    case 3: launch_tile<2, 2, 2, 1>(src, weights, output, part, plan, in_place, stream); break;
+    case 4: launch_tile<4, 1, 1, 1>(src, weights, output, part, plan, in_place, stream); break;
+    default: launch_tile<2, 2, 1, 1>(src, weights, output, part, plan, in_place, stream);
+  }
+  const hipError_t err = hipGetLastError();
+  if (temporary) temp_free_async(packed, stream);
+  if (err != hipSuccess) return report_hip_error(err, "conv_gather_f16_kernel");
+  return SNN_HIP_OK;
+}
+
+// The input gradient of a stride-1 convolution as a forward convolution of
+// dY: channels and features trade places, padding becomes window - 1 - pad.
+bool as_forward_of_dy(const snn_hip_conv2d_params& p,
+                      snn_hip_conv2d_params* q) {
+  if (p.stride_rows != 1 || p.stride_cols != 1) return false;
+  if (p.pad_rows > p.window_rows - 1 || p.pad_cols > p.window_cols - 1)
+    return false;
+  *q = p;
+  q->channels = p.features;
+  q->features = p.channels;
+  q->in_rows = p.out_rows;
+  q->in_cols = p.out_cols;
+  q->out_rows = p.in_rows;
+  q->out_cols = p.in_cols;
+  q->pad_rows = p.window_rows - 1 - p.pad_rows;
+  q->pad_cols = p.window_cols - 1 - p.pad_cols;
+  return true;
+}
+
+// The forward convolution the LDS-tile kernel would run, if it is wanted.
+bool rowtile_params(int direction, const snn_hip_conv2d_params& p,
+                    snn_hip_conv2d_params* q) {
+  if (direction == SNN_HIP_FORWARD)
+    *q = p;
+  else if (!as_forward_of_dy(p, q))
+    return false;
+  return conv2d_rowtile_f16_wanted(*q);
+}
+
+// 1x1, stride 1, no padding: a plain row-major GEMM over the pixels, X * W for
+// the forward and dY * W^T for the gradient.
+bool is_rows_gemm(int direction, const snn_hip_conv2d_params& p) {
+  const size_t pixels = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols;
+  if (p.window_rows != 1 || p.window_cols != 1 || p.stride_rows != 1 ||
+      p.stride_cols != 1 || p.pad_rows != 0 || p.pad_cols != 0 ||
+      p.out_rows != p.in_rows || p.out_cols != p.in_cols ||
+      pixels > static_cast<size_t>(INT_MAX))
+    return false;
+  const int m = static_cast<int>(pixels);
+  return direction == SNN_HIP_FORWARD
+             ? gemm_rows_f16_supports(m, p.channels, p.features)
+             : gemm_nt_f16_supports(m, p.features, p.channels);
+}
+
+// A handful of products per output and few outputs: one launch of the direct
+// kernel (16x16x8 -> 8, 1x1, at batch 2: 6.5 us against 10.3 with the filter's
+// pack in front; a 3x3 of 20 channels 20.3 against 10.5).
+bool is_tiny(int direction, const snn_hip_conv2d_params& p) {
+  const bool grad = direction == SNN_HIP_INPUT_BACKPROP;
+  const size_t products = static_cast<size_t>(p.window_rows) * p.window_cols *
+                          (grad ? p.features : p.channels);
+  const size_t outputs =
+      grad ? static_cast<size_t>(p.batch) * p.in_rows * p.in_cols * p.channels
+           : static_cast<size_t>(p.batch) * p.out_rows * p.out_cols * p.features;
+  return products <= 32 && outputs <= (size_t{1} << 16);
+}
+
+}  // namespace
+
+size_t conv2d_f16_workspace_halves(int direction,
+                                   const snn_hip_conv2d_params& p) {
+  snn_hip_conv2d_params q;
+  if (is_rows_gemm(direction, p)) return 0;
+  if (rowtile_params(direction, p, &q))
+    return static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
+           p.features;
+  if (is_tiny(direction, p)) return 0;
+  // (with room for the packed filter also where the gradient's is read in
+  // place, for one that is not 16-byte aligned; that of a 1x1 layer would take
+  // a temporary)
+  const GatherPlan& plan = make_plan(direction, p);
+  const bool packs =
+      !plan.in_place || p.window_rows > 1 || p.window_cols > 1;
+  return plan.ok ? plan.workspace_halves(packs) : 0;
+}
+
+int launch_conv2d_f16(int direction, const _Float16* input,
+                      const _Float16* filter, _Float16* output,
+                      const snn_hip_conv2d_params& p, _Float16* workspace,
+                      size_t workspace_elems, hipStream_t stream) {
+  auto aligned = [](const void* ptr) {
+    return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0;
+  };
+  if (!aligned(output)) return -1;
+  if (is_rows_gemm(direction, p) && aligned(input) && aligned(filter)) {
+    const int m = p.batch * p.in_rows * p.in_cols;
+    return direction == SNN_HIP_FORWARD
+               ? launch_gemm_rows_f16(input, filter, output, m, p.channels,
+                                      p.features, stream)
+               : launch_gemm_nt_f16(input, filter, output, m, p.features,
+                                    p.channels, stream);
+  }
+  snn_hip_conv2d_params q;
+  if (rowtile_params(direction, p, &q) && aligned(input) && aligned(filter)) {
+    const size_t need = static_cast<size_t>(p.window_rows) * p.window_cols *
+                        p.channels * p.features;
+    _Float16* packed = workspace;
+    const bool temporary = workspace == nullptr || workspace_elems < need ||
+                           !aligned(workspace);
+    if (temporary) {
+      void* ptr = nullptr;
+      if (temp_malloc_async(&ptr, need * sizeof(_Float16), stream) !=
+          hipSuccess)
+        return SNN_HIP_ALLOCATION_PROBLEM;
+      packed = static_cast<_Float16*>(ptr);
+    }
+    const int status =
+        launch_conv2d_rowtile_f16(input, filter, output, q, packed, stream,
+                                  direction == SNN_HIP_INPUT_BACKPROP);
+    if (temporary) temp_free_async(packed, stream);
+    return status;
+  }
+  if (is_tiny(direction, p)) return -1;
+  const GatherPlan& plan = make_plan(direction, p);
+  if (!plan.ok || (!plan.widen && !aligned(input))) return -1;
+  return launch_gather(plan, input, filter, output, workspace, workspace_elems,
+                       stream);
+}
+
+}  // namespace snn

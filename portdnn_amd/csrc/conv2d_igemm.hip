@@ -89,16 +89,14 @@ __device__ inline float4 buffer_load4_as_float(__amdgpu_buffer_rsrc_t r,
 // the 3-channel stem), so four consecutive reduction indices are not four
 // consecutive floats of one tap; each is located and loaded on its own.
 template <int BM, int BN, int WM, int WN, bool B_K_INNER, bool STRIDED,
-          bool ATOMIC, bool SCALAR_A = false, typename T = float>
+          bool ATOMIC, bool SCALAR_A = false>
 __global__ void __launch_bounds__(kThreads)
-    conv_igemm_kernel(const T* __restrict__ src, const T* __restrict__ wgt,
-                      T* __restrict__ dst, Gather g, unsigned src_bytes,
+    conv_igemm_kernel(const float* __restrict__ src, const float* __restrict__ wgt,
+                      float* __restrict__ dst, Gather g, unsigned src_bytes,
                       unsigned wgt_bytes, unsigned n_tiles_n, unsigned n_tiles,
                       int chunks_per_split) {
   static_assert(WM * WN == 4, "four waves per work-group");
-  static_assert(sizeof(T) == 4 || (!ATOMIC && !SCALAR_A),
-                "half-precision tensors: plain stores, vector gather");
-  constexpr unsigned kEsz = sizeof(T);
+  constexpr unsigned kEsz = sizeof(float);
   constexpr int WTM = BM / WM, WTN = BN / WN;  // wave tile
   constexpr int TM = WTM / 32, TN = WTN / 32;  // MFMA blocks per wave
   static_assert(TM >= 1 && TN >= 1, "wave tile must hold a 32x32 block");
@@ -239,7 +237,7 @@ __global__ void __launch_bounds__(kThreads)
       ok = ok &
            (static_cast<unsigned>(iy) < static_cast<unsigned>(g.src_rows)) &
            (static_cast<unsigned>(ix) < static_cast<unsigned>(g.src_cols));
-      a_reg[i] = buffer_load4_as_float<T>(
+      a_reg[i] = buffer_load4(
           src_rsrc, ok ? static_cast<unsigned>(off) * kEsz : kOob);
     }
   };
@@ -282,7 +280,7 @@ __global__ void __launch_bounds__(kThreads)
         if (col < g.n_total)
           off = static_cast<unsigned>(q * g.n_total + col) * kEsz;
       }
-      b_reg[i] = buffer_load4_as_float<T>(wgt_rsrc, off);
+      b_reg[i] = buffer_load4(wgt_rsrc, off);
     }
   };
   auto store_tiles = [&](int stage) {
@@ -344,11 +342,11 @@ __global__ void __launch_bounds__(kThreads)
       for (int v = 0; v < 16; ++v) {
         const int m = m0 + wave_m * WTM + 32 * i + 8 * (v >> 2) + row_l + (v & 3);
         if (m < g.m_total) {
-          T* o = dst + static_cast<size_t>(m) * g.n_total + col;
+          float* o = dst + static_cast<size_t>(m) * g.n_total + col;
           if constexpr (ATOMIC)
             unsafeAtomicAdd(o, acc[i][j][v]);
           else
-            *o = static_cast<T>(acc[i][j][v]);
+            *o = acc[i][j][v];
         }
       }
     }
@@ -1954,11 +1952,11 @@ struct StrideClasses {
 // Every filter element to its place in the sub-filter of its class: per tap
 // a C x K matrix becomes K x C, 32 x 32 tiles through LDS so that reads and
 // writes are both contiguous.  Grid: (K tiles, C tiles, taps), 32 x 8 lanes.
-template <typename T>
 __global__ void __launch_bounds__(256)
-    stride_class_filters_kernel(const T* __restrict__ w, T* __restrict__ g,
+    stride_class_filters_kernel(const float* __restrict__ w,
+                                float* __restrict__ g,
                                 StrideClasses sc) {
-  __shared__ T tile[32][33];
+  __shared__ float tile[32][33];
   const int tap = blockIdx.z;
   const int s = tap % sc.win_cols;
   const int r = tap / sc.win_cols;
@@ -1972,17 +1970,17 @@ __global__ void __launch_bounds__(256)
   const int v = sc.taps_c[cls] - 1 - s / sc.stride_cols;
   const int k0 = blockIdx.x * 32, c0 = blockIdx.y * 32;
   const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
-  const T* const src =
+  const float* const src =
       w + static_cast<size_t>(tap) * sc.channels * sc.features;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int c = c0 + ty + 8 * i, k = k0 + tx;
     tile[ty + 8 * i][tx] = (c < sc.channels && k < sc.features)
                                ? src[static_cast<size_t>(c) * sc.features + k]
-                               : static_cast<T>(0);
+                               : 0.f;
   }
   __syncthreads();
-  T* const dst =
+  float* const dst =
       g + sc.filter_base[cls] +
       static_cast<size_t>(u * sc.taps_c[cls] + v) * sc.features * sc.channels;
 #pragma unroll
@@ -1994,10 +1992,9 @@ __global__ void __launch_bounds__(256)
 }
 
 // dX from the dense results of the classes (zeros for a class no tap reaches).
-template <typename V>  // four elements: float4, or 8 bytes of binary16
 __global__ void __launch_bounds__(256)
-    interleave_stride_classes_kernel(const V* __restrict__ t,
-                                     V* __restrict__ dx, StrideClasses sc,
+    interleave_stride_classes_kernel(const float4* __restrict__ t,
+                                     float4* __restrict__ dx, StrideClasses sc,
                                      int in_rows, int in_cols, int cv,
                                      size_t n_vec) {
   const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -2009,7 +2006,7 @@ __global__ void __launch_bounds__(256)
   const int y = static_cast<int>(pix % in_rows);
   const size_t n = pix / in_rows;
   const int cls = (y % sc.stride_rows) * sc.stride_cols + x % sc.stride_cols;
-  V v = {};
+  float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
   if (sc.taps_r[cls] > 0 && sc.taps_c[cls] > 0)
     v = t[(sc.pixel_base[cls] +
            (n * sc.rows[cls] + y / sc.stride_rows) * sc.cols[cls] +
@@ -2182,98 +2179,6 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
   return SNN_HIP_OK;
 }
 
-// Half-precision input gradient for the shapes the LDS-tile kernel does not
-// take (strides, channel counts that are not multiples of 64): the general
-// implicit-GEMM kernel reading binary16 operands, one work-group per 64 x 64
-// tile of dX and no reduction split, so every output is stored once.
-bool conv2d_input_backprop_general_f16_supports(
-    const snn_hip_conv2d_params& p) {
-  const size_t x = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols *
-                   p.channels;
-  const size_t y = static_cast<size_t>(p.batch) * p.out_rows * p.out_cols *
-                   p.features;
-  const size_t w = static_cast<size_t>(p.window_rows) * p.window_cols *
-                   p.channels * p.features;
-  return p.features % 4 == 0 &&
-         max(max(x, y), w) * sizeof(_Float16) <= kMaxBufferBytes;
-}
-
-int launch_conv2d_input_backprop_general_f16(const _Float16* dy,
-                                             const _Float16* filter,
-                                             _Float16* dx,
-                                             const snn_hip_conv2d_params& p,
-                                             hipStream_t stream) {
-  Gather g;
-  fill_gather(p, SNN_HIP_INPUT_BACKPROP, &g);
-  constexpr int BM = 64, BN = 64;
-  const unsigned tiles_m = static_cast<unsigned>(ceil_div(g.m_total, BM));
-  const unsigned tiles_n = static_cast<unsigned>(ceil_div(g.n_total, BN));
-  const unsigned n_tiles = tiles_m * tiles_n;
-  const int n_chunks = ceil_div(g.k_total, kBK);
-  constexpr size_t kLdsBytes =
-      2 * sizeof(float) * (k_inner_floats(BM) + k_inner_floats(BN));
-  const unsigned src_bytes = static_cast<unsigned>(
-      static_cast<size_t>(g.batch) * g.src_rows * g.src_cols * g.src_ch * 2);
-  const unsigned wgt_bytes = static_cast<unsigned>(
-      static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
-      p.features * 2);
-  KernelTimer timer(stream);
-  if (g.div_rows != 1 || g.div_cols != 1) {
-    hipLaunchKernelGGL(
-        (conv_igemm_kernel<BM, BN, 2, 2, true, true, false, false, _Float16>),
-        dim3(n_tiles, 1), dim3(kThreads), kLdsBytes, stream, dy, filter, dx, g,
-        src_bytes, wgt_bytes, tiles_n, n_tiles, n_chunks);
-  } else {
-    hipLaunchKernelGGL(
-        (conv_igemm_kernel<BM, BN, 2, 2, true, false, false, false, _Float16>),
-        dim3(n_tiles, 1), dim3(kThreads), kLdsBytes, stream, dy, filter, dx, g,
-        src_bytes, wgt_bytes, tiles_n, n_tiles, n_chunks);
-  }
-  SNN_HIP_CHECK_LAUNCH();
-  return SNN_HIP_OK;
-}
-
-// Half-precision forward convolution for the shapes the binary16 kernels do
-// not take (channel counts that are not multiples of 64, windows of more than
-// 32 taps): the same general kernel, gathering X four channels at a time.
-bool conv2d_forward_general_f16_supports(const snn_hip_conv2d_params& p) {
-  const size_t x = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols *
-                   p.channels;
-  const size_t y = static_cast<size_t>(p.batch) * p.out_rows * p.out_cols *
-                   p.features;
-  const size_t w = static_cast<size_t>(p.window_rows) * p.window_cols *
-                   p.channels * p.features;
-  return p.channels % 4 == 0 && p.features % 4 == 0 &&
-         max(max(x, y), w) * sizeof(_Float16) <= kMaxBufferBytes;
-}
-
-int launch_conv2d_forward_general_f16(const _Float16* x, const _Float16* filter,
-                                      _Float16* y,
-                                      const snn_hip_conv2d_params& p,
-                                      hipStream_t stream) {
-  Gather g;
-  fill_gather(p, SNN_HIP_FORWARD, &g);
-  constexpr int BM = 64, BN = 64;
-  const unsigned tiles_m = static_cast<unsigned>(ceil_div(g.m_total, BM));
-  const unsigned tiles_n = static_cast<unsigned>(ceil_div(g.n_total, BN));
-  const unsigned n_tiles = tiles_m * tiles_n;
-  const int n_chunks = ceil_div(g.k_total, kBK);
-  constexpr size_t kLdsBytes =
-      2 * sizeof(float) * (k_inner_floats(BM) + row_inner_floats(BN));
-  const unsigned src_bytes = static_cast<unsigned>(
-      static_cast<size_t>(g.batch) * g.src_rows * g.src_cols * g.src_ch * 2);
-  const unsigned wgt_bytes = static_cast<unsigned>(
-      static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
-      p.features * 2);
-  KernelTimer timer(stream);
-  hipLaunchKernelGGL(
-      (conv_igemm_kernel<BM, BN, 2, 2, false, false, false, false, _Float16>),
-      dim3(n_tiles, 1), dim3(kThreads), kLdsBytes, stream, x, filter, y, g,
-      src_bytes, wgt_bytes, tiles_n, n_tiles, n_chunks);
-  SNN_HIP_CHECK_LAUNCH();
-  return SNN_HIP_OK;
-}
-
 bool conv2d_igemm_supports(int direction, const snn_hip_conv2d_params& p) {
   // buffer descriptors address at most kMaxBufferBytes
   const size_t x = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols *
@@ -2360,12 +2265,12 @@ int launch_batched_gemm_mfma_f32(const float* a, const float* b, float* c,
 }
 
 // The stride classes of an input gradient, each through `forward` (a
-// stride-1 forward convolution of T tensors: parameters, input, filter,
-// output), then interleaved.  Returns -1 when a class would need negative
+// stride-1 forward convolution: parameters, input, filter, output), then
+// interleaved.  Returns -1 when a class would need negative
 // padding (the caller then takes another path).
-template <typename T, typename V, typename Forward>
-int strided_input_backprop_by_classes(const T* input, const T* filter,
-                                      T* output,
+template <typename Forward>
+int strided_input_backprop_by_classes(const float* input, const float* filter,
+                                      float* output,
                                       const snn_hip_conv2d_params& p,
                                       hipStream_t stream, Forward forward) {
   StrideClasses sc;
@@ -2406,23 +2311,23 @@ int strided_input_backprop_by_classes(const T* input, const T* filter,
   if (ok) {
     void *g = nullptr, *t = nullptr;
     // (no room for the temporaries: the caller takes another path)
-    if (temp_malloc_async(&g, max(filter_elems, 4u) * sizeof(T), stream) !=
+    if (temp_malloc_async(&g, max(filter_elems, 4u) * sizeof(float), stream) !=
         hipSuccess) {
       (void)hipGetLastError();
       return -1;
     }
-    if (temp_malloc_async(&t, max(pixels, size_t{1}) * p.channels * sizeof(T),
+    if (temp_malloc_async(&t, max(pixels, size_t{1}) * p.channels * sizeof(float),
                           stream) != hipSuccess) {
       (void)hipGetLastError();
       temp_free_async(g, stream);
       return -1;
     }
     hipLaunchKernelGGL(
-        stride_class_filters_kernel<T>,
+        stride_class_filters_kernel,
         dim3(static_cast<unsigned>(ceil_div(p.features, 32)),
              static_cast<unsigned>(ceil_div(p.channels, 32)),
              static_cast<unsigned>(p.window_rows * p.window_cols)),
-        dim3(256), 0, stream, filter, static_cast<T*>(g), sc);
+        dim3(256), 0, stream, filter, static_cast<float*>(g), sc);
     int status = SNN_HIP_OK;
     for (int cls = 0; cls < p.stride_rows * p.stride_cols; ++cls) {
       if (sc.taps_r[cls] == 0 || status != SNN_HIP_OK) continue;
@@ -2433,17 +2338,17 @@ int strided_input_backprop_by_classes(const T* input, const T* filter,
       q.window_rows = sc.taps_r[cls]; q.window_cols = sc.taps_c[cls];
       q.stride_rows = q.stride_cols = 1;
       q.pad_rows = pad_r[cls];  q.pad_cols = pad_c[cls];
-      status = forward(q, input, static_cast<const T*>(g) + sc.filter_base[cls],
-                       static_cast<T*>(t) + sc.pixel_base[cls] * p.channels);
+      status = forward(q, input, static_cast<const float*>(g) + sc.filter_base[cls],
+                       static_cast<float*>(t) + sc.pixel_base[cls] * p.channels);
     }
     if (status == SNN_HIP_OK) {
       const size_t n_vec = static_cast<size_t>(p.batch) * p.in_rows *
                            p.in_cols * p.channels / 4;
       hipLaunchKernelGGL(
-          interleave_stride_classes_kernel<V>,
+          interleave_stride_classes_kernel,
           dim3(static_cast<unsigned>(ceil_div(n_vec, size_t{256}))),
-          dim3(256), 0, stream, static_cast<const V*>(t),
-          reinterpret_cast<V*>(output), sc, p.in_rows, p.in_cols,
+          dim3(256), 0, stream, static_cast<const float4*>(t),
+          reinterpret_cast<float4*>(output), sc, p.in_rows, p.in_cols,
           p.channels / 4, n_vec);
     }
     const hipError_t err = hipGetLastError();
@@ -2455,34 +2360,6 @@ int strided_input_backprop_by_classes(const T* input, const T* filter,
     return SNN_HIP_OK;
   }
   return -1;
-}
-
-bool conv2d_strided_input_backprop_f16_supports(
-    const snn_hip_conv2d_params& p) {
-  return (p.stride_rows > 1 || p.stride_cols > 1) &&
-         p.stride_rows * p.stride_cols <= kMaxStrideClasses &&
-         p.channels % 4 == 0 && p.features % 64 == 0 &&
-         static_cast<double>(p.batch) * p.out_rows * p.out_cols *
-                 p.window_rows * p.window_cols * p.channels * p.features >=
-             double(1 << 30);
-}
-
-// Binary16: the classes run on the binary16 forward kernels (dY's feature
-// count, the classes' channel count, in multiples of 64).  -1: not taken.
-int launch_conv2d_strided_input_backprop_f16(const _Float16* dy,
-                                             const _Float16* filter,
-                                             _Float16* dx,
-                                             const snn_hip_conv2d_params& p,
-                                             hipStream_t stream) {
-  typedef _Float16 half4v __attribute__((ext_vector_type(4)));
-  return strided_input_backprop_by_classes<_Float16, half4v>(
-      dy, filter, dx, p, stream,
-      [&](const snn_hip_conv2d_params& q, const _Float16* in,
-          const _Float16* fil, _Float16* out) {
-        if (conv2d_igemm_f16_supports(q))
-          return launch_conv2d_igemm_f16(in, fil, out, q, nullptr, 0, stream);
-        return launch_conv2d_forward_general_f16(in, fil, out, q, stream);
-      });
 }
 
 int launch_conv2d_igemm_f32(int direction, const float* input,
@@ -2564,7 +2441,7 @@ int launch_conv2d_igemm_f32(int direction, const float* input,
     // 2: 56x56x128 -> 128, 3x3, at batch 32 343 us against 90 forward).  By
     // stride classes every class is a dense stride-1 forward convolution of
     // dY on the fast kernels.
-    const int rc = strided_input_backprop_by_classes<float, float4>(
+    const int rc = strided_input_backprop_by_classes(
         input, filter, output, p, stream,
         [&](const snn_hip_conv2d_params& q, const float* in, const float* fil,
             float* out) {

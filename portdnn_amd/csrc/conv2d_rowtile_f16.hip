@@ -2,10 +2,9 @@
 // input tile resident in LDS: binary16 operands, fp32 accumulation, binary16
 // result.
 //
-// The implicit-GEMM kernel in conv2d_igemm_f16.hip gathers every input pixel
-// once per filter tap through the vector-memory pipeline and passes both
-// operands through LDS; at 32x32x16 f16 MFMA rates that makes LDS and the
-// texture path the limit, not the matrix cores.  Here a work-group owns a run
+// The gathering kernel in conv2d_gather_f16.hip loads every input pixel once
+// per filter tap and passes both operands through LDS; at 32x32x16 f16 MFMA
+// rates that makes LDS and the loads the limit, not the matrix cores.  Here a work-group owns a run
 // of consecutive output pixels (images, rows and columns flattened, so a tile
 // may start inside a row and run over an image boundary) and a slice of the
 // features:
@@ -666,18 +665,31 @@ bool launch_shape(const _Float16* input, const _Float16* wpk,
 
 }  // namespace
 
-bool conv2d_rowtile_f16_supports(const snn_hip_conv2d_params& p) {
+// Where this kernel is faster than the gathering one (conv2d_gather_f16.hip,
+// which shares a reduction between work-groups where there are few tiles):
+// short reductions at every size, and long ones with at least 1.5 wave tiles
+// per SIMD that leave two waves on each.  Measured with 3x3 windows, this
+// kernel / the other: 56x56x64 at batch 1 9.6 / 9.9 us, 128 50.7 / 58;
+// 28x28x128 at batch 32 19.4 / 18.7, 64 25.0 / 26.4; 14x14x256 at batch 64
+// 31.5 / 29.8, 128 39.1 / 42.6; 7x7x512 at batch 8 43 / 21, 128 56 / 52;
+// 112x112x128 at batch 4 (one work-group's tiles fill the LDS) 41 / 26.
+bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p) {
   const size_t x = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols *
                    p.channels;
   const size_t y = static_cast<size_t>(p.batch) * p.out_rows * p.out_cols *
                    p.features;
   if (p.stride_rows != 1 || p.stride_cols != 1) return false;
   if (p.channels % 64 != 0 || p.features % 64 != 0) return false;
-  // 1x1 windows have no taps to reuse an LDS tile over: the implicit-GEMM
-  // kernel measured as fast or faster there.
+  // 1x1 windows have no taps to reuse an LDS tile over
   if (p.window_rows * p.window_cols == 1) return false;
   if ((x > y ? x : y) * 2 > kMaxBufferBytes) return false;
-  return make_plan(p).lds_bytes != 0;
+  const RowTilePlan plan = make_plan(p);
+  if (plan.lds_bytes == 0) return false;
+  if (p.window_rows * p.window_cols * p.channels <= 576) return true;
+  const size_t wave_tiles = ceil_div(y / p.features, size_t{64}) *
+                            static_cast<size_t>(p.features / 64);
+  return wave_tiles >= 1536 &&
+         (plan.pb == 4 || 2 * plan.lds_bytes <= kMaxLdsBytes);
 }
 
 int launch_conv2d_rowtile_f16(const _Float16* input, const _Float16* filter,

@@ -301,16 +301,14 @@ int launch_matmul_f16(const _Float16* lhs, const _Float16* rhs,
     if (!transpose_rhs) {
       p.channels = k;
       p.features = n;
-      if (conv2d_igemm_f16_supports(p))
-        return launch_conv2d_igemm_f16(lhs, rhs, output, p, nullptr, 0,
-                                       stream);
     } else {
       p.channels = n;
       p.features = k;
-      if (conv2d_input_backprop_f16_supports(p))
-        return launch_conv2d_input_backprop_f16(lhs, rhs, output, p, nullptr,
-                                                0, stream);
     }
+    const int rc = launch_conv2d_f16(
+        transpose_rhs ? SNN_HIP_INPUT_BACKPROP : SNN_HIP_FORWARD, lhs, rhs,
+        output, p, nullptr, 0, stream);
+    if (rc >= 0) return rc;
   }
   const dim3 grid(static_cast<unsigned>(ceil_div(m, kTile)),
                   static_cast<unsigned>(ceil_div(n, kTile)),

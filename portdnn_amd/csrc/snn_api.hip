@@ -320,7 +320,7 @@ void im2col_workspace(const snn_hip_conv2d_params& p, int direction,
 // buffer of the filter gradient, counted in halves.
 size_t f16_workspace_halves(const snn_hip_conv2d_params& p, int direction) {
   if (direction != SNN_HIP_FILTER_BACKPROP)
-    return conv2d_f16_filter_pack_halves(direction, p);
+    return conv2d_f16_workspace_halves(direction, p);
   if (!conv2d_filter_backprop_f16_supports(p)) return 0;
   if (conv2d_filter_backprop_3x3_f16_supports(p))
     return 2 * conv2d_filter_backprop_3x3_f16_partial_floats(p);
@@ -572,33 +572,6 @@ int launch_f16_through_fp32(int direction, const _Float16* input,
                       p.window_rows * p.window_cols * p.channels * p.features;
   if (macs < double(1 << 24)) return -1;
   const ConvSizes sz = conv_sizes(p, direction);
-  // The 7x7 stride-2 three-channel stem, forward: the fp32 kernel rounds its
-  // output -- the large tensor -- to binary16 on the store, so only the image
-  // and the filter are widened (430 -> 328 us at batch 128).  (The filter
-  // gradient reading dY as binary16, one 2-byte load per lane where the fp32
-  // kernel has a 4-byte one, measured slower than the widening pass it saves:
-  // 623 against 444 us.)
-  if (direction == SNN_HIP_FORWARD && conv2d_stem_supports(p) &&
-      (reinterpret_cast<uintptr_t>(output) & 7u) == 0) {
-    auto padded = [](size_t floats) { return (floats + 63) / 64 * 64; };
-    void* block = nullptr;
-    if (temp_malloc_async(&block,
-                          (padded(sz.input) + padded(sz.filter)) * sizeof(float),
-                          s) == hipSuccess) {
-      float* const in32 = static_cast<float*>(block);
-      float* const fil32 = in32 + padded(sz.input);
-      convert(input, in32, sz.input, s);
-      convert(filter, fil32, sz.filter, s);
-      const int status =
-          launch_conv2d_stem_f32_to_f16(in32, fil32, output, p, s);
-      const hipError_t err = hipGetLastError();
-      temp_free_async(block, s);
-      if (status != SNN_HIP_OK) return status;
-      if (err != hipSuccess) return report_hip_error(err, "binary16 stem");
-      return SNN_HIP_OK;
-    }
-    (void)hipGetLastError();
-  }
   // One stream-ordered temporary for the three widened tensors and the
   // workspace the fp32 launch would otherwise allocate for itself (every
   // allocation costs tens of microseconds of host time).
@@ -638,59 +611,17 @@ int launch_gemm_path<_Float16>(int direction, const _Float16* input,
                                const snn_hip_conv2d_params& p, hipStream_t s,
                                _Float16* workspace, size_t workspace_elems,
                                const LaunchOptions*) {
-  // (a gradient of at most eight channels: the binary16 kernels' 64-channel
-  // tiles would be nearly empty, fp32 has kernels for such layers -- 224x224
-  // 3 <- 64, 3x3, at batch 8: 286 us on the general binary16 kernel over a
-  // copy widened to four channels, 69 us in fp32)
-  if (direction == SNN_HIP_INPUT_BACKPROP && p.channels <= 8) {
+  // (the 7x7 stride-2 stem's input gradient: fp32 has a kernel built for it)
+  if (direction == SNN_HIP_INPUT_BACKPROP &&
+      conv2d_stem_input_backprop_supports(p)) {
     const int rc = launch_f16_through_fp32(direction, input, filter, output, p, s);
     if (rc >= 0) return rc;
   }
-  if (direction == SNN_HIP_INPUT_BACKPROP && aligned16(output)) {
-    const int padded = launch_gemm_path_padded<_Float16>(
-        direction, input, filter, output, p, s, nullptr,
-        [](const snn_hip_conv2d_params& q) {
-          return conv2d_input_backprop_f16_supports(q) ||
-                 conv2d_input_backprop_general_f16_supports(q);
-        });
-    if (padded >= 0) return padded;
-  }
-  if (direction == SNN_HIP_FORWARD && conv2d_igemm_f16_supports(p) &&
-      aligned16(input) && aligned16(filter) && aligned16(output))
-    return launch_conv2d_igemm_f16(input, filter, output, p, workspace,
-                                   workspace_elems, s);
-  if (direction == SNN_HIP_FORWARD &&
-      conv2d_forward_general_f16_supports(p) && aligned16(input) &&
-      aligned16(filter) && aligned16(output))
-    return launch_conv2d_forward_general_f16(input, filter, output, p, s);
-  if (direction == SNN_HIP_INPUT_BACKPROP &&
-      conv2d_input_backprop_f16_supports(p) && aligned16(input) &&
-      aligned16(filter) && aligned16(output))
-    return launch_conv2d_input_backprop_f16(input, filter, output, p,
-                                            workspace, workspace_elems, s);
-  // (a strided input gradient from 2^30 multiply-adds: the fp32 launch splits
-  // it into stride classes, the general binary16 kernel multiplies the zeros
-  // of the taps that do not reach a pixel -- 1.39 ms against 67 us forward for
-  // 56x56x128 -> 128, 3x3 stride 2, at batch 128)
-  if (direction == SNN_HIP_INPUT_BACKPROP &&
-      conv2d_strided_input_backprop_f16_supports(p) && aligned16(input) &&
-      aligned16(filter) && aligned16(output)) {
-    const int rc =
-        launch_conv2d_strided_input_backprop_f16(input, filter, output, p, s);
+  if (direction != SNN_HIP_FILTER_BACKPROP) {
+    const int rc = launch_conv2d_f16(direction, input, filter, output, p,
+                                     workspace, workspace_elems, s);
     if (rc >= 0) return rc;
   }
-  if (direction == SNN_HIP_INPUT_BACKPROP &&
-      (p.stride_rows > 1 || p.stride_cols > 1) &&
-      static_cast<double>(p.batch) * p.out_rows * p.out_cols * p.window_rows *
-              p.window_cols * p.channels * p.features >= double(1 << 30)) {
-    const int rc = launch_f16_through_fp32(direction, input, filter, output, p, s);
-    if (rc >= 0) return rc;
-  }
-  if (direction == SNN_HIP_INPUT_BACKPROP &&
-      conv2d_input_backprop_general_f16_supports(p) && aligned16(input) &&
-      aligned16(filter))
-    return launch_conv2d_input_backprop_general_f16(input, filter, output, p,
-                                                    s);
   // (few (tap, channel) pairs -- a three-channel stem: fp32 has kernels built
   // for that; 64-channel tiles would be nearly empty)
   if (direction == SNN_HIP_FILTER_BACKPROP && p.channels <= 8 &&

@@ -204,73 +204,43 @@ int launch_conv2d_stem_filter_backprop_f32(const float* x, const float* dy,
                                            float* dw,
                                            const snn_hip_conv2d_params& p,
                                            hipStream_t stream);
-// The forward stem kernel with its output -- the large tensor -- rounded to
-// binary16 on the store and everything else fp32: what a binary16 stem launch
-// runs after widening its image and filter.
-int launch_conv2d_stem_f32_to_f16(const float* x, const float* w, _Float16* y,
-                                  const snn_hip_conv2d_params& p,
-                                  hipStream_t stream);
-
 // The same in half precision with fp32 accumulation (gemm_wreg_f16.hip):
 // k = 64, 128, 256 or 512.
 bool gemm_wreg_f16_supports(int m, int k, int n);
 void launch_gemm_wreg_f16(const _Float16* x, const _Float16* w, _Float16* y,
                           int m, int k, int n, hipStream_t stream);
 
-// Half-precision forward convolution on MFMA (conv2d_igemm_f16.hip).  The
-// workspace, when large enough, receives the re-laid-out filter.
-bool conv2d_igemm_f16_supports(const snn_hip_conv2d_params& p);
-int launch_conv2d_igemm_f16(const _Float16* input, const _Float16* filter,
-                            _Float16* output, const snn_hip_conv2d_params& p,
-                            _Float16* workspace, size_t workspace_elems,
-                            hipStream_t stream);
 // Row-major binary16 GEMM y[m][n] = sum_k x[m][k] w[k][n] with the filter slab
 // resident in LDS (gemm_rows_f16.hip): 1x1 stride-1 convolutions and matmul
 // with k a multiple of 64 and n a multiple of 64; needs no workspace.
 bool gemm_rows_f16_supports(int m, int k, int n);
 int launch_gemm_rows_f16(const _Float16* x, const _Float16* w, _Float16* y,
                          int m, int k, int n, hipStream_t stream);
-// Halves of caller workspace the half-precision forward and input-gradient
-// launchers use for the re-laid-out filter (0: none needed).
-size_t conv2d_f16_filter_pack_halves(int direction,
-                                     const snn_hip_conv2d_params& p);
-// Stride-1 input gradient in half precision: the forward kernels above run on
-// dY with the filter's taps mirrored and its channel / feature roles swapped.
-// `supports` is false when neither kernel takes the shape.
-bool conv2d_input_backprop_f16_supports(const snn_hip_conv2d_params& p);
-int launch_conv2d_input_backprop_f16(const _Float16* dy,
-                                     const _Float16* filter, _Float16* dx,
-                                     const snn_hip_conv2d_params& p,
-                                     _Float16* workspace,
-                                     size_t workspace_elems,
-                                     hipStream_t stream);
+// Row-major binary16 GEMM y[m][n] = sum_k x[m][k] w[n][k] (gemm_nt_f16.hip):
+// input gradients of 1x1 stride-1 convolutions and matmul with B transposed; k a
+// multiple of 64, x and w 16-byte aligned.
+bool gemm_nt_f16_supports(int m, int k, int n);
+int launch_gemm_nt_f16(const _Float16* x, const _Float16* w, _Float16* y, int m,
+                       int k, int n, hipStream_t stream);
 
-// Half-precision strided input gradient by stride classes (conv2d_igemm.hip):
-// every class of input pixels modulo the strides is a dense stride-1 forward
-// convolution of dY on the binary16 kernels.  Features in multiples of 64,
-// channels of 4, from 2^30 multiply-adds; the launch returns -1 when the
-// geometry does not fit (then nothing was launched).
-bool conv2d_strided_input_backprop_f16_supports(const snn_hip_conv2d_params& p);
-int launch_conv2d_strided_input_backprop_f16(const _Float16* output_gradient,
-                                             const _Float16* filter,
-                                             _Float16* input_gradient,
-                                             const snn_hip_conv2d_params& p,
-                                             hipStream_t stream);
+// Half-precision forward convolution and input gradient on the binary16 matrix
+// cores (conv2d_gather_f16.hip): stride-1 unpadded 1x1 layers on the row-major
+// GEMM kernels above, stride-1 layers that fill the GPU on the LDS-tile kernel, every
+// other window (up to 12 x 12), stride (input gradient: up to 16 classes) and
+// channel count on the gathering kernel.  The launch returns -1 when none takes
+// the shape or there is no room for its temporaries; `workspace` of
+// conv2d_f16_workspace_halves halves, 16-byte aligned, saves those.
+size_t conv2d_f16_workspace_halves(int direction,
+                                   const snn_hip_conv2d_params& p);
+int launch_conv2d_f16(int direction, const _Float16* input,
+                      const _Float16* filter, _Float16* output,
+                      const snn_hip_conv2d_params& p, _Float16* workspace,
+                      size_t workspace_elems, hipStream_t stream);
 
-// Half-precision forward convolution for the shapes the binary16 kernels do
-// not take (conv2d_igemm.hip): the general implicit-GEMM kernel reading
-// binary16 operands.  Channels and features in multiples of 4.
-bool conv2d_forward_general_f16_supports(const snn_hip_conv2d_params& p);
-int launch_conv2d_forward_general_f16(const _Float16* input,
-                                      const _Float16* filter, _Float16* output,
-                                      const snn_hip_conv2d_params& p,
-                                      hipStream_t stream);
-
-// Half-precision gradients on the fp32 matrix instructions
-// (conv2d_igemm.hip): the filter gradient for channel counts in multiples of
-// 64 (fp32 accumulation buffer in the workspace when it holds twice the
-// filter's element count, else a stream-ordered temporary), and the input
-// gradient for the shapes launch_conv2d_input_backprop_f16 does not take.
+// Half-precision filter gradient on the fp32 matrix instructions
+// (conv2d_igemm.hip) for channel counts in multiples of 64: fp32 accumulation
+// buffer in the workspace when it holds twice the filter's element count, else
+// a stream-ordered temporary.
 // conv2d_filter_backprop_f16.hip: 3x3 stride-1 SAME filter gradient on the
 // binary16 matrix cores (channels and features multiples of 64).  `part` is
 // scratch of ..._partial_floats(p) floats for the partial tiles.
@@ -298,13 +268,6 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
                                       _Float16* workspace,
                                       size_t workspace_elems,
                                       hipStream_t stream);
-bool conv2d_input_backprop_general_f16_supports(
-    const snn_hip_conv2d_params& p);
-int launch_conv2d_input_backprop_general_f16(const _Float16* dy,
-                                             const _Float16* filter,
-                                             _Float16* dx,
-                                             const snn_hip_conv2d_params& p,
-                                             hipStream_t stream);
 
 // Half-precision stride-1 forward convolution with the input tile resident
 // in LDS (conv2d_rowtile_f16.hip).  `packed` receives the filter in MFMA
@@ -313,7 +276,8 @@ int launch_conv2d_input_backprop_general_f16(const _Float16* dy,
 // gradient's: `p` then describes the gradient as a forward convolution of dY
 // (channels = the original features and vice versa, padding window - 1 - pad)
 // and `filter` is still the original HWCF tensor.
-bool conv2d_rowtile_f16_supports(const snn_hip_conv2d_params& p);
+// `wanted`: it takes the shape and is the faster one.
+bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p);
 int launch_conv2d_rowtile_f16(const _Float16* input, const _Float16* filter,
                               _Float16* output, const snn_hip_conv2d_params& p,
                               _Float16* packed, hipStream_t stream,

@@ -1,0 +1,95 @@
+"""Binary16 forward convolutions and input gradients at the sizes where the
+gathering kernel can go wrong: edges of its tiles, ragged channel and feature
+counts, stride classes with few, unequal or no taps, reductions shared by
+work-groups, filters that are not 16-byte aligned.
+
+Bound: the result is rounded to binary16 once (2^-11 of its magnitude) and its
+n products are added in fp32, each addition rounding by at most 2^-24 of a
+partial sum, which for the U[-1,1] operands here is of the size of the outputs:
+|gpu - ref| <= 2^-11 |ref| + n 2^-24 S + 2^-24 (subnormals), S the largest |ref|.
+"""
+import numpy as np
+import pytest
+import torch
+
+from portdnn_amd import ops
+from portdnn_amd.capi import ALGO, DIRECTION, DTYPE
+from test_gpu_parity import ORACLE_FN, dev, oracle_params, uniform
+
+pytestmark = pytest.mark.gpu
+
+
+def assert_rounded_once(got, ref, n_products, what):
+    got = np.asarray(got, dtype=np.float64).reshape(-1)
+    ref = np.asarray(ref, dtype=np.float64).reshape(-1)
+    size = np.abs(ref)
+    bound = 2.0**-11 * size + n_products * 2.0**-24 * size.max() + 2.0**-24
+    err = np.abs(got - ref)
+    assert np.all(err <= bound), (what, err.max(), np.argmax(err - bound))
+
+
+# batch, rows, cols, channels, features, window, stride, same
+SHAPES = [
+    (2, 9, 7, 8, 8, 1, 1, True),        # the smallest pieces
+    (1, 13, 11, 20, 30, 3, 2, True),    # no multiples of 8; nothing full
+    (3, 10, 13, 35, 45, 5, 1, False),   # odd counts: widened, 2-byte stores
+    (2, 17, 16, 36, 68, 3, 1, True),    # multiples of 4: 8-byte stores
+    (2, 12, 15, 24, 40, 3, 3, True),    # nine classes
+    (2, 15, 14, 40, 24, 2, 3, False),   # classes that no tap reaches
+    (2, 16, 16, 64, 136, 1, 2, True),   # 1x1 strided: three empty classes
+    (1, 16, 17, 32, 33, 1, 4, False),   # ... sixteen classes, odd features
+    (1, 18, 18, 16, 16, 12, 1, True),   # the largest window
+    (1, 20, 20, 8, 12, 13, 2, True),    # one larger: another kernel
+    (4, 16, 16, 96, 128, 3, 1, True),   # whole tiles of 128
+    (1, 23, 23, 96, 129, 3, 1, True),   # one feature and one pixel past them
+    (2, 7, 7, 512, 72, 3, 1, True),     # long reduction, few tiles: shared
+    (5, 9, 9, 264, 264, 3, 2, True),    # ... by classes of unequal length
+    (9, 57, 43, 72, 96, 3, 2, True),    # many tiles, ragged rows
+    (16, 40, 40, 64, 200, 3, 2, True),  # tiles of 256 pixels
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("direction", [DIRECTION.FORWARD,
+                                       DIRECTION.INPUT_BACKPROP])
+def test_conv_f16_shapes(shape, direction):
+    batch, rows, cols, channels, features, window, stride, same = shape
+    p = ops.conv_params(batch, rows, cols, channels, features, window, stride,
+                        same)
+    rng = np.random.default_rng(4100 + rows + channels + features)
+    n_a, n_b, n_out = ops.conv_sizes(p, direction)
+    a = uniform(rng, n_a).astype(np.float16)
+    b = uniform(rng, n_b).astype(np.float16)
+    ref = ORACLE_FN[direction](a.astype(np.float32), b.astype(np.float32),
+                               oracle_params(p, features), acc64=True)
+    da, db = dev(a, torch.float16), dev(b, torch.float16)
+    shifted = torch.empty(n_b + 1, dtype=torch.float16, device="cuda")[1:]
+    shifted.copy_(db)
+    n = window * window * (channels if direction == DIRECTION.FORWARD
+                           else features)
+    _, rec = ops.workspace_size(p, direction, ALGO.IM2COL, DTYPE.F16)
+    block = torch.full((rec + 4096,), 7.0, dtype=torch.float16, device="cuda")
+    for fil, ws in ((db, None), (db, block[:rec] if rec else None),
+                    (shifted, None)):
+        guard = torch.full((n_out + 4096,), 7.0, dtype=torch.float16,
+                           device="cuda")
+        got = ops.conv2d(da, fil, p, direction, ALGO.IM2COL, workspace=ws,
+                         out=guard[:n_out])
+        assert_rounded_once(got.float().cpu().numpy(), ref, n,
+                            (shape, direction, ws is None, fil is db))
+        assert torch.all(guard[n_out:] == 7.0)
+    assert torch.all(block[rec:] == 7.0)
+
+
+@pytest.mark.parametrize("m,k,n", [(32, 64, 64), (33, 40, 24), (257, 100, 130),
+                                   (640, 1000, 30)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_matmul_f16_ragged(m, k, n, trans_b):
+    rng = np.random.default_rng(4200 + m + k + n)
+    a = uniform(rng, m * k).astype(np.float16)
+    b = uniform(rng, k * n).astype(np.float16)
+    bm = b.reshape(n, k).T if trans_b else b.reshape(k, n)
+    ref = a.reshape(m, k).astype(np.float64) @ bm.astype(np.float64)
+    got = ops.matmul(dev(a, torch.float16), dev(b, torch.float16), 1, m, k, n,
+                     trans_b=trans_b)
+    assert_rounded_once(got.float().cpu().numpy(), ref, k, (m, k, n, trans_b))
