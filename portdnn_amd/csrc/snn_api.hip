@@ -319,6 +319,15 @@ void im2col_workspace(const snn_hip_conv2d_params& p, int direction,
 // (forward, stride-1 input gradient) or the fp32 partial tiles / accumulation
 // buffer of the filter gradient, counted in halves.
 size_t f16_workspace_halves(const snn_hip_conv2d_params& p, int direction) {
+  if (direction == SNN_HIP_FORWARD && conv2d_few_f16_forward_supports(p))
+    return 0;
+  if (direction == SNN_HIP_INPUT_BACKPROP &&
+      conv2d_few_f16_input_backprop_supports(p))
+    return 0;
+  if (direction == SNN_HIP_FILTER_BACKPROP) {
+    const size_t floats = conv2d_few_f16_filter_backprop_partial_floats(p);
+    if (floats != 0) return 2 * floats;
+  }
   if (direction != SNN_HIP_FILTER_BACKPROP)
     return conv2d_f16_workspace_halves(direction, p);
   if (!conv2d_filter_backprop_f16_supports(p)) return 0;
@@ -611,11 +620,18 @@ int launch_gemm_path<_Float16>(int direction, const _Float16* input,
                                const snn_hip_conv2d_params& p, hipStream_t s,
                                _Float16* workspace, size_t workspace_elems,
                                const LaunchOptions*) {
-  // (the 7x7 stride-2 stem's input gradient: fp32 has a kernel built for it)
-  if (direction == SNN_HIP_INPUT_BACKPROP &&
-      conv2d_stem_input_backprop_supports(p)) {
-    const int rc = launch_f16_through_fp32(direction, input, filter, output, p, s);
-    if (rc >= 0) return rc;
+  if (aligned16(input) && aligned16(filter) && aligned16(output)) {
+    if (direction == SNN_HIP_FORWARD && conv2d_few_f16_forward_supports(p))
+      return launch_conv2d_few_f16_forward(input, filter, output, p, s);
+    if (direction == SNN_HIP_INPUT_BACKPROP &&
+        conv2d_few_f16_input_backprop_supports(p))
+      return launch_conv2d_few_f16_input_backprop(input, filter, output, p, s);
+    if (direction == SNN_HIP_FILTER_BACKPROP &&
+        conv2d_few_f16_filter_backprop_partial_floats(p) != 0) {
+      const int rc = launch_conv2d_few_f16_filter_backprop(
+          input, filter, output, p, workspace, workspace_elems, s);
+      if (rc >= 0) return rc;
+    }
   }
   if (direction != SNN_HIP_FILTER_BACKPROP) {
     const int rc = launch_conv2d_f16(direction, input, filter, output, p,

@@ -241,6 +241,29 @@ int launch_conv2d_f16(int direction, const _Float16* input,
 // (conv2d_igemm.hip) for channel counts in multiples of 64: fp32 accumulation
 // buffer in the workspace when it holds twice the filter's element count, else
 // a stream-ordered temporary.
+// conv2d_few_f16.hip: one to four channels at stride 2, features in multiples
+// of 8 up to 96.  All operands 16-byte aligned.  The filter gradient keeps
+// partial sums in the workspace when it is given the room (else in a
+// stream-ordered temporary; -1 when there is none).
+bool conv2d_few_f16_forward_supports(const snn_hip_conv2d_params& p);
+bool conv2d_few_f16_input_backprop_supports(const snn_hip_conv2d_params& p);
+// 0: not supported
+size_t conv2d_few_f16_filter_backprop_partial_floats(
+    const snn_hip_conv2d_params& p);
+int launch_conv2d_few_f16_forward(const _Float16* x, const _Float16* w,
+                                  _Float16* y, const snn_hip_conv2d_params& p,
+                                  hipStream_t stream);
+int launch_conv2d_few_f16_input_backprop(const _Float16* dy, const _Float16* w,
+                                         _Float16* dx,
+                                         const snn_hip_conv2d_params& p,
+                                         hipStream_t stream);
+int launch_conv2d_few_f16_filter_backprop(const _Float16* x,
+                                          const _Float16* dy, _Float16* dw,
+                                          const snn_hip_conv2d_params& p,
+                                          _Float16* workspace,
+                                          size_t workspace_elems,
+                                          hipStream_t stream);
+
 // conv2d_filter_backprop_f16.hip: 3x3 stride-1 SAME filter gradient on the
 // binary16 matrix cores (channels and features multiples of 64).  `part` is
 // scratch of ..._partial_floats(p) floats for the partial tiles.
