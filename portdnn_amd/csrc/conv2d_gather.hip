@@ -1,6 +1,6 @@
-// Half-precision forward convolution and input gradient for every window,
-// stride and channel count, as an implicit GEMM on MFMA (gfx950): binary16
-// operands, fp32 accumulation, binary16 result.
+// Forward convolution and input gradient for every window, stride and channel
+// count, as an implicit GEMM on MFMA (gfx950): binary16 or fp32 operands, fp32
+// accumulation, one rounding of a binary16 result.
 //
 //   forward         Y[pixel][f]  = sum over (tap, c) X[pixel o tap][c] * W[tap][c][f]
 //   input gradient  dX[pixel][c] = sum over (tap, f) dY[pixel o tap][f] * W[tap'][c][f]
@@ -13,11 +13,11 @@
 // classes run in one launch, the one with the most taps first, and store their
 // pixels straight into dX; a class that no tap reaches stores zeros.
 //
-// The reduction runs over 16-byte pieces -- eight channels of one tap -- of a
-// pixel, flattened over (tap, piece): chunks of 32 channels are four pieces,
+// The reduction runs over 16-byte pieces -- eight binary16 or four fp32 channels
+// of one tap -- of a pixel, flattened over (tap, piece): a chunk is four pieces,
 // which may belong to different taps, so channel counts that are no multiple
-// of 32 waste nothing but the last chunk's tail.  Source tensors whose channel
-// count is no multiple of 8 are copied once with the count rounded up.
+// of a chunk's waste nothing but the last chunk's tail.  Source tensors whose
+// channel count fills no whole pieces are copied once with the count rounded up.
 //
 //   * A work-group owns BM pixels x BN features.  Per chunk both tiles, [row][4
 //     pieces], arrive in one of three LDS buffers by loads that write LDS
@@ -28,13 +28,24 @@
 //   * Which of its four positions in an LDS row a piece takes is XORed with
 //     bits of the row, so that the ds_read_b128 of 8 or 16 consecutive rows
 //     touch different banks.
-//   * A forward filter (and a gradient's whose feature count is no multiple of
-//     8) is packed first, [32 features][chunk][row][4 pieces] in the same
-//     swizzled order (2-5 us), zeros where channels or features end.  The
+//   * A binary16 forward filter (and a gradient's whose feature count fills no
+//     whole pieces) is packed first, [32 features][chunk][row][4 pieces] in the
+//     same swizzled order (2-5 us), zeros where channels or features end.  The
 //     gradient's is read in place: its reduction index is the contiguous one.
+//     So is a forward fp32 filter, whose tile lies in LDS as it does in memory,
+//     [16 (tap, channel)][features]: an fp32 instruction wants one value of a
+//     lane, which that layout gives it without conflicts.
 //   * Features are the MFMA rows and pixels the columns, with the features of
 //     a block permuted in the packed filter so that a lane ends with 16
-//     consecutive features of one pixel (two 16-byte stores).
+//     consecutive features of one pixel (16-byte stores).
+//   * An fp32 instruction (32x32x2) takes as long as a binary16 one but sums two
+//     products instead of sixteen: there the matrix units are the bound, and
+//     the tap arithmetic of every lane costs nothing beside them.
+//   * A strided gradient of few channels (a three-channel first layer) would
+//     fill 3 of the 32 matrix rows.  Its classes are merged: the pixels of a
+//     block of stride x stride share one window of ceil(window / stride) source
+//     pixels, and (class, channel) are the rows, with zeros packed for taps that
+//     do not reach a class (12 of 32 rows, 49 of 64 taps of a 7x7 stride 2).
 #include <algorithm>
 #include <climits>
 #include <cmath>
@@ -55,9 +66,21 @@ typedef float float4v __attribute__((ext_vector_type(4)));
 typedef unsigned int uint2v __attribute__((ext_vector_type(2)));
 typedef unsigned int uint4v __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void* lds_ptr;
+template <typename T>
+struct PieceOf;
+template <> struct PieceOf<_Float16> { typedef half8 type; };
+template <> struct PieceOf<float> { typedef float4v type; };
+template <typename T>
+constexpr int kPiece = 16 / static_cast<int>(sizeof(T));  // channels
+
+// Where the filter operand comes from: packed tiles, the gradient's filter as it
+// is (reduction index contiguous), the forward fp32 filter as it is (features
+// contiguous).
+enum FilterFrom { kPacked, kInPlace, kRows };
+
 constexpr unsigned kOob = 0x7FFFFFF0u;
 constexpr size_t kMaxBufferBytes = 0x7FFFFFF0u;
-constexpr int kRowBytes = 64;     // one chunk (32 halves) of one row
+constexpr int kRowBytes = 64;     // one chunk of one row
 constexpr int kMaxClasses = 16;
 constexpr int kMaxWindow = 12;    // the two tap masks of a pixel share a word
 
@@ -100,12 +123,14 @@ struct Gather {
   int step_r, step_c;    // source step per class pixel
   int out_rows, out_cols, out_step_r, out_step_c;
   int channels, features;
-  int win_cols;          // columns of the whole filter
+  int win_rows, win_cols;  // of the whole filter
   int n_tiles_n;
   int n_splits;          // work-groups that share a tile's reduction
   unsigned n_tiles;      // tiles of all classes
   int n_classes;
   int mirrored;          // input gradient: w[tap][feature][channel]
+  int merged;            // channels per pixel of merged classes, or 0
+  int relu;              // of a forward launch with bias and activation
   GatherClass cls[kMaxClasses];
 };
 
@@ -137,6 +162,12 @@ __host__ __device__ constexpr int feature_of_row(unsigned row) {
                           4 * ((row >> 3) & 1) + (row & 3));
 }
 
+// What a bias and an activation make of a sum.
+__device__ __forceinline__ float bias_act(float v, float bias, int relu) {
+  v += bias;
+  return relu != 0 ? fmaxf(v, 0.f) : v;
+}
+
 // (a function of its own: the compiler drops the host side of a kernel template
 // whose body names the LDS-direct load)
 __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t rsrc,
@@ -156,19 +187,35 @@ constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 struct TileOf { int m, cls, n; };
 __device__ __forceinline__ TileOf tile_of(unsigned tile, const Gather& g) {
   const unsigned n = tile % g.n_tiles_n, t = tile / g.n_tiles_n;
-  return {static_cast<int>(t / g.n_classes), static_cast<int>(t % g.n_classes),
+  const unsigned m = t / g.n_classes;
+  return {static_cast<int>(m), static_cast<int>((t + m) % g.n_classes),
           static_cast<int>(n)};
+}
+
+// Output element of feature f of a merged block, or -1 outside the image.
+__device__ __forceinline__ int merged_element(const Gather& g,
+                                              const GatherClass& cls, Pixel px,
+                                              int f) {
+  const int k = f / g.merged, c = f - k * g.merged;
+  const int a = k / g.out_step_c, b = k - a * g.out_step_c;
+  const int y = px.y * g.out_step_r + cls.out_r0 + a;
+  const int x = px.x * g.out_step_c + cls.out_c0 + b;
+  return y >= 0 && y < g.out_rows && x >= 0 && x < g.out_cols &&
+                 f < g.features
+             ? ((px.n * g.out_rows + y) * g.out_cols + x) * g.merged + c
+             : -1;
 }
 
 // Filter pack (the first n_pack_groups work-groups, one lane per 16-byte
 // piece) and, behind it, the copy of a source tensor to whole pieces.
+template <typename T>
 __global__ void __launch_bounds__(256)
-    gather_prepare_kernel(const _Float16* __restrict__ w,
-                          _Float16* __restrict__ wpk, Gather g,
-                          unsigned n_pack_lanes, unsigned n_pack_groups,
-                          const _Float16* __restrict__ src,
-                          _Float16* __restrict__ wide, unsigned n_pieces) {
-  half8 v;
+    gather_prepare_kernel(const T* __restrict__ w, T* __restrict__ wpk,
+                          Gather g, unsigned n_pack_lanes,
+                          unsigned n_pack_groups, const T* __restrict__ src,
+                          T* __restrict__ wide, unsigned n_pieces) {
+  constexpr int kE = kPiece<T>;
+  typename PieceOf<T>::type v;
   if (blockIdx.x < n_pack_groups) {
     const unsigned idx = blockIdx.x * 256 + threadIdx.x;
     if (idx >= n_pack_lanes) return;
@@ -180,47 +227,56 @@ __global__ void __launch_bounds__(256)
     const unsigned nb = local / cls.n_chunks, chunk = local % cls.n_chunks;
     const int q = static_cast<int>(chunk * 4 + (slot ^ swz(row & 15)));
     const int tap = divide(q, g.by_cp);
-    const int c = (q - tap * g.cp) * 8;
+    const int c = (q - tap * g.cp) * kE;
     const int tr = divide(tap, cls.by_win_c), ts = tap - tr * cls.win_c;
-    const int f = nb * 32 + feature_of_row(row);
-    const bool ok = tr < cls.win_r && f < g.features;
-    const int valid = ok ? min(8, g.channels - c) : 0;
-    const size_t at_tap =
-        static_cast<size_t>((cls.tap_r0 + tr * cls.tap_rs) * g.win_cols +
-                            cls.tap_c0 + ts * cls.tap_cs);
-    const _Float16* from =
-        g.mirrored ? w + (at_tap * g.features + f) * g.channels + c
-                   : w + (at_tap * g.channels + c) * g.features + f;
+    int f = nb * 32 + feature_of_row(row), per_tap = g.features;
+    bool ok = tr < cls.win_r && f < g.features;
+    int wr = cls.tap_r0 + tr * cls.tap_rs, wc = cls.tap_c0 + ts * cls.tap_cs;
+    if (g.merged != 0) {
+      const int member = f / g.merged;
+      f -= member * g.merged;
+      per_tap = g.merged;
+      wr += member / g.out_step_c;
+      wc += member % g.out_step_c;
+      ok = ok && wr < g.win_rows && wc < g.win_cols;
+    }
+    const int valid = ok ? min(kE, g.channels - c) : 0;
+    const size_t at_tap = static_cast<size_t>(wr * g.win_cols + wc);
+    const T* from = g.mirrored ? w + (at_tap * per_tap + f) * g.channels + c
+                               : w + (at_tap * g.channels + c) * g.features + f;
     const size_t stride = g.mirrored ? 1 : static_cast<size_t>(g.features);
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      v[e] = e < valid ? from[e * stride] : static_cast<_Float16>(0.f);
-    *reinterpret_cast<half8*>(wpk + static_cast<size_t>(idx) * 8) = v;
+    for (int e = 0; e < kE; ++e)
+      v[e] = e < valid ? from[e * stride] : static_cast<T>(0.f);
+    *reinterpret_cast<decltype(v)*>(wpk + static_cast<size_t>(idx) * kE) = v;
     return;
   }
   const unsigned idx = (blockIdx.x - n_pack_groups) * 256 + threadIdx.x;
   if (idx >= n_pieces) return;
   const unsigned pixel = divide(idx, g.by_cp);
-  const int c = static_cast<int>(idx - pixel * g.cp) * 8;
-  const _Float16* from = src + static_cast<size_t>(pixel) * g.channels + c;
+  const int c = static_cast<int>(idx - pixel * g.cp) * kE;
+  const T* from = src + static_cast<size_t>(pixel) * g.channels + c;
 #pragma unroll
-  for (int e = 0; e < 8; ++e)
-    v[e] = c + e < g.channels ? from[e] : static_cast<_Float16>(0.f);
-  *reinterpret_cast<half8*>(wide + static_cast<size_t>(idx) * 8) = v;
+  for (int e = 0; e < kE; ++e)
+    v[e] = c + e < g.channels ? from[e] : static_cast<T>(0.f);
+  *reinterpret_cast<decltype(v)*>(wide + static_cast<size_t>(idx) * kE) = v;
 }
 
 // WM x WN waves of TM x TN blocks of 32 pixels x 32 features.  UNIFORM: whole
-// chunks per tap (channels in multiples of 32), tap bookkeeping in scalar
-// registers; otherwise every lane works out the tap of its own piece.  IN_PLACE:
-// `wpk` is the gradient's filter itself, w[tap][feature][channel].
-template <int WM, int WN, int TM, int TN, bool UNIFORM, bool IN_PLACE>
+// chunks per tap, tap bookkeeping in scalar registers; otherwise every lane
+// works out the tap of its own piece.  FROM: what `wpk` is.
+template <typename T, int WM, int WN, int TM, int TN, bool UNIFORM, int FROM>
 __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
-    conv_gather_f16_kernel(const _Float16* __restrict__ src,
-                           const _Float16* __restrict__ wpk,
-                           _Float16* __restrict__ dst,
-                           float* __restrict__ part, Gather g,
-                           unsigned src_bytes, unsigned wpk_bytes,
-                           unsigned dst_bytes, unsigned n_groups) {
+    conv_gather_kernel(const T* __restrict__ src, const T* __restrict__ wpk,
+                       const float* __restrict__ bias, T* __restrict__ dst,
+                       float* __restrict__ part, Gather g, unsigned src_bytes,
+                       unsigned wpk_bytes, unsigned dst_bytes,
+                       unsigned n_groups) {
+  typedef typename PieceOf<T>::type Piece;
+  constexpr bool IN_PLACE = FROM == kInPlace;
+  constexpr int kE = kPiece<T>;
+  constexpr unsigned kSize = sizeof(T);
+  static_assert(FROM != kRows || kSize == 4, "one value per lane");
   constexpr int NW = WM * WN;
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   constexpr int LA = BM / 16 / NW;                      // loads per wave, chunk
@@ -249,11 +305,11 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
   const int n_chunks = min(cls.n_chunks - chunk0, per_split);
 
   // A class that no tap reaches: zeros, whole runs of features per pixel.
-  if (cls.n_chunks == 0 && (g.features & 7) == 0) {
+  if (cls.n_chunks == 0 && (g.features & (kE - 1)) == 0) {
     if (split != 0) return;
     const __amdgpu_buffer_rsrc_t out = make_rsrc(dst, dst_bytes);
-    for (int i = threadIdx.x; i < BM * (BN / 8); i += 64 * NW) {
-      const int m = m0 + i / (BN / 8), f = n0 + i % (BN / 8) * 8;
+    for (int i = threadIdx.x; i < BM * (BN / kE); i += 64 * NW) {
+      const int m = m0 + i / (BN / kE), f = n0 + i % (BN / kE) * kE;
       const Pixel px = pixel_of(m, cls);
       const unsigned pixel =
           (px.n * g.out_rows + px.y * g.out_step_r + cls.out_r0) * g.out_cols +
@@ -261,7 +317,7 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
       const uint4v zero = {0u, 0u, 0u, 0u};
       __builtin_amdgcn_raw_buffer_store_b128(
           zero, out, m < cls.pixels && f < g.features
-                         ? (pixel * g.features + f) * 2u : kOob, 0, 0);
+                         ? (pixel * g.features + f) * kSize : kOob, 0, 0);
     }
     return;
   }
@@ -300,9 +356,16 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
       const int f = n0 + b_block[i] / 2 * 32 +
                     feature_of_row((b_block[i] & 1) * 16 + (lane >> 2));
       // (2^31 stays out of range whatever is added)
-      b_off[i] = f < g.features ? static_cast<unsigned>(f * g.channels) * 2u +
+      b_off[i] = f < g.features ? static_cast<unsigned>(f * g.channels) * kSize +
                                       (UNIFORM ? piece * 16u : 0u)
                                 : 0x80000000u;
+    } else if constexpr (FROM == kRows) {
+      // 1 KB of the tile: whole runs of BN features of 256 / BN filter rows
+      // (columns past the last feature belong to the next row, and to outputs
+      // that are not stored; rows past the last one load zeros)
+      const int at = b_block[i] * 256 + lane * 4;
+      b_off[i] = static_cast<unsigned>((chunk0 * 16 + at / BN) * g.features +
+                                       n0 + at % BN) * 4u;
     } else {
       b_off[i] = ((cls.pack_block + static_cast<unsigned>(n0 / 32 + b_block[i] / 2) *
                                         cls.n_chunks) * 2 +
@@ -320,9 +383,10 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
     tap_r = tap / win_c;
     tap_c = tap - tap_r * win_c;
   }
-  unsigned b_chunk = IN_PLACE ? 0u : chunk0 * 2048u;
+  unsigned b_chunk = FROM == kPacked ? chunk0 * 2048u : 0u;
+  const unsigned b_step = FROM == kRows ? g.features * 64u : 2048u;
   // IN_PLACE: bytes from a tap to the next column's, the next row's
-  const int filter_row = cp * 8 * 2, filter_tap = g.features * filter_row;
+  const int filter_row = cp * 16, filter_tap = g.features * filter_row;
   const int tap_at = (cls.tap_r0 * g.win_cols + cls.tap_c0) * filter_tap;
   const int tap_dr = cls.tap_rs * g.win_cols * filter_tap;
   const int tap_dc = cls.tap_cs * filter_tap;
@@ -365,7 +429,7 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
                   IN_PLACE && !UNIFORM ? (b_off[i] | b_chunk) >= 0x80000000u
                                              ? kOob : b_off[i] + b_chunk
                                        : b_off[i] + b_chunk);
-    if constexpr (!IN_PLACE) b_chunk += 2048;
+    if constexpr (!IN_PLACE) b_chunk += b_step;
   };
 
   float16v acc[TN][TM];
@@ -383,24 +447,47 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
   const int ft_at = (BM + wn * TN * 32 + l32) * kRowBytes + in_row;
   // Operands of reduction step S (16 channels) of a chunk.  (Step 1 reads
   // pieces 2 and 3: bit 1 of the swizzled position flips.)
-  struct Operands { half8 a[TN], b[TM]; };
+  struct Operands { Piece a[TN], b[TM]; };
+  const int row_at = BM * kRowBytes + khalf * (4 * BN * 4) +
+                     (wn * TN * 32 + feature_of_row(l32)) * 4;
   auto fetch = [&](const char* buf, int s, Operands& o) {
 #pragma unroll
-    for (int i = 0; i < TN; ++i)
-      o.a[i] = *reinterpret_cast<const half8*>(
-          buf + (ft_at ^ (32 * s)) + i * 32 * kRowBytes);
+    for (int i = 0; i < TN; ++i) {
+      if constexpr (FROM == kRows) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          o.a[i][e] = *reinterpret_cast<const float*>(
+              buf + row_at + (8 * s + e) * (BN * 4) + i * 128);
+      } else {
+        o.a[i] = *reinterpret_cast<const Piece*>(
+            buf + (ft_at ^ (32 * s)) + i * 32 * kRowBytes);
+      }
+    }
 #pragma unroll
     for (int j = 0; j < TM; ++j)
-      o.b[j] = *reinterpret_cast<const half8*>(
+      o.b[j] = *reinterpret_cast<const Piece*>(
           buf + (px_at ^ (32 * s)) + j * 32 * kRowBytes);
   };
+  // (fp32: element e of the two lane halves is products 4 (2 s) + e and
+  // 4 (2 s + 1) + e of the chunk)
   auto multiply = [&](const Operands& o) {
+    if constexpr (kSize == 2) {
 #pragma unroll
-    for (int i = 0; i < TN; ++i)
+      for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TM; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-            o.a[i], o.b[j], acc[i][j], 0, 0, 0);
+        for (int j = 0; j < TM; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+              o.a[i], o.b[j], acc[i][j], 0, 0, 0);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
+                o.a[i][e], o.b[j][e], acc[i][j], 0, 0, 0);
+    }
   };
 
   // One chunk: its step 0 operands are in `even`, the next two chunks are
@@ -482,6 +569,44 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
   // A lane holds features f0 .. f0 + 7 and f0 + 16 .. f0 + 23 of one pixel per
   // block.
   const __amdgpu_buffer_rsrc_t dst_rsrc = make_rsrc(dst, dst_bytes);
+  if constexpr (kSize == 4) {
+    if (g.merged != 0) {
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        const int m = m0 + (wm * TM + j) * 32 + l32;
+        const Pixel px = pixel_of(m, cls);
+#pragma unroll
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const int f = n0 + (wn * TN + i) * 32 + 8 * khalf + v + v / 8 * 8;
+            const int at = merged_element(g, cls, px, f);
+            // (a variable of its own: a bit_cast of the vector's element takes
+            // its first one)
+            const float value = acc[i][j][v];
+            __builtin_amdgcn_raw_buffer_store_b32(
+                __builtin_bit_cast(unsigned, value), dst_rsrc,
+                m < cls.pixels && at >= 0 ? at * 4u : kOob, 0, 0);
+          }
+      }
+      return;
+    }
+    if (bias != nullptr || g.relu != 0) {
+      const __amdgpu_buffer_rsrc_t bias_rsrc =
+          make_rsrc(bias, bias != nullptr ? g.features * 4u : 0u);
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int f = n0 + (wn * TN + i) * 32 + 8 * khalf + v + v / 8 * 8;
+          const float add = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(bias_rsrc, f * 4u, 0, 0));
+#pragma unroll
+          for (int j = 0; j < TM; ++j)
+            acc[i][j][v] = bias_act(acc[i][j][v], add, g.relu);
+        }
+    }
+  }
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
     const int m = m0 + (wm * TM + j) * 32 + l32;
@@ -490,43 +615,67 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
     const int out_x = px.x * g.out_step_c + cls.out_c0;
     const unsigned at =
         static_cast<unsigned>(((px.n * g.out_rows + out_y) * g.out_cols + out_x) *
-                              g.features) * 2u;
+                              g.features) * kSize;
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
       const int f0 = n0 + (wn * TN + i) * 32 + 8 * khalf;
       const int count = m < cls.pixels ? g.features - f0 : 0;
-      const unsigned off = at + static_cast<unsigned>(f0) * 2u;
-      half8 lo, hi;
+      const unsigned off = at + static_cast<unsigned>(f0) * kSize;
+      if constexpr (kSize == 4) {
+        if ((g.features & 3) == 0) {
 #pragma unroll
-      for (int v = 0; v < 8; ++v) {
-        lo[v] = static_cast<_Float16>(acc[i][j][v]);
-        hi[v] = static_cast<_Float16>(acc[i][j][8 + v]);
-      }
-      const uint4v w0 = __builtin_bit_cast(uint4v, lo);
-      const uint4v w1 = __builtin_bit_cast(uint4v, hi);
-      if ((g.features & 7) == 0) {
-        __builtin_amdgcn_raw_buffer_store_b128(w0, dst_rsrc,
-                                               count > 0 ? off : kOob, 0, 0);
-        __builtin_amdgcn_raw_buffer_store_b128(
-            w1, dst_rsrc, count > 16 ? off + 32u : kOob, 0, 0);
-      } else if ((g.features & 3) == 0) {
-        const unsigned words[8] = {w0[0], w0[1], w0[2], w0[3],
-                                   w1[0], w1[1], w1[2], w1[3]};
+          for (int v = 0; v < 4; ++v) {
+            const float4v four = {acc[i][j][4 * v], acc[i][j][4 * v + 1],
+                                  acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]};
+            __builtin_amdgcn_raw_buffer_store_b128(
+                __builtin_bit_cast(uint4v, four), dst_rsrc,
+                count > 4 * v + v / 2 * 8 ? off + 16u * v + v / 2 * 32u : kOob,
+                0, 0);
+          }
+        } else {
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const uint2v two = {words[2 * v], words[2 * v + 1]};
-          __builtin_amdgcn_raw_buffer_store_b64(
-              two, dst_rsrc,
-              count > 4 * v + v / 2 * 8 ? off + 8u * v + v / 2 * 16u : kOob, 0,
-              0);
+          for (int v = 0; v < 16; ++v) {
+            const float value = acc[i][j][v];
+            __builtin_amdgcn_raw_buffer_store_b32(
+                __builtin_bit_cast(unsigned, value), dst_rsrc,
+                count > v + v / 8 * 8 ? off + 4u * v + v / 8 * 32u : kOob, 0,
+                0);
+          }
         }
       } else {
+        half8 lo, hi;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          const _Float16 h = v < 8 ? lo[v] : hi[v - 8];
-          __builtin_amdgcn_raw_buffer_store_b16(
-              __builtin_bit_cast(unsigned short, h), dst_rsrc,
-              count > v + v / 8 * 8 ? off + 2u * v + v / 8 * 16u : kOob, 0, 0);
+        for (int v = 0; v < 8; ++v) {
+          lo[v] = static_cast<_Float16>(acc[i][j][v]);
+          hi[v] = static_cast<_Float16>(acc[i][j][8 + v]);
+        }
+        const uint4v w0 = __builtin_bit_cast(uint4v, lo);
+        const uint4v w1 = __builtin_bit_cast(uint4v, hi);
+        if ((g.features & 7) == 0) {
+          __builtin_amdgcn_raw_buffer_store_b128(w0, dst_rsrc,
+                                                 count > 0 ? off : kOob, 0, 0);
+          __builtin_amdgcn_raw_buffer_store_b128(
+              w1, dst_rsrc, count > 16 ? off + 32u : kOob, 0, 0);
+        } else if ((g.features & 3) == 0) {
+          const unsigned words[8] = {w0[0], w0[1], w0[2], w0[3],
+                                     w1[0], w1[1], w1[2], w1[3]};
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const uint2v two = {words[2 * v], words[2 * v + 1]};
+            __builtin_amdgcn_raw_buffer_store_b64(
+                two, dst_rsrc,
+                count > 4 * v + v / 2 * 8 ? off + 8u * v + v / 2 * 16u : kOob,
+                0, 0);
+          }
+        } else {
+#pragma unroll
+          for (int v = 0; v < 16; ++v) {
+            const _Float16 h = v < 8 ? lo[v] : hi[v - 8];
+            __builtin_amdgcn_raw_buffer_store_b16(
+                __builtin_bit_cast(unsigned short, h), dst_rsrc,
+                count > v + v / 8 * 8 ? off + 2u * v + v / 8 * 16u : kOob, 0,
+                0);
+          }
         }
       }
     }
@@ -535,10 +684,11 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
 
 // Sums the splits of every tile in order and rounds: one float4 -- four
 // consecutive features of a pixel -- per lane.
-template <int WM, int WN, int TM, int TN>
+template <typename T, int WM, int WN, int TM, int TN>
 __global__ void __launch_bounds__(256)
     gather_reduce_kernel(const float4v* __restrict__ part,
-                         _Float16* __restrict__ dst, Gather g) {
+                         const float* __restrict__ bias, T* __restrict__ dst,
+                         Gather g) {
   constexpr unsigned BM = 32 * WM * TM, BN = 32 * WN * TN;
   constexpr unsigned kTileVecs = BM * BN / 4;
   const unsigned at = blockIdx.x * 256 + threadIdx.x;
@@ -555,23 +705,41 @@ __global__ void __launch_bounds__(256)
                 static_cast<int>((wave % WN * TN + i) * 32) +
                 feature_of_row(8 * v + 4 * (lane / 32));
   if (m >= cls.pixels || f >= g.features) return;
-  if (cls.n_chunks == 0 && (g.features & 7) == 0) return;  // stored already
+  if (cls.n_chunks == 0 && (g.features & (kPiece<T> - 1)) == 0)
+    return;  // stored already
   float4v sum = {0.f, 0.f, 0.f, 0.f};
   const float4v* from = part + at;
 #pragma unroll 4
   for (int s = 0; s < g.n_splits; ++s)
     sum += from[static_cast<size_t>(s) * g.n_tiles * kTileVecs];
   const Pixel px = pixel_of(m, cls);
-  _Float16* const out =
+  if constexpr (sizeof(T) == 4) {
+    if (g.merged != 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int to = merged_element(g, cls, px, f + e);
+        if (to >= 0) dst[to] = sum[e];
+      }
+      return;
+    }
+    if (bias != nullptr || g.relu != 0) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        sum[e] = bias_act(
+            sum[e], bias != nullptr && f + e < g.features ? bias[f + e] : 0.f,
+            g.relu);
+    }
+  }
+  T* const out =
       dst + (static_cast<size_t>(px.n * g.out_rows + px.y * g.out_step_r +
                                  cls.out_r0) * g.out_cols +
              px.x * g.out_step_c + cls.out_c0) * g.features + f;
-  typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-  half4 r;
+  typedef T Four __attribute__((ext_vector_type(4)));
+  Four r;
 #pragma unroll
-  for (int e = 0; e < 4; ++e) r[e] = static_cast<_Float16>(sum[e]);
+  for (int e = 0; e < 4; ++e) r[e] = static_cast<T>(sum[e]);
   if ((g.features & 3) == 0) {
-    *reinterpret_cast<half4*>(out) = r;
+    *reinterpret_cast<Four*>(out) = r;
   } else {
     for (int e = 0; e < 4 && f + e < g.features; ++e) out[e] = r[e];
   }
@@ -582,17 +750,17 @@ struct GatherPlan {
   bool ok = false;
   int batch = 0;
   size_t src_pixels = 0;
-  bool widen = false;       // source channels are no multiple of 8
+  bool widen = false;       // source channels fill no whole pieces
   size_t out_elems = 0;
   size_t pack_blocks = 0;   // 2 KB blocks of packed filter
-  size_t wide_halves = 0;   // of the widened source
+  size_t wide_bytes = 0;    // of the widened source
   size_t part_floats = 0;   // of the tiles whose reduction is shared
-  int tile = 0;             // index into kTiles
+  int tile = 0;             // index into the tile shapes of the type
   int n_splits = 1;
   size_t filter_elems = 0;
-  bool in_place = false;    // the filter may be read as it is
-  size_t workspace_halves(bool packs) const {
-    return (packs ? pack_blocks * 1024 : 0) + wide_halves + 2 * part_floats;
+  FilterFrom from = kPacked;
+  size_t workspace_bytes(bool packs) const {
+    return (packs ? pack_blocks * 2048 : 0) + wide_bytes + 4 * part_floats;
   }
 };
 
@@ -602,12 +770,30 @@ struct TileShape {
   int pixels, features;
   double alone_us, share_us;
 };
-constexpr TileShape kTiles[] = {
+constexpr TileShape kTilesF16[] = {
     {256, 128, 0.57, 0.46}, {256, 64, 0.34, 0.376}, {128, 128, 0.27, 0.24},
     {128, 64, 0.245, 0.17},  {128, 32, 0.23, 0.135}, {64, 64, 0.22, 0.103}};
-constexpr int kNumTiles = sizeof(kTiles) / sizeof(kTiles[0]);
+// (fp32: eight matrix instructions of 64 cycles per chunk and SIMD, in either
+// shape, which one wastes fewer columns decides.  128 x 64 and 128 x 128 need
+// fewer loads per product but were no faster on any of forty shapes: 17x27x27
+// 96 -> 256, 5x5, 158 / 163 us against 162)
+constexpr TileShape kTilesF32[] = {{128, 32, 0.36, 0.27}, {64, 64, 0.36, 0.265}};
+constexpr int kMergedTile = 0;
+template <typename T>
+struct Tiles;
+template <>
+struct Tiles<_Float16> {
+  static constexpr const TileShape* shapes = kTilesF16;
+  static constexpr int count = sizeof(kTilesF16) / sizeof(kTilesF16[0]);
+};
+template <>
+struct Tiles<float> {
+  static constexpr const TileShape* shapes = kTilesF32;
+  static constexpr int count = sizeof(kTilesF32) / sizeof(kTilesF32[0]);
+};
 constexpr int kNumCus = 256;
-constexpr int kMaxSplits = 16;
+template <typename T>
+constexpr int kMaxSplits = sizeof(T) == 4 ? 32 : 16;  // (half the chunk)
 
 int tuned(const char* name, int otherwise) {
 #ifdef SNN_HIP_TUNING
@@ -623,13 +809,15 @@ int tuned(const char* name, int otherwise) {
 // second launch and the partial tiles written and read.  The constants were
 // measured; against forced choices the model's was within about 10 % of the
 // best on forty shapes from 1x7x7x512 to 16x224x224x64.
-void choose_tile(GatherPlan* plan) {
+template <typename T>
+void choose_tile(GatherPlan* plan, bool may_split) {
   const Gather& g = plan->g;
   int pixels = 0;
-  double chunks = 0;
+  double chunks = 0, longest = 0;
   for (int k = 0; k < g.n_classes; ++k) {
     pixels = std::max(pixels, g.cls[k].pixels);
     chunks += g.cls[k].n_chunks;
+    longest = std::max(longest, static_cast<double>(g.cls[k].n_chunks));
   }
   chunks /= g.n_classes;
   auto tiles_of = [&](const TileShape& t) {
@@ -637,14 +825,15 @@ void choose_tile(GatherPlan* plan) {
            ceil_div(g.features, t.features);
   };
   double best = 1e30;
-  for (int i = 0; i < kNumTiles; ++i) {
-    const TileShape& t = kTiles[i];
+  for (int i = 0; i < Tiles<T>::count; ++i) {
+    if (g.merged != 0 && i != kMergedTile) continue;
+    const TileShape& t = Tiles<T>::shapes[i];
     const double tiles = tiles_of(t);
-    for (int splits = 1; splits <= kMaxSplits; splits *= 2) {
-      if (splits > 1 && chunks / splits < 4) break;
+    for (int splits = 1; splits <= (may_split ? kMaxSplits<T> : 1); splits *= 2) {
+      if (splits > 1 && longest / splits < 4) break;
       const double rounds = std::ceil(tiles * splits / kNumCus);
-      double us = std::ceil(chunks / splits) *
-                      std::max(t.alone_us, rounds * t.share_us) +
+      double us = std::max(std::ceil(longest / splits) * t.alone_us,
+                           std::ceil(chunks / splits) * rounds * t.share_us) +
                   0.5 * rounds;
       if (splits > 1)
         us += 3.0 + splits * tiles * t.pixels * t.features * 8 / 3e6;
@@ -657,17 +846,29 @@ void choose_tile(GatherPlan* plan) {
   }
   plan->tile = tuned("SNN_HIP_GATHER_TILE", plan->tile);
   plan->n_splits = tuned("SNN_HIP_GATHER_SPLITS", plan->n_splits);
-  const TileShape& t = kTiles[plan->tile];
+  const TileShape& t = Tiles<T>::shapes[plan->tile];
   plan->part_floats =
       plan->n_splits > 1 ? static_cast<size_t>(plan->n_splits * tiles_of(t)) *
                                t.pixels * t.features
                          : 0;
 }
 
-GatherPlan compute_plan(int direction, const snn_hip_conv2d_params& p) {
+// (a workspace may be asked for with parameters that no launch would take)
+bool positive(const snn_hip_conv2d_params& p) {
+  return p.batch > 0 && p.in_rows > 0 && p.in_cols > 0 && p.channels > 0 &&
+         p.features > 0 && p.out_rows > 0 && p.out_cols > 0 &&
+         p.window_rows > 0 && p.window_cols > 0 && p.stride_rows > 0 &&
+         p.stride_cols > 0 && p.pad_rows >= 0 && p.pad_cols >= 0;
+}
+
+template <typename T>
+GatherPlan compute_plan(int direction, const snn_hip_conv2d_params& p,
+                        bool may_split) {
+  constexpr int kE = kPiece<T>;
   GatherPlan plan;
   if (direction != SNN_HIP_FORWARD && direction != SNN_HIP_INPUT_BACKPROP)
     return plan;
+  if (!positive(p)) return plan;
   const bool grad = direction == SNN_HIP_INPUT_BACKPROP;
   if (p.window_rows > kMaxWindow || p.window_cols > kMaxWindow) return plan;
   if (grad && p.stride_rows * p.stride_cols > kMaxClasses) return plan;
@@ -678,21 +879,32 @@ GatherPlan compute_plan(int direction, const snn_hip_conv2d_params& p) {
   g.out_cols = grad ? p.in_cols : p.out_cols;
   g.channels = grad ? p.features : p.channels;
   g.features = grad ? p.channels : p.features;
-  g.cp = (g.channels + 7) / 8;
+  g.cp = (g.channels + kE - 1) / kE;
   g.by_cp = divisor(g.cp);
   g.step_r = grad ? 1 : p.stride_rows;
   g.step_c = grad ? 1 : p.stride_cols;
   g.out_step_r = grad ? p.stride_rows : 1;
   g.out_step_c = grad ? p.stride_cols : 1;
+  g.win_rows = p.window_rows;
   g.win_cols = p.window_cols;
   g.mirrored = grad;
+  const int strides = p.stride_rows * p.stride_cols;
+  // (beyond four channels a class of its own fills more of its matrix rows)
+  g.merged = sizeof(T) == 4 && grad && strides > 1 && p.channels <= 4 &&
+                     p.channels * strides <= 32 &&
+                     p.window_rows >= p.stride_rows &&
+                     p.window_cols >= p.stride_cols
+                 ? p.channels : 0;
+  if (g.merged != 0) g.features = p.channels * strides;
+  g.relu = 0;
   plan.batch = p.batch;
   plan.src_pixels = static_cast<size_t>(p.batch) * g.src_rows * g.src_cols;
-  plan.widen = g.channels % 8 != 0;
-  if (plan.widen) plan.wide_halves = plan.src_pixels * g.cp * 8;
+  plan.widen = g.channels % kE != 0;
+  if (plan.widen) plan.wide_bytes = plan.src_pixels * g.cp * 16;
+  plan.out_elems = static_cast<size_t>(p.batch) * g.out_rows * g.out_cols *
+                   (grad ? p.channels : p.features);
   if (plan.src_pixels * g.cp * 16 > kMaxBufferBytes ||
-      static_cast<size_t>(p.batch) * g.out_rows * g.out_cols * g.features * 2 >
-          kMaxBufferBytes)
+      plan.out_elems * sizeof(T) > kMaxBufferBytes)
     return plan;
   g.n_classes = 0;
   if (!grad) {
@@ -702,6 +914,28 @@ GatherPlan compute_plan(int direction, const snn_hip_conv2d_params& p) {
     c.win_r = p.window_rows; c.win_c = p.window_cols;
     c.out_r0 = 0; c.out_c0 = 0;
     c.tap_r0 = 0; c.tap_rs = 1; c.tap_c0 = 0; c.tap_cs = 1;
+  } else if (g.merged != 0) {
+    // A block's pixels are first + stride * i + 0 ... stride - 1 along an axis,
+    // with padded coordinates stride * (b + i) + 0 ...; tap t of the shared
+    // window is source position b + i - (taps - 1) + t and, for member a, filter
+    // tap a + stride * (taps - 1 - t).
+    auto axis = [](int in, int window, int stride, int pad, int* count,
+                   int* first, int* taps, int* off) {
+      const int b = pad / stride;
+      *first = b * stride - pad;
+      *count = (in - 1 + pad) / stride - b + 1;
+      *taps = (window + stride - 1) / stride;
+      *off = b - (*taps - 1);
+    };
+    GatherClass& c = g.cls[g.n_classes++];
+    axis(p.in_rows, p.window_rows, p.stride_rows, p.pad_rows, &c.rows,
+         &c.out_r0, &c.win_r, &c.off_r);
+    axis(p.in_cols, p.window_cols, p.stride_cols, p.pad_cols, &c.cols,
+         &c.out_c0, &c.win_c, &c.off_c);
+    c.tap_r0 = p.stride_rows * (c.win_r - 1);
+    c.tap_c0 = p.stride_cols * (c.win_c - 1);
+    c.tap_rs = -p.stride_rows;
+    c.tap_cs = -p.stride_cols;
   } else {
     // One axis of a class: input positions first, first + stride, ... are
     // reached by taps a, a + stride, ... at source position
@@ -741,19 +975,26 @@ GatherPlan compute_plan(int direction, const snn_hip_conv2d_params& p) {
   }
   plan.filter_elems = static_cast<size_t>(p.window_rows) * p.window_cols *
                       p.channels * p.features;
-  plan.in_place = grad && !plan.widen && plan.filter_elems * 2 <= kMaxBufferBytes / 2;
-  plan.out_elems =
-      static_cast<size_t>(p.batch) * g.out_rows * g.out_cols * g.features;
-  choose_tile(&plan);
+  if (!plan.widen && g.merged == 0 &&
+      plan.filter_elems * sizeof(T) <= kMaxBufferBytes / 2) {
+    if (grad)
+      plan.from = kInPlace;
+    else if (sizeof(T) == 4 && p.features % 4 == 0)
+      plan.from = kRows;
+  }
+  choose_tile<T>(&plan, may_split);
   plan.ok = plan.pack_blocks * 2048 <= kMaxBufferBytes / 2 && g.n_classes > 0;
   return plan;
 }
 
 // The plan of the most recent shape is kept per thread: layers are usually
 // launched many times with the same parameters.
-const GatherPlan& make_plan(int direction, const snn_hip_conv2d_params& p) {
+template <typename T>
+const GatherPlan& make_plan(int direction, const snn_hip_conv2d_params& p,
+                            bool may_split = true) {
   struct Cached {
     int direction = -1;
+    bool may_split = false;
     snn_hip_conv2d_params params;
     GatherPlan plan;
   };
@@ -762,110 +1003,140 @@ const GatherPlan& make_plan(int direction, const snn_hip_conv2d_params& p) {
 #ifdef SNN_HIP_TUNING
   c.direction = -1;
 #endif
-  if (c.direction != direction || std::memcmp(&c.params, &p, sizeof(p)) != 0) {
-    c.plan = compute_plan(direction, p);
+  if (c.direction != direction || c.may_split != may_split ||
+      std::memcmp(&c.params, &p, sizeof(p)) != 0) {
+    c.plan = compute_plan<T>(direction, p, may_split);
     c.params = p;
+    c.may_split = may_split;
     c.direction = direction;
   }
   return c.plan;
 }
 
-template <int WM, int WN, int TM, int TN>
-void launch_tile(const _Float16* src, const _Float16* wpk, _Float16* dst,
-                 float* part, const GatherPlan& plan, bool in_place,
-                 hipStream_t stream) {
+// A launch's operands: the source as whole pieces, the filter as `from` says.
+template <typename T>
+struct GatherOperands {
+  const T* src;
+  const T* filter;
+  const float* bias;
+  T* dst;
+  float* part;
+  FilterFrom from;
+};
+
+template <typename T, int WM, int WN, int TM, int TN, bool UNIFORM, int FROM>
+void launch_kernel(const GatherOperands<T>& ops, const GatherPlan& plan,
+                   const Gather& g, hipStream_t stream) {
+  const unsigned n_groups = g.n_tiles * static_cast<unsigned>(g.n_splits);
+  const unsigned src_bytes = static_cast<unsigned>(plan.src_pixels * g.cp * 16);
+  const unsigned filter_bytes = static_cast<unsigned>(
+      FROM == kPacked ? plan.pack_blocks * 2048
+                      : plan.filter_elems * sizeof(T));
+  const unsigned dst_bytes = static_cast<unsigned>(plan.out_elems * sizeof(T));
+  KernelTimer timer(stream);
+  hipLaunchKernelGGL((conv_gather_kernel<T, WM, WN, TM, TN, UNIFORM, FROM>),
+                     dim3(n_groups), dim3(64 * WM * WN), 0, stream, ops.src,
+                     ops.filter, ops.bias, ops.dst, ops.part, g, src_bytes,
+                     filter_bytes, dst_bytes, n_groups);
+}
+
+template <typename T, int WM, int WN, int TM, int TN>
+void launch_tile(const GatherOperands<T>& ops, const GatherPlan& plan,
+                 bool relu, hipStream_t stream) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
   Gather g = plan.g;
+  g.relu = relu;
   g.n_tiles_n = ceil_div(g.features, BN);
   int pixels = 0;
   for (int k = 0; k < g.n_classes; ++k)
     pixels = std::max(pixels, g.cls[k].pixels);
-  const unsigned n_tiles = static_cast<unsigned>(ceil_div(pixels, BM)) *
-                           static_cast<unsigned>(g.n_classes * g.n_tiles_n);
-  g.n_tiles = n_tiles;
+  g.n_tiles = static_cast<unsigned>(ceil_div(pixels, BM)) *
+              static_cast<unsigned>(g.n_classes * g.n_tiles_n);
   g.n_splits = plan.n_splits;
-  const unsigned n_groups = n_tiles * static_cast<unsigned>(g.n_splits);
-  const unsigned src_bytes = static_cast<unsigned>(plan.src_pixels * g.cp * 16);
-  const unsigned wpk_bytes = static_cast<unsigned>(
-      in_place ? plan.filter_elems * 2 : plan.pack_blocks * 2048);
-  const unsigned dst_bytes = static_cast<unsigned>(plan.out_elems * 2);
-  {
-    KernelTimer timer(stream);
-    if (in_place && g.cp % 4 == 0)
-      hipLaunchKernelGGL((conv_gather_f16_kernel<WM, WN, TM, TN, true, true>),
-                         dim3(n_groups), dim3(64 * WM * WN), 0, stream, src,
-                         wpk, dst, part, g, src_bytes, wpk_bytes, dst_bytes,
-                         n_groups);
-    else if (in_place)
-      hipLaunchKernelGGL((conv_gather_f16_kernel<WM, WN, TM, TN, false, true>),
-                         dim3(n_groups), dim3(64 * WM * WN), 0, stream, src,
-                         wpk, dst, part, g, src_bytes, wpk_bytes, dst_bytes,
-                         n_groups);
-    else if (g.cp % 4 == 0)
-      hipLaunchKernelGGL((conv_gather_f16_kernel<WM, WN, TM, TN, true, false>),
-                         dim3(n_groups), dim3(64 * WM * WN), 0, stream, src,
-                         wpk, dst, part, g, src_bytes, wpk_bytes, dst_bytes,
-                         n_groups);
+  if constexpr (sizeof(T) == 4) {
+    if (ops.from == kInPlace)
+      launch_kernel<T, WM, WN, TM, TN, false, kInPlace>(ops, plan, g, stream);
+    else if (ops.from == kRows)
+      launch_kernel<T, WM, WN, TM, TN, false, kRows>(ops, plan, g, stream);
     else
-      hipLaunchKernelGGL((conv_gather_f16_kernel<WM, WN, TM, TN, false, false>),
-                         dim3(n_groups), dim3(64 * WM * WN), 0, stream, src,
-                         wpk, dst, part, g, src_bytes, wpk_bytes, dst_bytes,
-                         n_groups);
+      launch_kernel<T, WM, WN, TM, TN, false, kPacked>(ops, plan, g, stream);
+  } else {
+    const bool uniform = g.cp % 4 == 0;
+    if (ops.from == kInPlace && uniform)
+      launch_kernel<T, WM, WN, TM, TN, true, kInPlace>(ops, plan, g, stream);
+    else if (ops.from == kInPlace)
+      launch_kernel<T, WM, WN, TM, TN, false, kInPlace>(ops, plan, g, stream);
+    else if (uniform)
+      launch_kernel<T, WM, WN, TM, TN, true, kPacked>(ops, plan, g, stream);
+    else
+      launch_kernel<T, WM, WN, TM, TN, false, kPacked>(ops, plan, g, stream);
   }
   if (g.n_splits > 1)
-    hipLaunchKernelGGL((gather_reduce_kernel<WM, WN, TM, TN>),
-                       dim3(n_tiles * (BM * BN / 1024)), dim3(256), 0, stream,
-                       reinterpret_cast<const float4v*>(part), dst, g);
+    hipLaunchKernelGGL((gather_reduce_kernel<T, WM, WN, TM, TN>),
+                       dim3(g.n_tiles * (BM * BN / 1024)), dim3(256), 0, stream,
+                       reinterpret_cast<const float4v*>(ops.part), ops.bias,
+                       ops.dst, g);
 }
 
 // Returns -1 when there is no room for its temporaries.
-int launch_gather(const GatherPlan& plan, const _Float16* input,
-                  const _Float16* filter, _Float16* output,
-                  _Float16* workspace, size_t workspace_elems,
-                  hipStream_t stream) {
+template <typename T>
+int launch_gather(const GatherPlan& plan, const T* input, const T* filter,
+                  T* output, T* workspace, size_t workspace_elems,
+                  const float* bias, bool relu, hipStream_t stream) {
   const Gather& g = plan.g;
-  const bool in_place =
-      plan.in_place && (reinterpret_cast<uintptr_t>(filter) & 15u) == 0;
-  const size_t need = plan.workspace_halves(!in_place);
-  _Float16* packed = workspace;
+  const FilterFrom from =
+      (reinterpret_cast<uintptr_t>(filter) & 15u) == 0 ? plan.from : kPacked;
+  const size_t need = plan.workspace_bytes(from == kPacked);
+  char* packed = reinterpret_cast<char*>(workspace);
   const bool temporary =
-      need != 0 && (workspace == nullptr || workspace_elems < need ||
-                    (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0);
+      need != 0 &&
+      (workspace == nullptr || workspace_elems < ceil_div(need, sizeof(T)) ||
+       (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0);
   if (temporary) {
     void* ptr = nullptr;
-    if (temp_malloc_async(&ptr, need * sizeof(_Float16), stream) !=
-        hipSuccess) {
+    if (temp_malloc_async(&ptr, need, stream) != hipSuccess) {
       (void)hipGetLastError();
       return -1;
     }
-    packed = static_cast<_Float16*>(ptr);
+    packed = static_cast<char*>(ptr);
   }
   // (every part is a multiple of 16 bytes)
-  const size_t pack_blocks = in_place ? 0 : plan.pack_blocks;
-  _Float16* const wide = packed + pack_blocks * 1024;
-  float* const part = reinterpret_cast<float*>(wide + plan.wide_halves);
+  const size_t pack_blocks = from == kPacked ? plan.pack_blocks : 0;
+  T* const wide = reinterpret_cast<T*>(packed + pack_blocks * 2048);
   const unsigned pack_lanes = static_cast<unsigned>(pack_blocks * 128);
   const unsigned pack_groups = ceil_div(pack_lanes, 256u);
   const unsigned pieces =
       plan.widen ? static_cast<unsigned>(plan.src_pixels * g.cp) : 0u;
   const unsigned groups = pack_groups + ceil_div(pieces, 256u);
   if (groups > 0)
-    hipLaunchKernelGGL(gather_prepare_kernel, dim3(groups), dim3(256), 0,
-                       stream, filter, packed, g, pack_lanes, pack_groups,
-                       input, wide, pieces);
-  const _Float16* const src = plan.widen ? wide : input;
-  const _Float16* const weights = in_place ? filter : packed;
-  switch (plan.tile) {
-    case 0: launch_tile<2, 2, 4, 2>(src, weights, output, part, plan, in_place, stream); break;
-    case 1: launch_tile<4, 1, 2, 2>(src, weights, output, part, plan, in_place, stream); break;
-    case 2: launch_tile<2, 2, 2, 2>(src, weights, output, part, plan, in_place, stream); break;
-    case 3: launch_tile<2, 2, 2, 1>(src, weights, output, part, plan, in_place, stream); break;
-    case 4: launch_tile<4, 1, 1, 1>(src, weights, output, part, plan, in_place, stream); break;
-    default: launch_tile<2, 2, 1, 1>(src, weights, output, part, plan, in_place, stream);
+    hipLaunchKernelGGL(gather_prepare_kernel<T>, dim3(groups), dim3(256), 0,
+                       stream, filter, reinterpret_cast<T*>(packed), g,
+                       pack_lanes, pack_groups, input, wide, pieces);
+  const GatherOperands<T> ops = {
+      plan.widen ? wide : input,
+      from == kPacked ? reinterpret_cast<const T*>(packed) : filter,
+      bias,
+      output,
+      reinterpret_cast<float*>(packed + pack_blocks * 2048 + plan.wide_bytes),
+      from};
+  if constexpr (sizeof(T) == 4) {
+    if (plan.tile == 0)
+      launch_tile<T, 4, 1, 1, 1>(ops, plan, relu, stream);
+    else
+      launch_tile<T, 2, 2, 1, 1>(ops, plan, relu, stream);
+  } else {
+    switch (plan.tile) {
+      case 0: launch_tile<T, 2, 2, 4, 2>(ops, plan, relu, stream); break;
+      case 1: launch_tile<T, 4, 1, 2, 2>(ops, plan, relu, stream); break;
+      case 2: launch_tile<T, 2, 2, 2, 2>(ops, plan, relu, stream); break;
+      case 3: launch_tile<T, 2, 2, 2, 1>(ops, plan, relu, stream); break;
+      case 4: launch_tile<T, 4, 1, 1, 1>(ops, plan, relu, stream); break;
+      default: launch_tile<T, 2, 2, 1, 1>(ops, plan, relu, stream);
+    }
   }
   const hipError_t err = hipGetLastError();
   if (temporary) temp_free_async(packed, stream);
-  if (err != hipSuccess) return report_hip_error(err, "conv_gather_f16_kernel");
+  if (err != hipSuccess) return report_hip_error(err, "conv_gather_kernel");
   return SNN_HIP_OK;
 }
 
@@ -939,10 +1210,10 @@ size_t conv2d_f16_workspace_halves(int direction,
   // (with room for the packed filter also where the gradient's is read in
   // place, for one that is not 16-byte aligned; that of a 1x1 layer would take
   // a temporary)
-  const GatherPlan& plan = make_plan(direction, p);
+  const GatherPlan& plan = make_plan<_Float16>(direction, p);
   const bool packs =
-      !plan.in_place || p.window_rows > 1 || p.window_cols > 1;
-  return plan.ok ? plan.workspace_halves(packs) : 0;
+      plan.from == kPacked || p.window_rows > 1 || p.window_cols > 1;
+  return plan.ok ? plan.workspace_bytes(packs) / 2 : 0;
 }
 
 int launch_conv2d_f16(int direction, const _Float16* input,
@@ -982,10 +1253,128 @@ int launch_conv2d_f16(int direction, const _Float16* input,
     return status;
   }
   if (is_tiny(direction, p)) return -1;
-  const GatherPlan& plan = make_plan(direction, p);
+  const GatherPlan& plan = make_plan<_Float16>(direction, p);
   if (!plan.ok || (!plan.widen && !aligned(input))) return -1;
-  return launch_gather(plan, input, filter, output, workspace, workspace_elems,
-                       stream);
+  return launch_gather<_Float16>(plan, input, filter, output, workspace,
+                                 workspace_elems, nullptr, false, stream);
+}
+
+// Where the gathering kernel is faster than the other fp32 kernels behind the
+// Tiled / Im2col / Matmul tags (times: there / here).
+bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
+  if (direction == SNN_HIP_FILTER_BACKPROP) return false;
+#ifdef SNN_HIP_TUNING
+  if (const char* env = std::getenv("SNN_HIP_GATHER_F32"))
+    if (env[0] == '0' || env[0] == '1') return env[0] == '1';
+#endif
+  const bool grad = direction == SNN_HIP_INPUT_BACKPROP;
+  const bool strided = p.stride_rows > 1 || p.stride_cols > 1;
+  const long long products = static_cast<long long>(p.window_rows) *
+                             p.window_cols * (grad ? p.features : p.channels);
+  const double macs = static_cast<double>(p.batch) * p.out_rows * p.out_cols *
+                      p.window_rows * p.window_cols * p.channels * p.features;
+  const double outputs =
+      grad ? static_cast<double>(p.batch) * p.in_rows * p.in_cols * p.channels
+           : static_cast<double>(p.batch) * p.out_rows * p.out_cols * p.features;
+  // One short loop per output (14x14x33 -> 64, 1x1: 5.3 / 17.8 us).
+  if (products <= 64 && outputs <= (1 << 16)) return false;
+  // Few outputs of a long reduction meet through atomics there, in one pass less
+  // (2x19x14 720 -> 80, 3x3 stride 2: 12.5 / 13.7 us; 4x14x14 144 -> 224, 5x5,
+  // 24 / 26 and its gradient 24 / 30; but 3x14x14 192 <- 128, 3x3, 12.7 / 12.0).
+  const bool whole = p.channels % 4 == 0 && p.features % 4 == 0;
+  if (whole && (!grad || !strided) &&
+      products >= (grad ? 2000 : 3000) && outputs < (1 << 18))
+    return false;
+  // 1x1, stride 1: plain products.  The kernels for these want reductions of
+  // whole chunks of 32, and tiles of 64 columns that are not mostly padding:
+  // 15x213x277 16 -> 84 120 / 101 us, its gradient 126 / 91; 3x201x151
+  // 288 -> 80 65 / 55; but 32x56x56 256 -> 64 33 / 41 and 32 / 47.
+  const bool plain = p.window_rows == 1 && p.window_cols == 1 && !strided &&
+                     p.pad_rows == 0 && p.pad_cols == 0 &&
+                     p.out_rows == p.in_rows && p.out_cols == p.in_cols;
+  const int reduced = grad ? p.features : p.channels;
+  const int columns = grad ? p.channels : p.features;
+  if (plain && p.features % 4 == 0 && reduced % 32 == 0) {
+    const int padded = (columns + 63) / 64 * 64;
+    return macs >= double(1 << 29) && 5 * (padded - columns) > padded;
+  }
+  if (!grad) {
+    if (p.features % 4 != 0) return true;  // nothing else but copies takes it
+    // The source is copied to whole pieces first: 5x14x10 166 -> 96, 3x3,
+    // 67 / 15 us; 18x168x218 3 -> 32, 7x7 stride 2, 48 / 37; but
+    // 8x224x224 3 -> 64, 3x3, 38 / 45 and 3x186x186 3 -> 48, 7x7, 13 / 15.
+    if (p.channels % 4 != 0)
+      return !conv2d_stem_supports(p) &&
+             (products >= 200 || (products >= 100 && macs >= double(1 << 29)));
+    // 27x27x96 -> 256, 5x5, at batch 17: 144 / 158 us on the rows-in-LDS
+    // kernel; where that does not apply 16x28x28 192 -> 96 146 / 115,
+    // 13x95x95 208 -> 28, 3x3, 280 / 140, 64x28x28 32 -> 32 60 / 35.
+    return !conv2d_small_supports(p) && !conv2d_rowtile_supports(p) &&
+           !conv2d_rowsplit_supports(p);
+  }
+  if (conv2d_stem_input_backprop_supports(p)) return false;
+  if (strided && p.channels <= 4)  // merged classes
+    // 37x104x104 3 <- 58, 7x7 stride 2, 1570 / 88 us, 7x111x144 3 <- 36, 3x3,
+    // 61 / 12; but 112x112 3 <- 32 at batch 1 8.6 / 11.7 (the filter's pack).
+    return macs >= double(1 << 23);
+  // (products of dY and the filter per output pixel, gathered: 8x224x224
+  // 3 <- 64, 3x3, 66 / 148 us; but 8x64x64 8 <- 32 15.6 / 10.4)
+  if (p.channels < 16 && p.features % 32 == 0) return macs < double(1 << 27);
+  // (16x28x28 192 <- 96, 5x5, 109 / 118 us and 48 <- 64, 7x7, 58 / 67 on tiles
+  // of 64 x 64, where those compute no more columns than tiles of 32 would)
+  if (!strided && p.features % 32 == 0 && (p.channels + 31) / 32 % 2 == 0 &&
+      macs >= double(1 << 30))
+    return false;
+  snn_hip_conv2d_params q;
+  if (as_forward_of_dy(p, &q) &&
+      (conv2d_rowtile_supports(q) || conv2d_rowsplit_supports(q)))
+    return false;
+  // 32x56x56 128 <- 128, 3x3 stride 2, 140 / 92 us; 256 <- 512, 1x1 stride 2,
+  // 95 / 90; 17x27x27 96 <- 256, 5x5, 178 / 160; 5x82x107 16 <- 75 129 / 68.
+  return true;
+}
+
+size_t conv2d_gather_f32_workspace_floats(int direction,
+                                          const snn_hip_conv2d_params& p) {
+  if (!positive(p) || !conv2d_gather_f32_wanted(direction, p)) return 0;
+  const GatherPlan& plan = make_plan<float>(direction, p);
+  return plan.ok ? plan.workspace_bytes(plan.from == kPacked) / 4 : 0;
+}
+
+int launch_conv2d_gather_f32(int direction, const float* input,
+                             const float* filter, float* output,
+                             const snn_hip_conv2d_params& p, float* workspace,
+                             size_t workspace_elems, hipStream_t stream,
+                             const LaunchOptions* epilogue) {
+  auto aligned = [](const void* ptr) {
+    return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0;
+  };
+  const GatherPlan* plan = &make_plan<float>(direction, p);
+  if (!plan->ok || !aligned(output) || (!plan->widen && !aligned(input)))
+    return -1;
+  // A stream that records a graph gives no temporaries: without them (the
+  // caller's workspace has no room either) the reduction stays whole, and what
+  // cannot do without is left to the kernels that need none.
+  const bool packs = plan->from == kPacked || !aligned(filter);
+  const size_t room =
+      workspace != nullptr && aligned(workspace) ? workspace_elems * 4 : 0;
+  if (plan->workspace_bytes(packs) > room) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess ||
+        status != hipStreamCaptureStatusNone) {
+      (void)hipGetLastError();
+      plan = &make_plan<float>(direction, p, false);
+      if (plan->workspace_bytes(packs) > room) return -1;
+    }
+  }
+  const bool fuse = direction == SNN_HIP_FORWARD && epilogue != nullptr &&
+                    epilogue->wanted();
+  const int rc = launch_gather<float>(
+      *plan, input, filter, output, workspace, workspace_elems,
+      fuse ? epilogue->bias : nullptr, fuse && epilogue->relu, stream);
+  if (rc == SNN_HIP_OK && fuse && epilogue->applied != nullptr)
+    *epilogue->applied = true;
+  return rc;
 }
 
 }  // namespace snn

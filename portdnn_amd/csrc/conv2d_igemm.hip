@@ -2390,7 +2390,8 @@ int launch_conv2d_igemm_f32(int direction, const float* input,
       p.channels % 4 == 0 && p.features % 4 == 0 &&
       static_cast<size_t>(p.batch) * p.out_rows * p.out_cols >= 1024 &&
       SNN_TUNING_ENV("SNN_HIP_STRIDED_1X1_OFF") == nullptr) {
-    // A strided 1x1 layer (a ResNet shortcut): only the input pixels at
+    // A strided 1x1 layer with more stride classes than the gathering kernel
+    // takes (strides from 5): only the input pixels at
     // multiples of the stride receive a gradient, and theirs is the stride-1
     // input gradient over the output pixels.  That product runs dense into a
     // stream-ordered temporary on the stride-1 kernels, and one pass writes
@@ -2436,6 +2437,8 @@ int launch_conv2d_igemm_f32(int direction, const float* input,
       static_cast<double>(p.batch) * p.out_rows * p.out_cols * p.window_rows *
               p.window_cols * p.channels * p.features >= double(1 << 30) &&
       SNN_TUNING_ENV("SNN_HIP_STRIDE_CLASSES_OFF") == nullptr) {
+    // Windows beyond the gathering kernel's 12 x 12, and few channels under
+    // features in multiples of 32.
     // The general strided kernel walks every tap for every input pixel and
     // multiplies zeros for those that do not reach it (3/4 of them at stride
     // 2: 56x56x128 -> 128, 3x3, at batch 32 343 us against 90 forward).  By

@@ -2,7 +2,7 @@
 // input tile resident in LDS: binary16 operands, fp32 accumulation, binary16
 // result.
 //
-// The gathering kernel in conv2d_gather_f16.hip loads every input pixel once
+// The gathering kernel in conv2d_gather.hip loads every input pixel once
 // per filter tap and passes both operands through LDS; at 32x32x16 f16 MFMA
 // rates that makes LDS and the loads the limit, not the matrix cores.  Here a work-group owns a run
 // of consecutive output pixels (images, rows and columns flattened, so a tile
@@ -665,7 +665,7 @@ bool launch_shape(const _Float16* input, const _Float16* wpk,
 
 }  // namespace
 
-// Where this kernel is faster than the gathering one (conv2d_gather_f16.hip,
+// Where this kernel is faster than the gathering one (conv2d_gather.hip,
 // which shares a reduction between work-groups where there are few tiles):
 // short reductions at every size, and long ones with at least 1.5 wave tiles
 // per SIMD that leave two waves on each.  Measured with 3x3 windows, this

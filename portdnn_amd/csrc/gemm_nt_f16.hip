@@ -6,7 +6,7 @@
 //
 // A work-group owns a BM x BN tile and walks the reduction in chunks of 64
 // halves -- one 128-byte line of every row, which is what these products, bound
-// by the bytes they move, want: the gathering kernel of conv2d_gather_f16.hip,
+// by the bytes they move, want: the gathering kernel of conv2d_gather.hip,
 // whose chunks are half a line, takes 58 us where this one takes 55.8
 // (401408x64x256, 257 MB) and 15.0 against 12.4 at a quarter of the rows.  Both
 // tiles pass through registers into two LDS stages; lane l supplies

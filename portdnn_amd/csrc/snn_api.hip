@@ -385,6 +385,14 @@ int workspace_size(const snn_hip_conv2d_params& p, int direction,
       conv2d_filter_backprop_direct_f32_wanted(p))
     *recommended = std::max(
         *recommended, conv2d_filter_backprop_direct_f32_partial_floats(p));
+  // The gathering kernel behind the same tags: its packed filter, widened source
+  // and partial tiles.
+  if (!filbk && p.input_format == 0 &&
+      (algorithm == SNN_HIP_ALGO_TILED || algorithm == SNN_HIP_ALGO_IM2COL ||
+       algorithm == SNN_HIP_ALGO_MATMUL) &&
+      algorithm_supports(p, direction, algorithm) == algorithm)
+    *recommended = std::max(*recommended,
+                            conv2d_gather_f32_workspace_floats(direction, p));
   return SNN_HIP_OK;
 }
 
@@ -669,6 +677,12 @@ int launch_gemm_path<float>(int direction, const float* input,
   const bool atomics_only = direction == SNN_HIP_FILTER_BACKPROP &&
                             epilogue != nullptr && epilogue->deterministic &&
                             !conv2d_filter_backprop_direct_f32_wanted(p, true);
+  if (conv2d_gather_f32_wanted(direction, p)) {
+    const int rc =
+        launch_conv2d_gather_f32(direction, input, filter, output, p, workspace,
+                                 workspace_elems, s, epilogue);
+    if (rc >= 0) return rc;
+  }
   if ((direction == SNN_HIP_FORWARD && aligned16(input)) ||
       (direction == SNN_HIP_INPUT_BACKPROP && aligned16(output))) {
     const int padded = launch_gemm_path_padded<float>(

@@ -224,7 +224,7 @@ int launch_gemm_nt_f16(const _Float16* x, const _Float16* w, _Float16* y, int m,
                        int k, int n, hipStream_t stream);
 
 // Half-precision forward convolution and input gradient on the binary16 matrix
-// cores (conv2d_gather_f16.hip): stride-1 unpadded 1x1 layers on the row-major
+// cores (conv2d_gather.hip): stride-1 unpadded 1x1 layers on the row-major
 // GEMM kernels above, stride-1 layers that fill the GPU on the LDS-tile kernel, every
 // other window (up to 12 x 12), stride (input gradient: up to 16 classes) and
 // channel count on the gathering kernel.  The launch returns -1 when none takes
@@ -236,6 +236,20 @@ int launch_conv2d_f16(int direction, const _Float16* input,
                       const _Float16* filter, _Float16* output,
                       const snn_hip_conv2d_params& p, _Float16* workspace,
                       size_t workspace_elems, hipStream_t stream);
+
+// Forward convolution (with bias and activation, if asked for) and input
+// gradient in fp32 on the same gathering kernel: every window, stride, channel
+// and feature count.  Needs a temporary (or `workspace`, in floats) where the
+// reduction is shared, the channels of the source are no multiple of 4, or a
+// forward filter's features are not; returns -1 where it does not apply.
+int launch_conv2d_gather_f32(int direction, const float* input,
+                             const float* filter, float* output,
+                             const snn_hip_conv2d_params& p, float* workspace,
+                             size_t workspace_elems, hipStream_t stream,
+                             const LaunchOptions* epilogue);
+bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p);
+size_t conv2d_gather_f32_workspace_floats(int direction,
+                                          const snn_hip_conv2d_params& p);
 
 // Half-precision filter gradient on the fp32 matrix instructions
 // (conv2d_igemm.hip) for channel counts in multiples of 64: fp32 accumulation
