@@ -51,6 +51,7 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <type_traits>
 
 #include "gemm_tile.h"
 #include "snn_kernels.h"
@@ -131,6 +132,9 @@ struct Gather {
   int mirrored;          // input gradient: w[tap][feature][channel]
   int merged;            // channels per pixel of merged classes, or 0
   int relu;              // of a forward launch with bias and activation
+  // A copy to whole pieces that takes every copy_step'th pixel of an image of
+  // copy_rows x copy_cols (0: all pixels).
+  int copy_rows, copy_cols, copy_step_r, copy_step_c;
   GatherClass cls[kMaxClasses];
 };
 
@@ -255,7 +259,13 @@ __global__ void __launch_bounds__(256)
   if (idx >= n_pieces) return;
   const unsigned pixel = divide(idx, g.by_cp);
   const int c = static_cast<int>(idx - pixel * g.cp) * kE;
-  const T* from = src + static_cast<size_t>(pixel) * g.channels + c;
+  size_t from_pixel = pixel;
+  if (g.copy_rows != 0) {  // (the copy's pixels are the output's)
+    const Pixel px = pixel_of(static_cast<int>(pixel), g.cls[0]);
+    from_pixel = (static_cast<size_t>(px.n) * g.copy_rows +
+                  px.y * g.copy_step_r) * g.copy_cols + px.x * g.copy_step_c;
+  }
+  const T* from = src + from_pixel * g.channels + c;
 #pragma unroll
   for (int e = 0; e < kE; ++e)
     v[e] = c + e < g.channels ? from[e] : static_cast<T>(0.f);
@@ -607,6 +617,81 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
         }
     }
   }
+  // Features that fill no whole 16-byte pieces (fp32: four, binary16: eight) go
+  // out through LDS, block by block, as rows of 32 consecutive features: one
+  // store instruction covers two to eight pixels' runs instead of 2 or 4 bytes of
+  // 64 pixels each (83x23x23x64 -> 391, 3x3, binary16:
+  // 96 -> 47 us; 32x28x28x128 -> 131, 3x3, fp32: 96 -> 92).  Word
+  // w of pixel row r lies at w XOR (bits of r), which keeps both the writes of 32
+  // rows and the reads along a row off each other's banks.
+  const bool by_rows = (g.features & (kPiece<T> - 1)) != 0;
+  constexpr int kOutRow = 32 * kSize;
+  constexpr int kBlocksPerBuf = STAGE / (32 * kOutRow);
+  static_assert(2 * kBlocksPerBuf >= WM * WN,
+                "a block of every wave in two buffers of the reduction");
+  char* const out_stage =
+      wave < kBlocksPerBuf
+          ? buf0 + wave * (32 * kOutRow)
+          : buf1 + (wave - kBlocksPerBuf) * (32 * kOutRow);
+  auto word_at = [&](int row, int word) {
+    const int bits = kSize == 4 ? row : row >> 1;
+    return reinterpret_cast<unsigned*>(out_stage + row * kOutRow +
+                                       (word ^ bits) * 4);
+  };
+  if (by_rows) __syncthreads();  // every wave is done with the last chunk
+  // UNIT: bytes per lane.
+  auto store_rows = [&](int n, unsigned at_mine, auto unit) {
+    constexpr int UNIT = decltype(unit)::value;
+    constexpr int PER_PIXEL = 32 * kSize / UNIT, PIXELS = 64 / PER_PIXEL;
+    const int at_lane = lane % PER_PIXEL * UNIT;
+    const int f = n + at_lane / kSize;
+#pragma unroll 2
+    for (int it = 0; it < 32 / PIXELS; ++it) {
+      const int row = it * PIXELS + lane / PER_PIXEL;
+      const unsigned at = static_cast<unsigned>(
+          __shfl(static_cast<int>(at_mine), row));
+      const unsigned* const word = word_at(row, at_lane / 4);
+      const unsigned off = f < g.features && at != kOob
+                               ? at + static_cast<unsigned>(f) * kSize : kOob;
+      if constexpr (UNIT == 2) {
+        __builtin_amdgcn_raw_buffer_store_b16(
+            static_cast<unsigned short>(*word >> (at_lane % 4 * 8)), dst_rsrc,
+            off, 0, 0);
+      } else if constexpr (UNIT == 4) {
+        __builtin_amdgcn_raw_buffer_store_b32(
+            *word, dst_rsrc, off, 0, 0);
+      } else {
+        const uint2v two = {*word, *word_at(row, at_lane / 4 + 1)};
+        __builtin_amdgcn_raw_buffer_store_b64(two, dst_rsrc, off, 0, 0);
+      }
+    }
+  };
+  // 32-bit words of a block's 16 values of this lane.
+  constexpr int kWords = 4 * kSize;
+  auto words_of = [&](const float16v& sums, unsigned (&words)[kWords]) {
+    if constexpr (kSize == 4) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const float value = sums[v];
+        words[v] = __builtin_bit_cast(unsigned, value);
+      }
+    } else {
+      half8 lo, hi;
+#pragma unroll
+      for (int v = 0; v < 8; ++v) {
+        lo[v] = static_cast<_Float16>(sums[v]);
+        hi[v] = static_cast<_Float16>(sums[8 + v]);
+      }
+      const uint4v w0 = __builtin_bit_cast(uint4v, lo);
+      const uint4v w1 = __builtin_bit_cast(uint4v, hi);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        words[v] = w0[v];
+        words[4 + v] = w1[v];
+      }
+    }
+  };
+  constexpr int kHalf = kWords / 2;  // words 0 ... kHalf - 1: features f0 ... + 7
 #pragma unroll
   for (int j = 0; j < TM; ++j) {
     const int m = m0 + (wm * TM + j) * 32 + l32;
@@ -616,67 +701,50 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
     const unsigned at =
         static_cast<unsigned>(((px.n * g.out_rows + out_y) * g.out_cols + out_x) *
                               g.features) * kSize;
+    if (by_rows) {
+      const unsigned at_mine = m < cls.pixels ? at : kOob;
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        unsigned words[kWords];
+        words_of(acc[i][j], words);
+#pragma unroll
+        for (int v = 0; v < kWords; ++v)
+          *word_at(l32, kHalf * khalf + v + v / kHalf * kHalf) = words[v];
+        // (LDS operations of a wave are done in order)
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const int n = n0 + (wn * TN + i) * 32;
+        if constexpr (kSize == 4) {
+          store_rows(n, at_mine, std::integral_constant<int, 4>{});
+        } else {
+          if ((g.features & 1) != 0)
+            store_rows(n, at_mine, std::integral_constant<int, 2>{});
+          else if ((g.features & 3) != 0)
+            store_rows(n, at_mine, std::integral_constant<int, 4>{});
+          else
+            store_rows(n, at_mine, std::integral_constant<int, 8>{});
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+      continue;
+    }
 #pragma unroll
     for (int i = 0; i < TN; ++i) {
       const int f0 = n0 + (wn * TN + i) * 32 + 8 * khalf;
       const int count = m < cls.pixels ? g.features - f0 : 0;
       const unsigned off = at + static_cast<unsigned>(f0) * kSize;
-      if constexpr (kSize == 4) {
-        if ((g.features & 3) == 0) {
+      unsigned words[kWords];
+      words_of(acc[i][j], words);
 #pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const float4v four = {acc[i][j][4 * v], acc[i][j][4 * v + 1],
-                                  acc[i][j][4 * v + 2], acc[i][j][4 * v + 3]};
-            __builtin_amdgcn_raw_buffer_store_b128(
-                __builtin_bit_cast(uint4v, four), dst_rsrc,
-                count > 4 * v + v / 2 * 8 ? off + 16u * v + v / 2 * 32u : kOob,
-                0, 0);
-          }
-        } else {
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const float value = acc[i][j][v];
-            __builtin_amdgcn_raw_buffer_store_b32(
-                __builtin_bit_cast(unsigned, value), dst_rsrc,
-                count > v + v / 8 * 8 ? off + 4u * v + v / 8 * 32u : kOob, 0,
-                0);
-          }
-        }
-      } else {
-        half8 lo, hi;
-#pragma unroll
-        for (int v = 0; v < 8; ++v) {
-          lo[v] = static_cast<_Float16>(acc[i][j][v]);
-          hi[v] = static_cast<_Float16>(acc[i][j][8 + v]);
-        }
-        const uint4v w0 = __builtin_bit_cast(uint4v, lo);
-        const uint4v w1 = __builtin_bit_cast(uint4v, hi);
-        if ((g.features & 7) == 0) {
-          __builtin_amdgcn_raw_buffer_store_b128(w0, dst_rsrc,
-                                                 count > 0 ? off : kOob, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b128(
-              w1, dst_rsrc, count > 16 ? off + 32u : kOob, 0, 0);
-        } else if ((g.features & 3) == 0) {
-          const unsigned words[8] = {w0[0], w0[1], w0[2], w0[3],
-                                     w1[0], w1[1], w1[2], w1[3]};
-#pragma unroll
-          for (int v = 0; v < 4; ++v) {
-            const uint2v two = {words[2 * v], words[2 * v + 1]};
-            __builtin_amdgcn_raw_buffer_store_b64(
-                two, dst_rsrc,
-                count > 4 * v + v / 2 * 8 ? off + 8u * v + v / 2 * 16u : kOob,
-                0, 0);
-          }
-        } else {
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            const _Float16 h = v < 8 ? lo[v] : hi[v - 8];
-            __builtin_amdgcn_raw_buffer_store_b16(
-                __builtin_bit_cast(unsigned short, h), dst_rsrc,
-                count > v + v / 8 * 8 ? off + 2u * v + v / 8 * 16u : kOob, 0,
-                0);
-          }
-        }
+      for (int v = 0; v < kWords / 4; ++v) {
+        const int first = kPiece<T> * v + v * 4 / kHalf * 8;
+        const uint4v four = {words[4 * v], words[4 * v + 1], words[4 * v + 2],
+                             words[4 * v + 3]};
+        __builtin_amdgcn_raw_buffer_store_b128(
+            four, dst_rsrc, count > first ? off + first * kSize : kOob, 0, 0);
       }
     }
   }
@@ -897,6 +965,21 @@ GatherPlan compute_plan(int direction, const snn_hip_conv2d_params& p,
                  ? p.channels : 0;
   if (g.merged != 0) g.features = p.channels * strides;
   g.relu = 0;
+  // A strided 1x1 window sees one pixel of stride x stride: only those are
+  // copied (64x57x57 255 -> 63, stride 2, binary16: 70 -> 30 us).
+  g.copy_rows = g.copy_cols = 0;
+  if (!grad && g.channels % kE != 0 && strides > 1 && p.window_rows == 1 &&
+      p.window_cols == 1 && p.pad_rows == 0 && p.pad_cols == 0 &&
+      (p.out_rows - 1LL) * p.stride_rows < p.in_rows &&
+      (p.out_cols - 1LL) * p.stride_cols < p.in_cols) {
+    g.copy_rows = p.in_rows;
+    g.copy_cols = p.in_cols;
+    g.copy_step_r = p.stride_rows;
+    g.copy_step_c = p.stride_cols;
+    g.src_rows = p.out_rows;
+    g.src_cols = p.out_cols;
+    g.step_r = g.step_c = 1;
+  }
   plan.batch = p.batch;
   plan.src_pixels = static_cast<size_t>(p.batch) * g.src_rows * g.src_cols;
   plan.widen = g.channels % kE != 0;
@@ -1303,6 +1386,12 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
     // The source is copied to whole pieces first: 5x14x10 166 -> 96, 3x3,
     // 67 / 15 us; 18x168x218 3 -> 32, 7x7 stride 2, 48 / 37; but
     // 8x224x224 3 -> 64, 3x3, 38 / 45 and 3x186x186 3 -> 48, 7x7, 13 / 15.
+    // A 1x1 window reads no more than the copy does: 25x43x43 454 -> 176 123 /
+    // 115 us, but 8x56x56 257 -> 64 21 / 30, 14x156x156 922 -> 32, stride 2,
+    // 151 / 205.
+    if (p.channels % 4 != 0 && p.window_rows == 1 && p.window_cols == 1 &&
+        p.features <= 128)
+      return false;
     if (p.channels % 4 != 0)
       return !conv2d_stem_supports(p) &&
              (products >= 200 || (products >= 100 && macs >= double(1 << 29)));

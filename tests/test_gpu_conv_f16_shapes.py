@@ -32,8 +32,8 @@ def assert_rounded_once(got, ref, n_products, what):
 SHAPES = [
     (2, 9, 7, 8, 8, 1, 1, True),        # the smallest pieces
     (1, 13, 11, 20, 30, 3, 2, True),    # no multiples of 8; nothing full
-    (3, 10, 13, 35, 45, 5, 1, False),   # odd counts: widened, 2-byte stores
-    (2, 17, 16, 36, 68, 3, 1, True),    # multiples of 4: 8-byte stores
+    (3, 10, 13, 35, 45, 5, 1, False),   # odd counts: widened, 2-byte runs
+    (2, 17, 16, 36, 68, 3, 1, True),    # multiples of 4: 8-byte runs
     (2, 12, 15, 24, 40, 3, 3, True),    # nine classes
     (2, 15, 14, 40, 24, 2, 3, False),   # classes that no tap reaches
     (2, 16, 16, 64, 136, 1, 2, True),   # 1x1 strided: three empty classes
@@ -46,6 +46,9 @@ SHAPES = [
     (5, 9, 9, 264, 264, 3, 2, True),    # ... by classes of unequal length
     (9, 57, 43, 72, 96, 3, 2, True),    # many tiles, ragged rows
     (16, 40, 40, 64, 200, 3, 2, True),  # tiles of 256 pixels
+    (3, 21, 22, 35, 45, 1, 2, True),    # strided 1x1, odd: copied subsampled
+    (2, 17, 19, 30, 66, 1, 3, False),   # ... even counts, VALID
+    (20, 20, 21, 64, 203, 3, 1, True),  # many tiles, runs of odd features
 ]
 
 

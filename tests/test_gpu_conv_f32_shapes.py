@@ -22,7 +22,7 @@ pytestmark = pytest.mark.gpu
 SHAPES = [
     (2, 9, 7, 8, 8, 3, 1, True),        # the smallest pieces
     (1, 13, 11, 20, 30, 3, 2, True),    # features of no whole piece
-    (3, 10, 13, 35, 45, 5, 1, False),   # odd counts: widened, 4-byte stores
+    (3, 10, 13, 35, 45, 5, 1, False),   # odd counts: widened, 4-byte runs
     (2, 12, 15, 24, 40, 3, 3, True),    # nine classes
     (2, 15, 14, 40, 24, 2, 3, False),   # classes that no tap reaches
     (2, 16, 16, 64, 136, 1, 2, True),   # 1x1 strided: three empty classes
@@ -39,6 +39,9 @@ SHAPES = [
     (31, 50, 64, 1, 200, 5, 3, True),   # ... nine classes of one channel
     (20, 60, 60, 2, 40, 6, 4, True),    # ... sixteen of two
     (60, 45, 44, 4, 68, 2, 2, True),    # ... one tap per class
+    (3, 21, 22, 35, 45, 1, 2, True),    # strided 1x1, odd: copied subsampled
+    (2, 17, 19, 30, 66, 1, 3, False),   # ... even counts, VALID
+    (20, 20, 21, 64, 203, 3, 1, True),  # many tiles, runs of odd features
 ]
 
 
