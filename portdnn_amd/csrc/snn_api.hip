@@ -303,6 +303,85 @@ void im2col_workspace(const snn_hip_conv2d_params& p, int direction,
   *recommended = static_cast<size_t>(p.batch) * in_t + filter_t;
 }
 
+// Filter gradients whose channel or feature counts are no multiples of 4 (of 8
+// for a binary16 first layer) on the kernels for those that are: X and dY are
+// copied with the counts rounded up (zeros in the new columns) and the gradient
+// is copied back without them.  The kernel that takes any count loads one value
+// per lane and step: in binary16 52 multiply-adds per ns on its 64 x 64 tiles,
+// where four at a time reach 280 (53x83x83 112 -> 139, 3x3: 1545 -> 440 us); in
+// fp32 both are bound by the matrix units at 47, but up to eight channels have a
+// kernel without the empty tiles (39x214x214 3 -> 50, 7x7 stride 2: 1772 ->
+// 191).  The copies move 3.5 TB/s; their three launches and a temporary cost
+// about 12 us.
+struct WidenedFilterGradient {
+  snn_hip_conv2d_params q;
+  // elements, each part a multiple of 16 bytes; 0 where no copy is needed
+  size_t x = 0, dy = 0, dw = 0, inner = 0;
+  size_t total() const { return x + dy + dw + inner; }
+};
+
+size_t f16_workspace_halves(const snn_hip_conv2d_params& p, int direction);
+
+bool widened_filter_gradient(const snn_hip_conv2d_params& p, size_t elem,
+                             WidenedFilterGradient* plan) {
+  if (p.input_format != 0 || p.batch <= 0 || p.in_rows <= 0 ||
+      p.in_cols <= 0 || p.out_rows <= 0 || p.out_cols <= 0 ||
+      p.window_rows <= 0 || p.window_cols <= 0 || p.channels <= 0 ||
+      p.features <= 0)
+    return false;
+  const bool half = elem == 2, few = p.channels <= 8;
+  snn_hip_conv2d_params& q = plan->q;
+  q = p;
+  auto up = [](int n, int to) { return (n + to - 1) / to * to; };
+  if (!few) q.channels = up(p.channels, 4);
+  q.features = up(p.features, 4);
+  if (half && few) {
+    snn_hip_conv2d_params eight = p;
+    eight.features = up(p.features, 8);
+    if (conv2d_few_f16_filter_backprop_partial_floats(eight) != 0) q = eight;
+  }
+  if (q.channels == p.channels && q.features == p.features) return false;
+  if (few ? p.window_rows * p.window_cols * p.channels > 768 : !half)
+    return false;
+  const size_t x_pixels = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols;
+  const size_t y_pixels =
+      static_cast<size_t>(p.batch) * p.out_rows * p.out_cols;
+  const size_t filter_rows =
+      static_cast<size_t>(p.window_rows) * p.window_cols * q.channels;
+  // (the copies count pieces of four in 32 bits)
+  if (x_pixels * q.channels >= (size_t{1} << 32) ||
+      y_pixels * q.features >= (size_t{1} << 32))
+    return false;
+  if (few ? !(half && conv2d_few_f16_filter_backprop_partial_floats(q) != 0) &&
+                !conv2d_igemm_supports(SNN_HIP_FILTER_BACKPROP, q)
+          : !conv2d_filter_backprop_f16_supports(q))
+    return false;
+  auto part = [](size_t n) { return (n + 127) / 128 * 128; };
+  plan->x = q.channels != p.channels ? part(x_pixels * q.channels) : 0;
+  plan->dy = q.features != p.features ? part(y_pixels * q.features) : 0;
+  plan->dw = part(filter_rows * q.features);
+  plan->inner =
+      half ? part(f16_workspace_halves(q, SNN_HIP_FILTER_BACKPROP)) : 0;
+  const double macs = static_cast<double>(y_pixels) * p.window_rows *
+                      p.window_cols * p.channels * p.features;
+  const double tiles = macs * up(p.channels, 64) / p.channels *
+                       up(p.features, 64) / p.features;
+  const double copy_us = 12 + 2.0 * elem * (plan->x + plan->dy) / 3.5e6;
+  double before_us = tiles / (half && !few ? 52e6 : 47e6);
+  double after_us = copy_us + (few ? macs / 14e6 : tiles / 280e6);
+  if (half && few) {
+    // Around the fp32 kernel three conversions; what a binary16 first layer's
+    // kernel does instead is hidden behind its loads (26x155x155 3 -> 44, 3x3
+    // stride 2: 70 -> 36 us; 52x117x117 3 -> 45, 7x7: 714 -> 45).
+    if (p.features % 4 == 0) before_us = macs / 5.5e6;
+    before_us += 8 + 6.0 * (x_pixels * p.channels + y_pixels * p.features) /
+                         3.5e6;
+    if (conv2d_few_f16_filter_backprop_partial_floats(q) != 0)
+      after_us = copy_us + macs / 60e6;
+  }
+  return after_us < 0.75 * before_us;
+}
+
 // What a launch with `algorithm` needs.  Winograd forward / input backprop
 // follow the reference's F(2x2,3x3) formula (the three-stage chain uses all of
 // it, the fused kernel its transformed-filter part).  WinogradLarge runs the
@@ -327,6 +406,9 @@ size_t f16_workspace_halves(const snn_hip_conv2d_params& p, int direction) {
   if (direction == SNN_HIP_FILTER_BACKPROP) {
     const size_t floats = conv2d_few_f16_filter_backprop_partial_floats(p);
     if (floats != 0) return 2 * floats;
+    WidenedFilterGradient widened;
+    if (widened_filter_gradient(p, sizeof(_Float16), &widened))
+      return widened.total();
   }
   if (direction != SNN_HIP_FILTER_BACKPROP)
     return conv2d_f16_workspace_halves(direction, p);
@@ -385,6 +467,13 @@ int workspace_size(const snn_hip_conv2d_params& p, int direction,
       conv2d_filter_backprop_direct_f32_wanted(p))
     *recommended = std::max(
         *recommended, conv2d_filter_backprop_direct_f32_partial_floats(p));
+  WidenedFilterGradient widened;
+  if (filbk &&
+      (algorithm == SNN_HIP_ALGO_TILED || algorithm == SNN_HIP_ALGO_IM2COL ||
+       algorithm == SNN_HIP_ALGO_MATMUL) &&
+      algorithm_supports(p, direction, algorithm) == algorithm &&
+      widened_filter_gradient(p, sizeof(float), &widened))
+    *recommended = std::max(*recommended, widened.total());
   // The gathering kernel behind the same tags: its packed filter, widened source
   // and partial tiles.
   if (!filbk && p.input_format == 0 &&
@@ -537,6 +626,105 @@ int launch_gemm_path<float>(int direction, const float* input,
                             float* workspace, size_t workspace_elems,
                             const LaunchOptions* epilogue);
 
+// out[r][j] = j < in_cols ? in[r][j] : 0, four columns per lane: out_cols is a
+// multiple of 4, `out` 16-byte aligned, `in` of any alignment.
+template <typename T>
+__global__ void __launch_bounds__(256)
+    widen_columns_kernel(const T* __restrict__ in, unsigned in_cols,
+                         T* __restrict__ out, unsigned out_vecs,
+                         unsigned total) {
+  typedef T vec4 __attribute__((ext_vector_type(4)));
+  const unsigned i = blockIdx.x * 256 + threadIdx.x;
+  if (i >= total) return;
+  const unsigned r = i / out_vecs, j = (i - r * out_vecs) * 4;
+  const T* const from = in + static_cast<size_t>(r) * in_cols + j;
+  vec4 v;
+#pragma unroll
+  for (unsigned e = 0; e < 4; ++e)
+    v[e] = j + e < in_cols ? from[e] : static_cast<T>(0.f);
+  reinterpret_cast<vec4*>(out)[i] = v;
+}
+
+// out[t][c][f] = in[t][c][f] of a filter with `in_channels` x `in_features`.
+template <typename T>
+__global__ void __launch_bounds__(256)
+    narrow_filter_kernel(const T* __restrict__ in, int in_channels,
+                         int in_features, T* __restrict__ out, int channels,
+                         int features, size_t total) {
+  const size_t i = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= total) return;
+  const size_t row = i / features, tap = row / channels;
+  out[i] = in[(tap * in_channels + (row - tap * channels)) * in_features +
+              (i - row * features)];
+}
+
+template <typename T>
+void widen_columns(const T* in, int in_cols, T* out, int out_cols, size_t rows,
+                   hipStream_t s) {
+  const unsigned vecs = static_cast<unsigned>(rows * (out_cols / 4));
+  hipLaunchKernelGGL(widen_columns_kernel<T>, dim3(ceil_div(vecs, 256u)),
+                     dim3(256), 0, s, in, static_cast<unsigned>(in_cols), out,
+                     static_cast<unsigned>(out_cols / 4), vecs);
+}
+
+// Returns -1 when it does not apply or has no room for the copies.
+template <typename T>
+int launch_filter_gradient_widened(const T* x, const T* dy, T* dw,
+                                   const snn_hip_conv2d_params& p,
+                                   hipStream_t s, T* workspace,
+                                   size_t workspace_elems) {
+  WidenedFilterGradient plan;
+  if (!widened_filter_gradient(p, sizeof(T), &plan)) return -1;
+  const snn_hip_conv2d_params& q = plan.q;
+  T* block = workspace;
+  const bool temporary = workspace == nullptr || !aligned16(workspace) ||
+                         workspace_elems < plan.total();
+  if (temporary) {
+    // (a stream that records a graph gives no temporaries)
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    void* ptr = nullptr;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess ||
+        status != hipStreamCaptureStatusNone ||
+        temp_malloc_async(&ptr, plan.total() * sizeof(T), s) != hipSuccess) {
+      (void)hipGetLastError();
+      return -1;
+    }
+    block = static_cast<T*>(ptr);
+  }
+  T* const wide_x = block;
+  T* const wide_dy = wide_x + plan.x;
+  T* const wide_dw = wide_dy + plan.dy;
+  T* const inner = plan.inner != 0 ? wide_dw + plan.dw : nullptr;
+  if (plan.x != 0)
+    widen_columns(x, p.channels, wide_x, q.channels,
+                  static_cast<size_t>(p.batch) * p.in_rows * p.in_cols, s);
+  if (plan.dy != 0)
+    widen_columns(dy, p.features, wide_dy, q.features,
+                  static_cast<size_t>(p.batch) * p.out_rows * p.out_cols, s);
+  const int status = launch_gemm_path<T>(
+      SNN_HIP_FILTER_BACKPROP, plan.x != 0 ? wide_x : x,
+      plan.dy != 0 ? wide_dy : dy, wide_dw, q, s, inner, plan.inner, nullptr);
+  if (status == SNN_HIP_OK) {
+    const size_t total = static_cast<size_t>(p.window_rows) * p.window_cols *
+                         p.channels * p.features;
+    hipLaunchKernelGGL(
+        narrow_filter_kernel<T>,
+        dim3(static_cast<unsigned>(ceil_div(total, size_t{256}))), dim3(256), 0,
+        s, wide_dw, q.channels, q.features, dw, p.channels, p.features, total);
+  }
+  const hipError_t err = hipGetLastError();
+  if (temporary) temp_free_async(block, s);
+  if (status != SNN_HIP_OK) return status;
+  if (err != hipSuccess) return report_hip_error(err, "widened filter gradient");
+  return SNN_HIP_OK;
+}
+template <>
+int launch_gemm_path<_Float16>(int direction, const _Float16* input,
+                               const _Float16* filter, _Float16* output,
+                               const snn_hip_conv2d_params& p, hipStream_t s,
+                               _Float16* workspace, size_t workspace_elems,
+                               const LaunchOptions* epilogue);
+
 template <typename From, typename To>
 __global__ void __launch_bounds__(256)
     convert_kernel(const From* __restrict__ in, To* __restrict__ out, size_t n) {
@@ -646,6 +834,11 @@ int launch_gemm_path<_Float16>(int direction, const _Float16* input,
                                      workspace, workspace_elems, s);
     if (rc >= 0) return rc;
   }
+  if (direction == SNN_HIP_FILTER_BACKPROP) {
+    const int rc = launch_filter_gradient_widened<_Float16>(
+        input, filter, output, p, s, workspace, workspace_elems);
+    if (rc >= 0) return rc;
+  }
   // (few (tap, channel) pairs -- a three-channel stem: fp32 has kernels built
   // for that; 64-channel tiles would be nearly empty)
   if (direction == SNN_HIP_FILTER_BACKPROP && p.channels <= 8 &&
@@ -677,6 +870,12 @@ int launch_gemm_path<float>(int direction, const float* input,
   const bool atomics_only = direction == SNN_HIP_FILTER_BACKPROP &&
                             epilogue != nullptr && epilogue->deterministic &&
                             !conv2d_filter_backprop_direct_f32_wanted(p, true);
+  if (direction == SNN_HIP_FILTER_BACKPROP &&
+      (epilogue == nullptr || !epilogue->deterministic)) {
+    const int rc = launch_filter_gradient_widened<float>(
+        input, filter, output, p, s, workspace, workspace_elems);
+    if (rc >= 0) return rc;
+  }
   if (conv2d_gather_f32_wanted(direction, p)) {
     const int rc =
         launch_conv2d_gather_f32(direction, input, filter, output, p, workspace,
