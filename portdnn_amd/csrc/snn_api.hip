@@ -763,9 +763,9 @@ void convert(const From* in, To* out, size_t n, hipStream_t s) {
                        dim3(256), 0, s, in, out, n);
 }
 
-// A binary16 launch that no binary16 matrix-core kernel takes (three input
-// channels, channel or feature counts that are not multiples of 4, strided
-// input gradients) through the fp32 kernels: operands widened into
+// A binary16 launch that no binary16 matrix-core kernel takes (filter gradients
+// of at most eight channels outside the first-layer kernels, operands off
+// 16-byte alignment) through the fp32 kernels: operands widened into
 // stream-ordered temporaries, the fp32 launch -- every path it has -- and the
 // result rounded back.  Products and sums are then fp32 on binary16-rounded
 // operands, as in the binary16 kernels.  From 2^24 multiply-adds; returns -1
