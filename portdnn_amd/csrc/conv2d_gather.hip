@@ -166,6 +166,55 @@ __host__ __device__ constexpr int feature_of_row(unsigned row) {
                           4 * ((row >> 3) & 1) + (row & 3));
 }
 
+// Whether a pixel's sums hold products with zeros that are no taps of theirs.
+__device__ __forceinline__ bool window_cut(const Gather& g,
+                                           const GatherClass& cls, Pixel px) {
+  const int iy = px.y * g.step_r + cls.off_r;
+  const int ix = px.x * g.step_c + cls.off_c;
+  return g.merged != 0 || iy < 0 || iy + cls.win_r > g.src_rows || ix < 0 ||
+         ix + cls.win_c > g.src_cols;
+}
+
+// Feature f of a pixel over the taps that exist, with `w` the filter as the
+// caller has it; up to the first term that makes it a NaN (a tensor of NaNs
+// would otherwise be summed one product at a time).
+template <typename T>
+__device__ __forceinline__ float exact_sum(const T* __restrict__ src,
+                                           const T* __restrict__ w,
+                                           const Gather& g,
+                                           const GatherClass& cls, Pixel px,
+                                           int f) {
+  int member_r = 0, member_c = 0, per_tap = g.features;
+  if (g.merged != 0) {
+    const int member = f / g.merged;
+    f -= member * g.merged;
+    member_r = member / g.out_step_c;
+    member_c = member - member_r * g.out_step_c;
+    per_tap = g.merged;
+  }
+  const size_t stride = g.mirrored ? 1 : static_cast<size_t>(g.features);
+  float sum = 0.f;
+  for (int tr = 0; tr < cls.win_r; ++tr) {
+    const int y = px.y * g.step_r + cls.off_r + tr;
+    const int wr = cls.tap_r0 + tr * cls.tap_rs + member_r;
+    if (y < 0 || y >= g.src_rows || wr >= g.win_rows) continue;
+    for (int ts = 0; ts < cls.win_c; ++ts) {
+      const int x = px.x * g.step_c + cls.off_c + ts;
+      const int wc = cls.tap_c0 + ts * cls.tap_cs + member_c;
+      if (x < 0 || x >= g.src_cols || wc >= g.win_cols) continue;
+      const T* const from =
+          src + (static_cast<size_t>(px.n * g.src_rows + y) * g.src_cols + x) *
+                    g.cp * kPiece<T>;
+      const size_t at_tap = static_cast<size_t>(wr * g.win_cols + wc);
+      const T* const by = g.mirrored ? w + (at_tap * per_tap + f) * g.channels
+                                     : w + at_tap * g.channels * g.features + f;
+      for (int c = 0; c < g.channels && sum == sum; ++c)
+        sum += static_cast<float>(from[c]) * static_cast<float>(by[c * stride]);
+    }
+  }
+  return sum;
+}
+
 // What a bias and an activation make of a sum.
 __device__ __forceinline__ float bias_act(float v, float bias, int relu) {
   v += bias;
@@ -274,10 +323,12 @@ __global__ void __launch_bounds__(256)
 
 // WM x WN waves of TM x TN blocks of 32 pixels x 32 features.  UNIFORM: whole
 // chunks per tap, tap bookkeeping in scalar registers; otherwise every lane
-// works out the tap of its own piece.  FROM: what `wpk` is.
+// works out the tap of its own piece.  FROM: what `wpk` is; `w` is the caller's
+// filter.
 template <typename T, int WM, int WN, int TM, int TN, bool UNIFORM, int FROM>
 __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
     conv_gather_kernel(const T* __restrict__ src, const T* __restrict__ wpk,
+                       const T* __restrict__ w,
                        const float* __restrict__ bias, T* __restrict__ dst,
                        float* __restrict__ part, Gather g, unsigned src_bytes,
                        unsigned wpk_bytes, unsigned dst_bytes,
@@ -578,6 +629,74 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
 
   // A lane holds features f0 .. f0 + 7 and f0 + 16 .. f0 + 23 of one pixel per
   // block.
+  // Bit v of strange[..]: sum v of the block is a NaN that may not belong there.
+  // It is stored like the others and replaced afterwards, when no sums are held
+  // in registers any more.
+  unsigned strange[TM * TN] = {};
+  {
+    // (a maximum that keeps NaNs: two values per instruction)
+    float most = 0.f;
+#pragma unroll
+    for (int j = 0; j < TM; ++j)
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        float block = 0.f;
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          block = __builtin_elementwise_maximum(block, acc[i][j][v]);
+        most = __builtin_elementwise_maximum(most, block);
+      }
+    if (__builtin_amdgcn_ballot_w64(most != most) != 0) {
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        const int m = m0 + (wm * TM + j) * 32 + l32;
+        const bool cut =
+            m < cls.pixels && window_cut(g, cls, pixel_of(m, cls));
+#pragma unroll
+        for (int i = 0; i < TN; ++i) {
+          unsigned bits = 0;
+#pragma unroll
+          for (int v = 0; v < 16; ++v)
+            bits |= acc[i][j][v] != acc[i][j][v] ? 1u << v : 0u;
+          strange[j * TN + i] = cut ? bits : 0u;
+        }
+      }
+    }
+  }
+  auto replace_strange = [&]() {
+    unsigned all = 0;
+#pragma unroll
+    for (int b = 0; b < TM * TN; ++b) all |= strange[b];
+    if (__builtin_amdgcn_ballot_w64(all != 0) == 0) return;
+    __builtin_amdgcn_s_waitcnt(0);  // the stores of the NaNs
+    __builtin_amdgcn_sched_barrier(0);
+#pragma nounroll
+    for (int b = 0; b < TM * TN; ++b) {
+      unsigned bits = 0;
+#pragma unroll
+      for (int u = 0; u < TM * TN; ++u) bits = u == b ? strange[u] : bits;
+      const int j = b / TN, i = b - j * TN;
+      const Pixel px = pixel_of(m0 + (wm * TM + j) * 32 + l32, cls);
+      while (bits != 0) {
+        const int v = __builtin_ctz(bits);
+        bits &= bits - 1;
+        const int f = n0 + (wn * TN + i) * 32 + 8 * khalf + v + v / 8 * 8;
+        if (f >= g.features) continue;
+        float sum = exact_sum(src, w, g, cls, px, f);
+        if constexpr (kSize == 4) {
+          if (bias != nullptr || g.relu != 0)
+            sum = bias_act(sum, bias != nullptr ? bias[f] : 0.f, g.relu);
+        }
+        const int at =
+            g.merged != 0
+                ? merged_element(g, cls, px, f)
+                : ((px.n * g.out_rows + px.y * g.out_step_r + cls.out_r0) *
+                       g.out_cols + px.x * g.out_step_c + cls.out_c0) *
+                          g.features + f;
+        if (at >= 0) dst[at] = static_cast<T>(sum);
+      }
+    }
+  };
   const __amdgpu_buffer_rsrc_t dst_rsrc = make_rsrc(dst, dst_bytes);
   if constexpr (kSize == 4) {
     if (g.merged != 0) {
@@ -599,6 +718,7 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
                 m < cls.pixels && at >= 0 ? at * 4u : kOob, 0, 0);
           }
       }
+      replace_strange();
       return;
     }
     if (bias != nullptr || g.relu != 0) {
@@ -748,6 +868,7 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
       }
     }
   }
+  replace_strange();
 }
 
 // Sums the splits of every tile in order and rounds: one float4 -- four
@@ -755,6 +876,7 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
 template <typename T, int WM, int WN, int TM, int TN>
 __global__ void __launch_bounds__(256)
     gather_reduce_kernel(const float4v* __restrict__ part,
+                         const T* __restrict__ src, const T* __restrict__ w,
                          const float* __restrict__ bias, T* __restrict__ dst,
                          Gather g) {
   constexpr unsigned BM = 32 * WM * TM, BN = 32 * WN * TN;
@@ -781,6 +903,13 @@ __global__ void __launch_bounds__(256)
   for (int s = 0; s < g.n_splits; ++s)
     sum += from[static_cast<size_t>(s) * g.n_tiles * kTileVecs];
   const Pixel px = pixel_of(m, cls);
+  if ((sum[0] != sum[0] || sum[1] != sum[1] || sum[2] != sum[2] ||
+       sum[3] != sum[3]) && window_cut(g, cls, px)) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (sum[e] != sum[e] && f + e < g.features)
+        sum[e] = exact_sum(src, w, g, cls, px, f + e);
+  }
   if constexpr (sizeof(T) == 4) {
     if (g.merged != 0) {
 #pragma unroll
@@ -1101,6 +1230,7 @@ template <typename T>
 struct GatherOperands {
   const T* src;
   const T* filter;
+  const T* caller_filter;
   const float* bias;
   T* dst;
   float* part;
@@ -1119,8 +1249,8 @@ void launch_kernel(const GatherOperands<T>& ops, const GatherPlan& plan,
   KernelTimer timer(stream);
   hipLaunchKernelGGL((conv_gather_kernel<T, WM, WN, TM, TN, UNIFORM, FROM>),
                      dim3(n_groups), dim3(64 * WM * WN), 0, stream, ops.src,
-                     ops.filter, ops.bias, ops.dst, ops.part, g, src_bytes,
-                     filter_bytes, dst_bytes, n_groups);
+                     ops.filter, ops.caller_filter, ops.bias, ops.dst, ops.part,
+                     g, src_bytes, filter_bytes, dst_bytes, n_groups);
 }
 
 template <typename T, int WM, int WN, int TM, int TN>
@@ -1157,8 +1287,8 @@ void launch_tile(const GatherOperands<T>& ops, const GatherPlan& plan,
   if (g.n_splits > 1)
     hipLaunchKernelGGL((gather_reduce_kernel<T, WM, WN, TM, TN>),
                        dim3(g.n_tiles * (BM * BN / 1024)), dim3(256), 0, stream,
-                       reinterpret_cast<const float4v*>(ops.part), ops.bias,
-                       ops.dst, g);
+                       reinterpret_cast<const float4v*>(ops.part), ops.src,
+                       ops.caller_filter, ops.bias, ops.dst, g);
 }
 
 // Returns -1 when there is no room for its temporaries.
@@ -1198,6 +1328,7 @@ int launch_gather(const GatherPlan& plan, const T* input, const T* filter,
   const GatherOperands<T> ops = {
       plan.widen ? wide : input,
       from == kPacked ? reinterpret_cast<const T*>(packed) : filter,
+      filter,
       bias,
       output,
       reinterpret_cast<float*>(packed + pack_blocks * 2048 + plan.wide_bytes),

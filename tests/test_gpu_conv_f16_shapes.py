@@ -84,6 +84,37 @@ def test_conv_f16_shapes(shape, direction):
     assert torch.all(block[rec:] == 7.0)
 
 
+@pytest.mark.parametrize("shape,direction", [
+    ((9, 57, 43, 72, 96, 3, 2, True), DIRECTION.FORWARD),
+    ((9, 57, 43, 72, 96, 3, 2, True), DIRECTION.INPUT_BACKPROP),
+    ((2, 7, 7, 512, 72, 3, 1, True), DIRECTION.FORWARD),
+    ((20, 20, 21, 64, 203, 3, 1, True), DIRECTION.FORWARD),
+    ((20, 20, 21, 64, 203, 3, 1, True), DIRECTION.INPUT_BACKPROP),
+    ((16, 80, 80, 128, 128, 3, 2, True), DIRECTION.FORWARD)], ids=str)
+def test_conv_f16_infinite_filter_stays(shape, direction):
+    """An infinite weight reaches the outputs that it is a factor of, and not
+    those whose window has that tap outside the image."""
+    batch, rows, cols, channels, features, window, stride, same = shape
+    p = ops.conv_params(batch, rows, cols, channels, features, window, stride,
+                        same)
+    rng = np.random.default_rng(4150 + rows)
+    n_a, n_b, _ = ops.conv_sizes(p, direction)
+    a = uniform(rng, n_a).astype(np.float16)
+    b = uniform(rng, n_b).astype(np.float16)
+    b[0] = np.inf   # (the first tap ...
+    b[-1] = np.inf  # ... and the last: stride 2 has padding on one side only)
+    ref = ORACLE_FN[direction](a.astype(np.float32), b.astype(np.float32),
+                               oracle_params(p, features), acc64=True)
+    ref = np.asarray(ref, dtype=np.float64).reshape(-1)
+    got = ops.conv2d(dev(a, torch.float16), dev(b, torch.float16), p, direction,
+                     ALGO.IM2COL).float().cpu().numpy().reshape(-1)
+    ok = np.isfinite(ref)
+    assert ok.any() and not ok.all()
+    assert np.array_equal(np.isfinite(got), ok)
+    assert_rounded_once(got[ok], ref[ok], window * window *
+                        max(channels, features), (shape, direction))
+
+
 @pytest.mark.parametrize("m,k,n", [(32, 64, 64), (33, 40, 24), (257, 100, 130),
                                    (640, 1000, 30)])
 @pytest.mark.parametrize("trans_b", [False, True])

@@ -2,7 +2,7 @@
 gathering kernel can go wrong: edges of its tiles, ragged channel and feature
 counts, stride classes with few, unequal or no taps, merged classes of a few
 channels, reductions shared by work-groups, filters that are not 16-byte
-aligned, bias and activation, launches recorded into a graph.
+aligned, bias and activation, infinite operands, launches recorded into a graph.
 
 Bound: n products added in fp32, each addition rounding by at most 2^-24 of a
 partial sum, which for the U[-1,1] operands here stays below twice the largest
@@ -101,6 +101,69 @@ def test_conv_f32_bias_act(shape, relu):
     got = ops.conv2d_bias_act(dev(a), dev(b), dev(bias), p, ALGO.IM2COL,
                               relu=relu)
     check(got, ref, window * window * channels + 1, (shape, relu))
+
+
+# Merged classes (3x3, 7x7 and 5x5 windows, whole reductions and a shared one),
+# classes of their own, forward windows over the border.
+INFINITE = [
+    ((30, 47, 61, 3, 58, 3, 2, True), DIRECTION.INPUT_BACKPROP),
+    ((20, 50, 51, 3, 40, 7, 2, True), DIRECTION.INPUT_BACKPROP),
+    ((20, 60, 60, 2, 40, 6, 4, True), DIRECTION.INPUT_BACKPROP),
+    ((31, 50, 64, 1, 200, 5, 3, True), DIRECTION.INPUT_BACKPROP),
+    ((1, 24, 24, 3, 512, 7, 2, True), DIRECTION.INPUT_BACKPROP),
+    ((2, 12, 15, 24, 40, 3, 3, True), DIRECTION.INPUT_BACKPROP),
+    ((2, 7, 7, 480, 72, 3, 2, True), DIRECTION.INPUT_BACKPROP),
+    ((3, 10, 13, 35, 45, 5, 1, True), DIRECTION.FORWARD),
+    ((2, 7, 7, 480, 70, 3, 2, True), DIRECTION.FORWARD),
+    ((9, 57, 43, 72, 96, 3, 2, True), DIRECTION.FORWARD),
+]
+
+
+@pytest.mark.parametrize("shape,direction", INFINITE, ids=str)
+@pytest.mark.parametrize("operand", [0, 1], ids=["tensor", "filter"])
+def test_conv_f32_infinity_stays(shape, direction, operand):
+    """An infinite value reaches the outputs that it is a factor of and no
+    other: the finite rest is what it is without it."""
+    batch, rows, cols, channels, features, window, stride, same = shape
+    p = ops.conv_params(batch, rows, cols, channels, features, window, stride,
+                        same)
+    rng = np.random.default_rng(4700 + rows)
+    n_a, n_b, _ = ops.conv_sizes(p, direction)
+    a, b = uniform(rng, n_a), uniform(rng, n_b)
+    if operand == 0:  # in the middle of an image
+        forward = direction == DIRECTION.FORWARD
+        r, c = (rows, cols) if forward else (p.out_rows, p.out_cols)
+        a[(r // 2 * c + c // 2) * (channels if forward else features)] = np.inf
+    else:             # the first tap, which the border pixels do not have
+        b[0] = np.inf
+    ref = ORACLE_FN[direction](a, b, oracle_params(p, features), acc64=True)
+    ref = np.asarray(ref, dtype=np.float64).reshape(-1)
+    got = ops.conv2d(dev(a), dev(b), p, direction, ALGO.IM2COL)
+    ok = torch.from_numpy(np.isfinite(ref))
+    assert ok.any() and not ok.all()
+    assert torch.equal(torch.isfinite(got.cpu()), ok)
+    check(got.cpu()[ok], ref[ok.numpy()], window * window *
+          max(channels, features), (shape, direction, operand))
+
+
+def test_conv_f32_bias_act_infinity_stays():
+    shape = batch, rows, cols, channels, features, window, stride, same = (
+        3, 20, 21, 20, 30, 3, 2, True)
+    p = ops.conv_params(batch, rows, cols, channels, features, window, stride,
+                        same)
+    rng = np.random.default_rng(4800)
+    n_a, n_b, _ = ops.conv_sizes(p, DIRECTION.FORWARD)
+    a, b, bias = uniform(rng, n_a), uniform(rng, n_b), uniform(rng, features)
+    b[-1] = np.inf
+    ref = ORACLE_FN[DIRECTION.FORWARD](a, b, oracle_params(p, features),
+                                       acc64=True)
+    ref = np.asarray(ref, dtype=np.float64).reshape(-1, features) + bias
+    ref = np.maximum(ref, 0).reshape(-1)
+    got = ops.conv2d_bias_act(dev(a), dev(b), dev(bias), p, ALGO.IM2COL,
+                              relu=True)
+    ok = torch.from_numpy(np.isfinite(ref))
+    assert torch.equal(torch.isfinite(got.cpu()), ok) and not ok.all()
+    check(got.cpu()[ok], ref[ok.numpy()], window * window * channels + 1, shape)
 
 
 @pytest.mark.parametrize("shape,direction", [
