@@ -73,6 +73,8 @@ __device__ __forceinline__ half8 read_transposed(const char* rows03,
   return __builtin_bit_cast(half8, both);
 }
 
+constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
+
 // Waits for this wave's LDS operations and for the other waves; loads from
 // memory stay in flight.
 __device__ __forceinline__ void lds_barrier() {
@@ -373,7 +375,9 @@ __global__ void __launch_bounds__(256, KS < 3 ? 2 : 1)
 //     consecutive features of a pixel) and stays in registers, all features in
 //     every wave: a pixel operand serves 2 NP instructions.
 //   * Values of an operand outside the filter row belong to other pixels and are
-//     cleared, not multiplied by zero: they may be infinite.
+//     cleared, not multiplied by zero: they may be infinite.  Where a window leaves
+//     the image an infinite weight meets a zero; sums that are NaN there are
+//     worked out term by term.
 //
 // 128 x 224x224x3 -> 64, 7x7: 153 us with the image widened to eight channels
 // -> 99 us.
@@ -494,6 +498,7 @@ __global__ void __launch_bounds__(256, 2)
         px.at[h][i] = *reinterpret_cast<const uint4a4*>(from + 16 * i);
     }
   };
+  float most = 0.f;  // a NaN once any sum of this lane is
   auto multiply = [&](int item, const Pixels& px) {
     const int oy = item / n_pb, pb = item - oy * n_pb;
     float4v acc[NP][2];
@@ -521,6 +526,13 @@ __global__ void __launch_bounds__(256, 2)
         ((n * g.out_rows + oy0 + oy) * g.out_cols + ox) * g.features + 8 * q) *
         2u;
 #pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int e = 0; e < 2; ++e)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          most = __builtin_elementwise_maximum(most, acc[p][e][v]);
+#pragma unroll
     for (int p = 0; p < NP; ++p) {
       half8 out;
 #pragma unroll
@@ -547,6 +559,35 @@ __global__ void __launch_bounds__(256, 2)
     __builtin_amdgcn_sched_barrier(0);
     multiply(item, odd);
     item += 4;
+  }
+
+  // ---- NaNs of windows that leave the image -----------------------------------
+  if (__builtin_amdgcn_ballot_w64(most != most) == 0) return;
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // their stores
+  __builtin_amdgcn_sched_barrier(0);
+  for (item = wave; item < n_items; item += 4) {
+    const int oy = oy0 + item / n_pb, ox = 16 * (item % n_pb) + l16;
+    const int iy = 2 * oy - g.pad_rows, ix = 2 * ox - g.pad_cols;
+    if (ox >= g.out_cols || (iy >= 0 && iy + g.win_rows <= g.in_rows &&
+                             ix >= 0 && ix + g.win_cols <= g.in_cols))
+      continue;
+    _Float16* const out =
+        y + (static_cast<size_t>(n * g.out_rows + oy) * g.out_cols + ox) *
+                g.features;
+    for (int f = q; f < g.features; f += 4) {
+      const _Float16 had = *const_cast<const volatile _Float16*>(out + f);
+      if (had == had) continue;
+      float sum = 0.f;
+      for (int r = max(0, -iy); r < min(g.win_rows, g.in_rows - iy); ++r)
+        for (int e = max(0, -ix) * C;
+             e < min(g.win_cols, g.in_cols - ix) * C && sum == sum; ++e)
+          sum += static_cast<float>(
+                     x[(static_cast<size_t>(n * g.in_rows + iy + r) * g.in_cols +
+                        ix) * C + e]) *
+                 static_cast<float>(w[static_cast<size_t>(r * wc + e) *
+                                          g.features + f]);
+      out[f] = static_cast<_Float16>(sum);
+    }
   }
 }
 

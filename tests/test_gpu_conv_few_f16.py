@@ -106,3 +106,27 @@ def test_few_channels_f16_infinity_stays(shape, direction):
     assert_rounded_once(got[ok], ref[ok], max(
         p.window_rows * p.window_cols * max(p.channels, p.features),
         p.batch * p.out_rows * p.out_cols), (shape, direction))
+
+
+@pytest.mark.parametrize("shape", [SHAPES[0], SHAPES[2], SHAPES[3], SHAPES[6],
+                                   SHAPES[12]],
+                         ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("direction", DIRECTIONS[:2])
+def test_few_channels_f16_infinite_filter_stays(shape, direction):
+    """An infinite weight reaches the outputs that it is a factor of, and not
+    those whose window has that tap outside the image."""
+    p, rng = make(shape, 5300)
+    n_a, n_b, _ = ops.conv_sizes(p, direction)
+    a = uniform(rng, n_a).astype(np.float16)
+    b = uniform(rng, n_b).astype(np.float16)
+    b[0], b[-1] = np.inf, -np.inf  # the first tap and the last
+    ref = ORACLE_FN[direction](a.astype(np.float32), b.astype(np.float32),
+                               oracle_params(p, p.features), acc64=True)
+    ref = np.asarray(ref).reshape(-1)
+    got = ops.conv2d(dev(a, torch.float16), dev(b, torch.float16), p, direction,
+                     ALGO.IM2COL).float().cpu().numpy().reshape(-1)
+    ok = np.isfinite(ref)
+    assert ok.any() and not ok.all()
+    assert np.array_equal(np.isfinite(got), ok)
+    assert_rounded_once(got[ok], ref[ok], p.window_rows * p.window_cols *
+                        max(p.channels, p.features), (shape, direction))
