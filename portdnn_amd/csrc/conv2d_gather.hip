@@ -954,6 +954,7 @@ struct GatherPlan {
   size_t part_floats = 0;   // of the tiles whose reduction is shared
   int tile = 0;             // index into the tile shapes of the type
   int n_splits = 1;
+  double us = 0;            // of the products, by the model of choose_tile
   size_t filter_elems = 0;
   FilterFrom from = kPacked;
   size_t workspace_bytes(bool packs) const {
@@ -1036,6 +1037,7 @@ void choose_tile(GatherPlan* plan, bool may_split) {
         us += 3.0 + splits * tiles * t.pixels * t.features * 8 / 3e6;
       if (us < best) {
         best = us;
+        plan->us = us;
         plan->tile = i;
         plan->n_splits = splits;
       }
@@ -1398,17 +1400,72 @@ bool is_rows_gemm(int direction, const snn_hip_conv2d_params& p) {
              : gemm_nt_f16_supports(m, p.features, p.channels);
 }
 
-// A handful of products per output and few outputs: one launch of the direct
-// kernel (16x16x8 -> 8, 1x1, at batch 2: 6.5 us against 10.3 with the filter's
-// pack in front; a 3x3 of 20 channels 20.3 against 10.5).
-bool is_tiny(int direction, const snn_hip_conv2d_params& p) {
+// What a binary16 launch takes on each of the kernels that take any stride, in
+// us back to back.  Fitted to 2060 random layers of 1e4 to 1.5e9 multiply-adds
+// (windows 1 to 7, strides 1 to 3, 3 to 1024 channels and features): the middle
+// half of the estimates is within 5 % for the gathering kernel and 8 % for the
+// other two.  They meet where launches are short.  The gathering one has
+// up to two launches in front of its products, the filter's pack and the copy to
+// whole pieces (16x55x41 16 -> 12, 1x1: general 5.6, gathering 8.8; 2x24x24
+// 52 -> 20, 1x1 stride 2: 5.4 and 7.9), and a temporary for these costs 14 us of
+// host time where the caller brings no workspace.
+constexpr double kNever = 1e30;
+
+struct Products {
+  double pixels, columns, reduced, macs;
+};
+Products products_of(int direction, const snn_hip_conv2d_params& p) {
   const bool grad = direction == SNN_HIP_INPUT_BACKPROP;
-  const size_t products = static_cast<size_t>(p.window_rows) * p.window_cols *
-                          (grad ? p.features : p.channels);
-  const size_t outputs =
-      grad ? static_cast<size_t>(p.batch) * p.in_rows * p.in_cols * p.channels
-           : static_cast<size_t>(p.batch) * p.out_rows * p.out_cols * p.features;
-  return products <= 32 && outputs <= (size_t{1} << 16);
+  const double taps = static_cast<double>(p.window_rows) * p.window_cols;
+  const double y = static_cast<double>(p.batch) * p.out_rows * p.out_cols;
+  Products r;
+  r.pixels = grad ? static_cast<double>(p.batch) * p.in_rows * p.in_cols : y;
+  r.columns = grad ? p.channels : p.features;
+  r.reduced = taps * (grad ? p.features : p.channels);
+  r.macs = y * taps * p.channels * p.features;
+  return r;
+}
+
+double gather_f16_us(const GatherPlan& plan, bool packs, bool temporary) {
+  const double bytes = static_cast<double>(plan.wide_bytes) +
+                       (packs ? plan.pack_blocks * 2048.0 : 0.0);
+  return 4.0 + 0.8 * plan.us + (bytes > 0 ? 3.0 + bytes / 1.5e6 : 0.0) +
+         plan.out_elems / 2.5e6 + (temporary ? 14.0 : 0.0);
+}
+
+double general_f16_us(const Products& r) {
+  const double chunks = std::ceil(r.reduced / 32);
+  const double rounds =
+      std::ceil(r.pixels / 64) * std::ceil(r.columns / 64) / kNumCus;
+  return 3.0 + 0.9 * chunks + (0.45 * chunks + 0.4) * rounds +
+         r.pixels * r.columns / 6e6;
+}
+
+// One lane per output.  A gradient's lanes read the filter columns of as many
+// channels: with features in multiples of 4 those fall into few banks, and the
+// general kernel is there.
+double direct_f16_us(int direction, const snn_hip_conv2d_params& p,
+                     const Products& r) {
+  const double outputs = r.pixels * r.columns;
+  if (r.macs >= double(1 << 24)) return kNever;
+  if (direction == SNN_HIP_FORWARD)
+    return 2.9 + 0.09 * r.reduced + (0.146 * r.reduced + 2.7) * outputs / 1e6;
+  const double loop = static_cast<double>(p.features) *
+                      ceil_div(p.window_rows, p.stride_rows) *
+                      ceil_div(p.window_cols, p.stride_cols);
+  if (p.features % 4 != 0 && loop <= 16)
+    return 3.1 + 0.05 * loop + (0.11 * loop + 3.3) * outputs / 1e6 +
+           0.67 * p.window_rows * p.window_cols /
+               (p.stride_rows * p.stride_cols);
+  return r.reduced <= 32 && outputs <= (1 << 16) ? 5.5 : kNever;
+}
+
+bool stream_captures(hipStream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &status) == hipSuccess)
+    return status != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
 }
 
 }  // namespace
@@ -1420,25 +1477,32 @@ size_t conv2d_f16_workspace_halves(int direction,
   if (rowtile_params(direction, p, &q))
     return static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
            p.features;
-  if (is_tiny(direction, p)) return 0;
+  const GatherPlan& plan = make_plan<_Float16>(direction, p);
+  if (!plan.ok) return 0;
+  const Products r = products_of(direction, p);
+  if (std::min(conv2d_general_f16_supports(direction, p) ? general_f16_us(r)
+                                                         : kNever,
+               direct_f16_us(direction, p, r)) <
+      gather_f16_us(plan, plan.from == kPacked, false))
+    return 0;
   // (with room for the packed filter also where the gradient's is read in
   // place, for one that is not 16-byte aligned; that of a 1x1 layer would take
   // a temporary)
-  const GatherPlan& plan = make_plan<_Float16>(direction, p);
   const bool packs =
       plan.from == kPacked || p.window_rows > 1 || p.window_cols > 1;
-  return plan.ok ? plan.workspace_bytes(packs) / 2 : 0;
+  return plan.workspace_bytes(packs) / 2;
 }
 
 int launch_conv2d_f16(int direction, const _Float16* input,
                       const _Float16* filter, _Float16* output,
                       const snn_hip_conv2d_params& p, _Float16* workspace,
-                      size_t workspace_elems, hipStream_t stream) {
+                      size_t workspace_elems, hipStream_t stream,
+                      double otherwise_us) {
   auto aligned = [](const void* ptr) {
     return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0;
   };
-  if (!aligned(output)) return -1;
-  if (is_rows_gemm(direction, p) && aligned(input) && aligned(filter)) {
+  const bool both_aligned = aligned(input) && aligned(filter);
+  if (aligned(output) && is_rows_gemm(direction, p) && both_aligned) {
     const int m = p.batch * p.in_rows * p.in_cols;
     return direction == SNN_HIP_FORWARD
                ? launch_gemm_rows_f16(input, filter, output, m, p.channels,
@@ -1447,7 +1511,7 @@ int launch_conv2d_f16(int direction, const _Float16* input,
                                     p.channels, stream);
   }
   snn_hip_conv2d_params q;
-  if (rowtile_params(direction, p, &q) && aligned(input) && aligned(filter)) {
+  if (aligned(output) && rowtile_params(direction, p, &q) && both_aligned) {
     const size_t need = static_cast<size_t>(p.window_rows) * p.window_cols *
                         p.channels * p.features;
     _Float16* packed = workspace;
@@ -1466,11 +1530,44 @@ int launch_conv2d_f16(int direction, const _Float16* input,
     if (temporary) temp_free_async(packed, stream);
     return status;
   }
-  if (is_tiny(direction, p)) return -1;
-  const GatherPlan& plan = make_plan<_Float16>(direction, p);
-  if (!plan.ok || (!plan.widen && !aligned(input))) return -1;
-  return launch_gather<_Float16>(plan, input, filter, output, workspace,
-                                 workspace_elems, nullptr, false, stream);
+  const Products r = products_of(direction, p);
+  const bool general =
+      both_aligned && conv2d_general_f16_supports(direction, p) &&
+      (direction == SNN_HIP_INPUT_BACKPROP || aligned(output));
+  const double general_us = general ? general_f16_us(r) : kNever;
+  const double direct_us = direct_f16_us(direction, p, r);
+
+  const GatherPlan* plan = &make_plan<_Float16>(direction, p);
+  const bool packs = plan->from == kPacked || !aligned(filter);
+  const size_t room = workspace != nullptr && aligned(workspace)
+                          ? workspace_elems * sizeof(_Float16) : 0;
+  bool able = plan->ok && aligned(output) && (plan->widen || aligned(input));
+  bool temporary = able && plan->workspace_bytes(packs) > room;
+  if (temporary && stream_captures(stream)) {
+    // A launch that is recorded without room for the packed filter or the copy
+    // keeps its reduction whole, or takes a kernel that needs no temporary.
+    // (Layers of 64 channels and large ones with counts that no other kernel
+    // takes have only kernels with temporaries, or slow ones.)
+    plan = &make_plan<_Float16>(direction, p, false);
+    temporary = plan->workspace_bytes(packs) > room;
+    const bool other = otherwise_us < kNever || r.macs < double(1 << 24) ||
+                       (general && (direction == SNN_HIP_INPUT_BACKPROP ||
+                                    p.channels % 64 != 0));
+    able = !temporary || !other;
+  }
+  const double gather_us =
+      able ? gather_f16_us(*plan, packs, temporary) : kNever;
+  if (std::min(otherwise_us, direct_us) < std::min(general_us, gather_us))
+    return -1;
+  if (gather_us <= general_us && able) {
+    const int rc = launch_gather<_Float16>(*plan, input, filter, output,
+                                           workspace, workspace_elems, nullptr,
+                                           false, stream);
+    if (rc >= 0) return rc;
+  }
+  return general ? launch_conv2d_general_f16(direction, input, filter, output,
+                                             p, stream)
+                 : -1;
 }
 
 // Where the gathering kernel is faster than the other fp32 kernels behind the

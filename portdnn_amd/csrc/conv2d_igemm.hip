@@ -89,14 +89,16 @@ __device__ inline float4 buffer_load4_as_float(__amdgpu_buffer_rsrc_t r,
 // the 3-channel stem), so four consecutive reduction indices are not four
 // consecutive floats of one tap; each is located and loaded on its own.
 template <int BM, int BN, int WM, int WN, bool B_K_INNER, bool STRIDED,
-          bool ATOMIC, bool SCALAR_A = false>
+          bool ATOMIC, bool SCALAR_A = false, typename T = float>
 __global__ void __launch_bounds__(kThreads)
-    conv_igemm_kernel(const float* __restrict__ src, const float* __restrict__ wgt,
-                      float* __restrict__ dst, Gather g, unsigned src_bytes,
+    conv_igemm_kernel(const T* __restrict__ src, const T* __restrict__ wgt,
+                      T* __restrict__ dst, Gather g, unsigned src_bytes,
                       unsigned wgt_bytes, unsigned n_tiles_n, unsigned n_tiles,
                       int chunks_per_split) {
   static_assert(WM * WN == 4, "four waves per work-group");
-  constexpr unsigned kEsz = sizeof(float);
+  static_assert(sizeof(T) == 4 || (!ATOMIC && !SCALAR_A),
+                "half-precision tensors: plain stores, vector gather");
+  constexpr unsigned kEsz = sizeof(T);
   constexpr int WTM = BM / WM, WTN = BN / WN;  // wave tile
   constexpr int TM = WTM / 32, TN = WTN / 32;  // MFMA blocks per wave
   static_assert(TM >= 1 && TN >= 1, "wave tile must hold a 32x32 block");
@@ -237,7 +239,7 @@ __global__ void __launch_bounds__(kThreads)
       ok = ok &
            (static_cast<unsigned>(iy) < static_cast<unsigned>(g.src_rows)) &
            (static_cast<unsigned>(ix) < static_cast<unsigned>(g.src_cols));
-      a_reg[i] = buffer_load4(
+      a_reg[i] = buffer_load4_as_float<T>(
           src_rsrc, ok ? static_cast<unsigned>(off) * kEsz : kOob);
     }
   };
@@ -280,7 +282,7 @@ __global__ void __launch_bounds__(kThreads)
         if (col < g.n_total)
           off = static_cast<unsigned>(q * g.n_total + col) * kEsz;
       }
-      b_reg[i] = buffer_load4(wgt_rsrc, off);
+      b_reg[i] = buffer_load4_as_float<T>(wgt_rsrc, off);
     }
   };
   auto store_tiles = [&](int stage) {
@@ -342,11 +344,11 @@ __global__ void __launch_bounds__(kThreads)
       for (int v = 0; v < 16; ++v) {
         const int m = m0 + wave_m * WTM + 32 * i + 8 * (v >> 2) + row_l + (v & 3);
         if (m < g.m_total) {
-          float* o = dst + static_cast<size_t>(m) * g.n_total + col;
+          T* o = dst + static_cast<size_t>(m) * g.n_total + col;
           if constexpr (ATOMIC)
             unsafeAtomicAdd(o, acc[i][j][v]);
           else
-            *o = acc[i][j][v];
+            *o = static_cast<T>(acc[i][j][v]);
         }
       }
     }
@@ -2176,6 +2178,60 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
   const hipError_t err = hipGetLastError();
   if (temporary) temp_free_async(acc32, stream);
   if (err != hipSuccess) return report_hip_error(err, "f16 filter backprop");
+  return SNN_HIP_OK;
+}
+
+// Half-precision forward convolution and input gradient on the general
+// implicit-GEMM kernel reading binary16 operands: one launch and no temporary,
+// one work-group per 64 x 64 tile and no reduction split, so every output is
+// stored once.  The faster kernel for short launches only (the fp32 matrix
+// instruction, conversions on the way into LDS).
+bool conv2d_general_f16_supports(int direction,
+                                 const snn_hip_conv2d_params& p) {
+  const size_t x = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols *
+                   p.channels;
+  const size_t y = static_cast<size_t>(p.batch) * p.out_rows * p.out_cols *
+                   p.features;
+  const size_t w = static_cast<size_t>(p.window_rows) * p.window_cols *
+                   p.channels * p.features;
+  return (direction == SNN_HIP_INPUT_BACKPROP || p.channels % 4 == 0) &&
+         p.features % 4 == 0 &&
+         max(max(x, y), w) * sizeof(_Float16) <= kMaxBufferBytes;
+}
+
+int launch_conv2d_general_f16(int direction, const _Float16* src,
+                              const _Float16* filter, _Float16* dst,
+                              const snn_hip_conv2d_params& p,
+                              hipStream_t stream) {
+  Gather g;
+  fill_gather(p, direction, &g);
+  constexpr int BM = 64, BN = 64;
+  const unsigned tiles_m = static_cast<unsigned>(ceil_div(g.m_total, BM));
+  const unsigned tiles_n = static_cast<unsigned>(ceil_div(g.n_total, BN));
+  const unsigned n_tiles = tiles_m * tiles_n;
+  const int n_chunks = ceil_div(g.k_total, kBK);
+  const unsigned src_bytes = static_cast<unsigned>(
+      static_cast<size_t>(g.batch) * g.src_rows * g.src_cols * g.src_ch * 2);
+  const unsigned wgt_bytes = static_cast<unsigned>(
+      static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
+      p.features * 2);
+  KernelTimer timer(stream);
+  auto launch = [&](auto kernel, int b_floats) {
+    hipLaunchKernelGGL(
+        kernel, dim3(n_tiles, 1), dim3(kThreads),
+        2 * sizeof(float) * (k_inner_floats(BM) + b_floats), stream, src,
+        filter, dst, g, src_bytes, wgt_bytes, tiles_n, n_tiles, n_chunks);
+  };
+  if (direction == SNN_HIP_FORWARD)
+    launch(conv_igemm_kernel<BM, BN, 2, 2, false, false, false, false, _Float16>,
+           row_inner_floats(BN));
+  else if (g.div_rows != 1 || g.div_cols != 1)
+    launch(conv_igemm_kernel<BM, BN, 2, 2, true, true, false, false, _Float16>,
+           k_inner_floats(BN));
+  else
+    launch(conv_igemm_kernel<BM, BN, 2, 2, true, false, false, false, _Float16>,
+           k_inner_floats(BN));
+  SNN_HIP_CHECK_LAUNCH();
   return SNN_HIP_OK;
 }
 

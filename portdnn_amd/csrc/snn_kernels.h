@@ -223,19 +223,30 @@ bool gemm_nt_f16_supports(int m, int k, int n);
 int launch_gemm_nt_f16(const _Float16* x, const _Float16* w, _Float16* y, int m,
                        int k, int n, hipStream_t stream);
 
-// Half-precision forward convolution and input gradient on the binary16 matrix
-// cores (conv2d_gather.hip): stride-1 unpadded 1x1 layers on the row-major
-// GEMM kernels above, stride-1 layers that fill the GPU on the LDS-tile kernel, every
-// other window (up to 12 x 12), stride (input gradient: up to 16 classes) and
-// channel count on the gathering kernel.  The launch returns -1 when none takes
-// the shape or there is no room for its temporaries; `workspace` of
-// conv2d_f16_workspace_halves halves, 16-byte aligned, saves those.
+// Half-precision forward convolution and input gradient (conv2d_gather.hip):
+// stride-1 unpadded 1x1 layers on the row-major GEMM kernels above, stride-1
+// layers that fill the GPU on the LDS-tile kernel, every other window (up to
+// 12 x 12), stride (input gradient: up to 16 classes) and channel count on the
+// gathering kernel or, where that is the faster one, the general kernel below.
+// Returns -1 when the caller's own kernel is the faster one (`otherwise_us`, by
+// default the direct kernel's time), none of these takes the shape or there is
+// no room for temporaries; `workspace` of conv2d_f16_workspace_halves halves,
+// 16-byte aligned, saves those.
 size_t conv2d_f16_workspace_halves(int direction,
                                    const snn_hip_conv2d_params& p);
 int launch_conv2d_f16(int direction, const _Float16* input,
                       const _Float16* filter, _Float16* output,
                       const snn_hip_conv2d_params& p, _Float16* workspace,
-                      size_t workspace_elems, hipStream_t stream);
+                      size_t workspace_elems, hipStream_t stream,
+                      double otherwise_us = 1e30);
+// The general implicit-GEMM kernel on binary16 tensors (conv2d_igemm.hip): no
+// temporary.  Features (and forward channels) in multiples of 4; source and
+// filter, and a forward output, 16-byte aligned.
+bool conv2d_general_f16_supports(int direction, const snn_hip_conv2d_params& p);
+int launch_conv2d_general_f16(int direction, const _Float16* src,
+                              const _Float16* filter, _Float16* dst,
+                              const snn_hip_conv2d_params& p,
+                              hipStream_t stream);
 
 // Forward convolution (with bias and activation, if asked for) and input
 // gradient in fp32 on the same gathering kernel: every window, stride, channel

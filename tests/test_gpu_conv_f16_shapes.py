@@ -1,13 +1,16 @@
 """Binary16 forward convolutions and input gradients at the sizes where the
 gathering kernel can go wrong: edges of its tiles, ragged channel and feature
 counts, stride classes with few, unequal or no taps, reductions shared by
-work-groups, filters that are not 16-byte aligned.
+work-groups, filters that are not 16-byte aligned, infinite weights, launches
+recorded into a graph; and short launches, which other kernels take.
 
 Bound: the result is rounded to binary16 once (2^-11 of its magnitude) and its
 n products are added in fp32, each addition rounding by at most 2^-24 of a
 partial sum, which for the U[-1,1] operands here is of the size of the outputs:
 |gpu - ref| <= 2^-11 |ref| + n 2^-24 S + 2^-24 (subnormals), S the largest |ref|.
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -49,6 +52,10 @@ SHAPES = [
     (3, 21, 22, 35, 45, 1, 2, True),    # strided 1x1, odd: copied subsampled
     (2, 17, 19, 30, 66, 1, 3, False),   # ... even counts, VALID
     (20, 20, 21, 64, 203, 3, 1, True),  # many tiles, runs of odd features
+    (4, 29, 29, 36, 44, 1, 1, True),    # short: the general kernel, no launch
+    (3, 30, 28, 72, 20, 3, 2, True),    # ... in front of it; stride 2
+    (1, 67, 50, 96, 3, 3, 3, True),     # ... the direct kernel's gradient
+    (10, 58, 43, 6, 40, 1, 2, True),    # ... and forward
 ]
 
 
@@ -72,16 +79,87 @@ def test_conv_f16_shapes(shape, direction):
                            else features)
     _, rec = ops.workspace_size(p, direction, ALGO.IM2COL, DTYPE.F16)
     block = torch.full((rec + 4096,), 7.0, dtype=torch.float16, device="cuda")
-    for fil, ws in ((db, None), (db, block[:rec] if rec else None),
-                    (shifted, None)):
+    for fil, ws, at in ((db, None, 0), (db, block[:rec] if rec else None, 0),
+                        (shifted, None, 0), (db, None, 1)):
         guard = torch.full((n_out + 4096,), 7.0, dtype=torch.float16,
                            device="cuda")
         got = ops.conv2d(da, fil, p, direction, ALGO.IM2COL, workspace=ws,
-                         out=guard[:n_out])
+                         out=guard[at:at + n_out])
         assert_rounded_once(got.float().cpu().numpy(), ref, n,
-                            (shape, direction, ws is None, fil is db))
-        assert torch.all(guard[n_out:] == 7.0)
+                            (shape, direction, ws is None, fil is db, at))
+        assert torch.all(guard[:at] == 7.0)
+        assert torch.all(guard[at + n_out:] == 7.0)
     assert torch.all(block[rec:] == 7.0)
+
+
+def graph_node_types(graph):
+    """The node types of a torch.cuda.CUDAGraph made with keep_graph=True."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    raw = ctypes.c_void_p(graph.raw_cuda_graph())
+    count = ctypes.c_size_t()
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(count)) == 0
+    nodes = (ctypes.c_void_p * count.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(count)) == 0
+    types = []
+    for node in nodes:
+        kind = ctypes.c_int()
+        assert hip.hipGraphNodeGetType(ctypes.c_void_p(node),
+                                       ctypes.byref(kind)) == 0
+        types.append(kind.value)
+    return types
+
+
+def check_recorded(call, refill, n_products, what):
+    """Records call(out), which may launch kernels only, and compares three
+    replays on refilled operands with eager calls."""
+    out = call(None)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call(out)
+    assert set(graph_node_types(graph)) == {0}, what  # hipGraphNodeTypeKernel
+    graph.instantiate()
+    for seed in (1, 2, 3):
+        refill(seed)
+        want = call(None).float().cpu().numpy()
+        out.fill_(7.0)
+        graph.replay()
+        torch.cuda.synchronize()
+        # (both sides round once, and add in orders of their own)
+        got = out.float().cpu().numpy()
+        bound = 2 * (2.0**-11 * np.abs(want) + 2.0**-24 +
+                     n_products * 2.0**-24 * np.abs(want).max())
+        assert np.all(np.abs(got - want) <= bound), (what, seed)
+
+
+@pytest.mark.parametrize("shape,direction", [
+    ((2, 16, 16, 20, 32, 3, 1, True), DIRECTION.FORWARD),
+    ((2, 16, 16, 20, 32, 3, 1, True), DIRECTION.INPUT_BACKPROP),
+    ((9, 57, 43, 72, 96, 3, 2, True), DIRECTION.FORWARD),
+    ((9, 57, 43, 72, 96, 3, 2, True), DIRECTION.INPUT_BACKPROP),
+    ((2, 7, 7, 480, 72, 3, 2, True), DIRECTION.FORWARD),
+    ((2, 7, 7, 480, 72, 3, 2, True), DIRECTION.INPUT_BACKPROP),
+    ((2, 17, 16, 36, 68, 3, 1, True), DIRECTION.INPUT_BACKPROP),
+    ((2, 12, 12, 33, 40, 3, 1, True), DIRECTION.FORWARD),
+    ((2, 12, 12, 40, 33, 3, 1, True), DIRECTION.INPUT_BACKPROP)], ids=str)
+def test_conv_f16_recorded_without_a_workspace(shape, direction):
+    """Counts in multiples of 4, and small launches of any: kernels only."""
+    batch, rows, cols, channels, features, window, stride, same = shape
+    p = ops.conv_params(batch, rows, cols, channels, features, window, stride,
+                        same)
+    n_a, n_b, n_out = ops.conv_sizes(p, direction)
+    a = torch.empty(n_a, dtype=torch.float16, device="cuda")
+    b = torch.empty(n_b, dtype=torch.float16, device="cuda")
+
+    def refill(seed):
+        rng = np.random.default_rng(seed)
+        a.copy_(dev(uniform(rng, n_a), torch.float16))
+        b.copy_(dev(uniform(rng, n_b), torch.float16))
+
+    refill(0)
+    check_recorded(
+        lambda out: ops.conv2d(a, b, p, direction, ALGO.IM2COL, out=out),
+        refill, window * window * max(channels, features), (shape, direction))
 
 
 @pytest.mark.parametrize("shape,direction", [
