@@ -194,7 +194,8 @@ def test_conv_f16_infinite_filter_stays(shape, direction):
 
 
 @pytest.mark.parametrize("m,k,n", [(32, 64, 64), (33, 40, 24), (257, 100, 130),
-                                   (640, 1000, 30)])
+                                   (640, 1000, 30), (2588, 14, 56),
+                                   (97, 1189, 338)])
 @pytest.mark.parametrize("trans_b", [False, True])
 def test_matmul_f16_ragged(m, k, n, trans_b):
     rng = np.random.default_rng(4200 + m + k + n)
@@ -205,3 +206,21 @@ def test_matmul_f16_ragged(m, k, n, trans_b):
     got = ops.matmul(dev(a, torch.float16), dev(b, torch.float16), 1, m, k, n,
                      trans_b=trans_b)
     assert_rounded_once(got.float().cpu().numpy(), ref, k, (m, k, n, trans_b))
+
+
+@pytest.mark.parametrize("m,k,n", [(257, 100, 130), (96, 1189, 40)])
+@pytest.mark.parametrize("trans_b", [False, True])
+def test_matmul_f16_recorded(m, k, n, trans_b):
+    """A reduction of no whole chunks of 64: kernels only."""
+    a = torch.empty(m * k, dtype=torch.float16, device="cuda")
+    b = torch.empty(k * n, dtype=torch.float16, device="cuda")
+
+    def refill(seed):
+        rng = np.random.default_rng(seed)
+        a.copy_(dev(uniform(rng, m * k), torch.float16))
+        b.copy_(dev(uniform(rng, k * n), torch.float16))
+
+    refill(0)
+    check_recorded(
+        lambda out: ops.matmul(a, b, 1, m, k, n, trans_b=trans_b, out=out),
+        refill, k, (m, k, n, trans_b))
