@@ -1589,6 +1589,27 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
            : static_cast<double>(p.batch) * p.out_rows * p.out_cols * p.features;
   // One short loop per output (14x14x33 -> 64, 1x1: 5.3 / 17.8 us).
   if (products <= 64 && outputs <= (1 << 16)) return false;
+  // Features of no whole piece: a short loop per output as well, where the
+  // filter's pack and the copy would be launches of their own (13x15x19 8 -> 135,
+  // 1x1 stride 2: 4.3 / 7.9; gradient of 8x21x21 24 <- 2, 2x2: 4.4 / 7.9; 41 random
+  // layers, none slower, 0.55 of the time in the middle; but 12x134x134 4 -> 3 with
+  // 2^20 outputs 9.1 / 8.5).
+  const int loop = grad ? p.features * ceil_div(p.window_rows, p.stride_rows) *
+                              ceil_div(p.window_cols, p.stride_cols)
+                        : static_cast<int>(products) / 2;
+  if (p.features % 4 != 0 && loop < 8 && macs < double(1 << 23) &&
+      outputs < (1 << 19))
+    return false;
+  // At most one 64 x 64 tile per compute unit and a short reduction in whole
+  // pieces: latencies are all there is, and those are shorter there (25x14x18
+  // 56 -> 424, 1x1 stride 2: 4.8 / 6.3; 11x14x10 24 -> 88, 1x1: 4.2 / 5.5; gradient
+  // of 30x30 441 <- 52, 1x1: 4.7 / 6.3; 0.89 of the time in the middle of 185
+  // random layers, four of them up to 9 % slower).
+  const double tiles = std::ceil(outputs / (grad ? p.channels : p.features) / 64) *
+                       ceil_div(grad ? p.channels : p.features, 64);
+  if (p.features % 4 == 0 && (grad ? !strided : p.channels % 4 == 0) &&
+      products <= 96 && tiles <= kNumCus)
+    return false;
   // Few outputs of a long reduction meet through atomics there, in one pass less
   // (2x19x14 720 -> 80, 3x3 stride 2: 12.5 / 13.7 us; 4x14x14 144 -> 224, 5x5,
   // 24 / 26 and its gradient 24 / 30; but 3x14x14 192 <- 128, 3x3, 12.7 / 12.0).
