@@ -1822,7 +1822,8 @@ static int launch_filter_backprop(const float* x, const float* dy, float* dw,
   if (conv2d_stem_filter_backprop_supports(p) &&
       (reinterpret_cast<uintptr_t>(dw) & 15u) == 0 &&
       SNN_TUNING_ENV("SNN_HIP_STEM_OFF") == nullptr)
-    return launch_conv2d_stem_filter_backprop_f32(x, dy, dw, p, stream);
+    return launch_conv2d_stem_filter_backprop_f32(x, dy, dw, p, workspace,
+                                                  workspace_elems, stream);
   if (conv2d_filter_backprop_direct_f32_wanted(p, reproducible)) {
     // partial filters go to the workspace when it holds them, else to a
     // stream-ordered temporary

@@ -799,22 +799,37 @@ bool conv2d_stem_filter_backprop_supports(const snn_hip_conv2d_params& p) {
   return make_geom(p, &g) && p.out_cols <= 4 * kMaxTSteps;
 }
 
-// dw 16-byte aligned.  The partial filters (one of 147 x 64 floats per
-// work-group) live in a stream-ordered temporary.
+// One partial filter of 147 x 64 floats per work-group; 0: not supported.
+size_t conv2d_stem_filter_backprop_partial_floats(
+    const snn_hip_conv2d_params& p) {
+  StemGeom g;
+  if (!make_geom(p, &g) || p.out_cols > 4 * kMaxTSteps) return 0;
+  return static_cast<size_t>(p.batch) * g.n_bands * kPartFloats;
+}
+
+// dw 16-byte aligned.  The partial filters live in the workspace when it holds
+// them, else in a stream-ordered temporary.
 int launch_conv2d_stem_filter_backprop_f32(const float* x, const float* dy,
                                            float* dw,
                                            const snn_hip_conv2d_params& p,
+                                           float* workspace,
+                                           size_t workspace_elems,
                                            hipStream_t stream) {
   StemGeom g;
   if (!make_geom(p, &g) || p.out_cols > 4 * kMaxTSteps)
     return SNN_HIP_INVALID_ALGORITHM;
   const unsigned n_groups = static_cast<unsigned>(p.batch * g.n_bands);
-  void* ptr = nullptr;
-  if (temp_malloc_async(&ptr, static_cast<size_t>(n_groups) * kPartFloats *
-                                  sizeof(float),
-                        stream) != hipSuccess)
-    return SNN_HIP_ALLOCATION_PROBLEM;
-  float* part = static_cast<float*>(ptr);
+  const size_t part_floats = static_cast<size_t>(n_groups) * kPartFloats;
+  float* part = workspace;
+  const bool temporary = workspace == nullptr || workspace_elems < part_floats ||
+                         (reinterpret_cast<uintptr_t>(workspace) & 15u) != 0;
+  if (temporary) {
+    void* ptr = nullptr;
+    if (temp_malloc_async(&ptr, part_floats * sizeof(float), stream) !=
+        hipSuccess)
+      return SNN_HIP_ALLOCATION_PROBLEM;
+    part = static_cast<float*>(ptr);
+  }
   // the band's rows, and at the end the accumulators of four waves
   const size_t lds_bytes = std::max(
       (static_cast<size_t>(g.lds_rows + 1) * g.row_floats + 64) * sizeof(float),
@@ -835,7 +850,7 @@ int launch_conv2d_stem_filter_backprop_f32(const float* x, const float* dy,
                      reinterpret_cast<const float4v*>(part),
                      reinterpret_cast<float4v*>(dw), static_cast<int>(n_groups));
   const hipError_t err = hipGetLastError();
-  temp_free_async(part, stream);
+  if (temporary) temp_free_async(part, stream);
   if (err != hipSuccess) return report_hip_error(err, "stem filter backprop");
   return SNN_HIP_OK;
 }

@@ -361,7 +361,12 @@ bool widened_filter_gradient(const snn_hip_conv2d_params& p, size_t elem,
   plan->dy = q.features != p.features ? part(y_pixels * q.features) : 0;
   plan->dw = part(filter_rows * q.features);
   plan->inner =
-      half ? part(f16_workspace_halves(q, SNN_HIP_FILTER_BACKPROP)) : 0;
+      part(half ? f16_workspace_halves(q, SNN_HIP_FILTER_BACKPROP)
+           : conv2d_stem_filter_backprop_supports(q)
+               ? conv2d_stem_filter_backprop_partial_floats(q)
+           : conv2d_filter_backprop_direct_f32_wanted(q)
+               ? conv2d_filter_backprop_direct_f32_partial_floats(q)
+               : 0);
   const double macs = static_cast<double>(y_pixels) * p.window_rows *
                       p.window_cols * p.channels * p.features;
   const double tiles = macs * up(p.channels, 64) / p.channels *

@@ -189,8 +189,8 @@ int launch_conv2d_filter_backprop_direct_f16(const _Float16* input,
 bool conv2d_stem_supports(const snn_hip_conv2d_params& p);
 int launch_conv2d_stem_f32(const float* x, const float* w, float* y,
                            const snn_hip_conv2d_params& p, hipStream_t stream);
-// ... and its filter gradient (dw 16-byte aligned; partial filters in a
-// stream-ordered temporary).
+// ... and its gradients (dx and dw 16-byte aligned; the filter gradient's
+// partial filters in the workspace, or a stream-ordered temporary).
 bool conv2d_stem_input_backprop_supports(const snn_hip_conv2d_params& p);
 int launch_conv2d_stem_input_backprop_f32(const float* dy, const float* w,
                                           float* dx,
@@ -200,9 +200,13 @@ int launch_conv2d_stem_input_backprop_f32(const float* dy, const float* w,
 // the same bits every run)
 bool conv2d_stem_input_backprop_reproducible(const snn_hip_conv2d_params& p);
 bool conv2d_stem_filter_backprop_supports(const snn_hip_conv2d_params& p);
+size_t conv2d_stem_filter_backprop_partial_floats(
+    const snn_hip_conv2d_params& p);
 int launch_conv2d_stem_filter_backprop_f32(const float* x, const float* dy,
                                            float* dw,
                                            const snn_hip_conv2d_params& p,
+                                           float* workspace,
+                                           size_t workspace_elems,
                                            hipStream_t stream);
 // The same in half precision with fp32 accumulation (gemm_wreg_f16.hip):
 // k = 64, 128, 256 or 512.

@@ -1,6 +1,7 @@
 """Filter gradients whose channel or feature counts are rounded up in a copy:
 either count or both odd, only one of them, first layers, every window, with the
-queried workspace, without one, and with operands off 16-byte alignment.
+queried workspace, without one, recorded into a graph, and with operands off
+16-byte alignment.
 
 Bound: n products added in fp32, each addition rounding by at most 2^-24 of a
 partial sum, which for the U[-1,1] operands here stays below twice the largest
@@ -13,6 +14,7 @@ import torch
 
 from portdnn_amd import ops
 from portdnn_amd.capi import ALGO, DIRECTION, DTYPE
+from test_gpu_conv_f16_shapes import check_recorded
 from test_gpu_parity import ORACLE_FN, dev, oracle_params, uniform
 
 pytestmark = pytest.mark.gpu
@@ -69,3 +71,34 @@ def test_filter_gradient_widened(shape, dtype):
         assert np.all(err <= bound), (shape, ws is None, err.max())
         assert torch.all(guard[n_dw:] == 7.0)
     assert torch.all(block[rec:] == 7.0)
+
+
+@pytest.mark.parametrize("shape,dtype", [
+    ((8, 112, 112, 3, 61, 7, 2, True), DTYPE.F32),
+    ((20, 100, 99, 3, 42, 3, 2, True), DTYPE.F32),
+    ((10, 50, 50, 8, 33, 3, 1, True), DTYPE.F32),
+    ((16, 28, 28, 65, 66, 3, 1, True), DTYPE.F16),
+    ((20, 100, 99, 3, 44, 3, 2, True), DTYPE.F16)], ids=str)
+def test_filter_gradient_widened_recorded(shape, dtype):
+    """The queried workspace holds all that the launches need."""
+    batch, rows, cols, channels, features, window, stride, same = shape
+    p = ops.conv_params(batch, rows, cols, channels, features, window, stride,
+                        same)
+    kind = torch.float16 if dtype == DTYPE.F16 else torch.float32
+    n_x, n_dy, n_dw = ops.conv_sizes(p, DIRECTION.FILTER_BACKPROP)
+    x = torch.empty(n_x, dtype=kind, device="cuda")
+    dy = torch.empty(n_dy, dtype=kind, device="cuda")
+    _, rec = ops.workspace_size(p, DIRECTION.FILTER_BACKPROP, ALGO.IM2COL,
+                                dtype)
+    ws = torch.empty(rec, dtype=kind, device="cuda")
+
+    def refill(seed):
+        rng = np.random.default_rng(seed)
+        x.copy_(dev(uniform(rng, n_x), kind))
+        dy.copy_(dev(uniform(rng, n_dy), kind))
+
+    refill(0)
+    check_recorded(
+        lambda out: ops.conv2d(x, dy, p, DIRECTION.FILTER_BACKPROP, ALGO.IM2COL,
+                               workspace=ws, out=out),
+        refill, batch * p.out_rows * p.out_cols, (shape, dtype))
