@@ -103,6 +103,11 @@ def _ptr(t):
     return ctypes.c_void_p(t.data_ptr()) if t is not None else None
 
 
+def _at(t):
+    """The address for _native; a missing operand is the entry point's error."""
+    return None if t is None else t.data_ptr()
+
+
 def workspace_size(p, direction, algorithm, dtype=None):
     """(required, recommended) elements; with a capi.DTYPE the element type's
     own answer (snn_hip_conv2d_workspace_size_for)."""
@@ -165,8 +170,7 @@ def conv2d(inp, fil, p, direction=DIRECTION.FORWARD, algorithm=ALGO.DIRECT,
     code = _native.conv2d(
         _address(_CONV_FN[direction, dtype]), direction, inp.data_ptr(),
         inp.numel(), fil.data_ptr(), fil.numel(), out.data_ptr(), p, algorithm,
-        None if workspace is None else workspace.data_ptr(),
-        0 if workspace is None else workspace.numel(), _stream())
+        _at(workspace), 0 if workspace is None else workspace.numel(), _stream())
     if code:
         capi.check(code)
     return out
@@ -254,11 +258,9 @@ def conv2d_bias_act(inp, fil, bias, p, algorithm, relu=True, workspace=None,
         _, rec = workspace_size(p, DIRECTION.FORWARD, algorithm)
         workspace = torch.empty(rec, dtype=inp.dtype, device=inp.device)
     code = _native.conv2d_bias_act(
-        _address("snn_hip_conv2d_forward_bias_act_f32"), inp.data_ptr(),
-        fil.data_ptr(), None if bias is None else bias.data_ptr(),
-        out.data_ptr(), p, algorithm, 1 if relu else 0,
-        None if workspace is None else workspace.data_ptr(),
-        0 if workspace is None else workspace.numel(), _stream())
+        _address("snn_hip_conv2d_forward_bias_act_f32"), _at(inp), _at(fil),
+        _at(bias), out.data_ptr(), p, algorithm, 1 if relu else 0,
+        _at(workspace), 0 if workspace is None else workspace.numel(), _stream())
     if code:
         capi.check(code)
     return out
@@ -337,7 +339,7 @@ def pooling_max_grad(inp, out, dy, p, op=POOL_OP.MAX, dx=None):
         dx = torch.empty_like(inp)
     code = _native.pooling_max_grad(
         _address("snn_hip_pooling_max_grad" + _suffix(inp)), inp.data_ptr(),
-        out.data_ptr(), dy.data_ptr(), dx.data_ptr(), p, op, _stream())
+        _at(out), _at(dy), dx.data_ptr(), p, op, _stream())
     if code:
         capi.check(code)
     return dx
@@ -423,8 +425,8 @@ def binaryop(lhs, rhs, lhs_dims, rhs_dims, op, out=None):
             size *= max(a, b)
         out = torch.empty(size, dtype=lhs.dtype, device=lhs.device)
     code = _native.binaryop(
-        _address("snn_hip_binaryop" + _suffix(lhs)), lhs.data_ptr(),
-        rhs.data_ptr(), out.data_ptr(), lhs_dims, rhs_dims, op, _stream())
+        _address("snn_hip_binaryop" + _suffix(lhs)), lhs.data_ptr(), _at(rhs),
+        out.data_ptr(), lhs_dims, rhs_dims, op, _stream())
     if code:
         capi.check(code)
     return out

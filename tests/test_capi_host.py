@@ -7,6 +7,7 @@ import re
 
 import numpy as np
 import pytest
+import torch
 
 from golden_cases import GOLDEN_DIR
 from portdnn_amd import capi, ops
@@ -332,3 +333,31 @@ def test_missing_library_fails_loudly(monkeypatch, tmp_path):
     monkeypatch.setattr(capi, "_LIB_PATH", str(tmp_path / "libsnn_hip.so"))
     with pytest.raises(capi.SnnHipError):
         capi.lib()
+
+
+@pytest.mark.parametrize("name", [n for n in dir(ops._native)
+                                  if not n.startswith("_")])
+def test_native_calls_refuse_a_wrong_argument_count(name):
+    for args in ((), (0,) * 5000):
+        with pytest.raises(TypeError):
+            getattr(ops._native, name)(*args)
+
+
+def test_a_missing_operand_is_the_entry_points_error(monkeypatch):
+    """None for a tensor that the call does not need itself reaches the C ABI
+    as a null pointer, which it refuses before anything is launched."""
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    t = torch.empty(4)
+    pool = ops.PoolParams(in_rows=1, in_cols=1, out_rows=1, out_cols=1,
+                          window_rows=1, window_cols=1, stride_rows=1,
+                          stride_cols=1, batch=1, channels=4)
+    conv = ops.conv_params(1, 1, 1, 2, 2, 1, 1, True)
+    for call in (
+            lambda: ops.conv2d_bias_act(None, t, t, conv, ALGO.DIRECT, out=t),
+            lambda: ops.conv2d_bias_act(t, None, t, conv, ALGO.DIRECT, out=t),
+            lambda: ops.pooling_max_grad(t, None, t, pool, dx=t),
+            lambda: ops.pooling_max_grad(t, t, None, pool, dx=t),
+            lambda: ops.binaryop(t, None, (4,), (4,), ops.BINARY_OP.ADD,
+                                 out=t)):
+        with pytest.raises(capi.SnnHipError):
+            call()
