@@ -161,6 +161,16 @@ SNN_HIP_API const char* snn_hip_last_error(void);
 SNN_HIP_API int snn_hip_kernel_timing_enable(int enable);
 SNN_HIP_API int snn_hip_kernel_timing_read(double* total_ms, int* kernels);
 
+/* Diagnostics for tests of the tile shapes (no counterpart in portDNN): the
+ * tile and the shares of a reduction that the gathering kernel takes for a
+ * forward convolution or input gradient behind the Tiled, Im2col and Matmul
+ * tags, for aligned operands and a workspace of the recommended size.
+ * SNN_HIP_INVALID_ALGORITHM where such a launch runs on another kernel. */
+SNN_HIP_API int snn_hip_conv2d_gather_tile(const snn_hip_conv2d_params* params,
+                                           int direction, int dtype,
+                                           int* pixels, int* features,
+                                           int* splits);
+
 /* Diagnostics for the stream-ordered temporaries some launches take when the
  * caller passes no workspace (no counterpart in portDNN, whose temporaries
  * come from backend.allocate): bytes currently reserved by, and the high-water

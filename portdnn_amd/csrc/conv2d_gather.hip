@@ -1470,21 +1470,33 @@ bool stream_captures(hipStream_t stream) {
 
 }  // namespace
 
-size_t conv2d_f16_workspace_halves(int direction,
-                                   const snn_hip_conv2d_params& p) {
+bool conv2d_gather_tile_f16(int direction, const snn_hip_conv2d_params& p,
+                            GatherTile* tile) {
   snn_hip_conv2d_params q;
-  if (is_rows_gemm(direction, p)) return 0;
-  if (rowtile_params(direction, p, &q))
-    return static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
-           p.features;
+  if (is_rows_gemm(direction, p) || rowtile_params(direction, p, &q))
+    return false;
   const GatherPlan& plan = make_plan<_Float16>(direction, p);
-  if (!plan.ok) return 0;
+  if (!plan.ok) return false;
   const Products r = products_of(direction, p);
   if (std::min(conv2d_general_f16_supports(direction, p) ? general_f16_us(r)
                                                          : kNever,
                direct_f16_us(direction, p, r)) <
       gather_f16_us(plan, plan.from == kPacked, false))
-    return 0;
+    return false;
+  *tile = {kTilesF16[plan.tile].pixels, kTilesF16[plan.tile].features,
+           plan.n_splits};
+  return true;
+}
+
+size_t conv2d_f16_workspace_halves(int direction,
+                                   const snn_hip_conv2d_params& p) {
+  snn_hip_conv2d_params q;
+  if (!is_rows_gemm(direction, p) && rowtile_params(direction, p, &q))
+    return static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
+           p.features;
+  GatherTile tile;
+  if (!conv2d_gather_tile_f16(direction, p, &tile)) return 0;
+  const GatherPlan& plan = make_plan<_Float16>(direction, p);
   // (with room for the packed filter also where the gradient's is read in
   // place, for one that is not 16-byte aligned; that of a 1x1 layer would take
   // a temporary)
@@ -1670,6 +1682,15 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
   // 32x56x56 128 <- 128, 3x3 stride 2, 140 / 92 us; 256 <- 512, 1x1 stride 2,
   // 95 / 90; 17x27x27 96 <- 256, 5x5, 178 / 160; 5x82x107 16 <- 75 129 / 68.
   return true;
+}
+
+bool conv2d_gather_tile_f32(int direction, const snn_hip_conv2d_params& p,
+                            GatherTile* tile) {
+  if (!positive(p) || !conv2d_gather_f32_wanted(direction, p)) return false;
+  const GatherPlan& plan = make_plan<float>(direction, p);
+  *tile = {kTilesF32[plan.tile].pixels, kTilesF32[plan.tile].features,
+           plan.n_splits};
+  return plan.ok;
 }
 
 size_t conv2d_gather_f32_workspace_floats(int direction,

@@ -1374,6 +1374,32 @@ int snn_hip_conv2d_default_algorithm_for(const snn_hip_conv2d_params* params,
   return default_algorithm(*params, direction, dtype);
 }
 
+int snn_hip_conv2d_gather_tile(const snn_hip_conv2d_params* params,
+                               int direction, int dtype, int* pixels,
+                               int* features, int* splits) {
+  if (params == nullptr || pixels == nullptr || features == nullptr ||
+      splits == nullptr ||
+      (dtype != SNN_HIP_DTYPE_F32 && dtype != SNN_HIP_DTYPE_F16))
+    return SNN_HIP_INVALID_PARAMETER;
+  const snn_hip_conv2d_params& p = *params;
+  const int v = validate(p);
+  if (v != SNN_HIP_OK) return v;
+  const bool half = dtype == SNN_HIP_DTYPE_F16;
+  GatherTile tile;
+  if (p.input_format != 0 || p.groups != 1 ||
+      (direction != SNN_HIP_FORWARD && direction != SNN_HIP_INPUT_BACKPROP) ||
+      (half && (direction == SNN_HIP_FORWARD
+                    ? conv2d_few_f16_forward_supports(p)
+                    : conv2d_few_f16_input_backprop_supports(p))) ||
+      !(half ? conv2d_gather_tile_f16(direction, p, &tile)
+             : conv2d_gather_tile_f32(direction, p, &tile)))
+    return SNN_HIP_INVALID_ALGORITHM;
+  *pixels = tile.pixels;
+  *features = tile.features;
+  *splits = tile.splits;
+  return SNN_HIP_OK;
+}
+
 int snn_hip_depthwise_conv2d_forward_f32(
     const float* input, const float* filter, float* output,
     const snn_hip_depthwise_params* params, void* stream) {

@@ -243,6 +243,13 @@ int launch_conv2d_f16(int direction, const _Float16* input,
                       const snn_hip_conv2d_params& p, _Float16* workspace,
                       size_t workspace_elems, hipStream_t stream,
                       double otherwise_us = 1e30);
+// The tile that a launch with aligned operands and that workspace takes on the
+// gathering kernel; false where it runs on another one.
+struct GatherTile { int pixels, features, splits; };
+bool conv2d_gather_tile_f16(int direction, const snn_hip_conv2d_params& p,
+                            GatherTile* tile);
+bool conv2d_gather_tile_f32(int direction, const snn_hip_conv2d_params& p,
+                            GatherTile* tile);
 // The general implicit-GEMM kernel on binary16 tensors (conv2d_igemm.hip): no
 // temporary.  Features (and forward channels) in multiples of 4; source and
 // filter, and a forward output, 16-byte aligned.

@@ -132,6 +132,19 @@ def default_algorithm(p, direction, dtype=None):
         ctypes.byref(p), direction, dtype)
 
 
+def gather_tile(p, direction, dtype):
+    """(pixels, features, splits) of the gathering kernel's tile, or None where
+    such a launch runs on another kernel (snn_hip_conv2d_gather_tile)."""
+    pixels, features, splits = (ctypes.c_int() for _ in range(3))
+    code = capi.lib().snn_hip_conv2d_gather_tile(
+        ctypes.byref(p), direction, dtype, ctypes.byref(pixels),
+        ctypes.byref(features), ctypes.byref(splits))
+    if code == STATUS.INVALID_ALGORITHM:
+        return None
+    capi.check(code)
+    return pixels.value, features.value, splits.value
+
+
 _CONV_FN = {
     (DIRECTION.FORWARD, torch.float32): "snn_hip_conv2d_forward_f32",
     (DIRECTION.INPUT_BACKPROP, torch.float32):

@@ -361,3 +361,47 @@ def test_a_missing_operand_is_the_entry_points_error(monkeypatch):
                                  out=t)):
         with pytest.raises(capi.SnnHipError):
             call()
+
+
+@pytest.mark.parametrize("dtype,shape,direction,tile,shared", [
+    # (batch, rows, cols, channels, features, window, stride, same)
+    (capi.DTYPE.F16, (2, 7, 7, 512, 72, 3, 1, True), 0, (128, 32), True),
+    (capi.DTYPE.F16, (5, 9, 9, 264, 264, 3, 2, True), 1, (128, 32), True),
+    (capi.DTYPE.F16, (5, 41, 43, 70, 65, 1, 2, True), 0, (64, 64), False),
+    (capi.DTYPE.F16, (16, 40, 40, 64, 200, 3, 2, True), 0, (128, 64), False),
+    (capi.DTYPE.F16, (20, 20, 21, 64, 203, 3, 1, True), 0, (128, 128), False),
+    (capi.DTYPE.F16, (128, 56, 56, 128, 128, 3, 2, True), 0, (256, 128), False),
+    (capi.DTYPE.F16, (128, 56, 56, 128, 128, 3, 2, True), 1, (256, 128), False),
+    (capi.DTYPE.F16, (4, 29, 29, 36, 44, 1, 1, True), 0, None, None),
+    (capi.DTYPE.F16, (10, 58, 43, 6, 40, 1, 2, True), 0, None, None),
+    (capi.DTYPE.F16, (128, 224, 224, 3, 64, 7, 2, True), 0, None, None),
+    (capi.DTYPE.F32, (1, 24, 24, 3, 512, 7, 2, True), 1, (128, 32), True),
+    (capi.DTYPE.F32, (2, 7, 7, 480, 70, 3, 2, True), 0, (64, 64), True),
+    (capi.DTYPE.F32, (4, 41, 43, 35, 133, 1, 2, True), 0, (128, 32), False),
+    (capi.DTYPE.F32, (9, 57, 43, 72, 96, 3, 2, True), 1, (64, 64), False),
+    (capi.DTYPE.F32, (13, 15, 19, 8, 135, 1, 2, True), 0, None, None),
+    (capi.DTYPE.F32, (25, 14, 18, 56, 424, 1, 2, True), 0, None, None)],
+    ids=str)
+def test_gather_tile(dtype, shape, direction, tile, shared):
+    """The kernels and tiles that the GPU tests name for their shapes."""
+    got = ops.gather_tile(ops.conv_params(*shape), direction, dtype)
+    if tile is None:
+        assert got is None
+    else:
+        assert got is not None and got[:2] == tile
+        assert (got[2] > 1) == shared
+
+
+def test_gather_tile_refuses_bad_arguments():
+    fn = capi.lib().snn_hip_conv2d_gather_tile
+    v = [ctypes.c_int() for _ in range(3)]
+    out = [ctypes.byref(x) for x in v]
+    p = _conv()
+    assert fn(None, 0, 0, *out) == STATUS.INVALID_PARAMETER
+    assert fn(ctypes.byref(p), 0, 7, *out) == STATUS.INVALID_PARAMETER
+    assert fn(ctypes.byref(p), 0, 0, out[0], out[1], None) == \
+        STATUS.INVALID_PARAMETER
+    assert fn(ctypes.byref(_conv(batch=-1)), 0, 0, *out) != STATUS.OK
+    for direction in (DIRECTION.FILTER_BACKPROP, 5, -1):
+        assert fn(ctypes.byref(p), direction, 0, *out) == \
+            STATUS.INVALID_ALGORITHM

@@ -48,10 +48,13 @@ SHAPES = [
     (2, 7, 7, 512, 72, 3, 1, True),     # long reduction, few tiles: shared
     (5, 9, 9, 264, 264, 3, 2, True),    # ... by classes of unequal length
     (9, 57, 43, 72, 96, 3, 2, True),    # many tiles, ragged rows
-    (16, 40, 40, 64, 200, 3, 2, True),  # tiles of 256 pixels
+    (16, 40, 40, 64, 200, 3, 2, True),  # tiles of 128 pixels and of 64
     (3, 21, 22, 35, 45, 1, 2, True),    # strided 1x1, odd: copied subsampled
     (2, 17, 19, 30, 66, 1, 3, False),   # ... even counts, VALID
     (20, 20, 21, 64, 203, 3, 1, True),  # many tiles, runs of odd features
+    (5, 41, 43, 70, 65, 1, 2, True),    # large enough to be copied subsampled
+    (3, 33, 35, 130, 66, 1, 3, False),
+    (6, 40, 41, 64, 37, 1, 4, False),   # sixteen classes, odd features
     (4, 29, 29, 36, 44, 1, 1, True),    # short: the general kernel, no launch
     (3, 30, 28, 72, 20, 3, 2, True),    # ... in front of it; stride 2
     (1, 67, 50, 96, 3, 3, 3, True),     # ... the direct kernel's gradient
@@ -90,6 +93,35 @@ def test_conv_f16_shapes(shape, direction):
         assert torch.all(guard[:at] == 7.0)
         assert torch.all(guard[at + n_out:] == 7.0)
     assert torch.all(block[rec:] == 7.0)
+
+
+# The tiles of 256 pixels: packed filters (forward) and filters in place
+# (gradients whose features fill whole pieces), whole chunks per tap or not,
+# outputs in whole pieces or through LDS, a last tile with a remainder.
+TILES = [
+    ((33, 45, 23, 8, 16, 3, 1, True), 0, (256, 64)),
+    ((17, 45, 23, 32, 130, 2, 1, True), 0, (256, 64)),
+    ((33, 45, 23, 32, 16, 2, 1, True), 0, (256, 64)),
+    ((17, 45, 23, 20, 130, 2, 1, True), 0, (256, 64)),
+    ((33, 45, 23, 8, 65, 2, 1, True), 0, (256, 128)),
+    ((33, 45, 23, 32, 65, 2, 1, True), 0, (256, 128)),
+    ((9, 64, 40, 32, 136, 2, 1, True), 0, (256, 128)),
+    ((9, 64, 40, 20, 136, 2, 1, True), 0, (256, 128)),
+    ((66, 21, 23, 8, 32, 2, 3, True), 1, (256, 64)),
+    ((66, 21, 23, 20, 16, 2, 3, True), 1, (256, 64)),
+    ((66, 21, 23, 20, 65, 2, 3, True), 1, (256, 64)),
+    ((66, 21, 23, 96, 32, 2, 3, True), 1, (256, 128)),
+    ((66, 21, 23, 67, 32, 2, 3, True), 1, (256, 128)),
+    ((66, 21, 23, 67, 16, 2, 3, True), 1, (256, 128)),
+    ((66, 45, 23, 96, 65, 2, 3, True), 1, (256, 128)),
+]
+
+
+@pytest.mark.parametrize("shape,direction,tile", TILES, ids=str)
+def test_conv_f16_large_tiles(shape, direction, tile):
+    p = ops.conv_params(*shape)
+    assert ops.gather_tile(p, direction, DTYPE.F16)[:2] == tile
+    test_conv_f16_shapes(shape, direction)
 
 
 def graph_node_types(graph):

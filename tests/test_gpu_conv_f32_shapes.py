@@ -42,8 +42,11 @@ SHAPES = [
     (3, 21, 22, 35, 45, 1, 2, True),    # strided 1x1, odd: copied subsampled
     (2, 17, 19, 30, 66, 1, 3, False),   # ... even counts, VALID
     (20, 20, 21, 64, 203, 3, 1, True),  # many tiles, runs of odd features
+    (4, 41, 43, 35, 133, 1, 2, True),   # large enough to be copied subsampled
+    (3, 33, 35, 130, 66, 1, 3, False),
+    (4, 40, 41, 32, 33, 1, 4, False),   # sixteen classes, odd features
     (13, 15, 19, 8, 135, 1, 2, True),   # short launches: the direct kernel
-    (8, 21, 21, 24, 2, 2, 1, False),    # ... its gradient
+    (7, 45, 45, 6, 6, 1, 1, False),     # ... and its gradient
     (25, 14, 18, 56, 424, 1, 2, True),  # ... the implicit-GEMM kernel
     (1, 30, 30, 441, 52, 1, 1, True),   # ... its gradient
 ]
