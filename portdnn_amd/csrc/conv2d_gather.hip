@@ -1543,18 +1543,17 @@ int launch_conv2d_f16(int direction, const _Float16* input,
     return status;
   }
   const Products r = products_of(direction, p);
-  const bool general =
-      both_aligned && conv2d_general_f16_supports(direction, p) &&
-      (direction == SNN_HIP_INPUT_BACKPROP || aligned(output));
-  const double general_us = general ? general_f16_us(r) : kNever;
-  const double direct_us = direct_f16_us(direction, p, r);
-
   const GatherPlan* plan = &make_plan<_Float16>(direction, p);
   const bool packs = plan->from == kPacked || !aligned(filter);
   const size_t room = workspace != nullptr && aligned(workspace)
                           ? workspace_elems * sizeof(_Float16) : 0;
   bool able = plan->ok && aligned(output) && (plan->widen || aligned(input));
   bool temporary = able && plan->workspace_bytes(packs) > room;
+  // (where the gathering kernel does not apply, large launches are faster
+  // through fp32 copies: 2x64x64x64 -> 64, 13x13 stride 2: 53 / 330 us)
+  bool general = both_aligned && conv2d_general_f16_supports(direction, p) &&
+                 (direction == SNN_HIP_INPUT_BACKPROP || aligned(output)) &&
+                 (able || r.macs < double(1 << 24));
   if (temporary && stream_captures(stream)) {
     // A launch that is recorded without room for the packed filter or the copy
     // keeps its reduction whole, or takes a kernel that needs no temporary.
@@ -1567,6 +1566,8 @@ int launch_conv2d_f16(int direction, const _Float16* input,
                                     p.channels % 64 != 0));
     able = !temporary || !other;
   }
+  const double general_us = general ? general_f16_us(r) : kNever;
+  const double direct_us = direct_f16_us(direction, p, r);
   const double gather_us =
       able ? gather_f16_us(*plan, packs, temporary) : kNever;
   if (std::min(otherwise_us, direct_us) < std::min(general_us, gather_us))

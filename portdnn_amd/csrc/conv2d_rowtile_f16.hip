@@ -672,7 +672,9 @@ bool launch_shape(const _Float16* input, const _Float16* wpk,
 // kernel / the other: 56x56x64 at batch 1 9.6 / 9.9 us, 128 50.7 / 58;
 // 28x28x128 at batch 32 19.4 / 18.7, 64 25.0 / 26.4; 14x14x256 at batch 64
 // 31.5 / 29.8, 128 39.1 / 42.6; 7x7x512 at batch 8 43 / 21, 128 56 / 52;
-// 112x112x128 at batch 4 (one work-group's tiles fill the LDS) 41 / 26.
+// 112x112x128 at batch 4 (one work-group's tiles fill the LDS) 41 / 26.  Windows
+// beyond 12 x 12 the other one does not take (gradient of 2x64x64x64 <- 64,
+// 13x13: 89 us, through fp32 136).
 bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p) {
   const size_t x = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols *
                    p.channels;
@@ -685,7 +687,9 @@ bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p) {
   if ((x > y ? x : y) * 2 > kMaxBufferBytes) return false;
   const RowTilePlan plan = make_plan(p);
   if (plan.lds_bytes == 0) return false;
-  if (p.window_rows * p.window_cols * p.channels <= 576) return true;
+  if (p.window_rows * p.window_cols * p.channels <= 576 ||
+      p.window_rows > 12 || p.window_cols > 12)
+    return true;
   const size_t wave_tiles = ceil_div(y / p.features, size_t{64}) *
                             static_cast<size_t>(p.features / 64);
   return wave_tiles >= 1536 &&

@@ -43,6 +43,8 @@ SHAPES = [
     (1, 16, 17, 32, 33, 1, 4, False),   # ... sixteen classes, odd features
     (1, 18, 18, 16, 16, 12, 1, True),   # the largest window
     (1, 20, 20, 8, 12, 13, 2, True),    # one larger: another kernel
+    (2, 20, 21, 64, 64, 13, 1, True),   # ... the LDS-tile kernel
+    (2, 40, 41, 32, 64, 13, 2, True),   # ... fp32 copies
     (4, 16, 16, 96, 128, 3, 1, True),   # whole tiles of 128
     (1, 23, 23, 96, 129, 3, 1, True),   # one feature and one pixel past them
     (2, 7, 7, 512, 72, 3, 1, True),     # long reduction, few tiles: shared

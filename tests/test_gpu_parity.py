@@ -125,11 +125,10 @@ def test_stem_7x7_stride2(direction):
     (2, 224, 224, True),    # the stem layer itself
 ])
 def test_stem_in_half_precision(batch, rows, cols, same):
-    """A binary16 launch of the 7x7 stride-2 three-channel stem runs the fp32
-    stem kernels: forward, the image and the filter widened into a temporary
-    and the output rounded to binary16 by the kernel's own store; the
-    gradients through fp32 copies.  Against the oracle in double precision on the same
-    binary16-rounded operands; nothing written past the result."""
+    """A binary16 launch of the 7x7 stride-2 three-channel stem, all directions
+    on the binary16 kernels for layers of few channels.  Against the oracle in
+    double precision on the same binary16-rounded operands; nothing written past
+    the result."""
     p = ops.conv_params(batch, rows, cols, 3, 64, 7, 2, same)
     rng = np.random.default_rng(331 + rows + cols)
     for direction in (DIRECTION.FORWARD, DIRECTION.INPUT_BACKPROP,
@@ -433,7 +432,6 @@ def test_filter_gradient_from_registers(shape):
 
 @pytest.mark.parametrize("shape", [
     # batch, rows, cols, channels, features, window, stride, SAME
-    # (from 2^30 multiply-adds on; smaller launches keep the general kernel)
     (16, 56, 56, 128, 128, 3, 2, True),  # a ResNet 3x3 stride-2 layer
     (16, 57, 55, 128, 128, 3, 2, True),  # odd image
     (16, 57, 55, 128, 144, 3, 2, False), # VALID
@@ -441,16 +439,17 @@ def test_filter_gradient_from_registers(shape):
     (18, 45, 45, 128, 256, 3, 3, True),  # stride 3: one tap per class
     (4, 64, 64, 64, 96, 7, 2, True),     # 7x7 stride 2 over 64 channels
     (48, 40, 40, 128, 256, 2, 3, False), # stride above the window: empty classes
-    (4, 28, 28, 256, 256, 3, 2, True),   # below the threshold: general kernel
+    (4, 28, 28, 256, 256, 3, 2, True),
+    (2, 64, 64, 64, 64, 13, 2, True),    # a window beyond the gathering kernel's
 ])
 @pytest.mark.parametrize("dtype", ["f32", "f16"])
 def test_strided_input_gradient_by_stride_classes(shape, dtype):
     """A strided input gradient is computed class by class of input pixels
-    modulo the strides -- each a dense stride-1 forward convolution of dY with
-    the sub-filter of the taps that reach the class, on the stride-1 kernels
-    (binary16: on the binary16 ones when the feature count is a multiple of
-    64, else through fp32 copies) -- and interleaved into dX in one pass:
-    against the oracle over the whole tensor, every element of dX written (the
+    modulo the strides, each a dense stride-1 convolution of dY with the
+    sub-filter of the taps that reach the class: all classes in one launch of the
+    gathering kernel, or, for windows beyond its 12 x 12 and from 2^30
+    multiply-adds, one fp32 launch per class and a pass that interleaves them.
+    Against the oracle over the whole tensor, every element of dX written (the
     output starts as NaN)."""
     batch, rows, cols, ch, feats, window, stride, same = shape
     p = ops.conv_params(batch, rows, cols, ch, feats, window, stride, same)
@@ -1525,12 +1524,11 @@ def test_f16_conv_forward_lds_tile_kernel(shape):
     (8, 17, 19, 40, 72, 1, 1, False),
 ])
 def test_f16_conv_forward_general_kernel(shape):
-    """Half-precision forward convolutions outside the binary16 kernels'
-    shapes (channel counts that are not multiples of 64, more than 32 taps)
-    run on the general implicit-GEMM kernel reading binary16 operands with
-    fp32 accumulation, not one lane per output: against the oracle in double
-    precision on the same half-rounded operands; nothing written past the
-    result."""
+    """Half-precision forward convolutions outside the LDS-tile kernel's shapes
+    (channel counts that are not multiples of 64, more than 32 taps) run on the
+    gathering kernel or, where they are short, the general implicit-GEMM kernel,
+    not one lane per output: against the oracle in double precision on the same
+    half-rounded operands; nothing written past the result."""
     batch, rows, cols, ch, feats, window, stride, same = shape
     p = ops.conv_params(batch, rows, cols, ch, feats, window, stride, same)
     rng = np.random.default_rng(770 + rows + ch + window)
@@ -1554,7 +1552,7 @@ def test_f16_conv_forward_general_kernel(shape):
     (28, 128, 128, 3),   # LDS-tile kernel, four channel blocks
     (56, 64, 64, 3),     # LDS-tile kernel, one channel block
     (7, 512, 512, 3),    # LDS-tile kernel, 64 x 64 wave tiles
-    (28, 128, 512, 1),   # implicit-GEMM kernel, 128 x 128 work-group tile
+    (28, 128, 512, 1),   # row-major GEMM kernel
 ])
 def test_f16_conv_forward_full_batch_sampled(size, ch, feats, window):
     p = ops.conv_params(128, size, size, ch, feats, window, 1, window == 3)
@@ -1584,12 +1582,12 @@ def test_f16_conv_forward_full_batch_sampled(size, ch, feats, window):
     (2, 11, 13, 64, 64, 3, 3, 1, False),    # VALID: padding 2 on dY
     (3, 12, 10, 128, 128, 5, 5, 1, True),   # 25 mirrored taps
     (2, 9, 20, 128, 256, 1, 3, 1, True),    # 1 x 3 window
-    (7, 5, 5, 256, 320, 1, 1, 1, False),    # 1x1: implicit-GEMM kernel
+    (7, 5, 5, 256, 320, 1, 1, 1, False),    # 1x1: row-major GEMM kernel
     (2, 28, 28, 128, 512, 1, 1, 1, False),  # 1x1, 128 x 128 tiles
-    (2, 17, 9, 128, 64, 3, 3, 2, True),     # stride 2: general MFMA kernel
-    (2, 8, 8, 24, 40, 3, 3, 1, True),       # few channels: general MFMA kernel
+    (2, 17, 9, 128, 64, 3, 3, 2, True),     # stride 2: classes
+    (2, 8, 8, 24, 40, 3, 3, 1, True),       # few channels
     (3, 31, 29, 64, 132, 3, 3, 2, False),   # stride 2, VALID, ragged tiles
-    (2, 16, 16, 6, 10, 3, 3, 2, True),      # features not x4: direct kernel
+    (2, 16, 16, 6, 10, 3, 3, 2, True),      # few and odd
     (2, 9, 10, 64, 64, 2, 2, 1, True),      # even window: padding 0 before, 1 after
     (2, 12, 9, 64, 128, 4, 4, 1, True),     # even window: padding 1 before, 2 after
     (2, 10, 10, 64, 64, 2, 4, 1, False),    # VALID, rectangular even window
@@ -1624,7 +1622,7 @@ def test_f16_conv_input_backprop(shape):
     (4, 28, 28, 128, 512, 1, 1, False),   # 1x1 K = 4C
     (3, 17, 9, 128, 72, 3, 2, True),      # stride 2, ragged feature tile
     (2, 9, 9, 64, 200, 5, 1, False),      # VALID, 25 taps
-    (128, 28, 28, 128, 128, 3, 1, True),  # configuration 4's batch
+    (128, 28, 28, 128, 128, 3, 1, True),  # a full batch
 ])
 def test_f16_conv_filter_backprop_on_matrix_cores(shape):
     """Half-precision filter gradient (channel counts in multiples of 64: the
