@@ -10,8 +10,9 @@
 // convolution is split by classes: the dX pixels whose padded row and column
 // have one remainder modulo the strides are reached by the same sub-window of
 // taps, and form a dense stride-1 convolution of dY with that sub-filter.  All
-// classes run in one launch, the one with the most taps first, and store their
-// pixels straight into dX; a class that no tap reaches stores zeros.
+// classes run in one launch, their tiles side by side and rotated over the
+// work-groups (see TileOf), and store their pixels straight into dX; a class that
+// no tap reaches stores zeros.
 //
 // The reduction runs over 16-byte pieces -- eight binary16 or four fp32 channels
 // of one tap -- of a pixel, flattened over (tap, piece): a chunk is four pieces,
@@ -993,12 +994,8 @@ constexpr int kNumCus = 256;
 template <typename T>
 constexpr int kMaxSplits = sizeof(T) == 4 ? 32 : 16;  // (half the chunk)
 
-int tuned(const char* name, int otherwise) {
-#ifdef SNN_HIP_TUNING
-  const char* const env = std::getenv(name);
-  if (env != nullptr) return std::atoi(env);
-#endif
-  return otherwise;
+int tuned(const char* value, int otherwise) {
+  return value != nullptr ? std::atoi(value) : otherwise;
 }
 
 // Tile shape and splits of the reduction: the least time by a model of the
@@ -1043,8 +1040,9 @@ void choose_tile(GatherPlan* plan, bool may_split) {
       }
     }
   }
-  plan->tile = tuned("SNN_HIP_GATHER_TILE", plan->tile);
-  plan->n_splits = tuned("SNN_HIP_GATHER_SPLITS", plan->n_splits);
+  plan->tile = tuned(SNN_TUNING_ENV("SNN_HIP_GATHER_TILE"), plan->tile);
+  plan->n_splits =
+      tuned(SNN_TUNING_ENV("SNN_HIP_GATHER_SPLITS"), plan->n_splits);
   const TileShape& t = Tiles<T>::shapes[plan->tile];
   plan->part_floats =
       plan->n_splits > 1 ? static_cast<size_t>(plan->n_splits * tiles_of(t)) *
@@ -1214,9 +1212,6 @@ const GatherPlan& make_plan(int direction, const snn_hip_conv2d_params& p,
   };
   thread_local Cached cached[2];
   Cached& c = cached[direction == SNN_HIP_INPUT_BACKPROP ? 1 : 0];
-#ifdef SNN_HIP_TUNING
-  c.direction = -1;
-#endif
   if (c.direction != direction || c.may_split != may_split ||
       std::memcmp(&c.params, &p, sizeof(p)) != 0) {
     c.plan = compute_plan<T>(direction, p, may_split);
@@ -1587,10 +1582,8 @@ int launch_conv2d_f16(int direction, const _Float16* input,
 // Tiled / Im2col / Matmul tags (times: there / here).
 bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
   if (direction == SNN_HIP_FILTER_BACKPROP) return false;
-#ifdef SNN_HIP_TUNING
-  if (const char* env = std::getenv("SNN_HIP_GATHER_F32"))
-    if (env[0] == '0' || env[0] == '1') return env[0] == '1';
-#endif
+  if (const char* const env = SNN_TUNING_ENV("SNN_HIP_GATHER_F32"))
+    return std::atoi(env) != 0;
   const bool grad = direction == SNN_HIP_INPUT_BACKPROP;
   const bool strided = p.stride_rows > 1 || p.stride_cols > 1;
   const long long products = static_cast<long long>(p.window_rows) *

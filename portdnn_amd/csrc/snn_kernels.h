@@ -273,10 +273,6 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p);
 size_t conv2d_gather_f32_workspace_floats(int direction,
                                           const snn_hip_conv2d_params& p);
 
-// Half-precision filter gradient on the fp32 matrix instructions
-// (conv2d_igemm.hip) for channel counts in multiples of 64: fp32 accumulation
-// buffer in the workspace when it holds twice the filter's element count, else
-// a stream-ordered temporary.
 // conv2d_few_f16.hip: one to four channels at stride 2, features in multiples
 // of 8 up to 96.  All operands 16-byte aligned.  The filter gradient keeps
 // partial sums in the workspace when it is given the room (else in a
@@ -320,6 +316,10 @@ int launch_conv2d_filter_backprop_1x1_f16(const _Float16* x,
                                           float* part,
                                           const snn_hip_conv2d_params& p,
                                           hipStream_t stream);
+// The half-precision filter gradient (conv2d_igemm.hip): those two kernels, the
+// direct-operand one, and for other channel counts in multiples of 64 the fp32
+// matrix instructions with an fp32 accumulation buffer, in the workspace when it
+// holds twice the filter's element count, else in a stream-ordered temporary.
 bool conv2d_filter_backprop_f16_supports(const snn_hip_conv2d_params& p);
 int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
                                       _Float16* dw,
