@@ -1,7 +1,7 @@
 #!/usr/bin/env python3
 """Benchmark of the conv2d forward hot path on one MI355X.
 
-    python bench.py [--gpus 1] [--steps K] [--warmup W]
+    python bench.py [--gpus 1] [--steps K] [--warmup W] [--detail FILE]
 
 One step = one forward pass over the eight fp32 NHWC batch-32 ResNet layers of
 the benchmark configuration (3x3 s1 SAME at 56x56x64, 28x28x128, 14x14x256,
@@ -26,8 +26,11 @@ algorithm).  The same JSON line carries
                 the host cores on bounded samples: the tiled convolution on
                 the same eight layers (`value`), the depthwise and pooling
                 loops (`depthwise_gbs`, `maxpool_gbs`, `avgpool_gbs`) and the
-                single-image layer (`config0_tflops`),
-  detail        per-layer / per-algorithm TFLOP/s, gradients, half precision.
+                single-image layer (`config0_tflops`).
+
+Per-layer / per-algorithm TFLOP/s, gradients and half precision are measured in
+the same run and written to the file that --detail names (17 KB of JSON, which
+a line on stdout was cut short by).
 
 No executed fraction of a peak may exceed 1: `frac()` raises if one does.
 Fractions of the algorithmic flops (the direct convolution's count, the
@@ -99,6 +102,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=5)
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--no-detail", action="store_true")
+    ap.add_argument("--detail", metavar="FILE")
     args = ap.parse_args()
     if args.gpus != 1:
         sys.exit("bench.py measures one GPU: this build has no multi-GPU path "
@@ -894,8 +898,11 @@ def main():
                                "SAME at (56,64),(28,128),(14,256),(7,512) + "
                                "1x1 K=4C at each stage; default selector",
                    "batch": BATCH},
-        "roofline": roofline, "cpu_baseline": cpu, "detail": detail,
+        "roofline": roofline, "cpu_baseline": cpu,
     }
+    if args.detail is not None:
+        with open(args.detail, "w") as f:
+            json.dump(detail, f)
     print(json.dumps(line))
 
 
