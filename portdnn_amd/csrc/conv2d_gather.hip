@@ -130,6 +130,7 @@ struct Gather {
   int n_splits;          // work-groups that share a tile's reduction
   unsigned n_tiles;      // tiles of all classes
   int n_classes;
+  int round_shift, turn; // how the classes are rotated, see tile_of
   int mirrored;          // input gradient: w[tap][feature][channel]
   int merged;            // channels per pixel of merged classes, or 0
   int relu;              // of a forward launch with bias and activation
@@ -236,13 +237,22 @@ constexpr int vmcnt_imm(int n) { return 0x0F70 | (n & 15) | ((n >> 4) << 14); }
 // piece of dX are written side by side.  (Class after class, every work-group
 // in flight wrote the same half of the rows and columns, which are the same
 // half of the memory channels: 56x56x256 <- 512, 1x1 stride 2, at batch 128,
-// 168 -> 110 us;
-// 56x56x128 <- 128, 3x3, 73 -> 61.)
+// 168 -> 110 us.)  Work-groups go round the 32 compute units of an XCD, so the
+// order of the classes is rotated from piece to piece: by one where the tiles of
+// a class come round to the units they met before (after 2^round_shift pieces),
+// so that the long ones meet every unit, and for two, four or eight classes by one
+// per piece (`turn`), which mixes the memory channels.  One per piece alone left
+// the long tiles of four classes to eight units (fp32 9x84x84 40 <- 620, 1x1
+// stride 2, one class with products: 51 -> 19.5 us; 32x28x28 256 <- 256, 3x3: 86
+// -> 79; binary16 32x56x56 128 <- 128, 3x3: 20.6 -> 19.1), without it the largest
+// lose (binary16 128x56x56 128 <- 128, 3x3: 53 / 56).
 struct TileOf { int m, cls, n; };
 __device__ __forceinline__ TileOf tile_of(unsigned tile, const Gather& g) {
   const unsigned n = tile % g.n_tiles_n, t = tile / g.n_tiles_n;
   const unsigned m = t / g.n_classes;
-  return {static_cast<int>(m), static_cast<int>((t + m) % g.n_classes),
+  return {static_cast<int>(m),
+          static_cast<int>((t + m * g.turn + (m >> g.round_shift)) %
+                           g.n_classes),
           static_cast<int>(n)};
 }
 
@@ -1263,6 +1273,11 @@ void launch_tile(const GatherOperands<T>& ops, const GatherPlan& plan,
   g.n_tiles = static_cast<unsigned>(ceil_div(pixels, BM)) *
               static_cast<unsigned>(g.n_classes * g.n_tiles_n);
   g.n_splits = plan.n_splits;
+  // (the tiles of a class are this many work-groups apart)
+  const unsigned apart =
+      static_cast<unsigned>(g.n_classes * g.n_tiles_n * g.n_splits);
+  g.round_shift = std::max(0, 5 - __builtin_ctz(apart));
+  g.turn = g.round_shift > 0 && (g.n_classes & (g.n_classes - 1)) == 0;
   if constexpr (sizeof(T) == 4) {
     if (ops.from == kInPlace)
       launch_kernel<T, WM, WN, TM, TN, false, kInPlace>(ops, plan, g, stream);
