@@ -1451,23 +1451,24 @@ double general_f16_us(const Products& r) {
          r.pixels * r.columns / 6e6;
 }
 
-// One lane per output.  A gradient's lanes read the filter columns of as many
-// channels: with features in multiples of 4 those fall into few banks, and the
-// general kernel is there.
-double direct_f16_us(int direction, const snn_hip_conv2d_params& p,
-                     const Products& r) {
+// One lane per output, either type.  A gradient's lanes read the filter columns of
+// as many channels: with features in multiples of 4 those fall into few banks,
+// and other kernels are there.
+double direct_us(int direction, const snn_hip_conv2d_params& p,
+                 const Products& r, bool half) {
   const double outputs = r.pixels * r.columns;
   if (r.macs >= double(1 << 24)) return kNever;
   if (direction == SNN_HIP_FORWARD)
-    return 2.9 + 0.09 * r.reduced + (0.146 * r.reduced + 2.7) * outputs / 1e6;
+    return 2.9 + 0.09 * r.reduced + (0.15 * r.reduced + 2.7) * outputs / 1e6;
   const double loop = static_cast<double>(p.features) *
                       ceil_div(p.window_rows, p.stride_rows) *
                       ceil_div(p.window_cols, p.stride_cols);
   if (p.features % 4 != 0 && loop <= 16)
-    return 3.1 + 0.05 * loop + (0.11 * loop + 3.3) * outputs / 1e6 +
-           0.67 * p.window_rows * p.window_cols /
+    return 3.1 + 0.05 * loop +
+           (half ? 0.11 * loop + 3.3 : 0.06 * loop + 4.3) * outputs / 1e6 +
+           0.6 * p.window_rows * p.window_cols /
                (p.stride_rows * p.stride_cols);
-  return r.reduced <= 32 && outputs <= (1 << 16) ? 5.5 : kNever;
+  return half && r.reduced <= 32 && outputs <= (1 << 16) ? 5.5 : kNever;
 }
 
 bool stream_captures(hipStream_t stream) {
@@ -1490,7 +1491,7 @@ bool conv2d_gather_tile_f16(int direction, const snn_hip_conv2d_params& p,
   const Products r = products_of(direction, p);
   if (std::min(conv2d_general_f16_supports(direction, p) ? general_f16_us(r)
                                                          : kNever,
-               direct_f16_us(direction, p, r)) <
+               direct_us(direction, p, r, true)) <
       gather_f16_us(plan, plan.from == kPacked, false))
     return false;
   *tile = {kTilesF16[plan.tile].pixels, kTilesF16[plan.tile].features,
@@ -1577,10 +1578,10 @@ int launch_conv2d_f16(int direction, const _Float16* input,
     able = !temporary || !other;
   }
   const double general_us = general ? general_f16_us(r) : kNever;
-  const double direct_us = direct_f16_us(direction, p, r);
+  const double one_lane_us = direct_us(direction, p, r, true);
   const double gather_us =
       able ? gather_f16_us(*plan, packs, temporary) : kNever;
-  if (std::min(otherwise_us, direct_us) < std::min(general_us, gather_us))
+  if (std::min(otherwise_us, one_lane_us) < std::min(general_us, gather_us))
     return -1;
   if (gather_us <= general_us && able) {
     const int rc = launch_gather<_Float16>(*plan, input, filter, output,
@@ -1612,15 +1613,17 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
   if (products <= 64 && outputs <= (1 << 16)) return false;
   // Features of no whole piece: a short loop per output as well, where the
   // filter's pack and the copy would be launches of their own (13x15x19 8 -> 135,
-  // 1x1 stride 2: 4.3 / 7.9; gradient of 8x21x21 24 <- 2, 2x2: 4.4 / 7.9; 41 random
-  // layers, none slower, 0.55 of the time in the middle; but 12x134x134 4 -> 3 with
-  // 2^20 outputs 9.1 / 8.5).
-  const int loop = grad ? p.features * ceil_div(p.window_rows, p.stride_rows) *
-                              ceil_div(p.window_cols, p.stride_cols)
-                        : static_cast<int>(products) / 2;
-  if (p.features % 4 != 0 && loop < 8 && macs < double(1 << 23) &&
-      outputs < (1 << 19))
-    return false;
+  // 1x1 stride 2: 4.3 / 7.9; gradient of 8x21x21 24 <- 2, 2x2: 4.4 / 7.9; but
+  // 24x39x39 50 -> 6, 1x1: 17.2 / 15.5).  The estimate of this kernel's time is
+  // within 5 % for half of 262 random layers.
+  if (p.features % 4 != 0) {
+    const GatherPlan& plan = make_plan<float>(direction, p);
+    if (plan.ok &&
+        direct_us(direction, p, products_of(direction, p), false) <
+            7.3 + 0.87 * plan.us + plan.out_elems / 5.2e6 +
+                (plan.wide_bytes + plan.pack_blocks * 2048.0) / 1.8e6)
+      return false;
+  }
   // At most one 64 x 64 tile per compute unit and a short reduction in whole
   // pieces: latencies are all there is, and those are shorter there (25x14x18
   // 56 -> 424, 1x1 stride 2: 4.8 / 6.3; 11x14x10 24 -> 88, 1x1: 4.2 / 5.5; gradient

@@ -377,7 +377,7 @@ def test_a_missing_operand_is_the_entry_points_error(monkeypatch):
     (capi.DTYPE.F16, (128, 224, 224, 3, 64, 7, 2, True), 0, None, None),
     (capi.DTYPE.F32, (1, 24, 24, 3, 512, 7, 2, True), 1, (128, 32), True),
     (capi.DTYPE.F32, (2, 7, 7, 480, 70, 3, 2, True), 0, (64, 64), True),
-    (capi.DTYPE.F32, (4, 41, 43, 35, 133, 1, 2, True), 0, (128, 32), False),
+    (capi.DTYPE.F32, (9, 41, 43, 35, 133, 1, 2, True), 0, (128, 32), False),
     (capi.DTYPE.F32, (9, 57, 43, 72, 96, 3, 2, True), 1, (64, 64), False),
     (capi.DTYPE.F32, (13, 15, 19, 8, 135, 1, 2, True), 0, None, None),
     (capi.DTYPE.F32, (25, 14, 18, 56, 424, 1, 2, True), 0, None, None)],

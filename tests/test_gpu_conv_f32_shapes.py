@@ -42,7 +42,7 @@ SHAPES = [
     (3, 21, 22, 35, 45, 1, 2, True),    # strided 1x1, odd: copied subsampled
     (2, 17, 19, 30, 66, 1, 3, False),   # ... even counts, VALID
     (20, 20, 21, 64, 203, 3, 1, True),  # many tiles, runs of odd features
-    (4, 41, 43, 35, 133, 1, 2, True),   # large enough to be copied subsampled
+    (9, 41, 43, 35, 133, 1, 2, True),   # large enough to be copied subsampled
     (3, 33, 35, 130, 66, 1, 3, False),
     (4, 40, 41, 32, 33, 1, 4, False),   # sixteen classes, odd features
     (13, 15, 19, 8, 135, 1, 2, True),   # short launches: the direct kernel
