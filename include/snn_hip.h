@@ -216,12 +216,12 @@ SNN_HIP_API int snn_hip_conv2d_forward_f16(
     const snn_hip_conv2d_params* params, int algorithm, void* workspace,
     size_t workspace_elems, void* stream);
 /* The two gradients in half precision (fp32 accumulation), the reference's
- * launch<half, conv_type::InputBackprop / FilterBackprop>.  With channel
- * counts in multiples of 64 they run on the matrix cores (3x3 stride-1 SAME
- * and 1x1 filter gradients and stride-1 input gradients on binary16 matrix
- * instructions, other shapes on fp32 matrix instructions fed binary16
- * operands); shapes off those multiples run on the direct kernels.  No
- * half-precision launch requires a workspace; one of the size
+ * launch<half, conv_type::InputBackprop / FilterBackprop>.  Forward
+ * convolutions and input gradients of every shape run on binary16 matrix
+ * instructions (short ones on fp32 matrix instructions fed binary16 operands,
+ * or one lane per output), filter gradients on binary16 ones but for layers of
+ * few channels outside the kernels for those, which run in fp32 on widened
+ * copies.  No half-precision launch requires a workspace; one of the size
  * snn_hip_conv2d_workspace_size_for reports saves a stream-ordered
  * temporary. */
 SNN_HIP_API int snn_hip_conv2d_input_backprop_f16(

@@ -752,7 +752,7 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
   // out through LDS, block by block, as rows of 32 consecutive features: one
   // store instruction covers two to eight pixels' runs instead of 2 or 4 bytes of
   // 64 pixels each (83x23x23x64 -> 391, 3x3, binary16:
-  // 96 -> 47 us; 32x28x28x128 -> 131, 3x3, fp32: 96 -> 92).  Word
+  // 93 -> 47 us; 32x28x28x128 -> 131, 3x3, fp32: 96 -> 92).  Word
   // w of pixel row r lies at w XOR (bits of r), which keeps both the writes of 32
   // rows and the reads along a row off each other's banks.
   const bool by_rows = (g.features & (kPiece<T> - 1)) != 0;
