@@ -1596,7 +1596,10 @@ int launch_conv2d_f16(int direction, const _Float16* input,
 
 // Where the gathering kernel is faster than the other fp32 kernels behind the
 // Tiled / Im2col / Matmul tags (times: there / here).
-bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
+// With a bias and activation (`fused`) those kernels that do not add them on the
+// way are followed by a launch of 2 us.
+bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p,
+                              bool fused) {
   if (direction == SNN_HIP_FILTER_BACKPROP) return false;
   if (const char* const env = SNN_TUNING_ENV("SNN_HIP_GATHER_F32"))
     return std::atoi(env) != 0;
@@ -1619,7 +1622,8 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
   if (p.features % 4 != 0) {
     const GatherPlan& plan = make_plan<float>(direction, p);
     if (plan.ok &&
-        direct_us(direction, p, products_of(direction, p), false) <
+        direct_us(direction, p, products_of(direction, p), false) +
+                (fused ? 2.0 : 0.0) <
             7.3 + 0.87 * plan.us + plan.out_elems / 5.2e6 +
                 (plan.wide_bytes + plan.pack_blocks * 2048.0) / 1.8e6)
       return false;
@@ -1628,11 +1632,12 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
   // pieces: latencies are all there is, and those are shorter there (25x14x18
   // 56 -> 424, 1x1 stride 2: 4.8 / 6.3; 11x14x10 24 -> 88, 1x1: 4.2 / 5.5; gradient
   // of 30x30 441 <- 52, 1x1: 4.7 / 6.3; 0.89 of the time in the middle of 185
-  // random layers, four of them up to 9 % slower).
+  // random layers, four of them up to 9 % slower; but with bias and ReLU 8.0 /
+  // 6.0 and 6.2 / 5.2).
   const double tiles = std::ceil(outputs / (grad ? p.channels : p.features) / 64) *
                        ceil_div(grad ? p.channels : p.features, 64);
-  if (p.features % 4 == 0 && (grad ? !strided : p.channels % 4 == 0) &&
-      products <= 96 && tiles <= kNumCus)
+  if (!fused && p.features % 4 == 0 &&
+      (grad ? !strided : p.channels % 4 == 0) && products <= 96 && tiles <= kNumCus)
     return false;
   // Few outputs of a long reduction meet through atomics there, in one pass less
   // (2x19x14 720 -> 80, 3x3 stride 2: 12.5 / 13.7 us; 4x14x14 144 -> 224, 5x5,
@@ -1698,7 +1703,8 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p) {
 
 bool conv2d_gather_tile_f32(int direction, const snn_hip_conv2d_params& p,
                             GatherTile* tile) {
-  if (!positive(p) || !conv2d_gather_f32_wanted(direction, p)) return false;
+  if (!positive(p) || !conv2d_gather_f32_wanted(direction, p, false))
+    return false;
   const GatherPlan& plan = make_plan<float>(direction, p);
   *tile = {kTilesF32[plan.tile].pixels, kTilesF32[plan.tile].features,
            plan.n_splits};
@@ -1707,7 +1713,12 @@ bool conv2d_gather_tile_f32(int direction, const snn_hip_conv2d_params& p,
 
 size_t conv2d_gather_f32_workspace_floats(int direction,
                                           const snn_hip_conv2d_params& p) {
-  if (!positive(p) || !conv2d_gather_f32_wanted(direction, p)) return 0;
+  // (the query does not know of a bias)
+  if (!positive(p) ||
+      !(conv2d_gather_f32_wanted(direction, p, false) ||
+        (direction == SNN_HIP_FORWARD &&
+         conv2d_gather_f32_wanted(direction, p, true))))
+    return 0;
   const GatherPlan& plan = make_plan<float>(direction, p);
   return plan.ok ? plan.workspace_bytes(plan.from == kPacked) / 4 : 0;
 }

@@ -769,8 +769,8 @@ void convert(const From* in, To* out, size_t n, hipStream_t s) {
 }
 
 // A binary16 launch that no binary16 matrix-core kernel takes (filter gradients
-// of at most eight channels outside the first-layer kernels, operands off
-// 16-byte alignment) through the fp32 kernels: operands widened into
+// of at most eight channels outside the first-layer kernels, large layers with
+// windows beyond the gathering kernel's, operands off 16-byte alignment) through the fp32 kernels: operands widened into
 // stream-ordered temporaries, the fp32 launch -- every path it has -- and the
 // result rounded back.  Products and sums are then fp32 on binary16-rounded
 // operands, as in the binary16 kernels.  From 2^24 multiply-adds; returns -1
@@ -881,7 +881,10 @@ int launch_gemm_path<float>(int direction, const float* input,
         input, filter, output, p, s, workspace, workspace_elems);
     if (rc >= 0) return rc;
   }
-  if (conv2d_gather_f32_wanted(direction, p)) {
+  if (conv2d_gather_f32_wanted(
+          direction, p,
+          direction == SNN_HIP_FORWARD && epilogue != nullptr &&
+              epilogue->wanted())) {
     const int rc =
         launch_conv2d_gather_f32(direction, input, filter, output, p, workspace,
                                  workspace_elems, s, epilogue);

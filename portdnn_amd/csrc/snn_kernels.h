@@ -269,7 +269,8 @@ int launch_conv2d_gather_f32(int direction, const float* input,
                              const snn_hip_conv2d_params& p, float* workspace,
                              size_t workspace_elems, hipStream_t stream,
                              const LaunchOptions* epilogue);
-bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p);
+bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p,
+                              bool fused);
 size_t conv2d_gather_f32_workspace_floats(int direction,
                                           const snn_hip_conv2d_params& p);
 

@@ -90,7 +90,9 @@ def test_conv_f32_shapes(shape, direction):
 
 @pytest.mark.parametrize("shape", [(3, 20, 21, 20, 30, 3, 2, True),
                                    (2, 7, 7, 480, 72, 3, 2, True),
-                                   (5, 31, 29, 84, 16, 1, 1, True)],
+                                   (5, 31, 29, 84, 16, 1, 1, True),
+                                   (25, 14, 18, 56, 424, 1, 2, True),
+                                   (13, 15, 19, 8, 135, 1, 2, True)],
                          ids=lambda s: "x".join(map(str, s)))
 @pytest.mark.parametrize("relu", [False, True])
 def test_conv_f32_bias_act(shape, relu):
