@@ -1216,17 +1216,15 @@ const GatherPlan& make_plan(int direction, const snn_hip_conv2d_params& p,
                             bool may_split = true) {
   struct Cached {
     int direction = -1;
-    bool may_split = false;
     snn_hip_conv2d_params params;
     GatherPlan plan;
   };
-  thread_local Cached cached[2];
-  Cached& c = cached[direction == SNN_HIP_INPUT_BACKPROP ? 1 : 0];
-  if (c.direction != direction || c.may_split != may_split ||
+  thread_local Cached cached[2][2];
+  Cached& c = cached[may_split][direction == SNN_HIP_INPUT_BACKPROP];
+  if (c.direction != direction ||
       std::memcmp(&c.params, &p, sizeof(p)) != 0) {
     c.plan = compute_plan<T>(direction, p, may_split);
     c.params = p;
-    c.may_split = may_split;
     c.direction = direction;
   }
   return c.plan;
@@ -1417,9 +1415,10 @@ bool is_rows_gemm(int direction, const snn_hip_conv2d_params& p) {
 // other two.  They meet where launches are short.  The gathering one has
 // up to two launches in front of its products, the filter's pack and the copy to
 // whole pieces (16x55x41 16 -> 12, 1x1: general 5.6, gathering 8.8; 2x24x24
-// 52 -> 20, 1x1 stride 2: 5.4 and 7.9), and a temporary for these costs 14 us of
-// host time where the caller brings no workspace.
+// 52 -> 20, 1x1 stride 2: 5.4 and 7.9), and where the caller brings no workspace a
+// call with a temporary takes 22 us of host time, which only longer kernels hide.
 constexpr double kNever = 1e30;
+constexpr double kTemporaryUs = 22.0;
 
 struct Products {
   double pixels, columns, reduced, macs;
@@ -1439,8 +1438,10 @@ Products products_of(int direction, const snn_hip_conv2d_params& p) {
 double gather_f16_us(const GatherPlan& plan, bool packs, bool temporary) {
   const double bytes = static_cast<double>(plan.wide_bytes) +
                        (packs ? plan.pack_blocks * 2048.0 : 0.0);
-  return 4.0 + 0.8 * plan.us + (bytes > 0 ? 3.0 + bytes / 1.5e6 : 0.0) +
-         plan.out_elems / 2.5e6 + (temporary ? 14.0 : 0.0);
+  const double us = 4.0 + 0.8 * plan.us +
+                    (bytes > 0 ? 3.0 + bytes / 1.5e6 : 0.0) +
+                    plan.out_elems / 2.5e6;
+  return temporary ? std::max(us, kTemporaryUs) : us;
 }
 
 double general_f16_us(const Products& r) {
@@ -1463,12 +1464,38 @@ double direct_us(int direction, const snn_hip_conv2d_params& p,
   const double loop = static_cast<double>(p.features) *
                       ceil_div(p.window_rows, p.stride_rows) *
                       ceil_div(p.window_cols, p.stride_cols);
-  if (p.features % 4 != 0 && loop <= 16)
-    return 3.1 + 0.05 * loop +
-           (half ? 0.11 * loop + 3.3 : 0.06 * loop + 4.3) * outputs / 1e6 +
-           0.6 * p.window_rows * p.window_cols /
-               (p.stride_rows * p.stride_cols);
-  return half && r.reduced <= 32 && outputs <= (1 << 16) ? 5.5 : kNever;
+  const bool small = half && r.reduced <= 32 && outputs <= (1 << 16);
+  if (p.features % 4 == 0 || loop > 64 || (small && loop > 16))
+    return small ? 5.5 : kNever;
+  return (3.1 + 0.05 * loop +
+          (half ? 0.11 * loop + 3.3 : 0.06 * loop + 4.3) * outputs / 1e6 +
+          0.6 * p.window_rows * p.window_cols /
+              (p.stride_rows * p.stride_cols)) *
+         (loop <= 16 ? 1.0 : 2.0);  // (longer ones up to three times that)
+}
+
+// The same in fp32: this kernel, and the implicit-GEMM one for counts in
+// multiples of 4 and stride 1 (or forward), whose shared reductions meet through
+// atomics after a launch that clears the output.  (Half of 270 and of 970 layers
+// within 5 and 10 %.)
+double gather_f32_us(const GatherPlan& plan, bool packs, bool temporary) {
+  const double bytes = static_cast<double>(plan.wide_bytes) +
+                       (packs ? plan.pack_blocks * 2048.0 : 0.0);
+  const double us = 4.4 + 0.87 * plan.us +
+                    (bytes > 0 ? 2.9 + bytes / 1.8e6 : 0.0) +
+                    plan.out_elems / 5.2e6;
+  return temporary ? std::max(us, kTemporaryUs) : us;
+}
+
+double igemm_f32_us(const Products& r) {
+  const double chunks = std::ceil(r.reduced / 32);
+  const double tiles = std::ceil(r.pixels / 64) * std::ceil(r.columns / 64);
+  const double splits =
+      std::max(1.0, std::min(std::floor(640 / tiles), std::floor(chunks / 2)));
+  const bool shared = splits > 1;
+  return 4.1 + 0.65 * tiles * chunks / kNumCus +
+         0.25 * std::ceil(chunks / splits) + (shared ? 3.5 : 0.0) +
+         r.pixels * r.columns * (shared ? 2 : 1) / 2.3e6;
 }
 
 bool stream_captures(hipStream_t stream) {
@@ -1565,17 +1592,25 @@ int launch_conv2d_f16(int direction, const _Float16* input,
   bool general = both_aligned && conv2d_general_f16_supports(direction, p) &&
                  (direction == SNN_HIP_INPUT_BACKPROP || aligned(output)) &&
                  (able || r.macs < double(1 << 24));
-  if (temporary && stream_captures(stream)) {
-    // A launch that is recorded without room for the packed filter or the copy
-    // keeps its reduction whole, or takes a kernel that needs no temporary.
-    // (Layers of 64 channels and large ones with counts that no other kernel
-    // takes have only kernels with temporaries, or slow ones.)
-    plan = &make_plan<_Float16>(direction, p, false);
-    temporary = plan->workspace_bytes(packs) > room;
-    const bool other = otherwise_us < kNever || r.macs < double(1 << 24) ||
-                       (general && (direction == SNN_HIP_INPUT_BACKPROP ||
-                                    p.channels % 64 != 0));
-    able = !temporary || !other;
+  if (temporary) {
+    const GatherPlan& whole = make_plan<_Float16>(direction, p, false);
+    const bool whole_temporary = whole.workspace_bytes(packs) > room;
+    if (stream_captures(stream)) {
+      // A launch that is recorded without room for the packed filter or the
+      // copy keeps its reduction whole, or takes a kernel that needs no
+      // temporary.  (Layers of 64 channels and large ones with counts that no
+      // other kernel takes have only kernels with temporaries, or slow ones.)
+      plan = &whole;
+      temporary = whole_temporary;
+      const bool other = otherwise_us < kNever || r.macs < double(1 << 24) ||
+                         (general && (direction == SNN_HIP_INPUT_BACKPROP ||
+                                      p.channels % 64 != 0));
+      able = !temporary || !other;
+    } else if (gather_f16_us(whole, packs, whole_temporary) <
+               gather_f16_us(*plan, packs, true)) {
+      plan = &whole;
+      temporary = whole_temporary;
+    }
   }
   const double general_us = general ? general_f16_us(r) : kNever;
   const double one_lane_us = direct_us(direction, p, r, true);
@@ -1624,8 +1659,7 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p,
     if (plan.ok &&
         direct_us(direction, p, products_of(direction, p), false) +
                 (fused ? 2.0 : 0.0) <
-            7.3 + 0.87 * plan.us + plan.out_elems / 5.2e6 +
-                (plan.wide_bytes + plan.pack_blocks * 2048.0) / 1.8e6)
+            gather_f32_us(plan, true, false))
       return false;
   }
   // At most one 64 x 64 tile per compute unit and a short reduction in whole
@@ -1734,23 +1768,41 @@ int launch_conv2d_gather_f32(int direction, const float* input,
   const GatherPlan* plan = &make_plan<float>(direction, p);
   if (!plan->ok || !aligned(output) || (!plan->widen && !aligned(input)))
     return -1;
-  // A stream that records a graph gives no temporaries: without them (the
-  // caller's workspace has no room either) the reduction stays whole, and what
-  // cannot do without is left to the kernels that need none.
+  const bool fuse = direction == SNN_HIP_FORWARD && epilogue != nullptr &&
+                    epilogue->wanted();
   const bool packs = plan->from == kPacked || !aligned(filter);
   const size_t room =
       workspace != nullptr && aligned(workspace) ? workspace_elems * 4 : 0;
   if (plan->workspace_bytes(packs) > room) {
-    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(stream, &status) != hipSuccess ||
-        status != hipStreamCaptureStatusNone) {
-      (void)hipGetLastError();
-      plan = &make_plan<float>(direction, p, false);
-      if (plan->workspace_bytes(packs) > room) return -1;
+    const GatherPlan& whole = make_plan<float>(direction, p, false);
+    const bool whole_temporary = whole.workspace_bytes(packs) > room;
+    if (stream_captures(stream)) {
+      // Recorded without room the reduction stays whole, and what cannot do
+      // without a temporary is left to the kernels that need none.
+      plan = &whole;
+      if (whole_temporary) return -1;
+    } else {
+      // The host time of a temporary is as much as a short launch: the
+      // reduction stays whole, or another kernel that needs none takes over,
+      // where that is estimated to be the faster one (18x18x18 36 -> 100,
+      // 3x3 stride 2: 21.3 -> 12.3 us).
+      const double split_us = gather_f32_us(*plan, packs, true);
+      const double whole_us = gather_f32_us(whole, packs, whole_temporary);
+      if (whole_us < split_us) plan = &whole;
+      const bool all_aligned = aligned(input) && aligned(filter);
+      const Products r = products_of(direction, p);
+      const double other_us =
+          p.features % 4 != 0 ? direct_us(direction, p, r, false)
+          : p.channels % 4 == 0 && all_aligned &&
+                  (direction == SNN_HIP_FORWARD ||
+                   (p.stride_rows == 1 && p.stride_cols == 1))
+              ? igemm_f32_us(r)
+              : kNever;
+      if ((epilogue == nullptr || !epilogue->deterministic) &&
+          other_us + (fuse ? 2.0 : 0.0) < std::min(split_us, whole_us))
+        return -1;
     }
   }
-  const bool fuse = direction == SNN_HIP_FORWARD && epilogue != nullptr &&
-                    epilogue->wanted();
   const int rc = launch_gather<float>(
       *plan, input, filter, output, workspace, workspace_elems,
       fuse ? epilogue->bias : nullptr, fuse && epilogue->relu, stream);

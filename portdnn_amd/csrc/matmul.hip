@@ -307,7 +307,7 @@ int launch_matmul_f16(const _Float16* lhs, const _Float16* rhs,
     }
     // What the kernel below takes.  A product whose reduction fills no whole
     // chunks of 64 needs a temporary over there, for B packed or for A in whole
-    // 16-byte pieces, 14 us of host time: 2588x14x56 4.6 us here, 24.1 there,
+    // 16-byte pieces, 22 us of host time a call: 2588x14x56 4.6 us here, 24.1 there,
     // 97x1189x338 135 and 28.  (The estimate is within 5 % for half of 395
     // random products.)
     const double rounds = static_cast<double>(ceil_div(m, kTile)) *

@@ -49,6 +49,8 @@ SHAPES = [
     (7, 45, 45, 6, 6, 1, 1, False),     # ... and its gradient
     (25, 14, 18, 56, 424, 1, 2, True),  # ... the implicit-GEMM kernel
     (1, 30, 30, 441, 52, 1, 1, True),   # ... its gradient
+    (18, 18, 18, 36, 100, 3, 2, True),  # shared, or without a workspace whole
+    (5, 37, 27, 32, 40, 3, 1, True),
 ]
 
 
