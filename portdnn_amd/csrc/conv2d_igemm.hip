@@ -2069,7 +2069,8 @@ bool conv2d_filter_backprop_f16_supports(const snn_hip_conv2d_params& p) {
           max(x, y) * sizeof(_Float16) <= kMaxBufferBytes &&
           static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
                   p.features * sizeof(float) <= kMaxBufferBytes) ||
-         conv2d_filter_backprop_direct_f16_supports(p);
+         conv2d_filter_backprop_direct_f16_supports(p) ||
+         conv2d_filter_backprop_window_f16_supports(p);
 }
 
 int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
@@ -2093,33 +2094,41 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
                           p.channels * p.features;
   const bool ws_aligned =
       workspace != nullptr && (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0;
-  const bool is_3x3 = conv2d_filter_backprop_3x3_f16_supports(p);
-  if ((is_3x3 || conv2d_filter_backprop_1x1_f16_supports(p)) &&
+  const bool windowed = conv2d_filter_backprop_window_f16_supports(p);
+  if ((windowed || conv2d_filter_backprop_1x1_f16_supports(p)) &&
       (reinterpret_cast<uintptr_t>(dw) & 7u) == 0 &&
       SNN_TUNING_ENV("SNN_HIP_FILBK_F16_OFF") == nullptr) {
     // binary16 matrix instructions; the partial tiles go to the workspace
-    // when it holds them, else to a stream-ordered temporary
+    // when it holds them, else to a stream-ordered temporary (or, when there is
+    // none, to the kernel below, which needs less)
     const size_t part_floats =
-        is_3x3 ? conv2d_filter_backprop_3x3_f16_partial_floats(p)
-               : conv2d_filter_backprop_1x1_f16_partial_floats(p);
+        windowed ? conv2d_filter_backprop_window_f16_partial_floats(p)
+                 : conv2d_filter_backprop_1x1_f16_partial_floats(p);
     float* part = reinterpret_cast<float*>(workspace);
     const bool own = !ws_aligned || workspace_elems < 2 * part_floats;
+    bool room = true;
     if (own) {
       void* ptr = nullptr;
       if (temp_malloc_async(&ptr, part_floats * sizeof(float), stream) !=
-          hipSuccess)
-        return SNN_HIP_ALLOCATION_PROBLEM;
+          hipSuccess) {
+        if (!conv2d_filter_backprop_direct_f16_supports(p))
+          return SNN_HIP_ALLOCATION_PROBLEM;
+        (void)hipGetLastError();
+        room = false;
+      }
       part = static_cast<float*>(ptr);
     }
-    const int status =
-        is_3x3
-            ? launch_conv2d_filter_backprop_3x3_f16(x, dy, dw, part, p, stream)
-            : launch_conv2d_filter_backprop_1x1_f16(x, dy, dw, part, p, stream);
-    const hipError_t err = hipGetLastError();
-    if (own) temp_free_async(part, stream);
-    if (status != SNN_HIP_OK) return status;
-    if (err != hipSuccess) return report_hip_error(err, "f16 filter backprop");
-    return SNN_HIP_OK;
+    if (room) {
+      const int status =
+          windowed
+              ? launch_conv2d_filter_backprop_window_f16(x, dy, dw, part, p, stream)
+              : launch_conv2d_filter_backprop_1x1_f16(x, dy, dw, part, p, stream);
+      const hipError_t err = hipGetLastError();
+      if (own) temp_free_async(part, stream);
+      if (status != SNN_HIP_OK) return status;
+      if (err != hipSuccess) return report_hip_error(err, "f16 filter backprop");
+      return SNN_HIP_OK;
+    }
   }
   if (conv2d_filter_backprop_direct_f16_supports(p)) {
     // every other shape with at least 256 output pixels: binary16 operands
@@ -2143,6 +2152,7 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
     if (err != hipSuccess) return report_hip_error(err, "f16 filter backprop");
     return SNN_HIP_OK;
   }
+  if (p.channels % 64 != 0 || p.features % 4 != 0) return -1;
   float* acc32 = reinterpret_cast<float*>(workspace);
   bool temporary = false;
   if (workspace == nullptr || workspace_elems < 2 * dw_elems ||

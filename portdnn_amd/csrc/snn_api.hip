@@ -418,8 +418,8 @@ size_t f16_workspace_halves(const snn_hip_conv2d_params& p, int direction) {
   if (direction != SNN_HIP_FILTER_BACKPROP)
     return conv2d_f16_workspace_halves(direction, p);
   if (!conv2d_filter_backprop_f16_supports(p)) return 0;
-  if (conv2d_filter_backprop_3x3_f16_supports(p))
-    return 2 * conv2d_filter_backprop_3x3_f16_partial_floats(p);
+  if (conv2d_filter_backprop_window_f16_supports(p))
+    return 2 * conv2d_filter_backprop_window_f16_partial_floats(p);
   if (conv2d_filter_backprop_1x1_f16_supports(p))
     return 2 * conv2d_filter_backprop_1x1_f16_partial_floats(p);
   if (conv2d_filter_backprop_direct_f16_supports(p))
@@ -853,9 +853,11 @@ int launch_gemm_path<_Float16>(int direction, const _Float16* input,
   }
   if (direction == SNN_HIP_FILTER_BACKPROP &&
       conv2d_filter_backprop_f16_supports(p) && aligned16(input) &&
-      aligned16(filter))
-    return launch_conv2d_filter_backprop_f16(input, filter, output, p,
-                                             workspace, workspace_elems, s);
+      aligned16(filter)) {
+    const int rc = launch_conv2d_filter_backprop_f16(
+        input, filter, output, p, workspace, workspace_elems, s);
+    if (rc >= 0) return rc;
+  }
   {
     const int rc = launch_f16_through_fp32(direction, input, filter, output, p, s);
     if (rc >= 0) return rc;

@@ -171,6 +171,8 @@ size_t conv2d_filter_backprop_direct_f32_partial_floats(
     const snn_hip_conv2d_params& p);
 size_t conv2d_filter_backprop_direct_f16_partial_floats(
     const snn_hip_conv2d_params& p);
+// estimated time of the f16 form with multiples of 4
+double conv2d_filter_backprop_direct_f16_us(const snn_hip_conv2d_params& p);
 int launch_conv2d_filter_backprop_direct_f32(const float* input,
                                              const float* output_gradient,
                                              float* filter_gradient,
@@ -297,17 +299,19 @@ int launch_conv2d_few_f16_filter_backprop(const _Float16* x,
                                           size_t workspace_elems,
                                           hipStream_t stream);
 
-// conv2d_filter_backprop_f16.hip: 3x3 stride-1 SAME filter gradient on the
-// binary16 matrix cores (channels and features multiples of 64).  `part` is
-// scratch of ..._partial_floats(p) floats for the partial tiles.
-bool conv2d_filter_backprop_3x3_f16_supports(const snn_hip_conv2d_params& p);
-size_t conv2d_filter_backprop_3x3_f16_partial_floats(
+// conv2d_filter_backprop_window_f16.hip: filter gradients of 3x3 (stride 1 and 2)
+// and 5x5 windows on the binary16 matrix cores, channels and features in
+// multiples of 8, where it is the faster one.  x, dy 16-byte and dw 8-byte
+// aligned; `part` is scratch of ..._partial_floats(p) floats for the partial
+// tiles.
+bool conv2d_filter_backprop_window_f16_supports(const snn_hip_conv2d_params& p);
+size_t conv2d_filter_backprop_window_f16_partial_floats(
     const snn_hip_conv2d_params& p);
-int launch_conv2d_filter_backprop_3x3_f16(const _Float16* x,
-                                          const _Float16* dy, _Float16* dw,
-                                          float* part,
-                                          const snn_hip_conv2d_params& p,
-                                          hipStream_t stream);
+int launch_conv2d_filter_backprop_window_f16(const _Float16* x,
+                                             const _Float16* dy, _Float16* dw,
+                                             float* part,
+                                             const snn_hip_conv2d_params& p,
+                                             hipStream_t stream);
 // The same for 1x1 stride-1 unpadded layers (one flat stream of pixels).
 bool conv2d_filter_backprop_1x1_f16_supports(const snn_hip_conv2d_params& p);
 size_t conv2d_filter_backprop_1x1_f16_partial_floats(
@@ -320,7 +324,8 @@ int launch_conv2d_filter_backprop_1x1_f16(const _Float16* x,
 // The half-precision filter gradient (conv2d_igemm.hip): those two kernels, the
 // direct-operand one, and for other channel counts in multiples of 64 the fp32
 // matrix instructions with an fp32 accumulation buffer, in the workspace when it
-// holds twice the filter's element count, else in a stream-ordered temporary.
+// holds twice the filter's element count, else in a stream-ordered temporary.  -1
+// where none of them takes the operands.
 bool conv2d_filter_backprop_f16_supports(const snn_hip_conv2d_params& p);
 int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
                                       _Float16* dw,
