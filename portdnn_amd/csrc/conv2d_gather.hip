@@ -1395,14 +1395,16 @@ bool rowtile_params(int direction, const snn_hip_conv2d_params& p,
 
 // 1x1, stride 1, no padding: a plain row-major GEMM over the pixels, X * W for
 // the forward and dY * W^T for the gradient.
+bool is_pixel_gemm(const snn_hip_conv2d_params& p) {
+  return p.window_rows == 1 && p.window_cols == 1 && p.stride_rows == 1 &&
+         p.stride_cols == 1 && p.pad_rows == 0 && p.pad_cols == 0 &&
+         p.out_rows == p.in_rows && p.out_cols == p.in_cols &&
+         static_cast<size_t>(p.batch) * p.in_rows * p.in_cols <=
+             static_cast<size_t>(INT_MAX);
+}
 bool is_rows_gemm(int direction, const snn_hip_conv2d_params& p) {
-  const size_t pixels = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols;
-  if (p.window_rows != 1 || p.window_cols != 1 || p.stride_rows != 1 ||
-      p.stride_cols != 1 || p.pad_rows != 0 || p.pad_cols != 0 ||
-      p.out_rows != p.in_rows || p.out_cols != p.in_cols ||
-      pixels > static_cast<size_t>(INT_MAX))
-    return false;
-  const int m = static_cast<int>(pixels);
+  if (!is_pixel_gemm(p)) return false;
+  const int m = p.batch * p.in_rows * p.in_cols;
   return direction == SNN_HIP_FORWARD
              ? gemm_rows_f16_supports(m, p.channels, p.features)
              : gemm_nt_f16_supports(m, p.features, p.channels);
@@ -1552,6 +1554,14 @@ int launch_conv2d_f16(int direction, const _Float16* input,
     return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0;
   };
   const bool both_aligned = aligned(input) && aligned(filter);
+  if (aligned(output) && both_aligned && is_pixel_gemm(p)) {
+    const bool grad = direction == SNN_HIP_INPUT_BACKPROP;
+    const int m = p.batch * p.in_rows * p.in_cols;
+    const int k = grad ? p.features : p.channels;
+    const int n = grad ? p.channels : p.features;
+    if (gemm_short_f16_wanted(m, k, n, grad))
+      return launch_gemm_short_f16(input, filter, output, m, k, n, grad, stream);
+  }
   if (aligned(output) && is_rows_gemm(direction, p) && both_aligned) {
     const int m = p.batch * p.in_rows * p.in_cols;
     return direction == SNN_HIP_FORWARD

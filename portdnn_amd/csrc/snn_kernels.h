@@ -229,6 +229,14 @@ bool gemm_nt_f16_supports(int m, int k, int n);
 int launch_gemm_nt_f16(const _Float16* x, const _Float16* w, _Float16* y, int m,
                        int k, int n, hipStream_t stream);
 
+// Both products with few tiles of 32 x 64 (gemm_short_f16.hip): the waves of a
+// work-group share the reduction.  k and n in multiples of 8, operands 16-byte
+// aligned.  `wanted`: it takes the shape and is the faster one.
+bool gemm_short_f16_wanted(int m, int k, int n, bool transpose_w);
+int launch_gemm_short_f16(const _Float16* x, const _Float16* w, _Float16* y,
+                          int m, int k, int n, bool transpose_w,
+                          hipStream_t stream);
+
 // Half-precision forward convolution and input gradient (conv2d_gather.hip):
 // stride-1 unpadded 1x1 layers on the row-major GEMM kernels above, stride-1
 // layers that fill the GPU on the LDS-tile kernel, every other window (up to
