@@ -1,6 +1,7 @@
 // The C ABI of libsnn_hip.so: parameter validation, algorithm support rules,
 // workspace sizing and dispatch to the kernel launchers.
 #include <atomic>
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -908,6 +909,34 @@ int launch_gemm_path<float>(int direction, const float* input,
   return launch_conv2d_direct<float>(direction, input, filter, output, p, s);
 }
 
+// Whether a Winograd launch of few units of work (32 tiles x 32 features) is
+// slower than the kernels behind the Tiled tag, which transform no filter first.
+// On 90 random layers of 1024 pixels and more, both directions: below 128 units
+// and with chunks of the channel range to split, Winograd zero-fills the output
+// and adds through atomics, 17 us and more against 9 us + 0.0225 us per million
+// multiply-adds (single image 56x56x128 -> 128: 25.8 / 16.5 us; of 30 such layers
+// two are slower here, 28.6 against 24.8 the most); with fewer than eight chunks
+// it takes 8 us + 1.15 per chunk (single image 56x56x64: 12.4, one launch of the
+// kernel for small layers 6.8; 38x28x64 -> 96 at batch 5: 12.5 / 14.5); a single
+// chunk of 16 channels runs on its slower kernel (42x32x16 -> 416 at batch 3: 12.3
+// / 9.8; 75x98x16 -> 416: 28 / 23).
+bool winograd_loses(int direction, const snn_hip_conv2d_params& p) {
+  const bool backprop = direction == SNN_HIP_INPUT_BACKPROP;
+  const int in_ch = backprop ? p.features : p.channels;
+  const int out_ch = backprop ? p.channels : p.features;
+  const int rows = backprop ? p.in_rows : p.out_rows;
+  const int cols = backprop ? p.in_cols : p.out_cols;
+  const double tiles =
+      static_cast<double>(p.batch) * ceil_div(rows, 2) * ceil_div(cols, 2);
+  const double units = std::ceil(tiles / 32) * (out_ch / 32);
+  const int chunks = in_ch / 16;
+  if (!backprop && conv2d_small_supports(p)) return true;
+  if (chunks == 1) return true;
+  if (units >= 128) return false;
+  const double macs_m = 9e-6 * p.batch * rows * cols * in_ch * out_ch;
+  return chunks >= 8 || 9 + 0.0225 * macs_m < 8 + 1.15 * chunks;
+}
+
 // Winograd / WinogradLarge: F(2x2,3x3) for forward and input backprop of 3x3
 // stride-1 convolutions and F(3x3,2x2) for their filter gradient; F(2,3)
 // along the window's axis for the 1x3 / 3x1 windows the selector also accepts
@@ -932,6 +961,25 @@ int launch_winograd_path<float>(int direction, const float* input,
                                 hipStream_t s, const LaunchOptions* epilogue) {
   // SNN_HIP_WINO_UNFUSED is a development switch that forces the three-stage
   // chain on shapes the fused kernel would take.
+  // Neither where a filter is or was transformed ahead, nor in place of a
+  // reproducible launch (the others add through atomics) unless on the kernel for
+  // small layers, nor where the other launch would take a temporary.
+  const bool plain = epilogue == nullptr ||
+                     (!epilogue->prepare_only && !epilogue->filter_prepared);
+  const bool reproducible = epilogue != nullptr && epilogue->deterministic;
+  const bool fused_epilogue = direction == SNN_HIP_FORWARD &&
+                              epilogue != nullptr && epilogue->wanted();
+  if (plain && direction != SNN_HIP_FILTER_BACKPROP &&
+      conv2d_winograd_fused_supports(direction, p) && aligned16(input) &&
+      aligned16(filter) && aligned16(output) && aligned16(workspace) &&
+      winograd_loses(direction, p) &&
+      (!reproducible ||
+       (direction == SNN_HIP_FORWARD && conv2d_small_supports(p) &&
+        !conv2d_gather_f32_wanted(direction, p, fused_epilogue))) &&
+      (!conv2d_gather_f32_wanted(direction, p, fused_epilogue) ||
+       conv2d_gather_f32_workspace_floats(direction, p) <= workspace_elems))
+    return launch_gemm_path<float>(direction, input, filter, output, p, s,
+                                   workspace, workspace_elems, epilogue);
   // (the input gradient's filter transform reads the filter 16 bytes at a time)
   if (conv2d_winograd_fused_supports(direction, p) && aligned16(input) &&
       aligned16(output) && aligned16(workspace) &&

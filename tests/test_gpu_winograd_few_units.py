@@ -1,0 +1,57 @@
+"""fp32 Winograd launches of few units of work: plain ones run on the kernels
+behind the Tiled tag where those are faster, ones with a filter transformed ahead
+stay on the Winograd kernels (whole and split channel ranges)."""
+import numpy as np
+import pytest
+import torch
+
+from portdnn_amd import ops
+from portdnn_amd.capi import ALGO, DIRECTION
+from test_gpu_parity import (ORACLE_FN, assert_close, dev, oracle_params,
+                             uniform)
+
+pytestmark = pytest.mark.gpu
+
+# batch, rows, cols, channels, features, same
+SHAPES = [
+    (1, 56, 56, 64, 64, True),    # the kernel for small layers
+    (3, 13, 11, 16, 64, True),    # one chunk of 16 channels
+    (2, 9, 10, 128, 32, False),   # eight chunks
+    (1, 7, 7, 512, 512, True),    # split channel range
+    (5, 6, 5, 48, 96, True),      # a line of the rule on each side
+    (5, 38, 28, 64, 96, True),
+]
+
+
+@pytest.mark.parametrize("direction", [DIRECTION.FORWARD,
+                                       DIRECTION.INPUT_BACKPROP])
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+def test_winograd_few_units(shape, direction):
+    batch, rows, cols, channels, features, same = shape
+    if direction == DIRECTION.INPUT_BACKPROP:
+        channels, features = features, channels
+    p = ops.conv_params(batch, rows, cols, channels, features, 3, 1, same)
+    rng = np.random.default_rng(8100 + rows)
+    n_a, n_b, _ = ops.conv_sizes(p, direction)
+    a, b = uniform(rng, n_a), uniform(rng, n_b)
+    ref = np.asarray(ORACLE_FN[direction](
+        a, b, oracle_params(p, features), acc64=True)).reshape(-1)
+    da, db = dev(a), dev(b)
+    _, rec = ops.workspace_size(p, direction, ALGO.WINOGRAD)
+    ws = torch.empty(rec, dtype=torch.float32, device="cuda")
+    plain = ops.conv2d(da, db, p, direction, ALGO.WINOGRAD, workspace=ws)
+    assert_close(plain.cpu().numpy(), ref, (shape, direction))
+    ops.conv2d_prepare_filter(db, p, direction, ALGO.WINOGRAD, ws)
+    for _ in range(2):
+        got = ops.conv2d_prepared(da, db, p, direction, ALGO.WINOGRAD, ws)
+        assert_close(got.cpu().numpy(), ref, (shape, direction, "prepared"))
+    same_bits = [ops.conv2d_deterministic(da, db, p, direction, ALGO.WINOGRAD,
+                                          ws) for _ in range(2)]
+    assert torch.equal(*same_bits)
+    assert_close(same_bits[0].cpu().numpy(), ref, (shape, "deterministic"))
+    if direction == DIRECTION.FORWARD:
+        bias = uniform(rng, features)
+        want = np.maximum(ref.reshape(-1, features) + bias, 0).reshape(-1)
+        got = ops.conv2d_bias_act(da, db, dev(bias), p, ALGO.WINOGRAD,
+                                  relu=True, workspace=ws)
+        assert_close(got.cpu().numpy(), want, (shape, "bias"))
