@@ -1383,16 +1383,6 @@ bool as_forward_of_dy(const snn_hip_conv2d_params& p,
   return true;
 }
 
-// The forward convolution the LDS-tile kernel would run, if it is wanted.
-bool rowtile_params(int direction, const snn_hip_conv2d_params& p,
-                    snn_hip_conv2d_params* q) {
-  if (direction == SNN_HIP_FORWARD)
-    *q = p;
-  else if (!as_forward_of_dy(p, q))
-    return false;
-  return conv2d_rowtile_f16_wanted(*q);
-}
-
 // 1x1, stride 1, no padding: a plain row-major GEMM over the pixels, X * W for
 // the forward and dY * W^T for the gradient.
 bool is_pixel_gemm(const snn_hip_conv2d_params& p) {
@@ -1401,6 +1391,13 @@ bool is_pixel_gemm(const snn_hip_conv2d_params& p) {
          p.out_rows == p.in_rows && p.out_cols == p.in_cols &&
          static_cast<size_t>(p.batch) * p.in_rows * p.in_cols <=
              static_cast<size_t>(INT_MAX);
+}
+bool is_short_gemm(int direction, const snn_hip_conv2d_params& p) {
+  const bool grad = direction == SNN_HIP_INPUT_BACKPROP;
+  return is_pixel_gemm(p) &&
+         gemm_short_f16_wanted(p.batch * p.in_rows * p.in_cols,
+                               grad ? p.features : p.channels,
+                               grad ? p.channels : p.features, grad);
 }
 bool is_rows_gemm(int direction, const snn_hip_conv2d_params& p) {
   if (!is_pixel_gemm(p)) return false;
@@ -1476,6 +1473,27 @@ double direct_us(int direction, const snn_hip_conv2d_params& p,
          (loop <= 16 ? 1.0 : 2.0);  // (longer ones up to three times that)
 }
 
+// The forward convolution the LDS-tile kernel would run, if it is wanted.
+bool rowtile_params(int direction, const snn_hip_conv2d_params& p,
+                    snn_hip_conv2d_params* q) {
+  if (direction == SNN_HIP_FORWARD)
+    *q = p;
+  else if (!as_forward_of_dy(p, q))
+    return false;
+  double other_us = kNever;
+  if (p.window_rows == 3 && p.window_cols == 3 && p.stride_rows == 1 &&
+      p.stride_cols == 1 && p.channels % 64 == 0 && p.features % 64 == 0) {
+    const GatherPlan& plan = make_plan<_Float16>(direction, p);
+    // (the estimate was fitted to shorter layers: 13x198x148 256 -> 64, no padding,
+    // takes 227 us there)
+    const bool longer = products_of(direction, p).macs > 1.5e9;
+    if (plan.ok)
+      other_us = gather_f16_us(plan, plan.from == kPacked, false) *
+                 (longer ? 1.2 : 1.0);
+  }
+  return conv2d_rowtile_f16_wanted(*q, other_us);
+}
+
 // The same in fp32: this kernel, and the implicit-GEMM one for counts in
 // multiples of 4 and stride 1 (or forward), whose shared reductions meet through
 // atomics after a launch that clears the output.  (Half of 270 and of 970 layers
@@ -1510,8 +1528,10 @@ bool stream_captures(hipStream_t stream) {
 
 }  // namespace
 
-bool conv2d_gather_tile_f16(int direction, const snn_hip_conv2d_params& p,
-                            GatherTile* tile) {
+namespace {
+
+bool gather_tile_f16(int direction, const snn_hip_conv2d_params& p,
+                     GatherTile* tile) {
   snn_hip_conv2d_params q;
   if (is_rows_gemm(direction, p) || rowtile_params(direction, p, &q))
     return false;
@@ -1528,6 +1548,13 @@ bool conv2d_gather_tile_f16(int direction, const snn_hip_conv2d_params& p,
   return true;
 }
 
+}  // namespace
+
+bool conv2d_gather_tile_f16(int direction, const snn_hip_conv2d_params& p,
+                            GatherTile* tile) {
+  return !is_short_gemm(direction, p) && gather_tile_f16(direction, p, tile);
+}
+
 size_t conv2d_f16_workspace_halves(int direction,
                                    const snn_hip_conv2d_params& p) {
   snn_hip_conv2d_params q;
@@ -1535,7 +1562,9 @@ size_t conv2d_f16_workspace_halves(int direction,
     return static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
            p.features;
   GatherTile tile;
-  if (!conv2d_gather_tile_f16(direction, p, &tile)) return 0;
+  // (that of a short product, too, which takes it when an operand is not 16-byte
+  // aligned)
+  if (!gather_tile_f16(direction, p, &tile)) return 0;
   const GatherPlan& plan = make_plan<_Float16>(direction, p);
   // (with room for the packed filter also where the gradient's is read in
   // place, for one that is not 16-byte aligned; that of a 1x1 layer would take
@@ -1554,13 +1583,12 @@ int launch_conv2d_f16(int direction, const _Float16* input,
     return (reinterpret_cast<uintptr_t>(ptr) & 15u) == 0;
   };
   const bool both_aligned = aligned(input) && aligned(filter);
-  if (aligned(output) && both_aligned && is_pixel_gemm(p)) {
+  if (aligned(output) && both_aligned && is_short_gemm(direction, p)) {
     const bool grad = direction == SNN_HIP_INPUT_BACKPROP;
-    const int m = p.batch * p.in_rows * p.in_cols;
-    const int k = grad ? p.features : p.channels;
-    const int n = grad ? p.channels : p.features;
-    if (gemm_short_f16_wanted(m, k, n, grad))
-      return launch_gemm_short_f16(input, filter, output, m, k, n, grad, stream);
+    return launch_gemm_short_f16(input, filter, output,
+                                 p.batch * p.in_rows * p.in_cols,
+                                 grad ? p.features : p.channels,
+                                 grad ? p.channels : p.features, grad, stream);
   }
   if (aligned(output) && is_rows_gemm(direction, p) && both_aligned) {
     const int m = p.batch * p.in_rows * p.in_cols;

@@ -25,13 +25,16 @@
 //
 // Each wave owns 2 feature blocks x 4 pixel blocks (64 features x 128
 // pixels, 128 accumulator registers): per 16-deep reduction step it reads
-// 4 KB from LDS and 2 KB of filter for 8 MFMAs.  Layers with too few such
-// tiles to fill the SIMDs use 2 x 2 blocks per wave instead.
+// 4 KB from LDS and 2 KB of filter for 8 MFMAs; or, where that balances the
+// compute units better, 2 x 2 blocks.  224x224x64 at batch 16, 3x3: 86 us (69
+// without the stores, 71 without the loads, 55 with neither).
 //
 // portDNN's half build accumulates in half (e.g. `DataType out_val{0}` with
 // T = cl::sycl::half in src/conv2d/direct/kernels_nhwc.h:92); accumulating in
 // fp32 is more accurate and stays inside the 1e-2 relative bar against it.
 #include <algorithm>
+#include <array>
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -51,6 +54,7 @@ typedef unsigned int uint4v __attribute__((ext_vector_type(4)));
 constexpr unsigned kOob = 0x7FFFFFF0u;
 constexpr int kStoreAux = 2;  // the output is written once: stream it (slc)
 constexpr size_t kMaxBufferBytes = 0x7FFFFFF0u;
+constexpr int kNumCus = 256;
 constexpr int kFA = 2;  // feature blocks (of 32) per wave
 constexpr size_t kMaxLdsBytes = 160 * 1024;
 
@@ -115,12 +119,15 @@ __global__ void __launch_bounds__(256)
 
 // s_waitcnt immediates that wait on the vector-memory counter only.
 constexpr int kWaitVm0 = 0x0F70;
+constexpr int kWaitLgkm0 = 0xC07F;  // (LDS reads)
 constexpr int kWaitVm4 = 0x0F74;
 constexpr int kWaitVm8 = 0x0F78;
 
 // WF x WP waves: WF feature groups of 64, WP pixel groups of PB * 32.  KC =
-// channels per LDS tile.  MULTI: more than one channel block (two LDS tiles,
-// the next one loading while the current one is multiplied).  WIN3: 3x3
+// channels per LDS tile.  BUFS: 1, one channel block; 2, more than one and two LDS
+// tiles, the next one loading while the current one is multiplied; 3, more than
+// one and one LDS tile, so that two work-groups fit a CU and one loads while the
+// other multiplies (3x3 windows only).  WIN3: 3x3
 // window, whose reduction loop is unrolled over a filter row with all tap
 // bookkeeping resolved at compile time.
 //
@@ -134,7 +141,7 @@ constexpr int kWaitVm8 = 0x0F78;
 // bytes = 1 KB of consecutive LDS per instruction; the lanes that fall on pad
 // pieces load from out of range), so a whole tile is in flight without
 // holding registers; out-of-range offsets (padding pixels) store zeros.
-template <int WF, int WP, int PB, int KC, bool MULTI, bool WIN3>
+template <int WF, int WP, int PB, int KC, int BUFS, bool WIN3>
 __global__ void __launch_bounds__(64 * WF * WP)
     __attribute__((amdgpu_waves_per_eu(2, 2)))
     conv_rowtile_f16_kernel(const _Float16* __restrict__ src,
@@ -144,6 +151,8 @@ __global__ void __launch_bounds__(64 * WF * WP)
                             unsigned dst_bytes, unsigned n_groups) {
   constexpr int NT = 64 * WF * WP;
   constexpr int NW = WF * WP;
+  constexpr bool MULTI = BUFS != 1;  // more than one channel block
+  constexpr bool AHEAD = BUFS == 2;  // the next one loads meanwhile
   constexpr int KS = KC / 16;        // MFMA reduction steps per tap
   constexpr int UPT = KS / 2;        // units of two steps per tap
   constexpr int PPS = KC / 8;        // 16-byte pieces of data per slot
@@ -172,7 +181,7 @@ __global__ void __launch_bounds__(64 * WF * WP)
   const int buf_bytes = n_blocks * 1024;
   unsigned char* const bufs = lds;
   unsigned* const table =
-      reinterpret_cast<unsigned*>(lds + (MULTI ? 2 : 1) * buf_bytes);
+      reinterpret_cast<unsigned*>(lds + (AHEAD ? 2 : 1) * buf_bytes);
 
   // Global byte offset of channel 0 of every pixel slot (kOob for padding
   // and for the slots that only fill up the last block).
@@ -302,7 +311,7 @@ __global__ void __launch_bounds__(64 * WF * WP)
     // idle, so this path has none per unit: the loop runs over filter rows
     // with the three taps of a row (UPT units each) unrolled, which also
     // keeps the rotation of the three filter buffers static.
-    int cur_off = 0, nxt_off = buf_bytes;
+    int cur_off = 0, nxt_off = AHEAD ? buf_bytes : 0;
     // Byte offset inside a tile of this lane's fragment of tap (0, 0), step 0.
     // Slots are SLOTB bytes apart, so the taps of a filter row and the steps
     // of a tap are compile-time offsets from the row's address.
@@ -337,7 +346,7 @@ __global__ void __launch_bounds__(64 * WF * WP)
             const int v = sc * UPT + u;  // unit within the filter row
             half8 (&a_use)[2][kFA] = a_buf[v % kRot];
             half8 (&a_fill)[2][kFA] = a_buf[(v + 2) % kRot];
-            if constexpr (MULTI) {
+            if constexpr (AHEAD) {
               if (sc == 0 && u == 0) {
                 if (r == 0 && c + 1 < n_chunks)
                   start_tile(bufs + nxt_off,
@@ -372,7 +381,18 @@ __global__ void __launch_bounds__(64 * WF * WP)
         // can still be outstanding.  No fence: this tile's pixel fragments
         // have all been read into registers, and the barrier alone makes
         // every wave's part of the next tile visible.
-        __builtin_amdgcn_s_waitcnt(0x0F70 | (4 * kFA));
+        if constexpr (AHEAD) {
+          __builtin_amdgcn_s_waitcnt(0x0F70 | (4 * kFA));
+        } else if (c + 1 < n_chunks) {
+          // One buffer: once every wave is done with this tile the next one is
+          // loaded in its place (the CU's other work-group multiplies meanwhile).
+          __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_barrier();
+          __builtin_amdgcn_sched_barrier(0);
+          start_tile(bufs, static_cast<unsigned>((c + 1) * KC * 2));
+          __builtin_amdgcn_s_waitcnt(kWaitVm0);
+        }
         __builtin_amdgcn_sched_barrier(0);
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
@@ -417,7 +437,7 @@ __global__ void __launch_bounds__(64 * WF * WP)
         next_ks = 0;
       }
       load_a(a_fill, step + 2 * (DEPTH - 1));
-      if constexpr (MULTI) {
+      if constexpr (AHEAD) {
         if (tap == 0 && sub == 0 && chunk + 1 < n_chunks) {
           __builtin_amdgcn_sched_barrier(0);
           start_tile(nxt, static_cast<unsigned>((chunk + 1) * KC * 2));
@@ -512,10 +532,36 @@ struct RowTilePlan {
   int wp = 0;            // pixel groups of PB * 32 per work-group
   int pb = 0;            // pixel blocks of 32 per wave
   int kc = 0;            // channels per LDS tile
+  int bufs = 0;          // see BUFS
   size_t lds_bytes = 0;  // 0: shape not supported
   long score = 0;
+  double us = 0;         // estimated
   unsigned n_groups = 0;
 };
+
+// Padded rows a tile of `tile_pixels` consecutive output pixels spans: from the
+// padded row of its first pixel to the padded row of its last pixel plus the
+// window, the largest over all tiles (their position inside an image repeats every
+// image / gcd tiles).
+int rows_spanned(const snn_hip_conv2d_params& p, int tile_pixels) {
+  const int total = p.batch * p.out_rows * p.out_cols;
+  const int padded_rows = p.out_rows + p.window_rows - 1;
+  const int image = p.out_rows * p.out_cols;
+  const int period = std::min(ceil_div(total, tile_pixels),
+                              image / std::gcd(image, tile_pixels) + 1);
+  auto padded_row = [&](int pixel) {
+    const int row = pixel / p.out_cols;
+    return row / p.out_rows * padded_rows + row % p.out_rows;
+  };
+  int rows = 0;
+  for (int t = 0; t < period; ++t) {
+    const int first = t * tile_pixels;
+    const int last = std::min(total - first, tile_pixels) + first - 1;
+    rows = std::max(rows,
+                    padded_row(last) - padded_row(first) + p.window_rows);
+  }
+  return rows;
+}
 
 // Geometry for work-groups of `tile_pixels` consecutive output pixels;
 // lds_bytes == 0 when the tile does not fit.  The score estimates the useful
@@ -523,7 +569,7 @@ struct RowTilePlan {
 // waves per SIMD) times the pixels of a tile, discounted by the unused part
 // of the wave tiles.
 RowTilePlan plan_tile(const snn_hip_conv2d_params& p, int wf, int wp, int pb,
-                      int kc, int tile_pixels) {
+                      int kc, int bufs, int tile_pixels, int lds_rows) {
   RowTilePlan plan;
   RowTile& g = plan.g;
   g.batch = p.batch; g.in_rows = p.in_rows; g.in_cols = p.in_cols;
@@ -535,96 +581,133 @@ RowTilePlan plan_tile(const snn_hip_conv2d_params& p, int wf, int wp, int pb,
   g.tile_pixels = tile_pixels;
   g.padded_rows = p.out_rows + p.window_rows - 1;
   g.halo_cols = p.out_cols + p.window_cols - 1;
-  // Padded rows a tile spans: from the padded row of its first pixel to the
-  // padded row of its last pixel plus the window, the largest over all tiles
-  // (their position inside an image repeats every image / gcd tiles).
-  const long image = static_cast<long>(p.out_rows) * p.out_cols;
-  const long n_tiles = ceil_div(g.total_pixels, tile_pixels);
-  const long period = std::min<long>(
-      n_tiles, image / std::gcd<long>(image, tile_pixels) + 1);
-  auto padded_row = [&](long pixel) {
-    const long row = pixel / p.out_cols;
-    return row / p.out_rows * g.padded_rows + row % p.out_rows;
-  };
-  long lds_rows = 0;
-  for (long t = 0; t < period; ++t) {
-    const long first = t * tile_pixels;
-    const long last =
-        std::min<long>(first + tile_pixels, g.total_pixels) - 1;
-    lds_rows = std::max(lds_rows, padded_row(last) - padded_row(first) +
-                                      p.window_rows);
-  }
-  g.n_slots = static_cast<int>(lds_rows) * g.halo_cols;
+  g.n_slots = lds_rows * g.halo_cols;
   g.n_fslices = p.features / (64 * wf);
-  const int n_chunks = p.channels / kc;
   const size_t slot_bytes = static_cast<size_t>(kc) * 2 + 16;
   const size_t n_blocks = ceil_div(g.n_slots * slot_bytes, size_t{1024});
   const size_t n_table = n_blocks * 1024 / slot_bytes + 1;
   const size_t lds_bytes =
-      (n_chunks > 1 ? 2 : 1) * n_blocks * 1024 + n_table * 4;
+      (bufs == 2 ? 2 : 1) * n_blocks * 1024 + n_table * 4;
   if (lds_bytes > kMaxLdsBytes) return plan;
-  plan.wf = wf; plan.wp = wp; plan.pb = pb; plan.kc = kc;
+  plan.wf = wf; plan.wp = wp; plan.pb = pb; plan.kc = kc; plan.bufs = bufs;
   plan.lds_bytes = lds_bytes;
   const long resident =
       std::min<long>(kMaxLdsBytes / lds_bytes, 8 / (wf * wp));
   plan.score = resident * tile_pixels * tile_pixels / (wp * pb * 32);
-  plan.n_groups = static_cast<unsigned>(n_tiles) *
+  plan.n_groups = static_cast<unsigned>(ceil_div(g.total_pixels, tile_pixels)) *
                   static_cast<unsigned>(g.n_fslices);
+  // The estimated time: rounds of the work-groups that fit the compute units, each
+  // its products (faster per wave with two on a SIMD), then loads at 18 and stores
+  // at 10 bytes per cycle and CU -- on 200 layers the estimates that took a part of
+  // these as hidden behind the products were the worse ones, with one buffer and
+  // with two.
+  const int here =
+      std::min<int>(static_cast<int>(resident),
+                    std::max(1, ceil_div(static_cast<int>(plan.n_groups), kNumCus)));
+  const int n_chunks = p.channels / kc;
+  const int per_simd = ceil_div(here * wf * wp, 4);
+  const double products = n_chunks * p.window_rows * p.window_cols * (kc / 16) *
+                          64.0 * pb * (pb == 2 ? 1.12 : 1.0) *
+                          (per_simd == 1 ? 1.44 : 0.805 * per_simd);
+  const double memory =
+      here * (n_chunks * static_cast<double>(g.n_slots) * kc * 2 / 17.9 +
+              tile_pixels * 128.0 * wf / 10.0);
+  double rounds = static_cast<double>(plan.n_groups) / (kNumCus * here);
+  rounds = rounds < 4 ? std::ceil(rounds) : rounds + 0.5;
+  plan.us = 5.2 + rounds * (products + memory + 2340) / 2000;
   return plan;
 }
 
-// Tile sizes tried: the full capacity of the work-group (tiles then start
-// anywhere in a row), and every whole number of rows below it.
-RowTilePlan best_tile(const snn_hip_conv2d_params& p, int wf, int wp, int pb,
-                      int kc) {
+RowTilePlan compute_plan(const snn_hip_conv2d_params& p) {
   const int total = p.batch * p.out_rows * p.out_cols;
-  const int capacity = std::min(wp * pb * 32, total);
-  RowTilePlan best = plan_tile(p, wf, wp, pb, kc, capacity);
-  for (int rows = capacity / p.out_cols; rows >= 1; --rows) {
-    const RowTilePlan plan = plan_tile(p, wf, wp, pb, kc, rows * p.out_cols);
-    if (plan.lds_bytes != 0 && plan.score > best.score) best = plan;
-  }
+  const bool win3 = p.window_rows == 3 && p.window_cols == 3;
+  // rows spanned by tiles of 64, 128, 256, 512 pixels and of 1, 2, ... rows
+  int of_pixels[4] = {0, 0, 0, 0};
+  std::array<int, 65> of_rows{};
+  // Of the tile sizes -- the full capacity of the work-group (tiles then start
+  // anywhere in a row), and every whole number of rows below it -- the one of the
+  // best score.
+  auto best_tile = [&](int wf, int wp, int pb, int kc, int bufs) {
+    const int full = wp * pb * 32;
+    const int capacity = std::min(full, total);
+    int& spanned = of_pixels[full == 64 ? 0 : full == 128 ? 1 : full == 256 ? 2 : 3];
+    if (spanned == 0) spanned = rows_spanned(p, capacity);
+    RowTilePlan best = plan_tile(p, wf, wp, pb, kc, bufs, capacity, spanned);
+    for (int rows = std::min(64, capacity / p.out_cols); rows >= 1; --rows) {
+      // (not even a tile that lies in one image fits)
+      if (static_cast<size_t>(rows + p.window_rows - 1) *
+              (p.out_cols + p.window_cols - 1) * (kc * 2 + 16) *
+              (bufs == 2 ? 2 : 1) > kMaxLdsBytes)
+        continue;
+      if (of_rows[rows] == 0) of_rows[rows] = rows_spanned(p, rows * p.out_cols);
+      const RowTilePlan plan = plan_tile(p, wf, wp, pb, kc, bufs,
+                                         rows * p.out_cols, of_rows[rows]);
+      if (plan.lds_bytes != 0 && plan.score > best.score) best = plan;
+    }
+    return best;
+  };
+  // Work-groups of two or four waves, 64 features x 64 or 128 pixels each, on 64
+  // (all of them) or 32 channels at a time: the least estimated time.  On 200
+  // layers of 1e9 to 1.2e11 operations the estimates were within 10 % and the one
+  // taken 1.6 % slower than the fastest, on the average.  (By counting wave tiles
+  // and work-groups instead, images of some widths were left with two waves per
+  // CU: 149x149x64 at batch 8 84 us, now 38; 87x87x256 <- 192 at batch 9 196, now 75;
+  // and 224x224x64 at batch 16 with one work-group, whose loads, products and
+  // stores took turns: 105, with two that share the LDS 86.)
+  RowTilePlan best;
+  for (int wf = 1; wf <= (p.features % 128 == 0 ? 2 : 1); ++wf)
+    for (int waves = 2; waves <= 4; waves += 2)
+      for (int pb = 2; pb <= 4; pb += 2)
+        for (int bufs = 1; bufs <= 3; ++bufs) {
+          if ((bufs == 1) != (p.channels == 64) && bufs == 1) continue;
+          if (bufs == 3 && (waves != 4 || !win3)) continue;
+          const RowTilePlan plan =
+              best_tile(wf, waves / wf, pb, bufs == 1 ? 64 : 32, bufs);
+          if (plan.lds_bytes != 0 && (best.lds_bytes == 0 || plan.us < best.us))
+            best = plan;
+        }
   return best;
 }
 
-// One channel block: 64 channels per LDS tile.  Otherwise 32, so that two
-// double-buffered work-groups fit the LDS of a compute unit.  Waves own 64 features x 128
-// pixels when that makes at least 1.5 waves per SIMD, else 64 x 64; the
-// work-group is four waves when at least three work-groups per compute unit
-// result, else two.
-RowTilePlan compute_plan(const snn_hip_conv2d_params& p);
+bool takes(const snn_hip_conv2d_params& p) {
+  const size_t x = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols *
+                   p.channels;
+  const size_t y = static_cast<size_t>(p.batch) * p.out_rows * p.out_cols *
+                   p.features;
+  // (1x1 windows have no taps to reuse an LDS tile over)
+  return p.stride_rows == 1 && p.stride_cols == 1 && p.channels % 64 == 0 &&
+         p.features % 64 == 0 && p.channels > 0 && p.features > 0 &&
+         p.batch > 0 && p.out_rows > 0 && p.out_cols > 0 && p.in_rows > 0 &&
+         p.in_cols > 0 && p.window_rows * p.window_cols > 1 &&
+         (x > y ? x : y) * 2 <= kMaxBufferBytes;
+}
 
-// The plan of the most recent shape is kept per thread: layers are usually
-// launched many times with the same parameters.
-RowTilePlan make_plan(const snn_hip_conv2d_params& p) {
-  thread_local snn_hip_conv2d_params cached_params;
-  thread_local RowTilePlan cached_plan;
-  thread_local bool cached = false;
-  if (!cached || std::memcmp(&cached_params, &p, sizeof(p)) != 0) {
-    cached_plan = compute_plan(p);
-    cached_params = p;
-    cached = true;
+// The plans of a network's layers are kept per thread.
+const RowTilePlan& make_plan(const snn_hip_conv2d_params& p) {
+  struct Entry {
+    bool used = false;
+    snn_hip_conv2d_params params;
+    RowTilePlan plan;
+  };
+  constexpr size_t kEntries = 64;
+  thread_local std::array<Entry, kEntries> cache;
+  const unsigned hash = (((p.channels * 31u + p.features) * 31u + p.in_rows) *
+                             31u + p.in_cols) * 31u + p.batch * 7u +
+                        p.window_rows + p.pad_rows * 5u;
+  Entry& entry = cache[hash % kEntries];
+  if (!entry.used || std::memcmp(&entry.params, &p, sizeof p) != 0) {
+    entry.plan = takes(p) ? compute_plan(p) : RowTilePlan();
+    entry.params = p;
+    entry.used = true;
   }
-  return cached_plan;
+  return entry.plan;
 }
 
-RowTilePlan compute_plan(const snn_hip_conv2d_params& p) {
-  const int kc = p.channels == 64 ? 64 : 32;
-  const int wf = p.features % 128 == 0 ? 2 : 1;
-  const long pixels = static_cast<long>(p.batch) * p.out_rows * p.out_cols;
-  const long wave_tiles = (pixels + 127) / 128 * (p.features / 64);
-  const int pb = wave_tiles >= 1536 ? 4 : 2;
-  const RowTilePlan big = best_tile(p, wf, 4 / wf, pb, kc);
-  if (big.lds_bytes != 0 && big.n_groups >= 768) return big;
-  const RowTilePlan small = best_tile(p, wf, 2 / wf, pb, kc);
-  return small.lds_bytes != 0 ? small : big;
-}
-
-template <int WF, int WP, int PB, int KC, bool MULTI, bool WIN3>
+template <int WF, int WP, int PB, int KC, int BUFS, bool WIN3>
 void launch_plan(const _Float16* input, const _Float16* wpk, _Float16* output,
                  const snn_hip_conv2d_params& p, const RowTilePlan& plan,
                  size_t wgt_elems, hipStream_t stream) {
-  auto kernel = conv_rowtile_f16_kernel<WF, WP, PB, KC, MULTI, WIN3>;
+  auto kernel = conv_rowtile_f16_kernel<WF, WP, PB, KC, BUFS, WIN3>;
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void*>(kernel),
       hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLdsBytes);
@@ -647,18 +730,20 @@ bool launch_shape(const _Float16* input, const _Float16* wpk,
                   const RowTilePlan& plan, size_t wgt_elems,
                   hipStream_t stream) {
   if (plan.wf != WF || plan.wp != WP || plan.pb != PB) return false;
-  const bool multi = p.channels > plan.kc;
   const bool win3 = p.window_rows == 3 && p.window_cols == 3;
-#define SNN_ROWTILE_CASE(KC, MULTI, WIN3)                                     \
-  if (plan.kc == KC && multi == MULTI && win3 == WIN3) {                      \
-    launch_plan<WF, WP, PB, KC, MULTI, WIN3>(input, wpk, output, p, plan,     \
-                                             wgt_elems, stream);              \
+#define SNN_ROWTILE_CASE(KC, BUFS, WIN3)                                      \
+  if (plan.kc == KC && plan.bufs == BUFS && win3 == WIN3) {                   \
+    launch_plan<WF, WP, PB, KC, BUFS, WIN3>(input, wpk, output, p, plan,      \
+                                            wgt_elems, stream);               \
     return true;                                                              \
   }
-  SNN_ROWTILE_CASE(64, false, true)
-  SNN_ROWTILE_CASE(32, true, true)
-  SNN_ROWTILE_CASE(64, false, false)
-  SNN_ROWTILE_CASE(32, true, false)
+  SNN_ROWTILE_CASE(64, 1, true)
+  SNN_ROWTILE_CASE(32, 2, true)
+  if constexpr (WF * WP == 4) {
+    SNN_ROWTILE_CASE(32, 3, true)
+  }
+  SNN_ROWTILE_CASE(64, 1, false)
+  SNN_ROWTILE_CASE(32, 2, false)
 #undef SNN_ROWTILE_CASE
   return false;
 }
@@ -666,33 +751,22 @@ bool launch_shape(const _Float16* input, const _Float16* wpk,
 }  // namespace
 
 // Where this kernel is faster than the gathering one (conv2d_gather.hip,
-// which shares a reduction between work-groups where there are few tiles):
-// short reductions at every size, and long ones with at least 1.5 wave tiles
-// per SIMD that leave two waves on each.  Measured with 3x3 windows, this
-// kernel / the other: 56x56x64 at batch 1 9.6 / 9.9 us, 128 50.7 / 58;
-// 28x28x128 at batch 32 19.4 / 18.7, 64 25.0 / 26.4; 14x14x256 at batch 64
-// 31.5 / 29.8, 128 39.1 / 42.6; 7x7x512 at batch 8 43 / 21, 128 56 / 52;
-// 112x112x128 at batch 4 (one work-group's tiles fill the LDS) 41 / 26.  Windows
-// beyond 12 x 12 the other one does not take (gradient of 2x64x64x64 <- 64,
-// 13x13: 89 us, through fp32 136).
-bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p) {
-  const size_t x = static_cast<size_t>(p.batch) * p.in_rows * p.in_cols *
-                   p.channels;
-  const size_t y = static_cast<size_t>(p.batch) * p.out_rows * p.out_cols *
-                   p.features;
-  if (p.stride_rows != 1 || p.stride_cols != 1) return false;
-  if (p.channels % 64 != 0 || p.features % 64 != 0) return false;
-  // 1x1 windows have no taps to reuse an LDS tile over
-  if (p.window_rows * p.window_cols == 1) return false;
-  if ((x > y ? x : y) * 2 > kMaxBufferBytes) return false;
-  const RowTilePlan plan = make_plan(p);
+// which shares a reduction between work-groups where there are few tiles), whose
+// estimate is `other_us`: 3x3 windows by the estimates of both.  Other windows:
+// short reductions at every size, and long ones with at least 1.5 wave tiles per
+// SIMD that leave two waves on each.  Windows beyond 12 x 12 the other one does
+// not take (gradient of 2x64x64x64 <- 64, 13x13: 89 us, through fp32 136).
+bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p,
+                               double other_us) {
+  const RowTilePlan& plan = make_plan(p);
   if (plan.lds_bytes == 0) return false;
+  if (p.window_rows == 3 && p.window_cols == 3) return plan.us < other_us;
   if (p.window_rows * p.window_cols * p.channels <= 576 ||
       p.window_rows > 12 || p.window_cols > 12)
     return true;
-  const size_t wave_tiles = ceil_div(y / p.features, size_t{64}) *
-                            static_cast<size_t>(p.features / 64);
-  return wave_tiles >= 1536 &&
+  const size_t pixels = static_cast<size_t>(p.batch) * p.out_rows * p.out_cols;
+  return ceil_div(pixels, size_t{64}) * static_cast<size_t>(p.features / 64) >=
+             1536 &&
          (plan.pb == 4 || 2 * plan.lds_bytes <= kMaxLdsBytes);
 }
 
@@ -700,7 +774,7 @@ int launch_conv2d_rowtile_f16(const _Float16* input, const _Float16* filter,
                               _Float16* output, const snn_hip_conv2d_params& p,
                               _Float16* packed, hipStream_t stream,
                               bool transposed_filter) {
-  const RowTilePlan plan = make_plan(p);
+  const RowTilePlan& plan = make_plan(p);
   if (plan.lds_bytes == 0) return SNN_HIP_INVALID_ALGORITHM;
   static const bool print_plan = SNN_TUNING_ENV("SNN_HIP_F16_PLAN") != nullptr;
   if (print_plan)

@@ -349,8 +349,8 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
 // gradient's: `p` then describes the gradient as a forward convolution of dY
 // (channels = the original features and vice versa, padding window - 1 - pad)
 // and `filter` is still the original HWCF tensor.
-// `wanted`: it takes the shape and is the faster one.
-bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p);
+// `wanted`: it takes the shape and is faster than a kernel of `other_us`.
+bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p, double other_us);
 int launch_conv2d_rowtile_f16(const _Float16* input, const _Float16* filter,
                               _Float16* output, const snn_hip_conv2d_params& p,
                               _Float16* packed, hipStream_t stream,

@@ -1,0 +1,51 @@
+"""Binary16 3x3 layers of wide images on the LDS-tile kernel: one tile of all 64
+channels, two of 32 in turn, and one of 32 that is loaded again; whole rows per
+work-group and tiles that start inside a row; one and two feature groups.
+
+Bound: one rounding to binary16 and n fp32 additions.
+"""
+import numpy as np
+import pytest
+import torch
+
+from portdnn_amd import ops
+from portdnn_amd.capi import ALGO, DIRECTION, DTYPE
+from test_gpu_conv_f16_shapes import assert_rounded_once
+from test_gpu_parity import ORACLE_FN, dev, oracle_params, uniform
+
+pytestmark = pytest.mark.gpu
+
+# batch, rows, cols, source channels, produced channels, same
+SHAPES = [
+    (3, 37, 224, 64, 64, True),
+    (1, 61, 300, 64, 64, True),
+    (2, 47, 219, 64, 128, False),
+    (1, 41, 224, 192, 64, True),
+    (2, 29, 150, 64, 192, True),
+    (9, 30, 31, 64, 64, True),
+]
+
+
+@pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("direction",
+                         [DIRECTION.FORWARD, DIRECTION.INPUT_BACKPROP])
+def test_conv_rowtile_f16(shape, direction):
+    batch, rows, cols, source, produced, same = shape
+    channels, features = ((source, produced) if direction == DIRECTION.FORWARD
+                          else (produced, source))
+    p = ops.conv_params(batch, rows, cols, channels, features, 3, 1, same)
+    rng = np.random.default_rng(9100 + rows + cols)
+    n_a, n_b, n_out = ops.conv_sizes(p, direction)
+    a = uniform(rng, n_a).astype(np.float16)
+    b = uniform(rng, n_b).astype(np.float16)
+    ref = ORACLE_FN[direction](a.astype(np.float32), b.astype(np.float32),
+                               oracle_params(p, features), acc64=True)
+    _, rec = ops.workspace_size(p, direction, ALGO.IM2COL, DTYPE.F16)
+    block = torch.full((rec + 4096,), 7.0, dtype=torch.float16, device="cuda")
+    guard = torch.full((n_out + 4096,), 7.0, dtype=torch.float16, device="cuda")
+    got = ops.conv2d(dev(a, torch.float16), dev(b, torch.float16), p, direction,
+                     ALGO.IM2COL, workspace=block[:rec], out=guard[:n_out])
+    assert_rounded_once(got.float().cpu().numpy(), ref, 9 * source,
+                        (shape, direction))
+    assert torch.all(guard[n_out:] == 7.0)
+    assert torch.all(block[rec:] == 7.0)
