@@ -42,6 +42,17 @@
 //   * An fp32 instruction (32x32x2) takes as long as a binary16 one but sums two
 //     products instead of sixteen: there the matrix units are the bound, and
 //     the tap arithmetic of every lane costs nothing beside them.
+//   * Larger fp32 tiles (SPLIT) take every operand apart into three bfloat16 parts
+//     in registers and sum six products of parts -- all but those below 2^-26 of
+//     the whole -- on the bfloat16 instruction, a sixteenth of the time each; the
+//     five small ones in accumulators of their own.  Against 64 bits the sums are
+//     closer than the fp32 instruction's, whose every second product is rounded
+//     (17x27x27 96 -> 256, 5x5: 2.3e-7 and 6.0e-7 in the 2-norm; 56x56x64 -> 256,
+//     1x1: 4e-8 and 1.0e-7).  149 -> 131 us on that layer, 28x28x128 at batch 128,
+//     3x3 (Tiled) 257 -> 200, 147x147x48 -> 64, 5x5, 122 -> 99: 0.15 PFLOP/s, where
+//     the matrix units are busy 0.4 of the time and the splitting takes as many
+//     cycles of the vector units.  A conversion ahead, into three planes, would
+//     move half as many bytes again.
 //   * A strided gradient of few channels (a three-channel first layer) would
 //     fill 3 of the 32 matrix rows.  Its classes are merged: the pixels of a
 //     block of stride x stride share one window of ceil(window / stride) source
@@ -332,11 +343,57 @@ __global__ void __launch_bounds__(256)
   *reinterpret_cast<decltype(v)*>(wide + static_cast<size_t>(idx) * kE) = v;
 }
 
+// An fp32 value as the sum of three bfloat16 ones, the first rounded to nearest
+// (its remainder then has no bias, nor have the products left out), the others
+// cut off: every remainder is exact, and the last one fits.  (Integer operations:
+// the conversion instruction takes as long as four of them.)
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+struct Parts {
+  bf16x8 first, second, third;
+};
+__device__ __forceinline__ Parts split_parts(const float4v& e,
+                                             const float4v& o) {
+  uint4v first, second, third;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    unsigned f[2], s[2], t[2];
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int at = 2 * k + h;
+      const float v = at < 4 ? e[at & 3] : o[at & 3];
+      f[h] = (__builtin_bit_cast(unsigned, v) + 0x8000u) & 0xFFFF0000u;
+      const float rest = v - __builtin_bit_cast(float, f[h]);
+      s[h] = __builtin_bit_cast(unsigned, rest);
+      t[h] = __builtin_bit_cast(
+          unsigned, rest - __builtin_bit_cast(float, s[h] & 0xFFFF0000u));
+    }
+    // the upper halves of two values
+    first[k] = __builtin_amdgcn_perm(f[1], f[0], 0x07060302u);
+    second[k] = __builtin_amdgcn_perm(s[1], s[0], 0x07060302u);
+    third[k] = __builtin_amdgcn_perm(t[1], t[0], 0x07060302u);
+  }
+  return {__builtin_bit_cast(bf16x8, first), __builtin_bit_cast(bf16x8, second),
+          __builtin_bit_cast(bf16x8, third)};
+}
+__device__ __forceinline__ Parts split_parts(const half8&, const half8&) {
+  return {};
+}
+// Whether a sum over split operands has to be taken again without splitting: the
+// parts of an infinity are no numbers and rounding the first part up may overflow,
+// and the matrix units take parts below 2^-126 for zero, which a sum of magnitude
+// 2^-103 and more does not notice.
+__device__ __forceinline__ bool beyond_split(float v) {
+  constexpr unsigned kLeast = 24u << 23, kInfinity = 0x7F800000u;
+  const unsigned u = __builtin_bit_cast(unsigned, v) & 0x7FFFFFFFu;
+  return u != 0u && u - kLeast >= kInfinity - kLeast;
+}
+
 // WM x WN waves of TM x TN blocks of 32 pixels x 32 features.  UNIFORM: whole
 // chunks per tap, tap bookkeeping in scalar registers; otherwise every lane
 // works out the tap of its own piece.  FROM: what `wpk` is; `w` is the caller's
 // filter.
-template <typename T, int WM, int WN, int TM, int TN, bool UNIFORM, int FROM>
+template <typename T, int WM, int WN, int TM, int TN, bool UNIFORM, int FROM,
+          bool SPLIT>
 __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
     conv_gather_kernel(const T* __restrict__ src, const T* __restrict__ wpk,
                        const T* __restrict__ w,
@@ -562,6 +619,31 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
     }
   };
 
+  // SPLIT: all 16 products of a chunk and lane pair in six instructions.
+  float16v low[SPLIT ? TN : 1][SPLIT ? TM : 1];
+  auto multiply_split = [&](const Operands& e, const Operands& o) {
+    Parts a[TN], b[TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i) a[i] = split_parts(e.a[i], o.a[i]);
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      b[j] = split_parts(e.b[j], o.b[j]);
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        auto product = [](const bf16x8& p, const bf16x8& q, const float16v& c) {
+          return __builtin_amdgcn_mfma_f32_32x32x16_bf16(p, q, c, 0, 0, 0);
+        };
+        float16v& lo = low[i][j];
+        lo = product(a[i].third, b[j].first, lo);
+        lo = product(a[i].first, b[j].third, lo);
+        lo = product(a[i].second, b[j].second, lo);
+        lo = product(a[i].second, b[j].first, lo);
+        lo = product(a[i].first, b[j].second, lo);
+        acc[i][j] = product(a[i].first, b[j].first, acc[i][j]);
+      }
+    }
+  };
+
   // One chunk: its step 0 operands are in `even`, the next two chunks are
   // arriving.  Step 1 is read while step 0 multiplies; then every wave is done
   // with the buffer, the load of the chunk after next-but-one goes into it,
@@ -590,7 +672,62 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
     __builtin_amdgcn_sched_barrier(0);
     ++done;
   };
-  if (n_chunks > 0) {
+  // SPLIT: a chunk is read whole, and its buffer free once every wave has.
+  auto step_split = [&](char* cur, bool more1, bool more2, bool more3) {
+    fetch(cur, 0, even);
+    fetch(cur, 1, odd);
+    if (more1) {
+      __builtin_amdgcn_sched_barrier(0);
+      if (more2)
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(LA + LB) & ~0x0F00);  // and LDS
+      else
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0) & ~0x0F00);
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      if (more3) issue(cur);
+    }
+    multiply_split(even, odd);
+    ++done;
+  };
+  if constexpr (SPLIT) {
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) low[i][j][v] = 0.f;
+    if (n_chunks > 0) {
+      issue(buf0);
+      if (n_chunks > 1) issue(buf1);
+      if (n_chunks > 2) issue(buf2);
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+      __builtin_amdgcn_sched_barrier(0);
+      __builtin_amdgcn_s_barrier();
+      __builtin_amdgcn_sched_barrier(0);
+      while (done + 5 < n_chunks) {
+        step_split(buf0, true, true, true);
+        step_split(buf1, true, true, true);
+        step_split(buf2, true, true, true);
+      }
+      auto last = [&](char* cur) {
+        if (done < n_chunks)
+          step_split(cur, done + 1 < n_chunks, done + 2 < n_chunks,
+                     done + 3 < n_chunks);
+      };
+      last(buf0);
+      last(buf1);
+      last(buf2);
+      last(buf0);
+      last(buf1);
+    }
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[i][j][v] += low[i][j][v];
+  } else if (n_chunks > 0) {
     issue(buf0);
     if (n_chunks > 1) issue(buf1);
     if (n_chunks > 2) issue(buf2);
@@ -647,17 +784,22 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
   {
     // (a maximum that keeps NaNs: two values per instruction)
     float most = 0.f;
+    bool odd = false;
 #pragma unroll
     for (int j = 0; j < TM; ++j)
 #pragma unroll
       for (int i = 0; i < TN; ++i) {
         float block = 0.f;
 #pragma unroll
-        for (int v = 0; v < 16; ++v)
-          block = __builtin_elementwise_maximum(block, acc[i][j][v]);
+        for (int v = 0; v < 16; ++v) {
+          if constexpr (SPLIT)
+            odd |= beyond_split(acc[i][j][v]);
+          else
+            block = __builtin_elementwise_maximum(block, acc[i][j][v]);
+        }
         most = __builtin_elementwise_maximum(most, block);
       }
-    if (__builtin_amdgcn_ballot_w64(most != most) != 0) {
+    if (__builtin_amdgcn_ballot_w64(SPLIT ? odd : most != most) != 0) {
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
         const int m = m0 + (wm * TM + j) * 32 + l32;
@@ -668,8 +810,10 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
           unsigned bits = 0;
 #pragma unroll
           for (int v = 0; v < 16; ++v)
-            bits |= acc[i][j][v] != acc[i][j][v] ? 1u << v : 0u;
-          strange[j * TN + i] = cut ? bits : 0u;
+            bits |= (SPLIT ? beyond_split(acc[i][j][v])
+                           : acc[i][j][v] != acc[i][j][v]) ? 1u << v : 0u;
+          strange[j * TN + i] =
+              SPLIT ? (m < cls.pixels ? bits : 0u) : cut ? bits : 0u;
         }
       }
     }
@@ -884,7 +1028,7 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
 
 // Sums the splits of every tile in order and rounds: one float4 -- four
 // consecutive features of a pixel -- per lane.
-template <typename T, int WM, int WN, int TM, int TN>
+template <typename T, int WM, int WN, int TM, int TN, bool SPLIT>
 __global__ void __launch_bounds__(256)
     gather_reduce_kernel(const float4v* __restrict__ part,
                          const T* __restrict__ src, const T* __restrict__ w,
@@ -914,11 +1058,12 @@ __global__ void __launch_bounds__(256)
   for (int s = 0; s < g.n_splits; ++s)
     sum += from[static_cast<size_t>(s) * g.n_tiles * kTileVecs];
   const Pixel px = pixel_of(m, cls);
-  if ((sum[0] != sum[0] || sum[1] != sum[1] || sum[2] != sum[2] ||
-       sum[3] != sum[3]) && window_cut(g, cls, px)) {
+  auto strange = [](float v) { return SPLIT ? beyond_split(v) : v != v; };
+  if ((strange(sum[0]) || strange(sum[1]) || strange(sum[2]) ||
+       strange(sum[3])) && (SPLIT || window_cut(g, cls, px))) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (sum[e] != sum[e] && f + e < g.features)
+      if (strange(sum[e]) && f + e < g.features)
         sum[e] = exact_sum(src, w, g, cls, px, f + e);
   }
   if constexpr (sizeof(T) == 4) {
@@ -974,19 +1119,28 @@ struct GatherPlan {
 };
 
 // Tile shapes, with what one work-group needs per chunk: alone on its CU
-// (bound by the time a load takes) and its share of a CU that is full.
+// (bound by the time a load takes) and its share of a CU that is full; `split`:
+// see kTilesF32.
 struct TileShape {
   int pixels, features;
   double alone_us, share_us;
+  bool split;
 };
 constexpr TileShape kTilesF16[] = {
-    {256, 128, 0.57, 0.46}, {256, 64, 0.34, 0.376}, {128, 128, 0.27, 0.24},
-    {128, 64, 0.245, 0.17},  {128, 32, 0.23, 0.135}, {64, 64, 0.22, 0.103}};
+    {256, 128, 0.57, 0.46, false}, {256, 64, 0.34, 0.376, false},
+    {128, 128, 0.27, 0.24, false}, {128, 64, 0.245, 0.17, false},
+    {128, 32, 0.23, 0.135, false}, {64, 64, 0.22, 0.103, false}};
 // (fp32: eight matrix instructions of 64 cycles per chunk and SIMD, in either
 // shape, which one wastes fewer columns decides.  128 x 64 and 128 x 128 need
 // fewer loads per product but were no faster on any of forty shapes: 17x27x27
 // 96 -> 256, 5x5, 158 / 163 us against 162)
-constexpr TileShape kTilesF32[] = {{128, 32, 0.36, 0.27}, {64, 64, 0.36, 0.265}};
+// The larger ones split their operands (SPLIT), and a chunk takes `alone_us` and
+// `share_us` per work-group on the average CU: the rate hangs on the conversions
+// and on power more than on how the tiles fall on compute units.
+constexpr TileShape kTilesF32[] = {{128, 32, 0.36, 0.27, false},
+                                   {64, 64, 0.36, 0.265, false},
+                                   {128, 128, 0.10, 0.88, true},
+                                   {128, 64, 0.27, 0.45, true}};
 constexpr int kMergedTile = 0;
 template <typename T>
 struct Tiles;
@@ -1024,6 +1178,10 @@ void choose_tile(GatherPlan* plan, bool may_split) {
     chunks += g.cls[k].n_chunks;
     longest = std::max(longest, static_cast<double>(g.cls[k].n_chunks));
   }
+  double products = 0;  // multiply-adds, in whole chunks
+  for (int k = 0; k < g.n_classes; ++k)
+    products += static_cast<double>(g.cls[k].pixels) * g.cls[k].n_chunks * 4 *
+                kPiece<T> * g.features;
   chunks /= g.n_classes;
   auto tiles_of = [&](const TileShape& t) {
     return static_cast<double>(ceil_div(pixels, t.pixels)) * g.n_classes *
@@ -1034,14 +1192,22 @@ void choose_tile(GatherPlan* plan, bool may_split) {
     if (g.merged != 0 && i != kMergedTile) continue;
     const TileShape& t = Tiles<T>::shapes[i];
     const double tiles = tiles_of(t);
+    // (split operands: from about 2e9 multiply-adds on faster by 10 to 25 % where
+    // the estimate is lower; below as often slower, on 80 layers)
+    if (t.split && products < 2e9) continue;
     for (int splits = 1; splits <= (may_split ? kMaxSplits<T> : 1); splits *= 2) {
       if (splits > 1 && longest / splits < 4) break;
       const double rounds = std::ceil(tiles * splits / kNumCus);
-      double us = std::max(std::ceil(longest / splits) * t.alone_us,
-                           std::ceil(chunks / splits) * rounds * t.share_us) +
-                  0.5 * rounds;
+      const double filled = std::max(0.9, tiles * splits / kNumCus);
+      double us =
+          t.split ? chunks / longest * std::ceil(longest / splits) *
+                            (t.alone_us + t.share_us * filled) + 3.0 * filled
+                  : std::max(std::ceil(longest / splits) * t.alone_us,
+                             std::ceil(chunks / splits) * rounds * t.share_us) +
+                        0.5 * rounds;
       if (splits > 1)
-        us += 3.0 + splits * tiles * t.pixels * t.features * 8 / 3e6;
+        us += 3.0 + splits * tiles * t.pixels * t.features * 8 /
+                        (t.split ? 4.6e6 : 3e6);
       if (us < best) {
         best = us;
         plan->us = us;
@@ -1242,7 +1408,8 @@ struct GatherOperands {
   FilterFrom from;
 };
 
-template <typename T, int WM, int WN, int TM, int TN, bool UNIFORM, int FROM>
+template <typename T, int WM, int WN, int TM, int TN, bool UNIFORM, int FROM,
+          bool SPLIT>
 void launch_kernel(const GatherOperands<T>& ops, const GatherPlan& plan,
                    const Gather& g, hipStream_t stream) {
   const unsigned n_groups = g.n_tiles * static_cast<unsigned>(g.n_splits);
@@ -1252,13 +1419,13 @@ void launch_kernel(const GatherOperands<T>& ops, const GatherPlan& plan,
                       : plan.filter_elems * sizeof(T));
   const unsigned dst_bytes = static_cast<unsigned>(plan.out_elems * sizeof(T));
   KernelTimer timer(stream);
-  hipLaunchKernelGGL((conv_gather_kernel<T, WM, WN, TM, TN, UNIFORM, FROM>),
+  hipLaunchKernelGGL((conv_gather_kernel<T, WM, WN, TM, TN, UNIFORM, FROM, SPLIT>),
                      dim3(n_groups), dim3(64 * WM * WN), 0, stream, ops.src,
                      ops.filter, ops.caller_filter, ops.bias, ops.dst, ops.part,
                      g, src_bytes, filter_bytes, dst_bytes, n_groups);
 }
 
-template <typename T, int WM, int WN, int TM, int TN>
+template <typename T, int WM, int WN, int TM, int TN, bool SPLIT = false>
 void launch_tile(const GatherOperands<T>& ops, const GatherPlan& plan,
                  bool relu, hipStream_t stream) {
   constexpr int BM = 32 * WM * TM, BN = 32 * WN * TN;
@@ -1277,25 +1444,32 @@ void launch_tile(const GatherOperands<T>& ops, const GatherPlan& plan,
   g.round_shift = std::max(0, 5 - __builtin_ctz(apart));
   g.turn = g.round_shift > 0 && (g.n_classes & (g.n_classes - 1)) == 0;
   if constexpr (sizeof(T) == 4) {
-    if (ops.from == kInPlace)
-      launch_kernel<T, WM, WN, TM, TN, false, kInPlace>(ops, plan, g, stream);
+    // (scalar tap bookkeeping where the tap arithmetic of every lane would take
+    // vector instructions from the splitting: 3 % of the time)
+    const bool uniform = SPLIT && g.cp % 4 == 0;
+    if (uniform && ops.from == kInPlace)
+      launch_kernel<T, WM, WN, TM, TN, SPLIT, kInPlace, SPLIT>(ops, plan, g, stream);
+    else if (uniform && ops.from == kRows)
+      launch_kernel<T, WM, WN, TM, TN, SPLIT, kRows, SPLIT>(ops, plan, g, stream);
+    else if (ops.from == kInPlace)
+      launch_kernel<T, WM, WN, TM, TN, false, kInPlace, SPLIT>(ops, plan, g, stream);
     else if (ops.from == kRows)
-      launch_kernel<T, WM, WN, TM, TN, false, kRows>(ops, plan, g, stream);
+      launch_kernel<T, WM, WN, TM, TN, false, kRows, SPLIT>(ops, plan, g, stream);
     else
-      launch_kernel<T, WM, WN, TM, TN, false, kPacked>(ops, plan, g, stream);
+      launch_kernel<T, WM, WN, TM, TN, false, kPacked, SPLIT>(ops, plan, g, stream);
   } else {
     const bool uniform = g.cp % 4 == 0;
     if (ops.from == kInPlace && uniform)
-      launch_kernel<T, WM, WN, TM, TN, true, kInPlace>(ops, plan, g, stream);
+      launch_kernel<T, WM, WN, TM, TN, true, kInPlace, SPLIT>(ops, plan, g, stream);
     else if (ops.from == kInPlace)
-      launch_kernel<T, WM, WN, TM, TN, false, kInPlace>(ops, plan, g, stream);
+      launch_kernel<T, WM, WN, TM, TN, false, kInPlace, SPLIT>(ops, plan, g, stream);
     else if (uniform)
-      launch_kernel<T, WM, WN, TM, TN, true, kPacked>(ops, plan, g, stream);
+      launch_kernel<T, WM, WN, TM, TN, true, kPacked, SPLIT>(ops, plan, g, stream);
     else
-      launch_kernel<T, WM, WN, TM, TN, false, kPacked>(ops, plan, g, stream);
+      launch_kernel<T, WM, WN, TM, TN, false, kPacked, SPLIT>(ops, plan, g, stream);
   }
   if (g.n_splits > 1)
-    hipLaunchKernelGGL((gather_reduce_kernel<T, WM, WN, TM, TN>),
+    hipLaunchKernelGGL((gather_reduce_kernel<T, WM, WN, TM, TN, SPLIT>),
                        dim3(g.n_tiles * (BM * BN / 1024)), dim3(256), 0, stream,
                        reinterpret_cast<const float4v*>(ops.part), ops.src,
                        ops.caller_filter, ops.bias, ops.dst, g);
@@ -1344,10 +1518,12 @@ int launch_gather(const GatherPlan& plan, const T* input, const T* filter,
       reinterpret_cast<float*>(packed + pack_blocks * 2048 + plan.wide_bytes),
       from};
   if constexpr (sizeof(T) == 4) {
-    if (plan.tile == 0)
-      launch_tile<T, 4, 1, 1, 1>(ops, plan, relu, stream);
-    else
-      launch_tile<T, 2, 2, 1, 1>(ops, plan, relu, stream);
+    switch (plan.tile) {
+      case 0: launch_tile<T, 4, 1, 1, 1>(ops, plan, relu, stream); break;
+      case 1: launch_tile<T, 2, 2, 1, 1>(ops, plan, relu, stream); break;
+      case 2: launch_tile<T, 2, 2, 2, 2, true>(ops, plan, relu, stream); break;
+      default: launch_tile<T, 2, 2, 2, 1, true>(ops, plan, relu, stream);
+    }
   } else {
     switch (plan.tile) {
       case 0: launch_tile<T, 2, 2, 4, 2>(ops, plan, relu, stream); break;
@@ -1667,12 +1843,25 @@ int launch_conv2d_f16(int direction, const _Float16* input,
                  : -1;
 }
 
+namespace {
+
+// The kernels with the input rows in LDS take 6 us and 55 multiply-adds per ns at
+// their best; tiles with split operands are faster on layers that fill the
+// compute units with them.
+bool split_beats_rows(int direction, const snn_hip_conv2d_params& p,
+                      double macs) {
+  const GatherPlan& plan = make_plan<float>(direction, p);
+  return plan.ok && kTilesF32[plan.tile].split &&
+         gather_f32_us(plan, plan.from == kPacked, false) < 6 + macs / 55e6;
+}
+
 // Where the gathering kernel is faster than the other fp32 kernels behind the
 // Tiled / Im2col / Matmul tags (times: there / here).
 // With a bias and activation (`fused`) those kernels that do not add them on the
-// way are followed by a launch of 2 us.
-bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p,
-                              bool fused) {
+// way are followed by a launch of 2 us.  `over_rows`: also in place of the kernels
+// with the input rows in LDS, which need no temporary.
+bool gather_f32_wanted(int direction, const snn_hip_conv2d_params& p, bool fused,
+                       bool over_rows) {
   if (direction == SNN_HIP_FILTER_BACKPROP) return false;
   if (const char* const env = SNN_TUNING_ENV("SNN_HIP_GATHER_F32"))
     return std::atoi(env) != 0;
@@ -1748,8 +1937,9 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p,
     // 27x27x96 -> 256, 5x5, at batch 17: 144 / 158 us on the rows-in-LDS
     // kernel; where that does not apply 16x28x28 192 -> 96 146 / 115,
     // 13x95x95 208 -> 28, 3x3, 280 / 140, 64x28x28 32 -> 32 60 / 35.
-    return !conv2d_small_supports(p) && !conv2d_rowtile_supports(p) &&
-           !conv2d_rowsplit_supports(p);
+    if (conv2d_small_supports(p)) return false;
+    return !(conv2d_rowtile_supports(p) || conv2d_rowsplit_supports(p)) ||
+           (over_rows && split_beats_rows(direction, p, macs));
   }
   if (conv2d_stem_input_backprop_supports(p)) return false;
   if (strided && p.channels <= 4)  // merged classes
@@ -1763,14 +1953,21 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p,
   // of 64 x 64, where those compute no more columns than tiles of 32 would)
   if (!strided && p.features % 32 == 0 && (p.channels + 31) / 32 % 2 == 0 &&
       macs >= double(1 << 30))
-    return false;
+    return over_rows && split_beats_rows(direction, p, macs);
   snn_hip_conv2d_params q;
   if (as_forward_of_dy(p, &q) &&
       (conv2d_rowtile_supports(q) || conv2d_rowsplit_supports(q)))
-    return false;
+    return over_rows && split_beats_rows(direction, p, macs);
   // 32x56x56 128 <- 128, 3x3 stride 2, 140 / 92 us; 256 <- 512, 1x1 stride 2,
   // 95 / 90; 17x27x27 96 <- 256, 5x5, 178 / 160; 5x82x107 16 <- 75 129 / 68.
   return true;
+}
+
+}  // namespace
+
+bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p,
+                              bool fused) {
+  return gather_f32_wanted(direction, p, fused, true);
 }
 
 bool conv2d_gather_tile_f32(int direction, const snn_hip_conv2d_params& p,
@@ -1812,6 +2009,7 @@ int launch_conv2d_gather_f32(int direction, const float* input,
   const size_t room =
       workspace != nullptr && aligned(workspace) ? workspace_elems * 4 : 0;
   if (plan->workspace_bytes(packs) > room) {
+    if (!gather_f32_wanted(direction, p, fuse, false)) return -1;
     const GatherPlan& whole = make_plan<float>(direction, p, false);
     const bool whole_temporary = whole.workspace_bytes(packs) > room;
     if (stream_captures(stream)) {
