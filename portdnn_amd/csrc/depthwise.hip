@@ -990,57 +990,74 @@ __global__ void __launch_bounds__(kDwFilbkThreads)
     if (part != nullptr) {
       part[static_cast<size_t>(blockIdx.x) * 9 * C + (comp >> 2) * C + ch] =
           sum;
-      // the kernel that adds the partial filters up expects dF zero-filled
-      if (blockIdx.x == 0) dw[(comp >> 2) * C + ch] = 0.f;
     } else {
       atomicAdd(dw + (comp >> 2) * C + ch, sum);
     }
   }
 }
 
-// dF += the work-groups' partial filters part[group][e], four elements per
-// lane.  blockIdx.y and the four waves of a work-group split the groups into
-// gridDim.y * 4 slices; the launcher sizes gridDim.y so that a lane has at most
-// kDwFilbkReduceLoads groups to add, and their loads are all issued before the
-// first addition.  The waves combine through LDS and one float atomic per
-// element and work-group goes to dF, which the strip kernel has zero-filled.
+// dF = the sum of the work-groups' partial filters part[group][e], rounded to
+// T.  A work-group of 16 waves owns 16 vectors of four elements (256 B of every
+// partial filter, which is what keeps its loads whole lines) and splits the
+// groups over its 64 slices; the four slices of a wave meet by lane exchange,
+// the waves in LDS, so dF needs neither atomics nor a fill before them nor, in
+// binary16, a rounding pass after them.
+// Bound by the latency of two or so rounds of loads: a lane issues its loads,
+// kDwFilbkReduceLoads at a time, before the first addition.
+// 14x14x512 at batch 128 in binary16: one launch of 4.0 us, where four waves
+// per work-group, atomics into an fp32 copy of dF and a rounding pass took
+// 3.6 + 2.1 us; without that pass and the second temporary the three directions
+// of the layer take 43.7 us instead of 59.4.
 constexpr int kDwFilbkReduceLoads = 8;
+constexpr int kDwFilbkReduceVecs = 16;
+constexpr int kDwFilbkReduceThreads = 1024;
 
-__global__ void __launch_bounds__(256)
+template <typename T>
+__global__ void __launch_bounds__(kDwFilbkReduceThreads)
     dw_filbk_reduce_kernel(const float4* __restrict__ part,
-                           float* __restrict__ dw, int n_vec, int n_groups) {
-  __shared__ float4 sums[4][64];
-  const int lane = threadIdx.x & 63, sub = threadIdx.x >> 6;
-  const int v = blockIdx.x * 64 + lane;
-  const int n_slices = gridDim.y * 4;
+                           T* __restrict__ dw, int n_vec, int n_groups) {
+  constexpr int kWaves = kDwFilbkReduceThreads / 64;
+  constexpr int kSlices = kDwFilbkReduceThreads / kDwFilbkReduceVecs;
+  __shared__ float4 sums[kWaves][kDwFilbkReduceVecs];
+  const int col = threadIdx.x % kDwFilbkReduceVecs;
+  const int slice = threadIdx.x / kDwFilbkReduceVecs;
+  const int v = blockIdx.x * kDwFilbkReduceVecs + col;
   float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
   if (v < n_vec) {
-    for (int g0 = blockIdx.y * 4 + sub; g0 < n_groups;
-         g0 += kDwFilbkReduceLoads * n_slices) {
+    for (int g0 = slice; g0 < n_groups; g0 += kDwFilbkReduceLoads * kSlices) {
       float4 x[kDwFilbkReduceLoads];
 #pragma unroll
       for (int k = 0; k < kDwFilbkReduceLoads; ++k) {
         // a group index past the end re-reads the last group and is not added
-        const int g = min(g0 + k * n_slices, n_groups - 1);
+        const int g = min(g0 + k * kSlices, n_groups - 1);
         x[k] = part[static_cast<size_t>(g) * n_vec + v];
       }
 #pragma unroll
       for (int k = 0; k < kDwFilbkReduceLoads; ++k) {
-        if (g0 + k * n_slices < n_groups)
+        if (g0 + k * kSlices < n_groups)
           a = make_float4(a.x + x[k].x, a.y + x[k].y, a.z + x[k].z,
                           a.w + x[k].w);
       }
     }
   }
-  sums[sub][lane] = a;
+#pragma unroll
+  for (int m = kDwFilbkReduceVecs; m < 64; m *= 2) {
+    a.x += __shfl_xor(a.x, m);
+    a.y += __shfl_xor(a.y, m);
+    a.z += __shfl_xor(a.z, m);
+    a.w += __shfl_xor(a.w, m);
+  }
+  if ((threadIdx.x & 63) < kDwFilbkReduceVecs) sums[threadIdx.x / 64][col] = a;
   __syncthreads();
-  if (sub == 0 && v < n_vec) {
-    const float4 s0 = sums[0][lane], s1 = sums[1][lane], s2 = sums[2][lane],
-                 s3 = sums[3][lane];
-    atomicAdd(dw + 4 * v + 0, (s0.x + s1.x) + (s2.x + s3.x));
-    atomicAdd(dw + 4 * v + 1, (s0.y + s1.y) + (s2.y + s3.y));
-    atomicAdd(dw + 4 * v + 2, (s0.z + s1.z) + (s2.z + s3.z));
-    atomicAdd(dw + 4 * v + 3, (s0.w + s1.w) + (s2.w + s3.w));
+  // one lane per element of the 16 vectors
+  const int e = blockIdx.x * kDwFilbkReduceVecs * 4 + threadIdx.x;
+  if (threadIdx.x < kDwFilbkReduceVecs * 4 && e < n_vec * 4) {
+    const float* s = reinterpret_cast<const float*>(&sums[0][0]);
+    float total = 0.f;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w)
+      total += s[w * kDwFilbkReduceVecs * 4 + threadIdx.x];
+    dw[e] = Elem<T>::from_float(total);
   }
 }
 
@@ -1367,13 +1384,15 @@ int dw_scratch_on_current_device(float** out) {
 
 // Picks the strip height (4 or 8 output rows, whichever wastes fewer rows of
 // the last row block; 8 on a tie) and deals the strips to the work-groups.
-// The work-groups add their sums into the zero-filled dF with float atomics
-// while those stay few; otherwise their partial filters go to `static_scratch`
-// when the caller brings it (kDwScratchElems floats), else to a stream-ordered
-// temporary, and a second kernel adds them up (also the fallback when the
-// allocation fails).
+// In fp32 the work-groups add their sums into the zero-filled dF with float
+// atomics while those stay few; otherwise, and always in binary16 (whose dF
+// takes no fp32 atomics), their partial filters go to `static_scratch` when the
+// caller brings it (kDwScratchElems floats), else to a stream-ordered
+// temporary, and a second kernel adds and rounds them.  Where that allocation
+// fails the atomics are the fallback, in binary16 into an fp32 temporary of the
+// filter's size that one more pass rounds.
 template <typename T>
-static int launch_dw_filbk_strip(const T* x, const T* dy, float* dw,
+static int launch_dw_filbk_strip(const T* x, const T* dy, T* dw,
                                  const snn_hip_depthwise_params& p, int cvw,
                                  int grid_y, hipStream_t stream,
                                  float* static_scratch) {
@@ -1405,7 +1424,8 @@ static int launch_dw_filbk_strip(const T* x, const T* dy, float* dw,
   const size_t part_elems = static_cast<size_t>(grid_x) * dw_elems;
   float* part = nullptr;
   bool temporary = false;
-  if (part_elems > kMaxAtomics) {
+  constexpr bool kFloat = std::is_same<T, float>::value;
+  if (!kFloat || part_elems > kMaxAtomics) {
     if (static_scratch != nullptr) {
       if (part_elems > kDwScratchElems)
         return report_error(
@@ -1424,15 +1444,23 @@ static int launch_dw_filbk_strip(const T* x, const T* dy, float* dw,
       part = nullptr;
     }
   }
+  float* acc = nullptr;  // where the atomics go
   if (part == nullptr) {
+    if constexpr (kFloat) {
+      acc = dw;
+    } else if (temp_malloc_async(reinterpret_cast<void**>(&acc),
+                                 dw_elems * sizeof(float),
+                                 stream) != hipSuccess) {
+      return SNN_HIP_ALLOCATION_PROBLEM;
+    }
     hipLaunchKernelGGL(dw_zero_kernel, dim3(ceil_div(dw_elems, 256)),
-                       dim3(256), 0, stream, dw, dw_elems);
+                       dim3(256), 0, stream, acc, dw_elems);
   }
   const dim3 grid(static_cast<unsigned>(grid_x),
                   static_cast<unsigned>(grid_y));
   auto launch = [&](auto kernel) {
     hipLaunchKernelGGL(kernel, grid, dim3(kDwFilbkThreads), 0, stream, x, dy,
-                       dw, part, p, cvw, spg, n_strips, n_rb, n_cb);
+                       acc, part, p, cvw, spg, n_strips, n_rb, n_cb);
   };
   // Loads two output rows ahead of the arithmetic at stride 1, one at stride 2
   // (measured at batch 32: 112x112x32 30.1 / 27.5 / 26.5 / 26.4 us for 0 / 1 /
@@ -1450,14 +1478,17 @@ static int launch_dw_filbk_strip(const T* x, const T* dy, float* dw,
   }
   if (part != nullptr) {
     const int n_vec = dw_elems / 4;
-    hipLaunchKernelGGL(
-        dw_filbk_reduce_kernel,
-        dim3(static_cast<unsigned>(ceil_div(n_vec, 64)),
-             static_cast<unsigned>(
-                 ceil_div(grid_x, 4 * kDwFilbkReduceLoads))),
-        dim3(256), 0, stream, reinterpret_cast<const float4*>(part), dw, n_vec,
-        grid_x);
+    hipLaunchKernelGGL(dw_filbk_reduce_kernel<T>,
+                       dim3(static_cast<unsigned>(
+                           ceil_div(n_vec, kDwFilbkReduceVecs))),
+                       dim3(kDwFilbkReduceThreads), 0, stream,
+                       reinterpret_cast<const float4*>(part), dw, n_vec,
+                       grid_x);
     if (temporary) temp_free_async(part, stream);
+  } else if constexpr (!kFloat) {
+    hipLaunchKernelGGL(dw_round_kernel<T>, dim3(ceil_div(dw_elems, 256)),
+                       dim3(256), 0, stream, acc, dw, dw_elems);
+    temp_free_async(acc, stream);
   }
   return SNN_HIP_OK;
 }
@@ -1560,8 +1591,7 @@ int launch_depthwise(int direction, const T* input, const T* filter, T* output,
     bool done = false;
     if constexpr (std::is_same<T, _Float16>::value) {
       // binary16, 3x3, stride 1 or 2: the fp32 strip kernel reading binary16,
-      // its sums in an fp32 temporary of the filter's size that one more pass
-      // rounds (the general kernel below took 1.07 ms where this takes about
+      // its sums in fp32 until the last of them (the general kernel below took 1.07 ms where this takes about
       // what fp32 does: 112x112x32 at batch 128)
       if (p.channel_multiplier == 1 && p.channels % 4 == 0 &&
           p.window_rows == 3 && p.window_cols == 3 &&
@@ -1575,21 +1605,10 @@ int launch_depthwise(int direction, const T* input, const T* filter, T* output,
         int cvw = 1;
         while (cvw * 2 <= cv && cvw < 32) cvw *= 2;  // >= 8 pixel lanes
         const int grid_y = ceil_div(cv, cvw);
-        const int dw_elems = 9 * p.channels;
-        void* acc = nullptr;
-        if (temp_malloc_async(&acc, dw_elems * sizeof(float), stream) !=
-            hipSuccess)
-          return SNN_HIP_ALLOCATION_PROBLEM;
         const int status = launch_dw_filbk_strip<T>(
-            input, filter, static_cast<float*>(acc), p, cvw, grid_y, stream,
-            nullptr);
-        if (status == SNN_HIP_OK)
-          hipLaunchKernelGGL(dw_round_kernel<T>, dim3(ceil_div(dw_elems, 256)),
-                             dim3(256), 0, stream,
-                             static_cast<const float*>(acc), output, dw_elems);
-        const hipError_t err = hipGetLastError();
-        temp_free_async(acc, stream);
+            input, filter, output, p, cvw, grid_y, stream, nullptr);
         if (status != SNN_HIP_OK) return status;
+        const hipError_t err = hipGetLastError();
         if (err != hipSuccess)
           return report_hip_error(err, "binary16 depthwise filter backprop");
         return SNN_HIP_OK;
