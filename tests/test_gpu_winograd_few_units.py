@@ -1,6 +1,7 @@
-"""fp32 Winograd launches of few units of work: plain ones run on the kernels
-behind the Tiled tag where those are faster, ones with a filter transformed ahead
-stay on the Winograd kernels (whole and split channel ranges)."""
+"""fp32 Winograd launches of few units of work, which run on the kernels behind the
+Tiled tag where those are faster, with the filter transformed ahead as well: an
+aligned launch may then have written over the transformed filter, and one on an
+unaligned filter, which stays on the Winograd kernels, must not read it there."""
 import numpy as np
 import pytest
 import torch
@@ -45,6 +46,13 @@ def test_winograd_few_units(shape, direction):
     for _ in range(2):
         got = ops.conv2d_prepared(da, db, p, direction, ALGO.WINOGRAD, ws)
         assert_close(got.cpu().numpy(), ref, (shape, direction, "prepared"))
+    ws.fill_(float("nan"))
+    ops.conv2d_prepare_filter(db, p, direction, ALGO.WINOGRAD, ws)
+    ops.conv2d_prepared(da, db, p, direction, ALGO.WINOGRAD, ws)
+    unaligned = torch.empty(n_b + 1, dtype=torch.float32, device="cuda")[1:]
+    unaligned.copy_(db)
+    got = ops.conv2d_prepared(da, unaligned, p, direction, ALGO.WINOGRAD, ws)
+    assert_close(got.cpu().numpy(), ref, (shape, direction, "unaligned"))
     same_bits = [ops.conv2d_deterministic(da, db, p, direction, ALGO.WINOGRAD,
                                           ws) for _ in range(2)]
     assert torch.equal(*same_bits)
