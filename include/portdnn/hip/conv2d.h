@@ -380,9 +380,9 @@ SNNStatus launch_forward_bias_activation(
 // launch in two calls for callers that run many launches with one filter.
 // prepare_filter writes what the selected algorithm derives from the filter
 // alone into the workspace (nothing, for most paths); launch_prepared is
-// launch<float, ConvType> trusting those contents.  The caller keeps the
-// workspace untouched in between and passes the same filter, parameters and
-// selector to both.
+// launch<float, ConvType> trusting those contents, which it only reads: several
+// streams may share them.  The caller keeps the workspace untouched in between
+// and passes the same filter, parameters and selector to both.
 template <typename T, typename ConvType, typename Backend>
 SNNStatus prepare_filter(
     typename Backend::template pointer_type<T const> filter,

@@ -278,8 +278,10 @@ SNN_HIP_API int snn_hip_conv2d_deterministic_f32(
  * recomputing them: the caller guarantees that `workspace` (same pointer,
  * same size) still holds what a prepare call with the same filter values,
  * parameters, direction and algorithm wrote, and that nothing else wrote to
- * its first 16 * C * K elements since.  The one-call entry points never
- * trust a workspace: they always transform the filter they are given. */
+ * its first 16 * C * K elements since.  Where something was prepared the
+ * launch only reads the workspace, whichever kernel it takes, so that launches
+ * on several streams may share one.  The one-call entry points never trust a
+ * workspace: they always transform the filter they are given. */
 SNN_HIP_API int snn_hip_conv2d_prepare_filter_f32(
     int direction, const float* filter, const snn_hip_conv2d_params* params,
     int algorithm, float* workspace, size_t workspace_elems, void* stream);

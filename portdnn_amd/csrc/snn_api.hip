@@ -1,7 +1,6 @@
 // The C ABI of libsnn_hip.so: parameter validation, algorithm support rules,
 // workspace sizing and dispatch to the kernel launchers.
 #include <atomic>
-#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -909,32 +908,47 @@ int launch_gemm_path<float>(int direction, const float* input,
   return launch_conv2d_direct<float>(direction, input, filter, output, p, s);
 }
 
-// Whether a Winograd launch of few units of work (32 tiles x 32 features) is
-// slower than the kernels behind the Tiled tag, which transform no filter first.
-// On 90 random layers of 1024 pixels and more, both directions: below 128 units
-// and with chunks of the channel range to split, Winograd zero-fills the output
-// and adds through atomics, 17 us and more against 9 us + 0.0225 us per million
-// multiply-adds (single image 56x56x128 -> 128: 25.8 / 16.5 us; of 30 such layers
-// two are slower here, 28.6 against 24.8 the most); with fewer than eight chunks
-// it takes 8 us + 1.15 per chunk (single image 56x56x64: 12.4, one launch of the
-// kernel for small layers 6.8; 38x28x64 -> 96 at batch 5: 12.5 / 14.5); a single
-// chunk of 16 channels runs on its slower kernel (42x32x16 -> 416 at batch 3: 12.3
-// / 9.8; 75x98x16 -> 416: 28 / 23).
-bool winograd_loses(int direction, const snn_hip_conv2d_params& p) {
+// Whether an aligned Winograd launch runs on the kernels behind the Tiled tag, which
+// transform no filter first, because those are the faster ones.  A launch whose
+// filter was transformed ahead (`prepared`) writes nothing to its workspace, which
+// launches on other streams may be reading, and gives the bits of the launch that
+// transforms it unless that one adds through atomics.  So, by 220 random layers
+// (us; in brackets the Winograd launch without its transform):
+//   * The kernel for small layers, which needs no workspace, takes all: 12.4 (9.2) /
+//     6.7 on a single 56x56x64 image, 20.3 (16.3) / 9.8 at 5x10x10 128 -> 320; with
+//     a second round of work-groups 12.7 (9.4) / 10.3.
+//   * A single chunk of 16 channels runs on Winograd's slower kernel; tiles of the
+//     gathering kernel that share no reduction take it: 9.2 (6.2) / 6.6 at 22x22x16
+//     -> 64, 55.6 (51.8) / 43.7 at 9x56x42, 16 -> 736.
+//   * Fewer than 128 units of work (32 tiles x 32 features) with at least eight
+//     chunks zero-fill the output and add through atomics: 18.8 (14.9) / 11.4 at
+//     3x17x22, 128 -> 96; 57.6 (47.6) / 39.2 at 2x14x14, 704 -> 576.  Of 80, two
+//     are slower here, by 3 %.  Prepared launches stay: the others' partial sums
+//     lie in the workspace.
+// (Two to seven chunks would gain 10 to 30 % on shared reductions, 12.4 / 8.8 at
+// 3x14x18, 64 -> 64, but in other bits than a prepared launch's.)
+bool winograd_loses(int direction, const snn_hip_conv2d_params& p,
+                    size_t workspace_elems, const LaunchOptions* epilogue) {
   const bool backprop = direction == SNN_HIP_INPUT_BACKPROP;
+  const bool gathers = conv2d_gather_f32_wanted(
+      direction, p,
+      !backprop && epilogue != nullptr && epilogue->wanted());
+  if (!backprop && !gathers && conv2d_small_supports(p)) return true;
+  // (the others may add through atomics)
+  if (epilogue != nullptr && epilogue->deterministic) return false;
+  const size_t scratch =
+      gathers ? conv2d_gather_f32_workspace_floats(direction, p) : 0;
   const int in_ch = backprop ? p.features : p.channels;
   const int out_ch = backprop ? p.channels : p.features;
-  const int rows = backprop ? p.in_rows : p.out_rows;
-  const int cols = backprop ? p.in_cols : p.out_cols;
-  const double tiles =
-      static_cast<double>(p.batch) * ceil_div(rows, 2) * ceil_div(cols, 2);
-  const double units = std::ceil(tiles / 32) * (out_ch / 32);
   const int chunks = in_ch / 16;
-  if (!backprop && conv2d_small_supports(p)) return true;
-  if (chunks == 1) return true;
-  if (units >= 128) return false;
-  const double macs_m = 9e-6 * p.batch * rows * cols * in_ch * out_ch;
-  return chunks >= 8 || 9 + 0.0225 * macs_m < 8 + 1.15 * chunks;
+  if (chunks == 1) return gathers && scratch == 0;
+  const size_t tiles =
+      static_cast<size_t>(p.batch) *
+      ceil_div(backprop ? p.in_rows : p.out_rows, 2) *
+      ceil_div(backprop ? p.in_cols : p.out_cols, 2);
+  const size_t units = ceil_div(tiles, size_t{32}) * (out_ch / 32);
+  return chunks >= 8 && units < 128 && scratch <= workspace_elems &&
+         (epilogue == nullptr || !epilogue->filter_prepared);
 }
 
 // Winograd / WinogradLarge: F(2x2,3x3) for forward and input backprop of 3x3
@@ -961,45 +975,26 @@ int launch_winograd_path<float>(int direction, const float* input,
                                 hipStream_t s, const LaunchOptions* epilogue) {
   // SNN_HIP_WINO_UNFUSED is a development switch that forces the three-stage
   // chain on shapes the fused kernel would take.
-  // A launch whose filter was transformed ahead takes the same kernel, and gives the
-  // same bits, as one that transforms it (the call that only transforms does so: it
-  // does not know the alignment of the others' operands).  Of 60 such layers, timed
-  // without the transform, 0.92 of the time; ten are slower, 25.7 against 31.9 us the
-  // most.  Not in place of a
-  // reproducible launch (the others add through atomics) unless on the kernel for
-  // small layers, nor where the other launch would take a temporary.
-  const bool computes = epilogue == nullptr || !epilogue->prepare_only;
-  const bool reproducible = epilogue != nullptr && epilogue->deterministic;
-  const bool fused_epilogue = direction == SNN_HIP_FORWARD &&
-                              epilogue != nullptr && epilogue->wanted();
-  LaunchOptions transforming;
-  if (computes && direction != SNN_HIP_FILTER_BACKPROP &&
-      conv2d_winograd_fused_supports(direction, p) && aligned16(workspace) &&
-      winograd_loses(direction, p) &&
-      (!reproducible ||
-       (direction == SNN_HIP_FORWARD && conv2d_small_supports(p) &&
-        !conv2d_gather_f32_wanted(direction, p, fused_epilogue))) &&
-      (!conv2d_gather_f32_wanted(direction, p, fused_epilogue) ||
-       conv2d_gather_f32_workspace_floats(direction, p) <= workspace_elems)) {
-    if (aligned16(input) && aligned16(filter) && aligned16(output))
-      return launch_gemm_path<float>(direction, input, filter, output, p, s,
-                                     workspace, workspace_elems, epilogue);
-    // An aligned launch may have put its packed filter where the transformed one
-    // was.
-    if (epilogue != nullptr && epilogue->filter_prepared) {
-      transforming = *epilogue;
-      transforming.filter_prepared = false;
-      epilogue = &transforming;
-    }
-  }
+  const bool fused = direction != SNN_HIP_FILTER_BACKPROP &&
+                     conv2d_winograd_fused_supports(direction, p);
+  const bool prepared = epilogue != nullptr && epilogue->filter_prepared;
+  if (fused && aligned16(input) && aligned16(filter) && aligned16(output) &&
+      aligned16(workspace) &&
+      winograd_loses(direction, p, workspace_elems, epilogue))
+    return launch_gemm_path<float>(direction, input, filter, output, p, s,
+                                   prepared ? nullptr : workspace,
+                                   prepared ? 0 : workspace_elems, epilogue);
   // (the input gradient's filter transform reads the filter 16 bytes at a time)
-  if (conv2d_winograd_fused_supports(direction, p) && aligned16(input) &&
-      aligned16(output) && aligned16(workspace) &&
+  if (fused && aligned16(input) && aligned16(output) && aligned16(workspace) &&
       (direction != SNN_HIP_INPUT_BACKPROP || aligned16(filter)) &&
       SNN_TUNING_ENV("SNN_HIP_WINO_UNFUSED") == nullptr)
     return launch_conv2d_winograd_fused_f32(direction, input, filter, output,
                                             p, workspace, workspace_elems, s,
                                             epilogue);
+  // (the kernels below would write over the transformed filter)
+  if (fused && prepared)
+    return launch_gemm_path<float>(direction, input, filter, output, p, s,
+                                   nullptr, 0, epilogue);
   if (conv2d_winograd_supports(direction, p))
     return launch_conv2d_winograd_f32(
         direction, input, filter, output, p, workspace, workspace_elems, s,

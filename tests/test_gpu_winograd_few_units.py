@@ -1,7 +1,6 @@
 """fp32 Winograd launches of few units of work, which run on the kernels behind the
-Tiled tag where those are faster, with the filter transformed ahead as well: an
-aligned launch may then have written over the transformed filter, and one on an
-unaligned filter, which stays on the Winograd kernels, must not read it there."""
+Tiled tag where those are faster, with the filter transformed ahead as well where
+nothing is written over the transformed filter."""
 import numpy as np
 import pytest
 import torch
@@ -63,3 +62,48 @@ def test_winograd_few_units(shape, direction):
         got = ops.conv2d_bias_act(da, db, dev(bias), p, ALGO.WINOGRAD,
                                   relu=True, workspace=ws)
         assert_close(got.cpu().numpy(), want, (shape, "bias"))
+
+
+@pytest.mark.parametrize("direction", [DIRECTION.FORWARD,
+                                       DIRECTION.INPUT_BACKPROP])
+@pytest.mark.parametrize("shape", SHAPES + [
+    (1, 56, 56, 96, 96, True),    # tiles that would share a reduction ...
+    (2, 14, 14, 160, 96, True),   # ... and a split channel range
+    (3, 14, 14, 64, 64, True),
+    (9, 20, 42, 16, 736, True),
+], ids=lambda s: "x".join(map(str, s)))
+def test_prepared_workspace_is_only_read(shape, direction):
+    """What a filter was transformed to survives every prepared launch, aligned or
+    not, so that launches on other streams can read it meanwhile; and a layer whose
+    channel range is not split gives the bits of the one-call launch."""
+    batch, rows, cols, channels, features, same = shape
+    p = ops.conv_params(batch, rows, cols, *(
+        (channels, features) if direction == DIRECTION.FORWARD else
+        (features, channels)), 3, 1, same)
+    rng = np.random.default_rng(8200 + rows)
+    n_a, n_b, n_out = ops.conv_sizes(p, direction)
+    a, b = uniform(rng, n_a), uniform(rng, n_b)
+    ref = np.asarray(ORACLE_FN[direction](
+        a, b, oracle_params(p, p.features), acc64=True)).reshape(-1)
+    da, db = dev(a), dev(b)
+
+    def moved(t):
+        u = torch.empty(t.numel() + 1, dtype=t.dtype, device="cuda")[1:]
+        u.copy_(t.reshape(-1))
+        return u
+
+    _, rec = ops.workspace_size(p, direction, ALGO.WINOGRAD)
+    ws = torch.full((rec,), 7.0, device="cuda")
+    ops.conv2d_prepare_filter(db, p, direction, ALGO.WINOGRAD, ws)
+    held = ws.clone()
+    out = torch.empty(n_out + 4, device="cuda")
+    for x, w, y in ((da, db, out[:n_out]), (moved(da), db, out[:n_out]),
+                    (da, moved(db), out[:n_out]), (da, db, out[1:n_out + 1])):
+        y.fill_(float("nan"))
+        ops.conv2d_prepared(x, w, p, direction, ALGO.WINOGRAD, ws, out=y)
+        assert_close(y.cpu().numpy(), ref, (shape, direction))
+        assert torch.equal(ws.view(torch.int32), held.view(torch.int32))
+    if channels < 128:
+        two = ops.conv2d_prepared(da, db, p, direction, ALGO.WINOGRAD, ws)
+        one = ops.conv2d(da, db, p, direction, ALGO.WINOGRAD, workspace=ws)
+        assert torch.equal(one.view(torch.int32), two.view(torch.int32))
