@@ -43,16 +43,22 @@
 //     products instead of sixteen: there the matrix units are the bound, and
 //     the tap arithmetic of every lane costs nothing beside them.
 //   * Larger fp32 tiles (SPLIT) take every operand apart into three bfloat16 parts
-//     in registers and sum six products of parts -- all but those below 2^-26 of
-//     the whole -- on the bfloat16 instruction, a sixteenth of the time each; the
-//     five small ones in accumulators of their own.  Against 64 bits the sums are
-//     closer than the fp32 instruction's, whose every second product is rounded
-//     (17x27x27 96 -> 256, 5x5: 2.3e-7 and 6.0e-7 in the 2-norm; 56x56x64 -> 256,
-//     1x1: 4e-8 and 1.0e-7).  149 -> 131 us on that layer, 28x28x128 at batch 128,
-//     3x3 (Tiled) 257 -> 200, 147x147x48 -> 64, 5x5, 122 -> 99: 0.15 PFLOP/s, where
-//     the matrix units are busy 0.4 of the time and the splitting takes as many
-//     cycles of the vector units.  A conversion ahead, into three planes, would
-//     move half as many bytes again.
+//     in registers and sum six of the nine products of parts on the bfloat16
+//     instruction, a sixteenth of the time each; the five small ones in
+//     accumulators of their own.  What is left out (the second and third parts'
+//     products, and that of the third ones) is below 2^-23 of a product, 2^-26 in
+//     the root mean square and without a bias; an fp32 sum rounds by as much at
+//     every second product.  Against 64 bits the results are closer than the fp32
+//     instruction's: on 70 random layers of 36 to 8640 products, with activations of
+//     either sign, of one sign and half of them zero, 0.71 of its error in the
+//     2-norm and 0.93 in the worst value at the most (17x27x27 96 -> 256, 5x5:
+//     2.3e-7 and 6.0e-7).  Two more products take 13 us of 120 and change neither.
+//     With the fp32 instruction / here: that layer 144 / 120 us, 28x28x128 at batch
+//     128, 3x3, 259 / 215, 147x147x48 -> 64 at batch 8, 5x5, 218 / 208, 56x56x128,
+//     3x3 stride 2, at batch 32 80 / 71: 0.15 PFLOP/s, where the matrix units are
+//     busy 0.4 of the time and the splitting takes as many cycles of the vector
+//     units.  A conversion ahead, into three planes, would move half as many bytes
+//     again.
 //   * A strided gradient of few channels (a three-channel first layer) would
 //     fill 3 of the 32 matrix rows.  Its classes are merged: the pixels of a
 //     block of stride x stride share one window of ceil(window / stride) source
@@ -343,10 +349,17 @@ __global__ void __launch_bounds__(256)
   *reinterpret_cast<decltype(v)*>(wide + static_cast<size_t>(idx) * kE) = v;
 }
 
-// An fp32 value as the sum of three bfloat16 ones, the first rounded to nearest
-// (its remainder then has no bias, nor have the products left out), the others
-// cut off: every remainder is exact, and the last one fits.  (Integer operations:
-// the conversion instruction takes as long as four of them.)
+// An fp32 value times 2^24 as the sum of three bfloat16 ones, the first rounded to
+// nearest (its remainder then has no bias, nor have the products left out), the
+// others cut off: every remainder is exact, and the last one fits.  (Integer
+// operations: the conversion instruction takes as long as four of them.)
+// The matrix units take operands and sums below 2^-126 for zero.  No part of an
+// fp32 value lies below 2^-149, so none of a value times 2^24 is lost, nor is any
+// product of parts times 2^48 that an fp32 sum could hold; what grows beyond the
+// range by it gives an infinity or a NaN, and such a tile is taken again without
+// splitting.  (One instruction per value: 17x27x27 96 -> 256, 5x5, 114.5 -> 119.5
+// us; looking for the smallest value on the way takes 125.)
+constexpr float kSplitScale = 0x1p24f, kSplitUnscale = 0x1p-48f;
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 struct Parts {
   bf16x8 first, second, third;
@@ -360,7 +373,7 @@ __device__ __forceinline__ Parts split_parts(const float4v& e,
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int at = 2 * k + h;
-      const float v = at < 4 ? e[at & 3] : o[at & 3];
+      const float v = (at < 4 ? e[at & 3] : o[at & 3]) * kSplitScale;
       f[h] = (__builtin_bit_cast(unsigned, v) + 0x8000u) & 0xFFFF0000u;
       const float rest = v - __builtin_bit_cast(float, f[h]);
       s[h] = __builtin_bit_cast(unsigned, rest);
@@ -377,15 +390,6 @@ __device__ __forceinline__ Parts split_parts(const float4v& e,
 }
 __device__ __forceinline__ Parts split_parts(const half8&, const half8&) {
   return {};
-}
-// Whether a sum over split operands has to be taken again without splitting: the
-// parts of an infinity are no numbers and rounding the first part up may overflow,
-// and the matrix units take parts below 2^-126 for zero, which a sum of magnitude
-// 2^-103 and more does not notice.
-__device__ __forceinline__ bool beyond_split(float v) {
-  constexpr unsigned kLeast = 24u << 23, kInfinity = 0x7F800000u;
-  const unsigned u = __builtin_bit_cast(unsigned, v) & 0x7FFFFFFFu;
-  return u != 0u && u - kLeast >= kInfinity - kLeast;
 }
 
 // WM x WN waves of TM x TN blocks of 32 pixels x 32 features.  UNIFORM: whole
@@ -504,15 +508,21 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
 
   const int cp = g.cp, src_cols = g.src_cols, win_c = cls.win_c;
   const Divisor by_cp = g.by_cp, by_win_c = cls.by_win_c;
-  int tap_r = 0, tap_c = 0, c4 = 0;  // UNIFORM: of the next chunk to load
-  int q = chunk0 * 4 + piece;        // otherwise: the lane's next piece
-  if (UNIFORM && chunk0 > 0) {
-    const int tap = chunk0 * 4 / cp;
-    c4 = chunk0 * 4 - tap * cp;
-    tap_r = tap / win_c;
-    tap_c = tap - tap_r * win_c;
-  }
-  unsigned b_chunk = FROM == kPacked ? chunk0 * 2048u : 0u;
+  int tap_r, tap_c, c4;  // UNIFORM: of the next chunk to load
+  int q;                 // otherwise: the lane's next piece
+  unsigned b_chunk;
+  auto rewind = [&]() {  // to the first chunk
+    tap_r = tap_c = c4 = 0;
+    q = chunk0 * 4 + piece;
+    if (UNIFORM && chunk0 > 0) {
+      const int tap = chunk0 * 4 / cp;
+      c4 = chunk0 * 4 - tap * cp;
+      tap_r = tap / win_c;
+      tap_c = tap - tap_r * win_c;
+    }
+    b_chunk = FROM == kPacked ? chunk0 * 2048u : 0u;
+  };
+  rewind();
   const unsigned b_step = FROM == kRows ? g.features * 64u : 2048u;
   // IN_PLACE: bytes from a tap to the next column's, the next row's
   const int filter_row = cp * 16, filter_tap = g.features * filter_row;
@@ -690,6 +700,35 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
     multiply_split(even, odd);
     ++done;
   };
+  auto multiply_all = [&]() {
+    if (n_chunks <= 0) return;
+    issue(buf0);
+    if (n_chunks > 1) issue(buf1);
+    if (n_chunks > 2) issue(buf2);
+    // (all three: a wait for the first alone makes the compiler put a full
+    // wait into every turn of the loop)
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    fetch(buf0, 0, even);
+    while (done + 5 < n_chunks) {
+      step(buf0, buf1, true, true, true);
+      step(buf1, buf2, true, true, true);
+      step(buf2, buf0, true, true, true);
+    }
+    // at most five chunks are left
+    auto last = [&](char* cur, const char* next) {
+      if (done < n_chunks)
+        step(cur, next, done + 1 < n_chunks, done + 2 < n_chunks,
+             done + 3 < n_chunks);
+    };
+    last(buf0, buf1);
+    last(buf1, buf2);
+    last(buf2, buf0);
+    last(buf0, buf1);
+    last(buf1, buf2);
+  };
   if constexpr (SPLIT) {
 #pragma unroll
     for (int i = 0; i < TN; ++i)
@@ -721,39 +760,41 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
       last(buf0);
       last(buf1);
     }
+    // A tile with sums that are no numbers (the parts of an infinity are none) is
+    // taken again without splitting, by the whole work-group.
+    bool again = false;
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
       for (int j = 0; j < TM; ++j)
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] += low[i][j][v];
-  } else if (n_chunks > 0) {
-    issue(buf0);
-    if (n_chunks > 1) issue(buf1);
-    if (n_chunks > 2) issue(buf2);
-    // (all three: a wait for the first alone makes the compiler put a full
-    // wait into every turn of the loop)
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_barrier();
-    __builtin_amdgcn_sched_barrier(0);
-    fetch(buf0, 0, even);
-    while (done + 5 < n_chunks) {
-      step(buf0, buf1, true, true, true);
-      step(buf1, buf2, true, true, true);
-      step(buf2, buf0, true, true, true);
+        for (int v = 0; v < 16; ++v) {
+          const float sum = (acc[i][j][v] + low[i][j][v]) * kSplitUnscale;
+          acc[i][j][v] = sum;
+          again |= !(__builtin_fabsf(sum) < __builtin_inff());
+        }
+    __syncthreads();  // every wave is done with the last chunk
+    int* const agains = reinterpret_cast<int*>(buf0);
+    again = __builtin_amdgcn_ballot_w64(again) != 0;
+    if (lane == 0) agains[wave] = again ? 1 : 0;
+    __syncthreads();
+    int any = 0;
+#pragma unroll
+    for (int k = 0; k < NW; ++k) any |= agains[k];
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(any) != 0) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+      rewind();
+      done = 0;
+      multiply_all();
     }
-    // at most five chunks are left
-    auto last = [&](char* cur, const char* next) {
-      if (done < n_chunks)
-        step(cur, next, done + 1 < n_chunks, done + 2 < n_chunks,
-             done + 3 < n_chunks);
-    };
-    last(buf0, buf1);
-    last(buf1, buf2);
-    last(buf2, buf0);
-    last(buf0, buf1);
-    last(buf1, buf2);
+  } else {
+    multiply_all();
   }
 
   // A shared reduction: the fp32 tile in accumulator order, 1 KB per store.
@@ -784,22 +825,17 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
   {
     // (a maximum that keeps NaNs: two values per instruction)
     float most = 0.f;
-    bool odd = false;
 #pragma unroll
     for (int j = 0; j < TM; ++j)
 #pragma unroll
       for (int i = 0; i < TN; ++i) {
         float block = 0.f;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) {
-          if constexpr (SPLIT)
-            odd |= beyond_split(acc[i][j][v]);
-          else
-            block = __builtin_elementwise_maximum(block, acc[i][j][v]);
-        }
+        for (int v = 0; v < 16; ++v)
+          block = __builtin_elementwise_maximum(block, acc[i][j][v]);
         most = __builtin_elementwise_maximum(most, block);
       }
-    if (__builtin_amdgcn_ballot_w64(SPLIT ? odd : most != most) != 0) {
+    if (__builtin_amdgcn_ballot_w64(most != most) != 0) {
 #pragma unroll
       for (int j = 0; j < TM; ++j) {
         const int m = m0 + (wm * TM + j) * 32 + l32;
@@ -810,10 +846,8 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
           unsigned bits = 0;
 #pragma unroll
           for (int v = 0; v < 16; ++v)
-            bits |= (SPLIT ? beyond_split(acc[i][j][v])
-                           : acc[i][j][v] != acc[i][j][v]) ? 1u << v : 0u;
-          strange[j * TN + i] =
-              SPLIT ? (m < cls.pixels ? bits : 0u) : cut ? bits : 0u;
+            bits |= acc[i][j][v] != acc[i][j][v] ? 1u << v : 0u;
+          strange[j * TN + i] = cut ? bits : 0u;
         }
       }
     }
@@ -1028,7 +1062,7 @@ __global__ void __launch_bounds__(64 * WM * WN, TM * TN >= 4 ? 2 : 3)
 
 // Sums the splits of every tile in order and rounds: one float4 -- four
 // consecutive features of a pixel -- per lane.
-template <typename T, int WM, int WN, int TM, int TN, bool SPLIT>
+template <typename T, int WM, int WN, int TM, int TN>
 __global__ void __launch_bounds__(256)
     gather_reduce_kernel(const float4v* __restrict__ part,
                          const T* __restrict__ src, const T* __restrict__ w,
@@ -1058,12 +1092,11 @@ __global__ void __launch_bounds__(256)
   for (int s = 0; s < g.n_splits; ++s)
     sum += from[static_cast<size_t>(s) * g.n_tiles * kTileVecs];
   const Pixel px = pixel_of(m, cls);
-  auto strange = [](float v) { return SPLIT ? beyond_split(v) : v != v; };
-  if ((strange(sum[0]) || strange(sum[1]) || strange(sum[2]) ||
-       strange(sum[3])) && (SPLIT || window_cut(g, cls, px))) {
+  if ((sum[0] != sum[0] || sum[1] != sum[1] || sum[2] != sum[2] ||
+       sum[3] != sum[3]) && window_cut(g, cls, px)) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-      if (strange(sum[e]) && f + e < g.features)
+      if (sum[e] != sum[e] && f + e < g.features)
         sum[e] = exact_sum(src, w, g, cls, px, f + e);
   }
   if constexpr (sizeof(T) == 4) {
@@ -1139,8 +1172,8 @@ constexpr TileShape kTilesF16[] = {
 // and on power more than on how the tiles fall on compute units.
 constexpr TileShape kTilesF32[] = {{128, 32, 0.36, 0.27, false},
                                    {64, 64, 0.36, 0.265, false},
-                                   {128, 128, 0.10, 0.88, true},
-                                   {128, 64, 0.27, 0.45, true}};
+                                   {128, 128, 0.10, 0.92, true},
+                                   {128, 64, 0.27, 0.47, true}};
 constexpr int kMergedTile = 0;
 template <typename T>
 struct Tiles;
@@ -1469,7 +1502,7 @@ void launch_tile(const GatherOperands<T>& ops, const GatherPlan& plan,
       launch_kernel<T, WM, WN, TM, TN, false, kPacked, SPLIT>(ops, plan, g, stream);
   }
   if (g.n_splits > 1)
-    hipLaunchKernelGGL((gather_reduce_kernel<T, WM, WN, TM, TN, SPLIT>),
+    hipLaunchKernelGGL((gather_reduce_kernel<T, WM, WN, TM, TN>),
                        dim3(g.n_tiles * (BM * BN / 1024)), dim3(256), 0, stream,
                        reinterpret_cast<const float4v*>(ops.part), ops.src,
                        ops.caller_filter, ops.bias, ops.dst, g);

@@ -3,8 +3,9 @@ into bfloat16 parts: filters in place and packed, whole and broken chunks per ta
 ragged tiles, stride classes, shared reductions, bias and activation, infinities,
 the largest and very small values.
 
-Bound: n products added in fp32 as in the other fp32 convolutions; the products
-left out are below 2^-26 of a product each, a quarter of one rounding.
+Bound: n products added in fp32 as in the other fp32 convolutions; the products of
+parts left out are below 2^-23 of a product, two roundings (2^-26 in the root mean
+square).
 """
 import numpy as np
 import pytest
@@ -109,3 +110,31 @@ def test_split_operands_of_any_size(shape, direction, tile, operand):
         assert part.any()
         error = np.abs(got[part].astype(np.float64) - ref[part])
         assert error.max() <= 2 * n * 2.0**-24 * np.abs(ref[part]).max()
+
+
+@pytest.mark.parametrize("shape,direction,tile", [CASES[0], CASES[1], CASES[5],
+                                                  CASES[8]],
+                         ids=[IDS[i] for i in (0, 1, 5, 8)])
+@pytest.mark.parametrize("small,large", [(-110, 10), (-115, 15), (-120, 20),
+                                         (-130, 100), (-50, -60)])
+@pytest.mark.parametrize("operand", [0, 1])
+def test_split_operands_small_beside_large(shape, direction, tile, small, large,
+                                           operand):
+    """Operands whose later parts the matrix units would take for zero, with
+    partners that make ordinary sums of them, and operands whose products come near
+    the least: what the parts cannot hold is not missing from the sum.
+
+    Bound: every addition rounds half a unit of a partial sum, which grows with the
+    square root of its length."""
+    p, a, b, _ = operands(shape, direction, 3600)
+    both = []
+    for k, v in enumerate((a, b)):
+        v = np.where(v < 0, -1, 1) * (1 + np.abs(v) * np.float32(0.999))
+        both.append(np.ldexp(v, small if k == operand else large)
+                    .astype(np.float32))
+    a, b = both
+    ref = reference(p, direction, a, b).astype(np.float64)
+    got = ops.conv2d(dev(a), dev(b), p, direction,
+                     ALGO.IM2COL).cpu().numpy().reshape(-1).astype(np.float64)
+    error = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert error <= np.sqrt(products(p, direction)) * 2.0**-24
