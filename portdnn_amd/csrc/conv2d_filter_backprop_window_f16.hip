@@ -49,11 +49,11 @@
 //     60 us), so the partial tiles are stored, and a second kernel sums them
 //     and rounds to binary16.
 #include <algorithm>
-#include <array>
 #include <cmath>
 #include <cstring>
 
 #include "gemm_tile.h"
+#include "plan_cache.h"
 #include "snn_kernels.h"
 
 namespace snn {
@@ -823,25 +823,9 @@ WindowPlan wanted_plan(const snn_hip_conv2d_params& p) {
   return plan;
 }
 
-// The plans of a network's layers are kept per thread.
 const WindowPlan& make_plan(const snn_hip_conv2d_params& p) {
-  struct Entry {
-    bool used = false;
-    snn_hip_conv2d_params params;
-    WindowPlan plan;
-  };
-  constexpr size_t kEntries = 64;
-  thread_local std::array<Entry, kEntries> cache;
-  const unsigned hash = (((p.channels * 31u + p.features) * 31u + p.in_rows) *
-                             31u + p.in_cols) * 31u + p.batch * 7u +
-                        p.window_rows + p.stride_rows * 5u;
-  Entry& entry = cache[hash % kEntries];
-  if (!entry.used || std::memcmp(&entry.params, &p, sizeof p) != 0) {
-    entry.plan = wanted_plan(p);
-    entry.params = p;
-    entry.used = true;
-  }
-  return entry.plan;
+  thread_local PlanCache<WindowPlan> cache;
+  return cache.get(p, 0, [&] { return wanted_plan(p); });
 }
 
 template <typename ROWS>

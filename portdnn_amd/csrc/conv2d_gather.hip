@@ -68,10 +68,10 @@
 #include <climits>
 #include <cmath>
 #include <cstdlib>
-#include <cstring>
 #include <type_traits>
 
 #include "gemm_tile.h"
+#include "plan_cache.h"
 #include "snn_kernels.h"
 
 namespace snn {
@@ -1408,25 +1408,12 @@ GatherPlan compute_plan(int direction, const snn_hip_conv2d_params& p,
   return plan;
 }
 
-// The plan of the most recent shape is kept per thread: layers are usually
-// launched many times with the same parameters.
 template <typename T>
 const GatherPlan& make_plan(int direction, const snn_hip_conv2d_params& p,
                             bool may_split = true) {
-  struct Cached {
-    int direction = -1;
-    snn_hip_conv2d_params params;
-    GatherPlan plan;
-  };
-  thread_local Cached cached[2][2];
-  Cached& c = cached[may_split][direction == SNN_HIP_INPUT_BACKPROP];
-  if (c.direction != direction ||
-      std::memcmp(&c.params, &p, sizeof(p)) != 0) {
-    c.plan = compute_plan<T>(direction, p, may_split);
-    c.params = p;
-    c.direction = direction;
-  }
-  return c.plan;
+  thread_local PlanCache<GatherPlan> cache;
+  return cache.get(p, static_cast<unsigned>(direction) * 2 + may_split,
+                   [&] { return compute_plan<T>(direction, p, may_split); });
 }
 
 // A launch's operands: the source as whole pieces, the filter as `from` says.

@@ -31,10 +31,10 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
-#include <cstring>
 #include <numeric>
 
 #include "gemm_tile.h"
+#include "plan_cache.h"
 #include "snn_kernels.h"
 
 namespace snn {
@@ -418,16 +418,9 @@ SplitPlan compute_plan(const snn_hip_conv2d_params& p) {
   return best;
 }
 
-SplitPlan make_plan(const snn_hip_conv2d_params& p) {
-  thread_local snn_hip_conv2d_params cached_params;
-  thread_local SplitPlan cached_plan;
-  thread_local bool cached = false;
-  if (!cached || std::memcmp(&cached_params, &p, sizeof(p)) != 0) {
-    cached_plan = compute_plan(p);
-    cached_params = p;
-    cached = true;
-  }
-  return cached_plan;
+const SplitPlan& make_plan(const snn_hip_conv2d_params& p) {
+  thread_local PlanCache<SplitPlan> cache;
+  return cache.get(p, 0, [&] { return compute_plan(p); });
 }
 
 template <int FA, int PB, bool TRANSPOSED>
@@ -478,7 +471,7 @@ bool conv2d_rowsplit_supports(const snn_hip_conv2d_params& p) {
     if (p.channels < min_channels) return false;
   }
   if (std::max(std::max(x, y), w) * 4 > kMaxBufferBytes) return false;
-  const SplitPlan plan = make_plan(p);
+  const SplitPlan& plan = make_plan(p);
   if (plan.lds_bytes == 0) return false;
   // most compute units busy, most block slots real output
   const double blocks = static_cast<double>(plan.g.total_pixels) / 16.0 *
@@ -491,7 +484,7 @@ int launch_conv2d_rowsplit_f32(const float* input, const float* filter,
                                float* output, const snn_hip_conv2d_params& p,
                                hipStream_t stream, bool transposed_filter,
                                const LaunchOptions* epilogue) {
-  const SplitPlan plan = make_plan(p);
+  const SplitPlan& plan = make_plan(p);
   if (plan.lds_bytes == 0) return SNN_HIP_INVALID_ALGORITHM;
   static const bool print_plan =
       SNN_TUNING_ENV("SNN_HIP_ROWTILE_PLAN") != nullptr;

@@ -41,10 +41,10 @@
 #include <algorithm>
 #include <cstdio>
 #include <cstdlib>
-#include <cstring>
 #include <numeric>
 
 #include "gemm_tile.h"
+#include "plan_cache.h"
 #include "snn_kernels.h"
 
 namespace snn {
@@ -534,18 +534,9 @@ RowTilePlan compute_plan(const snn_hip_conv2d_params& p) {
   return best;
 }
 
-// The plan of the most recent shape is kept per thread: layers are usually
-// launched many times with the same parameters.
-RowTilePlan make_plan(const snn_hip_conv2d_params& p) {
-  thread_local snn_hip_conv2d_params cached_params;
-  thread_local RowTilePlan cached_plan;
-  thread_local bool cached = false;
-  if (!cached || std::memcmp(&cached_params, &p, sizeof(p)) != 0) {
-    cached_plan = compute_plan(p);
-    cached_params = p;
-    cached = true;
-  }
-  return cached_plan;
+const RowTilePlan& make_plan(const snn_hip_conv2d_params& p) {
+  thread_local PlanCache<RowTilePlan> cache;
+  return cache.get(p, 0, [&] { return compute_plan(p); });
 }
 
 template <int PB, bool MULTI, bool WIN3, bool TRANSPOSED>
@@ -630,7 +621,7 @@ bool conv2d_rowtile_supports(const snn_hip_conv2d_params& p) {
   // 1x1 windows have no taps to reuse an LDS tile over
   if (p.window_rows * p.window_cols == 1) return false;
   if (std::max(std::max(x, y), w) * 4 > kMaxBufferBytes) return false;
-  const RowTilePlan plan = make_plan(p);
+  const RowTilePlan& plan = make_plan(p);
   if (plan.lds_bytes == 0) return false;
   // Worth it when most compute units get a work-group and most of the wave
   // tiles' 16 x 16 blocks are real output: the share of block slots (rounds x
@@ -645,7 +636,7 @@ int launch_conv2d_rowtile_f32(const float* input, const float* filter,
                               float* output, const snn_hip_conv2d_params& p,
                               hipStream_t stream, bool transposed_filter,
                               const LaunchOptions* epilogue) {
-  const RowTilePlan plan = make_plan(p);
+  const RowTilePlan& plan = make_plan(p);
   if (plan.lds_bytes == 0) return SNN_HIP_INVALID_ALGORITHM;
   static const bool print_plan = SNN_TUNING_ENV("SNN_HIP_ROWTILE_PLAN") != nullptr;
   if (print_plan)

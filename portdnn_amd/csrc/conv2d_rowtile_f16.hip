@@ -37,10 +37,10 @@
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
-#include <cstring>
 #include <numeric>
 
 #include "gemm_tile.h"
+#include "plan_cache.h"
 #include "snn_kernels.h"
 
 namespace snn {
@@ -687,25 +687,9 @@ bool takes(const snn_hip_conv2d_params& p) {
          (x > y ? x : y) * 2 <= kMaxBufferBytes;
 }
 
-// The plans of a network's layers are kept per thread.
 const RowTilePlan& make_plan(const snn_hip_conv2d_params& p) {
-  struct Entry {
-    bool used = false;
-    snn_hip_conv2d_params params;
-    RowTilePlan plan;
-  };
-  constexpr size_t kEntries = 64;
-  thread_local std::array<Entry, kEntries> cache;
-  const unsigned hash = (((p.channels * 31u + p.features) * 31u + p.in_rows) *
-                             31u + p.in_cols) * 31u + p.batch * 7u +
-                        p.window_rows + p.pad_rows * 5u;
-  Entry& entry = cache[hash % kEntries];
-  if (!entry.used || std::memcmp(&entry.params, &p, sizeof p) != 0) {
-    entry.plan = takes(p) ? compute_plan(p) : RowTilePlan();
-    entry.params = p;
-    entry.used = true;
-  }
-  return entry.plan;
+  thread_local PlanCache<RowTilePlan> cache;
+  return cache.get(p, 0, [&] { return takes(p) ? compute_plan(p) : RowTilePlan(); });
 }
 
 template <int WF, int WP, int PB, int KC, int BUFS, bool WIN3>

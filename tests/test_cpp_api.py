@@ -28,6 +28,15 @@ def test_host_api_program():
     assert "0 failures" in out.stdout
 
 
+def test_plan_cache_program():
+    """The launch plans of a network's layers stay kept, whatever powers of two
+    their sizes are multiples of."""
+    out = subprocess.run([_exe("plan_cache_test")], stdout=subprocess.PIPE,
+                         stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert out.returncode == 0, out.stdout
+    assert "0 failures" in out.stdout
+
+
 @pytest.mark.gpu
 def test_gpu_api_program():
     """conv2d (every selector, three directions), depthwise, pooling and event
