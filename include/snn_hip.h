@@ -170,6 +170,13 @@ SNN_HIP_API int snn_hip_conv2d_gather_tile(const snn_hip_conv2d_params* params,
                                            int direction, int dtype,
                                            int* pixels, int* features,
                                            int* splits);
+/* The same for the binary16 kernels that keep pixels in LDS: `form` is, for a
+ * forward convolution or input gradient, how a work-group of the row-tile kernel
+ * holds its input (1: one tile of all channels, 2: two tiles in turn, 3: one tile
+ * that is loaded again), and for a filter gradient the work-groups that share a
+ * tile of the kernel for 3x3 and 5x5 windows. */
+SNN_HIP_API int snn_hip_conv2d_lds_form_f16(const snn_hip_conv2d_params* params,
+                                            int direction, int* form);
 
 /* Diagnostics for the stream-ordered temporaries some launches take when the
  * caller passes no workspace (no counterpart in portDNN, whose temporaries

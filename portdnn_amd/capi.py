@@ -122,6 +122,7 @@ SIGNATURES = {
                                    ctypes.POINTER(ctypes.c_int)],
     "snn_hip_conv2d_gather_tile": [_P, _I, _I, ctypes.POINTER(_I),
                                    ctypes.POINTER(_I), ctypes.POINTER(_I)],
+    "snn_hip_conv2d_lds_form_f16": [_P, _I, ctypes.POINTER(_I)],
     "snn_hip_conv2d_forward_f32": [_P, _P, _P, _P, _I, _P, _SZ, _P],
     "snn_hip_conv2d_input_backprop_f32": [_P, _P, _P, _P, _I, _P, _SZ, _P],
     "snn_hip_conv2d_filter_backprop_f32": [_P, _P, _P, _P, _I, _P, _SZ, _P],

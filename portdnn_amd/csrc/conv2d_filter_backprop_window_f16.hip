@@ -857,6 +857,11 @@ bool conv2d_filter_backprop_window_f16_supports(
   return make_plan(p).shape != kNone;
 }
 
+int conv2d_filter_backprop_window_f16_splits(const snn_hip_conv2d_params& p) {
+  const WindowPlan& plan = make_plan(p);
+  return plan.shape != kNone ? plan.g.n_splits : 0;
+}
+
 size_t conv2d_filter_backprop_window_f16_partial_floats(
     const snn_hip_conv2d_params& p) {
   const WindowPlan& plan = make_plan(p);

@@ -1751,6 +1751,13 @@ bool conv2d_gather_tile_f16(int direction, const snn_hip_conv2d_params& p,
   return !is_short_gemm(direction, p) && gather_tile_f16(direction, p, tile);
 }
 
+int conv2d_rowtile_form_f16(int direction, const snn_hip_conv2d_params& p) {
+  snn_hip_conv2d_params q;
+  return !is_short_gemm(direction, p) && !is_rows_gemm(direction, p) &&
+                 rowtile_params(direction, p, &q)
+             ? conv2d_rowtile_f16_buffers(q) : 0;
+}
+
 size_t conv2d_f16_workspace_halves(int direction,
                                    const snn_hip_conv2d_params& p) {
   snn_hip_conv2d_params q;

@@ -759,6 +759,11 @@ bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p,
          (plan.pb == 4 || 2 * plan.lds_bytes <= kMaxLdsBytes);
 }
 
+int conv2d_rowtile_f16_buffers(const snn_hip_conv2d_params& p) {
+  const RowTilePlan& plan = make_plan(p);
+  return plan.lds_bytes != 0 ? plan.bufs : 0;
+}
+
 int launch_conv2d_rowtile_f16(const _Float16* input, const _Float16* filter,
                               _Float16* output, const snn_hip_conv2d_params& p,
                               _Float16* packed, hipStream_t stream,

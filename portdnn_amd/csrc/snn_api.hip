@@ -1460,6 +1460,30 @@ int snn_hip_conv2d_gather_tile(const snn_hip_conv2d_params* params,
   return SNN_HIP_OK;
 }
 
+int snn_hip_conv2d_lds_form_f16(const snn_hip_conv2d_params* params,
+                                int direction, int* form) {
+  if (params == nullptr || form == nullptr ||
+      (direction != SNN_HIP_FORWARD && direction != SNN_HIP_INPUT_BACKPROP &&
+       direction != SNN_HIP_FILTER_BACKPROP))
+    return SNN_HIP_INVALID_PARAMETER;
+  const snn_hip_conv2d_params& p = *params;
+  const int v = validate(p);
+  if (v != SNN_HIP_OK) return v;
+  int taken = 0;
+  if (p.input_format == 0 && p.groups == 1) {
+    if (direction == SNN_HIP_FILTER_BACKPROP)
+      // (fewer channels may run in fp32)
+      taken = p.channels > 8 ? conv2d_filter_backprop_window_f16_splits(p) : 0;
+    else if (!(direction == SNN_HIP_FORWARD
+                   ? conv2d_few_f16_forward_supports(p)
+                   : conv2d_few_f16_input_backprop_supports(p)))
+      taken = conv2d_rowtile_form_f16(direction, p);
+  }
+  if (taken == 0) return SNN_HIP_INVALID_ALGORITHM;
+  *form = taken;
+  return SNN_HIP_OK;
+}
+
 int snn_hip_depthwise_conv2d_forward_f32(
     const float* input, const float* filter, float* output,
     const snn_hip_depthwise_params* params, void* stream) {

@@ -260,6 +260,9 @@ bool conv2d_gather_tile_f16(int direction, const snn_hip_conv2d_params& p,
                             GatherTile* tile);
 bool conv2d_gather_tile_f32(int direction, const snn_hip_conv2d_params& p,
                             GatherTile* tile);
+// conv2d_rowtile_f16_buffers of an aligned binary16 launch, 0 where it runs on
+// another kernel.
+int conv2d_rowtile_form_f16(int direction, const snn_hip_conv2d_params& p);
 // The general implicit-GEMM kernel on binary16 tensors (conv2d_igemm.hip): no
 // temporary.  Features (and forward channels) in multiples of 4; source and
 // filter, and a forward output, 16-byte aligned.
@@ -313,6 +316,8 @@ int launch_conv2d_few_f16_filter_backprop(const _Float16* x,
 // aligned; `part` is scratch of ..._partial_floats(p) floats for the partial
 // tiles.
 bool conv2d_filter_backprop_window_f16_supports(const snn_hip_conv2d_params& p);
+// ... and the work-groups that share a tile, or 0
+int conv2d_filter_backprop_window_f16_splits(const snn_hip_conv2d_params& p);
 size_t conv2d_filter_backprop_window_f16_partial_floats(
     const snn_hip_conv2d_params& p);
 int launch_conv2d_filter_backprop_window_f16(const _Float16* x,
@@ -351,6 +356,9 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
 // and `filter` is still the original HWCF tensor.
 // `wanted`: it takes the shape and is faster than a kernel of `other_us`.
 bool conv2d_rowtile_f16_wanted(const snn_hip_conv2d_params& p, double other_us);
+// LDS tiles: 1 of all channels, 2 in turn, 3: one that is loaded again; 0: none
+// takes the shape
+int conv2d_rowtile_f16_buffers(const snn_hip_conv2d_params& p);
 int launch_conv2d_rowtile_f16(const _Float16* input, const _Float16* filter,
                               _Float16* output, const snn_hip_conv2d_params& p,
                               _Float16* packed, hipStream_t stream,

@@ -145,6 +145,18 @@ def gather_tile(p, direction, dtype):
     return pixels.value, features.value, splits.value
 
 
+def lds_form_f16(p, direction):
+    """How a binary16 launch keeps its pixels in LDS, or None where it runs on
+    another kernel (snn_hip_conv2d_lds_form_f16)."""
+    form = ctypes.c_int()
+    code = capi.lib().snn_hip_conv2d_lds_form_f16(
+        ctypes.byref(p), direction, ctypes.byref(form))
+    if code == STATUS.INVALID_ALGORITHM:
+        return None
+    capi.check(code)
+    return form.value
+
+
 _CONV_FN = {
     (DIRECTION.FORWARD, torch.float32): "snn_hip_conv2d_forward_f32",
     (DIRECTION.INPUT_BACKPROP, torch.float32):

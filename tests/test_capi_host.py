@@ -405,3 +405,37 @@ def test_gather_tile_refuses_bad_arguments():
     for direction in (DIRECTION.FILTER_BACKPROP, 5, -1):
         assert fn(ctypes.byref(p), direction, 0, *out) == \
             STATUS.INVALID_ALGORITHM
+
+
+@pytest.mark.parametrize("shape,direction,form", [
+    ((128, 56, 56, 64, 64, 3, 1, True), DIRECTION.FORWARD, 1),
+    ((128, 28, 28, 128, 128, 3, 1, True), DIRECTION.INPUT_BACKPROP, 2),
+    ((16, 224, 224, 64, 64, 3, 1, True), DIRECTION.FORWARD, 3),
+    ((128, 56, 56, 128, 128, 3, 2, True), DIRECTION.FORWARD, None),
+    ((1, 14, 14, 64, 64, 3, 1, True), DIRECTION.FORWARD, None),
+    ((128, 56, 56, 64, 256, 1, 1, True), DIRECTION.FORWARD, None),
+    ((8, 14, 14, 1024, 256, 1, 1, True), DIRECTION.FORWARD, None),
+    ((128, 224, 224, 3, 64, 7, 2, True), DIRECTION.FORWARD, None),
+    ((2, 14, 14, 64, 72, 3, 1, True), DIRECTION.FILTER_BACKPROP, None),
+])
+def test_lds_form(shape, direction, form):
+    assert ops.lds_form_f16(ops.conv_params(*shape), direction) == form
+
+
+def test_lds_form_of_filter_gradients():
+    p = ops.conv_params(16, 224, 224, 64, 64, 3, 1, True)
+    assert ops.lds_form_f16(p, DIRECTION.FILTER_BACKPROP) > 1
+
+
+def test_lds_form_refuses_bad_arguments():
+    fn = capi.lib().snn_hip_conv2d_lds_form_f16
+    p = ops.conv_params(2, 9, 9, 8, 8, 3, 1, True)
+    out = ctypes.c_int()
+    ref = ctypes.byref(out)
+    assert fn(None, DIRECTION.FORWARD, ref) == STATUS.INVALID_PARAMETER
+    assert fn(ctypes.byref(p), DIRECTION.FORWARD, None) == \
+        STATUS.INVALID_PARAMETER
+    assert fn(ctypes.byref(p), 3, ref) == STATUS.INVALID_PARAMETER
+    p.batch = 0
+    assert fn(ctypes.byref(p), DIRECTION.FORWARD, ref) == \
+        STATUS.INVALID_PARAMETER

@@ -1,6 +1,7 @@
-"""Binary16 3x3 layers of wide images on the LDS-tile kernel: one tile of all 64
-channels, two of 32 in turn, and one of 32 that is loaded again; whole rows per
-work-group and tiles that start inside a row; one and two feature groups.
+"""Binary16 3x3 layers on the LDS-tile kernel: one tile of all 64 channels, two of 32
+in turn, and one of 32 that is loaded again; whole rows per work-group and tiles that
+start inside a row; one and two feature groups.  And wide images of few pixels, which
+the rule leaves to the gathering kernel.
 
 Bound: one rounding to binary16 and n fp32 additions.
 """
@@ -26,10 +27,47 @@ SHAPES = [
 ]
 
 
+F, I = DIRECTION.FORWARD, DIRECTION.INPUT_BACKPROP
+# ..., direction, form (ops.lds_form_f16)
+FORMS = [
+    ((7, 27, 39, 64, 192, True), F, 1),
+    ((14, 11, 54, 64, 128, True), F, 1),
+    ((8, 115, 53, 64, 64, False), I, 1),
+    ((11, 39, 77, 64, 128, False), I, 1),
+    ((13, 15, 49, 64, 128, True), F, 2),
+    ((10, 17, 121, 128, 64, True), F, 2),
+    ((1, 43, 119, 128, 256, True), F, 2),
+    ((11, 65, 23, 128, 192, True), I, 2),
+    ((13, 17, 75, 128, 256, True), I, 2),
+    ((2, 129, 169, 64, 64, True), F, 3),
+    ((3, 43, 107, 64, 256, True), F, 3),
+    ((2, 69, 91, 128, 256, True), F, 3),
+    ((5, 79, 185, 64, 64, True), I, 3),
+    ((6, 63, 185, 128, 64, True), I, 3),
+    ((5, 163, 78, 64, 128, False), I, 3),
+]
+
+
+@pytest.mark.parametrize(
+    "shape,direction,form", FORMS,
+    ids=["x".join(map(str, c[0])) + "fi"[c[1] == I] for c in FORMS])
+def test_conv_rowtile_f16_forms(shape, direction, form):
+    batch, rows, cols, source, produced, same = shape
+    channels, features = ((source, produced) if direction == F
+                          else (produced, source))
+    assert ops.lds_form_f16(
+        ops.conv_params(batch, rows, cols, channels, features, 3, 1, same),
+        direction) == form
+    check(shape, direction)
+
+
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
-@pytest.mark.parametrize("direction",
-                         [DIRECTION.FORWARD, DIRECTION.INPUT_BACKPROP])
+@pytest.mark.parametrize("direction", [F, I])
 def test_conv_rowtile_f16(shape, direction):
+    check(shape, direction)
+
+
+def check(shape, direction):
     batch, rows, cols, source, produced, same = shape
     channels, features = ((source, produced) if direction == DIRECTION.FORWARD
                           else (produced, source))

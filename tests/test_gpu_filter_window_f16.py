@@ -33,7 +33,9 @@ SHAPES = [
     (1, 15, 16, 56, 56, 5, 1, True),
     (2, 14, 14, 64, 56, 5, 1, False),
     (250, 1, 1, 64, 64, 5, 1, True),      # images smaller than the window
-    (2, 61, 67, 144, 144, 3, 1, True),    # many bands, partial tiles summed
+    (3, 111, 69, 144, 72, 3, 1, True),    # many bands, partial tiles summed
+    (6, 42, 95, 216, 232, 3, 2, True),    # ... in planes
+    (8, 74, 40, 64, 72, 5, 1, True),
     (1, 42, 55, 136, 200, 5, 1, True),
 ]
 
@@ -41,6 +43,7 @@ SHAPES = [
 @pytest.mark.parametrize("shape", SHAPES, ids=lambda s: "x".join(map(str, s)))
 def test_filter_window_f16(shape):
     p = ops.conv_params(*shape)
+    assert ops.lds_form_f16(p, DIRECTION.FILTER_BACKPROP) is not None
     rng = np.random.default_rng(6100 + shape[1] + shape[3])
     n_a, n_b, n_out = ops.conv_sizes(p, DIRECTION.FILTER_BACKPROP)
     a = uniform(rng, n_a).astype(np.float16)
