@@ -134,6 +134,8 @@ struct FbGeom {
   TapRow rows[kMaxGroups][kMaxEntries];
 };
 
+struct FbGeoms { FbGeom g[1]; };  // (see the kernel that sums)
+
 __device__ inline __amdgpu_buffer_rsrc_t make_rsrc(const void* p,
                                                    size_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0,
@@ -540,51 +542,111 @@ __global__ void __launch_bounds__(64 * kWaves)
   }
 }
 
-// One element of dW over the products that exist.  The kernel above multiplies
-// the zeros beside a band's dY and in the padding of X with whatever the other
-// operand holds there, which an infinity makes a NaN; a NaN sum is therefore
-// taken again by this one, by the whole work-group.
-__device__ inline float exact_gradient(const _Float16* __restrict__ x,
-                                       const _Float16* __restrict__ dy,
-                                       const FbGeom& g, int tap, int c, int k,
-                                       float* sums) {
+// The sum over the lanes of a wave of value `lane % 16`.
+__device__ inline float add_lanes(float16v& sums) {
+#pragma nounroll
+  for (int m = 1; m < 64; m *= 2)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const float other = __shfl_xor(sums[v], m);
+      sums[v] += other;
+    }
+  float mine = sums[0];
+#pragma unroll
+  for (int v = 1; v < 16; ++v)
+    mine = static_cast<int>(threadIdx.x & 15) == v ? sums[v] : mine;
+  return mine;
+}
+
+// Elements c ... c + 3, k ... k + 3 of dW's tap over the products that exist among
+// the pixels of one split, by one wave: number 4 channel + feature for lane % 16;
+// `open`: a bit for each that is wanted.  Stops where none of them can be a number
+// any more.
+__device__ inline float exact_part(const _Float16* __restrict__ x,
+                                   const _Float16* __restrict__ dy,
+                                   const FbGeom& g, int tap, int c, int k,
+                                   int split, unsigned open) {
   const int r = tap / g.win_cols, s = tap - r * g.win_cols;
-  const int total = g.batch * g.out_rows * g.out_cols;
-  float sum = 0.f;
-  for (int m = threadIdx.x; m < total && sum == sum; m += 256) {
-    const int row = m / g.out_cols;
-    const int n = row / g.out_rows;
-    const int iy = (row - n * g.out_rows) * g.stride_rows + r - g.pad_rows;
-    const int ix = (m - row * g.out_cols) * g.stride_cols + s - g.pad_cols;
-    if (iy < 0 || iy >= g.in_rows || ix < 0 || ix >= g.in_cols) continue;
-    sum += static_cast<float>(
-               x[(static_cast<size_t>(n * g.in_rows + iy) * g.in_cols + ix) *
-                     g.channels + c]) *
-           static_cast<float>(dy[static_cast<size_t>(m) * g.features + k]);
+  const int lane = threadIdx.x & 63;
+  const int first = split * g.per_split * g.group;
+  const int bands = min(g.n_subbands, first + g.per_split * g.group) - first;
+  const int total = bands * g.band * g.seg_cols;
+  // A pixel's place, and the digits of 64 pixels more: stepping takes no division.
+  struct Place { int col, row, seg, band, n; };
+  auto place = [&](int pixel, int first_band) {
+    const int rows = pixel / g.seg_cols, in = rows / g.band + first_band;
+    const int of_row = in / g.segs, n = of_row / g.bands_per_image;
+    return Place{pixel - rows * g.seg_cols, rows % g.band, in - of_row * g.segs,
+                 of_row - n * g.bands_per_image, n};
+  };
+  Place at = place(lane, first);
+  const Place more = place(64, 0);
+  float16v sums;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) sums[v] = 0.f;
+#pragma nounroll
+  for (int i = lane; i - lane < total; i += 64) {
+    const int oy = at.band * g.band + at.row;
+    const int ox = at.seg * g.seg_cols + at.col;
+    const int iy = oy * g.stride_rows + r - g.pad_rows;
+    const int ix = ox * g.stride_cols + s - g.pad_cols;
+    if (i < total && oy < g.out_rows && ox < g.out_cols && iy >= 0 &&
+        iy < g.in_rows && ix >= 0 && ix < g.in_cols) {
+      const half4v xs = *reinterpret_cast<const half4v*>(
+          x + (static_cast<size_t>(at.n * g.in_rows + iy) * g.in_cols + ix) *
+                  g.channels + c);
+      const half4v ys = *reinterpret_cast<const half4v*>(
+          dy + (static_cast<size_t>(at.n * g.out_rows + oy) * g.out_cols + ox) *
+                   g.features + k);
+#pragma unroll
+      for (int v = 0; v < 16; ++v)
+        sums[v] += static_cast<float>(xs[v / 4]) * static_cast<float>(ys[v % 4]);
+    }
+    auto carry = [](int& digit, int add, int radix, int over) {
+      digit += add + over;
+      const bool full = digit >= radix;
+      if (full) digit -= radix;
+      return full ? 1 : 0;
+    };
+    int over = carry(at.col, more.col, g.seg_cols, 0);
+    over = carry(at.row, more.row, g.band, over);
+    over = carry(at.seg, more.seg, g.segs, over);
+    over = carry(at.band, more.band, g.bands_per_image, over);
+    at.n += more.n + over;
+    unsigned numbers = 0;
+#pragma unroll
+    for (int v = 0; v < 16; ++v)
+      if (__builtin_amdgcn_ballot_w64(sums[v] != sums[v]) == 0)
+        numbers |= 1u << v;
+    if ((numbers & open) == 0) break;
   }
-  __syncthreads();
-  sums[threadIdx.x] = sum;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (static_cast<int>(threadIdx.x) < w)
-      sums[threadIdx.x] += sums[threadIdx.x + w];
-    __syncthreads();
-  }
-  return sums[0];
+  return add_lanes(sums);
 }
 
 // Sums the partial tiles and rounds: a work-group is 256 / n_groups
 // consecutive float4 of the filter x n_groups groups of splits (a power of two
 // up to 16).
+// The kernel above multiplies the zeros beside a band's dY and in the padding of X
+// with whatever the other operand holds there, which an infinity makes a NaN.  A sum
+// that is one has those partial sums that are taken again, over the products that
+// exist, one wave per four channels and features, until one is a NaN by these.
+// That part keeps to few registers and loads its arguments for itself, as the waves
+// in flight bound the rest (122 registers cost 14x14x256 at batch 128 3 us, 69 none).
+// 224x224x64 at batch 16, finite 87 us: one infinite dY 137, all infinite 90, an
+// infinity in the first row of every image, where the padding meets it, 758; over
+// the whole batch and one sum after the other these took 56735, 391 and 69977.
+// 56x56x128, 3x3 stride 2, at batch 128, finite 72: 87, 91 and 161.
 template <typename ROWS>
 __global__ void __launch_bounds__(256)
     filter_backprop_window_f16_reduce_kernel(const float4v* __restrict__ part,
                                              const _Float16* __restrict__ x,
                                              const _Float16* __restrict__ dy,
                                              _Float16* __restrict__ dw,
-                                             FbGeom g, int n_groups) {
+                                             FbGeoms gs, int n_groups) {
+  const FbGeom& g = gs.g[0];
   __shared__ float4v sums[256];
-  __shared__ int bad[4];
+  __shared__ int any_strange;
+  __shared__ int strange[64];  // of four channels each, a bit per channel
   constexpr int kTileVecs = ROWS::kTaps * kTile * kTile / 4;
   const int n_units = g.tap_groups * g.c_tiles * g.k_tiles;
   const int width = 256 / n_groups;
@@ -598,12 +660,13 @@ __global__ void __launch_bounds__(256)
   for (int sp = group; sp < g.n_splits; sp += n_groups)
     sum += part[(static_cast<size_t>(sp) * n_units + unit) * kTileVecs + local];
   sums[threadIdx.x] = sum;
-  if (threadIdx.x < 4) bad[threadIdx.x] = 0;
+  if (threadIdx.x < 64) strange[threadIdx.x] = 0;
+  if (threadIdx.x == 0) any_strange = 0;
   __syncthreads();
   // accumulator order of the partial tiles: local = ((tap * 4 + quarter) * 4 +
   // i4) * 64 + lane holds channel 32 (quarter & 1) + lane % 32 and features
   // 32 (quarter >> 1) + 8 i4 + 4 (lane / 32) ... + 3
-  auto place_of = [&](unsigned at, int* tap, int* c, int* k) {
+  auto place_of = [](const FbGeom& g, unsigned at, int* tap, int* c, int* k) {
     const unsigned u = at / kTileVecs, l = at - u * kTileVecs;
     const unsigned ln = l & 63, i4 = (l >> 6) & 3, quarter = (l >> 8) & 3;
     const int tg = u % g.tap_groups;
@@ -618,36 +681,79 @@ __global__ void __launch_bounds__(256)
   if (group == 0) {
     for (int i = 1; i < n_groups; ++i) sum += sums[i * width + lane_o];
     int tap, c, k;
-    place_of(o, &tap, &c, &k);
+    place_of(g, o, &tap, &c, &k);
     if (c < g.channels && k < g.features) {
-      half4v r;
+      if (sum[0] != sum[0] || sum[1] != sum[1] || sum[2] != sum[2] ||
+          sum[3] != sum[3]) {
+        atomicOr(&strange[lane_o >> 2], 1 << (lane_o & 3));
+        any_strange = 1;
+      } else {
+        half4v r;
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        r[v] = static_cast<_Float16>(sum[v]);
-        if (sum[v] != sum[v]) bad[v] = 1;
+        for (int v = 0; v < 4; ++v) r[v] = static_cast<_Float16>(sum[v]);
+        *reinterpret_cast<half4v*>(
+            dw + (static_cast<size_t>(tap) * g.channels + c) * g.features + k) = r;
       }
-      *reinterpret_cast<half4v*>(
-          dw + (static_cast<size_t>(tap) * g.channels + c) * g.features + k) = r;
     }
   }
   __syncthreads();
-  if ((bad[0] | bad[1] | bad[2] | bad[3]) == 0) return;
-  // (every lane of the work-group comes here; the sums in LDS are done with)
-  if (group == 0) sums[lane_o] = sum;
-  __syncthreads();
-  __shared__ float terms[256];
-  for (int i = 0; i < width; ++i) {
+  if (__builtin_amdgcn_readfirstlane(any_strange) == 0) return;
+  // (an index that is not known before: what follows would load its arguments in
+  // front of the sums)
+  const FbGeom& h = gs.g[__builtin_amdgcn_readfirstlane(any_strange) - 1];
+  const int units = h.tap_groups * h.c_tiles * h.k_tiles;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma nounroll
+  for (int i = wave; i < width / 4; i += 4) {
+    const int channels = strange[i];
+    if (channels == 0) continue;
+    const unsigned at = blockIdx.x * width + 4 * i;
+    const unsigned u = at / kTileVecs;
     int tap, c, k;
-    place_of(blockIdx.x * width + i, &tap, &c, &k);
-    if (c >= g.channels || k >= g.features) continue;
-    for (int v = 0; v < 4; ++v) {
-      if (sums[i][v] == sums[i][v]) continue;
-      const float fixed = exact_gradient(x, dy, g, tap, c, k + v, terms);
-      if (threadIdx.x == 0)
-        dw[(static_cast<size_t>(tap) * g.channels + c) * g.features + k + v] =
-            static_cast<_Float16>(fixed);
-      __syncthreads();
+    place_of(h, at, &tap, &c, &k);
+    float total = 0.f;  // number 4 channel + feature for lane % 16
+    unsigned open = 0;  // sums that may be numbers
+#pragma unroll
+    for (int ch = 0; ch < 4; ++ch)
+      if ((channels >> ch & 1) != 0) open |= 15u << (4 * ch);
+#pragma nounroll
+    for (int sp0 = 0; sp0 < h.n_splits && open != 0; sp0 += 64) {
+      unsigned again = 0;  // sums of this lane's split
+      {
+        float16v p;
+#pragma unroll
+        for (int ch = 0; ch < 4; ++ch) {
+          float4v four = {0.f, 0.f, 0.f, 0.f};
+          if (sp0 + lane < h.n_splits)
+            four = part[(static_cast<size_t>(sp0 + lane) * units + u) * kTileVecs +
+                        (at - u * kTileVecs) + ch];
+#pragma unroll
+          for (int v = 0; v < 4; ++v) {
+            const bool number = four[v] == four[v];
+            p[4 * ch + v] = number ? four[v] : 0.f;
+            if (!number) again |= 1u << (4 * ch + v);
+          }
+        }
+        total += add_lanes(p);
+      }
+      unsigned long long left = __builtin_amdgcn_ballot_w64(again != 0);
+#pragma nounroll
+      for (;;) {
+        open &= ~static_cast<unsigned>(
+            __builtin_amdgcn_ballot_w64(total != total));
+        if (left == 0 || open == 0) break;
+        const int from = __builtin_ctzll(left);
+        left &= left - 1;
+        const unsigned these =
+            static_cast<unsigned>(__shfl(static_cast<int>(again), from)) & open;
+        if (these == 0) continue;
+        const float exact = exact_part(x, dy, h, tap, c, k, sp0 + from, these);
+        if ((these >> (lane & 15) & 1u) != 0) total += exact;
+      }
     }
+    if (lane < 16 && (channels >> (lane >> 2) & 1) != 0)
+      dw[(static_cast<size_t>(tap) * h.channels + c + (lane >> 2)) * h.features +
+         k + (lane & 3)] = static_cast<_Float16>(total);
   }
 }
 
@@ -846,8 +952,8 @@ void launch_rows(const _Float16* x, const _Float16* dy, _Float16* dw,
     reduce_groups *= 2;
   hipLaunchKernelGGL(filter_backprop_window_f16_reduce_kernel<ROWS>,
                      dim3(vecs / (256 / reduce_groups)), dim3(256), 0, stream,
-                     reinterpret_cast<const float4v*>(part), x, dy, dw, g,
-                     reduce_groups);
+                     reinterpret_cast<const float4v*>(part), x, dy, dw,
+                     FbGeoms{{g}}, reduce_groups);
 }
 
 }  // namespace

@@ -96,3 +96,64 @@ def test_filter_window_f16_infinity_stays(shape, operand):
     assert np.array_equal(np.isfinite(got), ok)
     assert_rounded_once(got[ok], ref[ok], p.batch * p.out_rows * p.out_cols,
                         (shape, operand))
+
+
+@pytest.mark.parametrize("shape", [(4, 224, 224, 64, 64, 3, 1, True),
+                                   (28, 101, 112, 88, 72, 3, 2, True),
+                                   (8, 74, 40, 64, 72, 5, 1, True)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_filter_window_f16_infinities_of_many_splits(shape):
+    """What an overflow of a scaled loss leaves: infinities among gradients, whose
+    products with the zeros of a ReLU are NaNs by right, and beside the border, whose
+    products with the padding are none.  Such a launch takes at most a few times as
+    long as a finite one (30 for those of the border, in every image)."""
+    p = ops.conv_params(*shape)
+    assert ops.lds_form_f16(p, DIRECTION.FILTER_BACKPROP) > 4
+    rng = np.random.default_rng(6300 + shape[1])
+    n_a, n_b, _ = ops.conv_sizes(p, DIRECTION.FILTER_BACKPROP)
+    a = np.maximum(uniform(rng, n_a), 0).astype(np.float16)
+    b = uniform(rng, n_b).astype(np.float16)
+    _, rec = ops.workspace_size(p, DIRECTION.FILTER_BACKPROP, ALGO.IM2COL,
+                                DTYPE.F16)
+    ws = torch.empty(rec, dtype=torch.float16, device="cuda")
+    da, db = dev(a, torch.float16), dev(b, torch.float16)
+
+    def run():
+        return ops.conv2d(da, db, p, DIRECTION.FILTER_BACKPROP, ALGO.IM2COL,
+                          workspace=ws)
+
+    def least_ms():
+        times = []
+        for _ in range(6):
+            start, end = (torch.cuda.Event(enable_timing=True) for _ in "ab")
+            start.record()
+            run()
+            end.record()
+            end.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times[1:])
+
+    finite_ms = max(least_ms(), 0.03)
+    images = b.reshape(p.batch, p.out_rows, p.out_cols, p.features)
+    x = a.reshape(p.batch, p.in_rows, p.in_cols, p.channels)
+    images[1, 5, 7, 3] = np.inf        # inside
+    images[2, 0, p.out_cols - 1, 9] = -np.inf  # at the border
+    x[0, 0, 0, 5] = np.inf
+    x[p.batch - 1, p.in_rows - 1, 4, 60] = np.nan
+    da, db = dev(a, torch.float16), dev(b, torch.float16)
+    ref = np.asarray(ORACLE_FN[DIRECTION.FILTER_BACKPROP](
+        a.astype(np.float32), b.astype(np.float32),
+        oracle_params(p, p.features), acc64=True), dtype=np.float64).reshape(-1)
+    got = run().float().cpu().numpy().reshape(-1)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    ok = np.isfinite(ref)
+    assert ok.any() and np.isnan(ref).any() and np.isinf(ref).any()
+    assert_rounded_once(got[ok], ref[ok], p.batch * p.out_rows * p.out_cols,
+                        shape)
+    assert least_ms() < 10 * finite_ms
+    db[:] = np.inf
+    assert least_ms() < 10 * finite_ms
+    images[:, 0, 3, :] = np.inf
+    db = dev(b, torch.float16)
+    assert least_ms() < 30 * finite_ms
