@@ -35,10 +35,10 @@ class PlanCache {
   template <typename F>
   const Plan& get(const snn_hip_conv2d_params& p, unsigned form, F compute) {
     ++now_;
+    if (latest_ < used_ && matches(latest_, p, form)) return hit(latest_);
     const std::uint64_t hash = hash_of(p, form);
-    if (latest_ < used_ && matches(latest_, hash, p, form)) return hit(latest_);
     for (int k = 0; k < used_; ++k)
-      if (matches(k, hash, p, form)) return hit(k);
+      if (hashes_[k] == hash && matches(k, p, form)) return hit(k);
     const Plan plan = compute();
     if (entries_ == nullptr)
       entries_ = static_cast<Entry*>(std::malloc(kCapacity * sizeof(Entry)));
@@ -68,19 +68,18 @@ class PlanCache {
   };
 
   static std::uint64_t hash_of(const snn_hip_conv2d_params& p, unsigned form) {
-    static_assert(sizeof p % 4 == 0, "whole words");
-    unsigned words[sizeof p / 4];
+    constexpr int kWords = (sizeof p + 7) / 8;
+    std::uint64_t words[kWords] = {};
     std::memcpy(words, &p, sizeof p);
     std::uint64_t h = form;
-    for (const unsigned word : words) {
+    for (const std::uint64_t word : words) {
       h = (h ^ word) * 0x9E3779B97F4A7C15ull;
       h ^= h >> 32;
     }
     return h;
   }
-  bool matches(int k, std::uint64_t hash, const snn_hip_conv2d_params& p,
-               unsigned form) const {
-    return hashes_[k] == hash && entries_[k].form == form &&
+  bool matches(int k, const snn_hip_conv2d_params& p, unsigned form) const {
+    return entries_[k].form == form &&
            std::memcmp(&entries_[k].params, &p, sizeof p) == 0;
   }
   const Plan& hit(int k) {
