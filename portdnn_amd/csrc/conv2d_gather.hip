@@ -1172,8 +1172,8 @@ constexpr TileShape kTilesF16[] = {
 // and on power more than on how the tiles fall on compute units.
 constexpr TileShape kTilesF32[] = {{128, 32, 0.36, 0.27, false},
                                    {64, 64, 0.36, 0.265, false},
-                                   {128, 128, 0.10, 0.92, true},
-                                   {128, 64, 0.27, 0.47, true}};
+                                   {128, 128, 0.10, 0.88, true},
+                                   {128, 64, 0.27, 0.45, true}};
 constexpr int kMergedTile = 0;
 template <typename T>
 struct Tiles;
