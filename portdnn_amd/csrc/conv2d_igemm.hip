@@ -2100,7 +2100,7 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
       SNN_TUNING_ENV("SNN_HIP_FILBK_F16_OFF") == nullptr) {
     // binary16 matrix instructions; the partial tiles go to the workspace
     // when it holds them, else to a stream-ordered temporary (or, when there is
-    // none, to the kernel below, which needs less)
+    // none, the kernels below take the launch, which need less)
     const size_t part_floats =
         windowed ? conv2d_filter_backprop_window_f16_partial_floats(p)
                  : conv2d_filter_backprop_1x1_f16_partial_floats(p);
@@ -2111,8 +2111,6 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
       void* ptr = nullptr;
       if (temp_malloc_async(&ptr, part_floats * sizeof(float), stream) !=
           hipSuccess) {
-        if (!conv2d_filter_backprop_direct_f16_supports(p))
-          return SNN_HIP_ALLOCATION_PROBLEM;
         (void)hipGetLastError();
         room = false;
       }
@@ -2152,7 +2150,9 @@ int launch_conv2d_filter_backprop_f16(const _Float16* x, const _Float16* dy,
     if (err != hipSuccess) return report_hip_error(err, "f16 filter backprop");
     return SNN_HIP_OK;
   }
-  if (p.channels % 64 != 0 || p.features % 4 != 0) return -1;
+  if (p.channels % 64 != 0 || p.features % 4 != 0 ||
+      dw_elems * sizeof(float) > kMaxBufferBytes)
+    return -1;
   float* acc32 = reinterpret_cast<float*>(workspace);
   bool temporary = false;
   if (workspace == nullptr || workspace_elems < 2 * dw_elems ||

@@ -45,3 +45,14 @@ def test_gpu_api_program():
                          stderr=subprocess.STDOUT, text=True, timeout=300)
     assert out.returncode == 0, out.stdout[-4000:]
     assert "0 failures" in out.stdout
+
+
+@pytest.mark.gpu
+def test_gpu_no_temporary_program():
+    """Launches whose stream-ordered temporary cannot be had (the program refuses the
+    library's allocations) take a kernel that needs none, or say so."""
+    out = subprocess.run([_exe("gpu_no_temporary_test")],
+                         stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                         text=True, timeout=120)
+    assert out.returncode == 0, out.stdout[-4000:]
+    assert "0 failures" in out.stdout
