@@ -1809,10 +1809,21 @@ int launch_conv2d_f16(int direction, const _Float16* input,
     const bool temporary = workspace == nullptr || workspace_elems < need ||
                            !aligned(workspace);
     if (temporary) {
+      // An input gradient needs none on the gathering kernel, which reads its filter
+      // in place: recorded launches run there, and those whose temporary cannot be
+      // had.
+      const GatherPlan& whole = make_plan<_Float16>(direction, p, false);
+      const bool without =
+          whole.ok && whole.workspace_bytes(whole.from == kPacked) == 0;
       void* ptr = nullptr;
-      if (temp_malloc_async(&ptr, need * sizeof(_Float16), stream) !=
-          hipSuccess)
-        return SNN_HIP_ALLOCATION_PROBLEM;
+      if ((without && stream_captures(stream)) ||
+          temp_malloc_async(&ptr, need * sizeof(_Float16), stream) !=
+              hipSuccess) {
+        if (!without) return SNN_HIP_ALLOCATION_PROBLEM;
+        (void)hipGetLastError();
+        return launch_gather<_Float16>(whole, input, filter, output, nullptr, 0,
+                                       nullptr, false, stream);
+      }
       packed = static_cast<_Float16*>(ptr);
     }
     const int status =

@@ -109,9 +109,62 @@ void test_filter_gradient() {
     CHECK(hipFree(ptr) == hipSuccess);
 }
 
+// An input gradient on the row-tile kernel, whose packed filter has no room.
+void test_input_gradient() {
+  constexpr int kBatch = 11, kRows = 108, kCols = 37, kC = 64, kK = 64;
+  snn_hip_conv2d_params p{};
+  p.channels = kC;
+  p.features = kK;
+  p.batch = kBatch;
+  p.in_rows = p.out_rows = kRows;
+  p.in_cols = p.out_cols = kCols;
+  p.window_rows = p.window_cols = 3;
+  p.stride_rows = p.stride_cols = 1;
+  p.pad_rows = p.pad_cols = 1;
+  p.dilation_rows = p.dilation_cols = p.groups = 1;
+  int form = 0;
+  CHECK(snn_hip_conv2d_lds_form_f16(&p, SNN_HIP_INPUT_BACKPROP, &form) ==
+        SNN_HIP_OK);
+  const auto dy = values(size_t{kBatch} * kRows * kCols * kK, 3);
+  const auto w = values(9 * kC * kK, 4);
+  std::vector<std::uint16_t> dx(size_t{kBatch} * kRows * kCols * kC, 0xFFFF);
+  void* const d_dy = on_device(dy);
+  void* const d_w = on_device(w);
+  void* const d_dx = on_device(dx);
+  g_refused = 0;
+  CHECK_EQ(snn_hip_conv2d_input_backprop_f16(d_dy, d_w, d_dx, &p,
+                                             SNN_HIP_ALGO_IM2COL, nullptr, 0,
+                                             nullptr),
+           SNN_HIP_OK);
+  CHECK(g_refused > 0);
+  CHECK(hipMemcpy(dx.data(), d_dx, dx.size() * 2, hipMemcpyDeviceToHost) ==
+        hipSuccess);
+  int wrong = 0;
+  for (int pixel = 0; pixel < kBatch * kRows * kCols; pixel += 97) {
+    const int n = pixel / (kRows * kCols), y = pixel / kCols % kRows;
+    const int x = pixel % kCols;
+    for (int c = 0; c < kC; ++c) {
+      float sum = 0;
+      for (int r = 0; r < 3; ++r)
+        for (int s = 0; s < 3; ++s) {
+          const int oy = y + 1 - r, ox = x + 1 - s;
+          if (oy < 0 || oy >= kRows || ox < 0 || ox >= kCols) continue;
+          const size_t at = (size_t{1} * (n * kRows + oy) * kCols + ox) * kK;
+          for (int k = 0; k < kK; ++k)
+            sum += half_value(dy[at + k]) *
+                   half_value(w[((r * 3 + s) * kC + c) * kK + k]);
+        }
+      wrong += half_value(dx[static_cast<size_t>(pixel) * kC + c]) != sum;
+    }
+  }
+  CHECK_EQ(wrong, 0);
+  for (void* ptr : {d_dy, d_w, d_dx}) CHECK(hipFree(ptr) == hipSuccess);
+}
+
 }  // namespace
 
 int main() {
   test_filter_gradient();
+  test_input_gradient();
   return report("gpu_no_temporary_test");
 }

@@ -11,7 +11,7 @@ import torch
 
 from portdnn_amd import ops
 from portdnn_amd.capi import ALGO, DIRECTION, DTYPE
-from test_gpu_conv_f16_shapes import assert_rounded_once
+from test_gpu_conv_f16_shapes import assert_rounded_once, check_recorded
 from test_gpu_parity import ORACLE_FN, dev, oracle_params, uniform
 
 pytestmark = pytest.mark.gpu
@@ -87,3 +87,23 @@ def check(shape, direction):
                         (shape, direction))
     assert torch.all(guard[n_out:] == 7.0)
     assert torch.all(block[rec:] == 7.0)
+
+
+@pytest.mark.parametrize("shape", [c[0] for c in FORMS if c[1] == I][:4],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_input_gradient_recorded_without_a_workspace(shape):
+    """Kernels only: the gathering kernel reads the filter in place."""
+    batch, rows, cols, source, produced, same = shape
+    p = ops.conv_params(batch, rows, cols, produced, source, 3, 1, same)
+    n_a, n_b, n_out = ops.conv_sizes(p, I)
+    a = torch.empty(n_a, dtype=torch.float16, device="cuda")
+    b = torch.empty(n_b, dtype=torch.float16, device="cuda")
+
+    def refill(seed):
+        rng = np.random.default_rng(seed)
+        a.copy_(dev(uniform(rng, n_a), torch.float16))
+        b.copy_(dev(uniform(rng, n_b), torch.float16))
+
+    refill(0)
+    check_recorded(lambda out: ops.conv2d(a, b, p, I, ALGO.IM2COL, out=out),
+                   refill, 9 * source, shape)
