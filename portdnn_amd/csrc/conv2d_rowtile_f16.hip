@@ -26,7 +26,7 @@
 // Each wave owns 2 feature blocks x 4 pixel blocks (64 features x 128
 // pixels, 128 accumulator registers): per 16-deep reduction step it reads
 // 4 KB from LDS and 2 KB of filter for 8 MFMAs; or, where that balances the
-// compute units better, 2 x 2 blocks.  224x224x64 at batch 16, 3x3: 86 us (69
+// compute units better, 2 x 2 blocks.  224x224x64 at batch 16, 3x3: 85 us (69
 // without the stores, 71 without the loads, 55 with neither).
 //
 // portDNN's half build accumulates in half (e.g. `DataType out_val{0}` with
@@ -656,9 +656,9 @@ RowTilePlan compute_plan(const snn_hip_conv2d_params& p) {
   // layers of 1e9 to 1.2e11 operations the estimates were within 10 % and the one
   // taken 1.6 % slower than the fastest, on the average.  (By counting wave tiles
   // and work-groups instead, images of some widths were left with two waves per
-  // CU: 149x149x64 at batch 8 84 us, now 38; 87x87x256 <- 192 at batch 9 196, now 75;
-  // and 224x224x64 at batch 16 with one work-group, whose loads, products and
-  // stores took turns: 105, with two that share the LDS 86.)
+  // CU: 149x149x64 at batch 8 76 us, now 34; 150x150x64 -> 128 at batch 8 94, now
+  // 45; and 224x224x64 at batch 16 with one work-group, whose loads, products and
+  // stores took turns: 99, with two that share the LDS 85.)
   RowTilePlan best;
   for (int wf = 1; wf <= (p.features % 128 == 0 ? 2 : 1); ++wf)
     for (int waves = 2; waves <= 4; waves += 2)
