@@ -930,24 +930,27 @@ int launch_gemm_path<float>(int direction, const float* input,
 bool winograd_loses(int direction, const snn_hip_conv2d_params& p,
                     size_t workspace_elems, const LaunchOptions* epilogue) {
   const bool backprop = direction == SNN_HIP_INPUT_BACKPROP;
-  const bool gathers = conv2d_gather_f32_wanted(
-      direction, p,
-      !backprop && epilogue != nullptr && epilogue->wanted());
-  if (!backprop && !gathers && conv2d_small_supports(p)) return true;
-  // (the others may add through atomics)
-  if (epilogue != nullptr && epilogue->deterministic) return false;
-  const size_t scratch =
-      gathers ? conv2d_gather_f32_workspace_floats(direction, p) : 0;
   const int in_ch = backprop ? p.features : p.channels;
   const int out_ch = backprop ? p.channels : p.features;
   const int chunks = in_ch / 16;
-  if (chunks == 1) return gathers && scratch == 0;
   const size_t tiles =
       static_cast<size_t>(p.batch) *
       ceil_div(backprop ? p.in_rows : p.out_rows, 2) *
       ceil_div(backprop ? p.in_cols : p.out_cols, 2);
   const size_t units = ceil_div(tiles, size_t{32}) * (out_ch / 32);
-  return chunks >= 8 && units < 128 && scratch <= workspace_elems &&
+  const bool small = !backprop && conv2d_small_supports(p);
+  const bool splits = chunks >= 8 && units < 128;
+  if (!small && !splits && chunks != 1) return false;
+  const bool gathers = conv2d_gather_f32_wanted(
+      direction, p,
+      !backprop && epilogue != nullptr && epilogue->wanted());
+  if (small && !gathers) return true;
+  // (the others may add through atomics)
+  if (epilogue != nullptr && epilogue->deterministic) return false;
+  const size_t scratch =
+      gathers ? conv2d_gather_f32_workspace_floats(direction, p) : 0;
+  if (chunks == 1) return gathers && scratch == 0;
+  return splits && scratch <= workspace_elems &&
          (epilogue == nullptr || !epilogue->filter_prepared);
 }
 
