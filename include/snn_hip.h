@@ -170,6 +170,12 @@ SNN_HIP_API int snn_hip_conv2d_gather_tile(const snn_hip_conv2d_params* params,
                                            int direction, int dtype,
                                            int* pixels, int* features,
                                            int* splits);
+/* The tile of the fp32 kernel that takes its operands apart into binary16 values, for
+ * a forward convolution or input gradient with this tag; where it answers, such a
+ * launch runs there, also one for which the function above has an answer. */
+SNN_HIP_API int snn_hip_conv2d_halves_tile(const snn_hip_conv2d_params* params,
+                                           int direction, int algorithm,
+                                           int* pixels, int* features);
 /* The same for the binary16 kernels that keep pixels in LDS: `form` is, for a
  * forward convolution or input gradient, how a work-group of the row-tile kernel
  * holds its input (1: one tile of all channels, 2: two tiles in turn, 3: one tile

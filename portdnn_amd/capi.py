@@ -120,6 +120,8 @@ SIGNATURES = {
     "snn_hip_kernel_timing_enable": [_I],
     "snn_hip_kernel_timing_read": [ctypes.POINTER(ctypes.c_double),
                                    ctypes.POINTER(ctypes.c_int)],
+    "snn_hip_conv2d_halves_tile": [_P, _I, _I, ctypes.POINTER(_I),
+                                   ctypes.POINTER(_I)],
     "snn_hip_conv2d_gather_tile": [_P, _I, _I, ctypes.POINTER(_I),
                                    ctypes.POINTER(_I), ctypes.POINTER(_I)],
     "snn_hip_conv2d_lds_form_f16": [_P, _I, ctypes.POINTER(_I)],

@@ -2008,6 +2008,38 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p,
   return gather_f32_wanted(direction, p, fused, true);
 }
 
+double conv2d_gemm_f32_shares(int direction, const snn_hip_conv2d_params& p) {
+  if (conv2d_gather_f32_wanted(direction, p, false)) {
+    const GatherPlan& plan = make_plan<float>(direction, p);
+    if (plan.ok)
+      return kTilesF32[plan.tile].split ? plan.n_splits : 0.25 * plan.n_splits;
+  }
+  snn_hip_conv2d_params q = p;
+  if ((direction == SNN_HIP_FORWARD || as_forward_of_dy(p, &q)) &&
+      (conv2d_rowtile_supports(q) || conv2d_rowsplit_supports(q)))
+    return 0.25;
+  // (the launch's own rule; the estimate's is what a split is worth)
+  const Products r = products_of(direction, p);
+  const double tiles = std::ceil(r.pixels / 64) * std::ceil(r.columns / 64);
+  const double chunks = std::ceil(r.reduced / 32);
+  const double splits =
+      tiles < 640 ? std::min(std::ceil(2048 / tiles), std::floor(chunks / 8)) : 1.0;
+  return 0.25 * std::max(1.0, splits);
+}
+
+double conv2d_gemm_f32_us(int direction, const snn_hip_conv2d_params& p) {
+  if (conv2d_gather_f32_wanted(direction, p, false)) {
+    const GatherPlan& plan = make_plan<float>(direction, p);
+    if (plan.ok) return gather_f32_us(plan, plan.from == kPacked, false);
+  }
+  const Products r = products_of(direction, p);
+  snn_hip_conv2d_params q = p;
+  if ((direction == SNN_HIP_FORWARD || as_forward_of_dy(p, &q)) &&
+      (conv2d_rowtile_supports(q) || conv2d_rowsplit_supports(q)))
+    return 6 + r.macs / 55e6;
+  return igemm_f32_us(r);
+}
+
 bool conv2d_gather_tile_f32(int direction, const snn_hip_conv2d_params& p,
                             GatherTile* tile) {
   if (!positive(p) || !conv2d_gather_f32_wanted(direction, p, false))

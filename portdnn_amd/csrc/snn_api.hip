@@ -428,6 +428,8 @@ size_t f16_workspace_halves(const snn_hip_conv2d_params& p, int direction) {
          p.features;
 }
 
+bool halves_wanted(int direction, const snn_hip_conv2d_params& p);
+
 int workspace_size(const snn_hip_conv2d_params& p, int direction,
                    int algorithm, int dtype, size_t* required,
                    size_t* recommended) {
@@ -484,9 +486,13 @@ int workspace_size(const snn_hip_conv2d_params& p, int direction,
   if (!filbk && p.input_format == 0 &&
       (algorithm == SNN_HIP_ALGO_TILED || algorithm == SNN_HIP_ALGO_IM2COL ||
        algorithm == SNN_HIP_ALGO_MATMUL) &&
-      algorithm_supports(p, direction, algorithm) == algorithm)
+      algorithm_supports(p, direction, algorithm) == algorithm) {
     *recommended = std::max(*recommended,
                             conv2d_gather_f32_workspace_floats(direction, p));
+    if (halves_wanted(direction, p))
+      *recommended = std::max(*recommended,
+                              conv2d_halves_f32_workspace_floats(direction, p));
+  }
   return SNN_HIP_OK;
 }
 
@@ -864,6 +870,28 @@ int launch_gemm_path<_Float16>(int direction, const _Float16* input,
   }
   return launch_conv2d_direct<_Float16>(direction, input, filter, output, p, s);
 }
+// Whether a launch behind the Tiled, Im2col or Matmul tag goes to the kernel that
+// takes its operands apart into binary16 values, by the estimates of both.  Of 220 random layers with windows of 3x3 and
+// 5x5 120 run there, in 0.58 of the time in the geometric mean, none slower by more
+// than 6 % (17x27x27 96 -> 256, 5x5: 114 -> 54 us, its gradient 160 -> 77; 64x16x16
+// 256 -> 120, 3x3: 85 -> 40); small ones stay, whose reductions the others share
+// among work-groups (4x10x10 896 -> 192, 3x3: 25 -> 89).  A strided window reads
+// four times the pixels for a tile, and the estimate has missed that by a third.  1x1
+// windows have no taps to take an operand apart for, and 3x3 layers of whole chunks
+// come here behind the Winograd tag, which brings room for the filter.
+bool halves_wanted(int direction, const snn_hip_conv2d_params& p) {
+  if (direction == SNN_HIP_FILTER_BACKPROP || p.input_format != 0 ||
+      p.window_rows * p.window_cols == 1 ||
+      conv2d_winograd_fused_supports(direction, p))
+    return false;
+  const double us = conv2d_halves_f32_us(direction, p, false);
+  if (us < 0) return false;
+  if (const char* const env = SNN_TUNING_ENV("SNN_HIP_HALVES"))
+    return std::atoi(env) != 0;
+  const bool strided = p.stride_rows > 1 || p.stride_cols > 1;
+  return (strided ? 1.3 : 1.0) * us < conv2d_gemm_f32_us(direction, p);
+}
+
 template <>
 int launch_gemm_path<float>(int direction, const float* input,
                             const float* filter, float* output,
@@ -883,6 +911,14 @@ int launch_gemm_path<float>(int direction, const float* input,
         input, filter, output, p, s, workspace, workspace_elems);
     if (rc >= 0) return rc;
   }
+  // (A launch without room for the filter taken apart stays on the kernels that it
+  // had: a temporary costs more host time than most of them take, and a stream that
+  // records a graph gives none.)
+  if (workspace != nullptr && aligned16(workspace) && aligned16(input) &&
+      aligned16(output) && halves_wanted(direction, p) &&
+      workspace_elems >= conv2d_halves_f32_workspace_floats(direction, p))
+    return launch_conv2d_halves_f32(direction, input, filter, output, p,
+                                    workspace, false, false, s, epilogue);
   if (conv2d_gather_f32_wanted(
           direction, p,
           direction == SNN_HIP_FORWARD && epilogue != nullptr &&
@@ -954,6 +990,42 @@ bool winograd_loses(int direction, const snn_hip_conv2d_params& p,
          (epilogue == nullptr || !epilogue->filter_prepared);
 }
 
+// Whether an aligned fused Winograd launch runs on the kernel that takes its operands
+// apart into binary16 values.  By sizes alone (the filter taken apart fits the
+// workspace that every such launch has to bring): a filter is prepared for the
+// kernel that its launches then take.
+// Winograd's units (32 tiles x 32 features) go round 512 work-groups, two to a
+// compute unit; what a chunk of 16 channels takes was fitted to 40 random layers,
+// within 15 % (an odd number of chunks goes to its slower kernel).  28x28x128 at
+// batch 32: 50 -> 37 us with the filter's launch, 14x14x256 50 -> 37, 13x13
+// 512 -> 64 at batch 116 81 -> 63, 80x104 624 -> 224 170 -> 94; 56x56x64 at batch 32
+// is level, 87x87 96 -> 32 at batch 82 155 / 162.
+bool winograd_halves(int direction, const snn_hip_conv2d_params& p) {
+  const double us = conv2d_halves_f32_us(direction, p, true);
+  size_t required = 0, recommended = 0;
+  winograd_workspace(p, direction, 2, 2, 3, 3, &required, &recommended);
+  if (us < 0 || conv2d_halves_f32_workspace_floats(direction, p) > required)
+    return false;
+  if (const char* const env = SNN_TUNING_ENV("SNN_HIP_HALVES"))
+    return std::atoi(env) != 0;
+  const bool backprop = direction == SNN_HIP_INPUT_BACKPROP;
+  const int chunks = (backprop ? p.features : p.channels) / 16;
+  const size_t tiles =
+      static_cast<size_t>(p.batch) *
+      ceil_div(backprop ? p.in_rows : p.out_rows, 2) *
+      ceil_div(backprop ? p.in_cols : p.out_cols, 2);
+  const size_t units = ceil_div(tiles, size_t{32}) *
+                       ((backprop ? p.channels : p.features) / 32);
+  if (units < 128) return false;
+  double rounds = units / 512.0;
+  rounds = rounds <= 0.5 ? 0.6
+           : rounds < 4  ? std::max(1.0, std::ceil(2 * rounds) / 2)
+                         : rounds;
+  const double winograd_us =
+      7 + rounds * (chunks % 2 == 0 ? 1.9 + 2.2 * chunks : 1.5 + 3.3 * chunks);
+  return us < winograd_us;
+}
+
 // Winograd / WinogradLarge: F(2x2,3x3) for forward and input backprop of 3x3
 // stride-1 convolutions and F(3x3,2x2) for their filter gradient; F(2,3)
 // along the window's axis for the 1x3 / 3x1 windows the selector also accepts
@@ -987,6 +1059,10 @@ int launch_winograd_path<float>(int direction, const float* input,
     return launch_gemm_path<float>(direction, input, filter, output, p, s,
                                    prepared ? nullptr : workspace,
                                    prepared ? 0 : workspace_elems, epilogue);
+  if (fused && aligned16(input) && aligned16(output) && aligned16(workspace) &&
+      winograd_halves(direction, p))
+    return launch_conv2d_halves_f32(direction, input, filter, output, p,
+                                    workspace, true, prepared, s, epilogue);
   // (the input gradient's filter transform reads the filter 16 bytes at a time)
   if (fused && aligned16(input) && aligned16(output) && aligned16(workspace) &&
       (direction != SNN_HIP_INPUT_BACKPROP || aligned16(filter)) &&
@@ -1370,6 +1446,10 @@ int snn_hip_conv2d_prepare_filter_f32(int direction, const float* filter,
     return SNN_HIP_INSUFFICIENT_WORKSPACE;
   LaunchOptions options;
   options.prepare_only = true;
+  if (aligned16(workspace) && winograd_halves(direction, p))
+    return launch_conv2d_halves_f32(direction, nullptr, filter, nullptr, p,
+                                    workspace, true, false, as_stream(stream),
+                                    &options);
   return launch_conv2d_winograd_fused_f32(direction, nullptr, filter, nullptr,
                                           p, workspace, workspace_elems,
                                           as_stream(stream), &options);
@@ -1460,6 +1540,27 @@ int snn_hip_conv2d_gather_tile(const snn_hip_conv2d_params* params,
   *pixels = tile.pixels;
   *features = tile.features;
   *splits = tile.splits;
+  return SNN_HIP_OK;
+}
+
+int snn_hip_conv2d_halves_tile(const snn_hip_conv2d_params* params,
+                               int direction, int algorithm, int* pixels,
+                               int* features) {
+  if (params == nullptr || pixels == nullptr || features == nullptr)
+    return SNN_HIP_INVALID_PARAMETER;
+  const snn_hip_conv2d_params& p = *params;
+  const int v = validate(p);
+  if (v != SNN_HIP_OK) return v;
+  const bool winograd = (algorithm == SNN_HIP_ALGO_WINOGRAD ||
+                         algorithm == SNN_HIP_ALGO_WINOGRAD_LARGE) &&
+                        conv2d_winograd_fused_supports(direction, p);
+  if (p.input_format != 0 || p.groups != 1 ||
+      algorithm == SNN_HIP_ALGO_DIRECT ||
+      (direction != SNN_HIP_FORWARD && direction != SNN_HIP_INPUT_BACKPROP) ||
+      algorithm_supports(p, direction, algorithm) != algorithm ||
+      !(winograd ? winograd_halves(direction, p) : halves_wanted(direction, p)))
+    return SNN_HIP_INVALID_ALGORITHM;
+  conv2d_halves_f32_tile(direction, p, winograd, pixels, features);
   return SNN_HIP_OK;
 }
 

@@ -35,6 +35,23 @@ struct LaunchOptions {
   bool wanted() const { return bias != nullptr || relu; }
 };
 
+// fp32 forward convolution and stride-1 input gradient with operands taken apart
+// into two binary16 values (conv2d_halves_f32.hip).  The estimated time, below zero
+// for shapes it does not take; what it needs in front of its launch; `workspace`
+// has that much room and is aligned to 16 bytes; winograd: in place of Winograd's
+// kernels; prepared: a launch with options->prepare_only has left the filter there.
+double conv2d_halves_f32_us(int direction, const snn_hip_conv2d_params& p,
+                            bool winograd);
+size_t conv2d_halves_f32_workspace_floats(int direction,
+                                          const snn_hip_conv2d_params& p);
+void conv2d_halves_f32_tile(int direction, const snn_hip_conv2d_params& p,
+                            bool winograd, int* pixels, int* features);
+int launch_conv2d_halves_f32(int direction, const float* input,
+                             const float* filter, float* output,
+                             const snn_hip_conv2d_params& p, float* workspace,
+                             bool winograd, bool prepared, hipStream_t stream,
+                             const LaunchOptions* options);
+
 // Implicit-GEMM convolution on MFMA (conv2d_igemm.hip): the path behind the
 // Tiled and Im2col algorithm tags.  `supports` tells whether the shape meets
 // the kernel's vector-width requirements; pointers must be 16-byte aligned.
@@ -271,6 +288,15 @@ int launch_conv2d_general_f16(int direction, const _Float16* src,
                               const _Float16* filter, _Float16* dst,
                               const snn_hip_conv2d_params& p,
                               hipStream_t stream);
+
+// Estimated time of a forward or input-gradient launch on the gathering or the
+// implicit-GEMM kernels, whichever it takes.
+double conv2d_gemm_f32_us(int direction, const snn_hip_conv2d_params& p);
+
+// Into how many sums of their own such a launch divides its reductions, counted as a
+// quarter each where the fp32 instruction adds them, whose sums are twice as far from
+// 64 bits as those of operands in parts.
+double conv2d_gemm_f32_shares(int direction, const snn_hip_conv2d_params& p);
 
 // Forward convolution (with bias and activation, if asked for) and input
 // gradient in fp32 on the same gathering kernel: every window, stride, channel

@@ -145,6 +145,20 @@ def gather_tile(p, direction, dtype):
     return pixels.value, features.value, splits.value
 
 
+def halves_tile(p, direction, algorithm):
+    """(pixels, features) of the fp32 kernel whose operands are taken apart into
+    binary16 values, or None where such a launch runs on another kernel
+    (snn_hip_conv2d_halves_tile)."""
+    pixels, features = ctypes.c_int(), ctypes.c_int()
+    code = capi.lib().snn_hip_conv2d_halves_tile(
+        ctypes.byref(p), direction, algorithm, ctypes.byref(pixels),
+        ctypes.byref(features))
+    if code == STATUS.INVALID_ALGORITHM:
+        return None
+    capi.check(code)
+    return pixels.value, features.value
+
+
 def lds_form_f16(p, direction):
     """How a binary16 launch keeps its pixels in LDS, or None where it runs on
     another kernel (snn_hip_conv2d_lds_form_f16)."""

@@ -1,0 +1,215 @@
+"""fp32 convolutions whose operands are taken apart into two binary16 values: every
+tile, ragged pixels, channels and features, strips of columns, windows of 2 to 49
+taps, strides, bias and activation, prepared filters; values that binary16's range
+does not hold beside each other, infinities and NaNs.
+
+Bound: n products added in fp32, as in the other fp32 convolutions.  Taken apart, an
+operand is off by at most 2^-23 of itself and a product by 2^-22 of the two products
+of low parts; both are roundings of single products of either sign, and add
+2^-22 sqrt(n) of the sum's norm at the most.
+"""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from portdnn_amd import capi, ops
+from portdnn_amd.capi import ALGO, DIRECTION, DTYPE
+from test_gpu_conv_f32_shapes import check
+from test_gpu_parity import ORACLE_FN, dev, oracle_params, uniform
+
+pytestmark = pytest.mark.gpu
+
+F, I = DIRECTION.FORWARD, DIRECTION.INPUT_BACKPROP
+TILED, WINO = ALGO.IM2COL, ALGO.WINOGRAD
+# batch, rows, cols, channels, features, window, stride, same; direction; tag; tile
+CASES = [
+    ((8, 30, 29, 160, 132, 3, 1, True), F, TILED, (60, 128)),   # two image rows
+    ((8, 30, 29, 160, 132, 3, 1, True), I, TILED, (60, 128)),   # ragged channels
+    ((9, 41, 43, 100, 64, 3, 1, True), F, WINO, (64, 64)),
+    ((40, 8, 8, 256, 132, 3, 1, True), I, TILED, (64, 64)),     # whole images
+    ((3, 50, 60, 128, 160, 2, 1, True), F, TILED, (120, 64)),   # four taps
+    ((3, 50, 60, 128, 160, 2, 1, True), I, TILED, (40, 128)),   # strips
+    ((9, 41, 43, 100, 68, 4, 1, False), F, TILED, (60, 128)),   # sixteen taps
+    ((1, 80, 104, 112, 224, 3, 1, True), F, WINO, (240, 32)),
+    ((6, 57, 61, 40, 36, 7, 1, True), F, TILED, (93, 64)),      # 49 taps
+    ((4, 27, 27, 96, 256, 5, 1, True), F, TILED, (56, 64)),     # 25 taps
+    ((16, 27, 27, 96, 256, 5, 1, True), F, TILED, (126, 128)),
+    ((40, 33, 31, 64, 64, 3, 1, True), F, WINO, (176, 64)),     # several tiles each
+    ((12, 37, 39, 128, 256, 3, 2, True), F, TILED, (60, 128)),  # stride 2
+]
+IDS = ["x".join(map(str, c[0])) + "fi"[c[1] == I] for c in CASES]
+
+
+def operands(shape, direction, seed):
+    p = ops.conv_params(*shape)
+    rng = np.random.default_rng(seed + shape[1])
+    n_a, n_b, n_out = ops.conv_sizes(p, direction)
+    return p, uniform(rng, n_a), uniform(rng, n_b), n_out
+
+
+def reference(p, direction, a, b):
+    return np.asarray(ORACLE_FN[direction](
+        a, b, oracle_params(p, p.features), acc64=True)).reshape(-1)
+
+
+def products(p, direction):
+    return p.window_rows * p.window_cols * (
+        p.channels if direction == F else p.features)
+
+
+def launch(p, direction, tag, a, b, **kw):
+    _, rec = ops.workspace_size(p, direction, tag, DTYPE.F32)
+    ws = torch.full((rec + 1024,), 7.0, device="cuda")
+    out = ops.conv2d(dev(a), dev(b), p, direction, tag, workspace=ws[:rec], **kw)
+    assert torch.all(ws[rec:] == 7.0)
+    return out
+
+
+@pytest.mark.parametrize("shape,direction,tag,tile", CASES, ids=IDS)
+def test_taken_apart(shape, direction, tag, tile):
+    p, a, b, n_out = operands(shape, direction, 5100)
+    assert ops.halves_tile(p, direction, tag) == tile
+    ref = reference(p, direction, a, b)
+    guard = torch.full((n_out + 1024,), 7.0, device="cuda")
+    got = launch(p, direction, tag, a, b, out=guard[:n_out])
+    check(got, ref, products(p, direction), (shape, direction))
+    assert torch.all(guard[n_out:] == 7.0)
+    # (closer to 64 bits than additions in fp32: 3e-7 and more at these lengths)
+    error = got.cpu().numpy().astype(np.float64).reshape(-1) - ref
+    assert np.linalg.norm(error) <= 4e-7 * np.linalg.norm(ref.astype(np.float64))
+    again = launch(p, direction, tag, a, b)
+    assert torch.equal(again.view(torch.int32).reshape(-1),
+                       got.view(torch.int32).reshape(-1))
+
+
+@pytest.mark.parametrize("tag,shape", [
+    (TILED, (9, 41, 43, 100, 68, 4, 1, False)),
+    (TILED, (16, 27, 27, 96, 256, 5, 1, True)),   # in parts
+    (WINO, (16, 28, 28, 96, 128, 3, 1, True))])
+@pytest.mark.parametrize("relu", [False, True])
+def test_bias_and_relu(tag, shape, relu):
+    p, a, b, _ = operands(shape, F, 5200)
+    assert ops.halves_tile(p, F, tag) is not None
+    bias = uniform(np.random.default_rng(3), p.features)
+    ref = reference(p, F, a, b).reshape(-1, p.features) + bias
+    _, rec = ops.workspace_size(p, F, tag, DTYPE.F32)
+    got = ops.conv2d_bias_act(dev(a), dev(b), dev(bias), p, tag, relu=relu,
+                              workspace=torch.empty(rec, device="cuda"))
+    check(got, np.maximum(ref, 0) if relu else ref, products(p, F) + 1, shape)
+
+
+def compare(p, direction, tag, a, b, tolerance):
+    """The error of every output against the sum of its products' magnitudes."""
+    ref = reference(p, direction, a, b).astype(np.float64)
+    size = reference(p, direction, np.abs(a), np.abs(b)).astype(np.float64)
+    got = launch(p, direction, tag, a, b).cpu().numpy().reshape(-1)
+    error = np.abs(got.astype(np.float64) - ref)
+    # (and half the least fp32 number)
+    assert np.all(error <= tolerance * size + 2.0**-149)
+
+
+# Small: few enough that the reference in 64 bits is quick, but on this kernel.
+SHAPE = (8, 28, 28, 96, 96, 4, 1, True)
+
+
+@pytest.mark.parametrize("direction", [F, I])
+@pytest.mark.parametrize("operand", [0, 1])
+@pytest.mark.parametrize("exponents", [
+    (0, -20), (0, -26), (0, -27), (0, -40), (0, -52), (0, -60), (0, -126),
+    (40, -10), (100, -20), (-100, -126), (-120, -130), (100, 60)])
+def test_values_beside_larger_ones(direction, operand, exponents):
+    """Every other channel has the larger exponent and meets zeros, so that the
+    outputs are sums of the smaller values alone: no bit of them may be missing.
+    A binary16 pair holds 2^26 between them, a second pass 2^52, the fp32
+    instruction the rest."""
+    p, a, b, _ = operands(SHAPE, direction, 5300)
+    assert ops.halves_tile(p, direction, TILED) is not None
+    large, small = exponents
+    depth = p.channels if direction == F else p.features
+    odd = np.arange(depth) % 2 == 1
+    scale = np.where(odd, 2.0**small, 2.0**large)
+    # the reduction's channel is a's last dimension; b is [tap][c][f]
+    va = a.reshape(-1, depth).astype(np.float64)
+    vb = b.reshape(16, p.channels, p.features).astype(np.float64)
+    by = odd[None, :, None] if direction == F else odd[None, None, :]
+    if operand == 0:
+        va, vb = va * scale, np.where(by, vb, 0)
+    else:
+        vb = vb * (scale[None, :, None] if direction == F else scale)
+        va = np.where(odd, va, 0)
+    a, b = va.astype(np.float32).reshape(-1), vb.astype(np.float32).reshape(-1)
+    compare(p, direction, TILED, a, b, 2 * np.sqrt(16 * depth) * 2.0**-24)
+
+
+@pytest.mark.parametrize("direction", [F, I])
+@pytest.mark.parametrize("operand", [0, 1])
+def test_exponents_that_change(direction, operand):
+    """Blocks of channels, images and features of other sizes than their
+    neighbours, zeros among them."""
+    p, a, b, _ = operands(SHAPE, direction, 5400)
+    rng = np.random.default_rng(9)
+    depth = p.channels if direction == F else p.features
+    if operand == 0:
+        v = a.reshape(p.batch, -1, depth)
+        v *= np.exp2(rng.integers(-12, 12, (p.batch, 1, depth // 32, 1)) *
+                     np.ones((1, 1, 1, 32))).reshape(p.batch, 1, depth)
+        v[1, :, :32] = 0
+        v[2] = 0
+    else:
+        v = b.reshape(16, p.channels, p.features)
+        v *= np.exp2(rng.integers(-12, 12, (1, p.channels // 32, 1,
+                                            p.features // 32, 1)) *
+                     np.ones((1, 1, 32, 1, 32))).reshape(1, p.channels, -1)
+        v[:, :32, :32] = 0
+        v[:, 64:] = 0
+    compare(p, direction, TILED, a, b, 2 * np.sqrt(16 * depth) * 2.0**-24)
+
+
+@pytest.mark.parametrize("direction", [F, I])
+@pytest.mark.parametrize("operand", [0, 1])
+@pytest.mark.parametrize("value", [np.inf, np.nan, np.finfo(np.float32).max])
+def test_infinities_stay_with_their_outputs(direction, operand, value):
+    p, a, b, n_out = operands(SHAPE, direction, 5500)
+    # (the largest finite value once: sums of several overflow on the way in fp32)
+    (a, b)[operand][-1] = value
+    if not np.isfinite(value):
+        (a, b)[operand][:1] = value
+        (a, b)[operand][-5:] = value
+    ref = reference(p, direction, a, b)
+    got = launch(p, direction, TILED, a, b).cpu().numpy().reshape(-1)
+    ok = np.isfinite(ref)
+    assert ok.any()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    n = products(p, direction)
+    part = ok & (np.abs(ref) < 1e30)
+    error = np.abs(got[part].astype(np.float64) - ref[part])
+    assert error.max() <= 2 * n * 2.0**-24 * np.abs(ref[part]).max()
+
+
+def test_prepared_filter_without_a_pack():
+    """A prepared launch behind another tag than Winograd packs for itself."""
+    p, a, b, _ = operands(SHAPE, F, 5600)
+    _, rec = ops.workspace_size(p, F, TILED, DTYPE.F32)
+    ws = torch.full((rec,), float("nan"), device="cuda")
+    ops.conv2d_prepare_filter(dev(b), p, F, TILED, ws)
+    got = ops.conv2d_prepared(dev(a), dev(b), p, F, TILED, ws)
+    check(got, reference(p, F, a, b), products(p, F), "prepared")
+
+
+def test_short_workspace_and_bad_arguments():
+    """Without room for the filter such a launch runs on the kernels that need
+    none."""
+    p, a, b, _ = operands(SHAPE, F, 5700)
+    ref = reference(p, F, a, b)
+    for ws in (None, torch.empty(64, device="cuda")):
+        got = ops.conv2d(dev(a), dev(b), p, F, TILED, workspace=ws)
+        check(got, ref, products(p, F), "short workspace")
+    fn = capi.lib().snn_hip_conv2d_halves_tile
+    n = ctypes.c_int()
+    assert fn(None, F, TILED, ctypes.byref(n), ctypes.byref(n)) == \
+        capi.STATUS.INVALID_PARAMETER
+    assert ops.halves_tile(p, DIRECTION.FILTER_BACKPROP, TILED) is None
+    assert ops.halves_tile(p, F, ALGO.DIRECT) is None
