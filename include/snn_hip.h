@@ -176,6 +176,9 @@ SNN_HIP_API int snn_hip_conv2d_gather_tile(const snn_hip_conv2d_params* params,
 SNN_HIP_API int snn_hip_conv2d_halves_tile(const snn_hip_conv2d_params* params,
                                            int direction, int algorithm,
                                            int* pixels, int* features);
+/* The same for the filter gradient: the partial filters that are added up. */
+SNN_HIP_API int snn_hip_conv2d_filter_halves_partials(
+    const snn_hip_conv2d_params* params, int algorithm, int* partials);
 /* The same for the binary16 kernels that keep pixels in LDS: `form` is, for a
  * forward convolution or input gradient, how a work-group of the row-tile kernel
  * holds its input (1: one tile of all channels, 2: two tiles in turn, 3: one tile

@@ -122,6 +122,7 @@ SIGNATURES = {
                                    ctypes.POINTER(ctypes.c_int)],
     "snn_hip_conv2d_halves_tile": [_P, _I, _I, ctypes.POINTER(_I),
                                    ctypes.POINTER(_I)],
+    "snn_hip_conv2d_filter_halves_partials": [_P, _I, ctypes.POINTER(_I)],
     "snn_hip_conv2d_gather_tile": [_P, _I, _I, ctypes.POINTER(_I),
                                    ctypes.POINTER(_I), ctypes.POINTER(_I)],
     "snn_hip_conv2d_lds_form_f16": [_P, _I, ctypes.POINTER(_I)],

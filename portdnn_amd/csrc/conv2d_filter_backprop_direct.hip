@@ -749,6 +749,19 @@ size_t conv2d_filter_backprop_direct_f16_partial_floats(
          p.features;
 }
 
+// Fitted to 88 random layers of 3x3 and 5x5 windows with counts in multiples of 4
+// (half of them within a fiftieth, nine of ten within a quarter).
+double conv2d_filter_backprop_direct_f32_us(const snn_hip_conv2d_params& p) {
+  const Plan plan = make_plan(p);
+  const double dw_bytes = 4.0 * plan.g.taps * p.channels * p.features;
+  return 2.8 + plan.rounds * (plan.g.steps_per_wave * 0.51 + 3.1) +
+         (plan.splits > 1 ? 0.8e-6 * plan.splits * dw_bytes : 0);
+}
+
+double conv2d_filter_backprop_direct_f32_chain(const snn_hip_conv2d_params& p) {
+  return supports(p, true, sizeof(float)) ? 4.0 * make_plan(p).g.steps_per_wave : 0;
+}
+
 // Fitted to 110 random layers of 3x3 and 5x5 windows with counts in multiples of
 // 8 (within a third, most within a tenth).
 double conv2d_filter_backprop_direct_f16_us(const snn_hip_conv2d_params& p) {

@@ -429,6 +429,7 @@ size_t f16_workspace_halves(const snn_hip_conv2d_params& p, int direction) {
 }
 
 bool halves_wanted(int direction, const snn_hip_conv2d_params& p);
+bool filter_halves_wanted(const snn_hip_conv2d_params& p, bool winograd);
 
 int workspace_size(const snn_hip_conv2d_params& p, int direction,
                    int algorithm, int dtype, size_t* required,
@@ -455,6 +456,9 @@ int workspace_size(const snn_hip_conv2d_params& p, int direction,
       } else if (filbk && conv2d_winograd_filter_backprop_supports(p)) {
         *required = conv2d_winograd_filter_backprop_workspace(p);
         *recommended = *required;
+        if (filter_halves_wanted(p, true))
+          *recommended = std::max(
+              *recommended, conv2d_filter_halves_f32_partial_floats(p, true));
       }
       break;
     case SNN_HIP_ALGO_IM2COL:
@@ -474,6 +478,12 @@ int workspace_size(const snn_hip_conv2d_params& p, int direction,
       conv2d_filter_backprop_direct_f32_wanted(p))
     *recommended = std::max(
         *recommended, conv2d_filter_backprop_direct_f32_partial_floats(p));
+  if (filbk &&
+      (algorithm == SNN_HIP_ALGO_TILED || algorithm == SNN_HIP_ALGO_IM2COL) &&
+      algorithm_supports(p, direction, algorithm) == algorithm &&
+      filter_halves_wanted(p, false))
+    *recommended = std::max(*recommended,
+                            conv2d_filter_halves_f32_partial_floats(p, false));
   WidenedFilterGradient widened;
   if (filbk &&
       (algorithm == SNN_HIP_ALGO_TILED || algorithm == SNN_HIP_ALGO_IM2COL ||
@@ -630,6 +640,56 @@ int launch_gemm_path_padded(int direction, const T* input, const T* filter,
   if (err != hipSuccess) return report_hip_error(err, "padded features");
   return SNN_HIP_OK;
 }
+// Filter gradients on the binary16 instruction (conv2d_filter_halves_f32.hip): behind
+// the Winograd tag from 1024 output pixels on, where the default policy names that tag
+// (28x28x128 at batch 32: 37.6 us instead of 56.1, 64x64x256 at batch 8: 132 instead
+// of 195); behind the others in place of the kernel that holds all taps and channels
+// (163x212x24 at batch 7 -> 32: 39 us instead of 150) and of the one for tiles of 64
+// where its estimate is higher (17x27x27 96 -> 256, 5x5: 88 us instead of 180; 9x9x144
+// -> 528 at batch 5, below the line: 18.3 here, 11.1 there).
+bool filter_halves_wanted(const snn_hip_conv2d_params& p, bool winograd) {
+  const double us = conv2d_filter_halves_f32_us(p, winograd);
+  if (us < 0) return false;
+#ifdef SNN_HIP_TUNING
+  if (const char* s = std::getenv("SNN_HIP_FHALVES")) return std::atoi(s) != 0;
+#endif
+  if (p.channels < 16 || p.features < 16) return false;
+  if (winograd)
+    return static_cast<long long>(p.batch) * p.out_rows * p.out_cols >= 1024;
+  return !conv2d_filter_backprop_direct_f32_wanted(p) ||
+         1.05 * us < conv2d_filter_backprop_direct_f32_us(p);
+}
+
+// The filter gradient on the binary16 instruction behind the Tiled / Im2col tags.
+// Without room for the partial filters they go to a stream-ordered temporary, as those
+// of the kernel that the layer had do, so that a launch gives the same bits either
+// way; below zero: it stays on that kernel, where that one takes no temporary and none
+// can be had (a stream that records a graph), or sums through atomics.
+int launch_filter_halves(const float* x, const float* dy, float* dw,
+                         const snn_hip_conv2d_params& p, hipStream_t s,
+                         float* workspace, size_t workspace_elems) {
+  const size_t need = conv2d_filter_halves_f32_partial_floats(p, false);
+  if (need == 0 || (workspace != nullptr && aligned16(workspace) &&
+                    workspace_elems >= need))
+    return launch_conv2d_filter_halves_f32(x, dy, dw, p, false, workspace, s);
+  if (!conv2d_filter_backprop_direct_f32_wanted(p)) return -1;
+  if (conv2d_filter_backprop_direct_f32_partial_floats(p) == 0) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &status) != hipSuccess ||
+        status != hipStreamCaptureStatusNone)
+      return -1;
+  }
+  void* part = nullptr;
+  if (temp_malloc_async(&part, need * sizeof(float), s) != hipSuccess) {
+    (void)hipGetLastError();
+    return -1;
+  }
+  const int rc = launch_conv2d_filter_halves_f32(x, dy, dw, p, false,
+                                                 static_cast<float*>(part), s);
+  temp_free_async(part, s);
+  return rc;
+}
+
 template <>
 int launch_gemm_path<float>(int direction, const float* input,
                             const float* filter, float* output,
@@ -919,6 +979,12 @@ int launch_gemm_path<float>(int direction, const float* input,
       workspace_elems >= conv2d_halves_f32_workspace_floats(direction, p))
     return launch_conv2d_halves_f32(direction, input, filter, output, p,
                                     workspace, false, false, s, epilogue);
+  if (direction == SNN_HIP_FILTER_BACKPROP && aligned16(input) &&
+      aligned16(filter) && aligned16(output) && filter_halves_wanted(p, false)) {
+    const int rc = launch_filter_halves(input, filter, output, p, s, workspace,
+                                        workspace_elems);
+    if (rc >= 0) return rc;
+  }
   if (conv2d_gather_f32_wanted(
           direction, p,
           direction == SNN_HIP_FORWARD && epilogue != nullptr &&
@@ -1084,9 +1150,14 @@ int launch_winograd_path<float>(int direction, const float* input,
         epilogue != nullptr && epilogue->deterministic);
   if (direction == SNN_HIP_FILTER_BACKPROP &&
       conv2d_winograd_filter_backprop_supports(p) && aligned16(input) &&
-      aligned16(filter) && aligned16(output) && aligned16(workspace))
+      aligned16(filter) && aligned16(output) && aligned16(workspace)) {
+    if (filter_halves_wanted(p, true) &&
+        workspace_elems >= conv2d_filter_halves_f32_partial_floats(p, true))
+      return launch_conv2d_filter_halves_f32(input, filter, output, p, true,
+                                             workspace, s);
     return launch_conv2d_winograd_filter_backprop_f32(
         input, filter, output, p, workspace, workspace_elems, s);
+  }
   return launch_gemm_path<float>(direction, input, filter, output, p, s,
                                  nullptr, 0, epilogue);
 }
@@ -1561,6 +1632,23 @@ int snn_hip_conv2d_halves_tile(const snn_hip_conv2d_params* params,
       !(winograd ? winograd_halves(direction, p) : halves_wanted(direction, p)))
     return SNN_HIP_INVALID_ALGORITHM;
   conv2d_halves_f32_tile(direction, p, winograd, pixels, features);
+  return SNN_HIP_OK;
+}
+
+int snn_hip_conv2d_filter_halves_partials(const snn_hip_conv2d_params* params,
+                                        int algorithm, int* partials) {
+  if (params == nullptr || partials == nullptr) return SNN_HIP_INVALID_PARAMETER;
+  const snn_hip_conv2d_params& p = *params;
+  const int v = validate(p);
+  if (v != SNN_HIP_OK) return v;
+  const bool winograd = (algorithm == SNN_HIP_ALGO_WINOGRAD ||
+                         algorithm == SNN_HIP_ALGO_WINOGRAD_LARGE) &&
+                        conv2d_winograd_filter_backprop_supports(p);
+  if (p.input_format != 0 || p.groups != 1 || algorithm == SNN_HIP_ALGO_DIRECT ||
+      algorithm_supports(p, SNN_HIP_FILTER_BACKPROP, algorithm) != algorithm ||
+      !filter_halves_wanted(p, winograd))
+    return SNN_HIP_INVALID_ALGORITHM;
+  *partials = conv2d_filter_halves_f32_partials(p, winograd);
   return SNN_HIP_OK;
 }
 

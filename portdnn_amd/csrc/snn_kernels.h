@@ -52,6 +52,17 @@ int launch_conv2d_halves_f32(int direction, const float* input,
                              bool winograd, bool prepared, hipStream_t stream,
                              const LaunchOptions* options);
 
+// The same for the filter gradient of 3x3 and 5x5 windows at stride 1
+// (conv2d_filter_halves_f32.hip): estimated time (below zero: not for it), the
+// number of partial filters, and the floats of `workspace` that these take.
+double conv2d_filter_halves_f32_us(const snn_hip_conv2d_params& p, bool winograd);
+int conv2d_filter_halves_f32_partials(const snn_hip_conv2d_params& p, bool winograd);
+size_t conv2d_filter_halves_f32_partial_floats(const snn_hip_conv2d_params& p,
+                                               bool winograd);
+int launch_conv2d_filter_halves_f32(const float* x, const float* dy, float* dw,
+                                    const snn_hip_conv2d_params& p, bool winograd,
+                                    float* workspace, hipStream_t stream);
+
 // Implicit-GEMM convolution on MFMA (conv2d_igemm.hip): the path behind the
 // Tiled and Im2col algorithm tags.  `supports` tells whether the shape meets
 // the kernel's vector-width requirements; pointers must be 16-byte aligned.
@@ -189,6 +200,9 @@ size_t conv2d_filter_backprop_direct_f32_partial_floats(
 size_t conv2d_filter_backprop_direct_f16_partial_floats(
     const snn_hip_conv2d_params& p);
 // estimated time of the f16 form with multiples of 4
+double conv2d_filter_backprop_direct_f32_us(const snn_hip_conv2d_params& p);
+// Pixels of a wave's sums; 0 where the kernel does not take the layer.
+double conv2d_filter_backprop_direct_f32_chain(const snn_hip_conv2d_params& p);
 double conv2d_filter_backprop_direct_f16_us(const snn_hip_conv2d_params& p);
 int launch_conv2d_filter_backprop_direct_f32(const float* input,
                                              const float* output_gradient,

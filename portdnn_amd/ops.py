@@ -159,6 +159,19 @@ def halves_tile(p, direction, algorithm):
     return pixels.value, features.value
 
 
+def filter_halves_partials(p, algorithm):
+    """Partial filters of the fp32 filter gradient whose operands are taken apart into
+    binary16 values, or None where such a launch runs on another kernel
+    (snn_hip_conv2d_filter_halves_partials)."""
+    partials = ctypes.c_int()
+    code = capi.lib().snn_hip_conv2d_filter_halves_partials(
+        ctypes.byref(p), algorithm, ctypes.byref(partials))
+    if code == STATUS.INVALID_ALGORITHM:
+        return None
+    capi.check(code)
+    return partials.value
+
+
 def lds_form_f16(p, direction):
     """How a binary16 launch keeps its pixels in LDS, or None where it runs on
     another kernel (snn_hip_conv2d_lds_form_f16)."""
