@@ -609,12 +609,23 @@ bool supports(const snn_hip_conv2d_params& p, bool ragged, size_t elem) {
   if (!ragged && (p.channels % kTile != 0 || p.features % kTile != 0))
     return false;
   const size_t m = static_cast<size_t>(p.batch) * p.out_rows * p.out_cols;
-  if (m < 4 * kWaves * kMinStepsPerWave) return false;
+  // fp32 convolutions of fewer pixels (a wave without one adds nothing): down to one
+  // where the other kernel adds through atomics (7x9x384 -> 192, 3x3, at batch 2: 12.1
+  // us there, 8.9 here), down to 96 where it is a lane per element (12x9x256 -> 242,
+  // 5x5, at batch 2: 464, 21.5; 9x5x700 -> 528, 3x3, at batch 4: 855, 25.9) -- with
+  // fewer that one is slower as well, but its sums in order are a few hundredths
+  // closer to 64 bits.
+  const bool any = ragged && elem == sizeof(float);
+  const size_t least = !any ? 4 * kWaves * kMinStepsPerWave
+                       : p.channels % kTile == 0 && p.features % 4 == 0 ? 1
+                                                                        : 96;
+  if (m < least) return false;
   // every byte offset a lane forms, prefetch past the end included
-  const size_t rows = m + 16 * (kDepthH + 2);
-  if (rows * p.features * elem > kMaxBufferBytes) return false;
-  const size_t in_rows = static_cast<size_t>(p.batch + 1) * p.in_rows *
-                             p.in_cols + 16 * (kDepthH + 2);
+  constexpr size_t kAhead = 16 * (kDepthH + 2);
+  if ((m + kAhead) * p.features * elem > kMaxBufferBytes) return false;
+  const size_t image = static_cast<size_t>(p.out_rows) * p.out_cols;
+  const size_t in_rows =
+      (p.batch + (kAhead + image - 1) / image) * p.in_rows * p.in_cols + kAhead;
   if (in_rows * p.channels * elem > kMaxBufferBytes) return false;
   return static_cast<size_t>(p.window_rows) * p.window_cols * p.channels *
              p.features * sizeof(float) <= kMaxBufferBytes;
