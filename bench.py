@@ -14,7 +14,8 @@ algorithm).  The same JSON line carries
                 peak: `achieved` = algorithmic flops per launch over its
                 average duration, timed with HIP events on the launch stream;
                 `frac_algorithmic` = achieved / peak, `frac` = the part of it
-                the matrix cores really execute (16/36 for Winograd) / peak;
+                the matrix cores really execute (16/36 for Winograd, 3 binary16 ones
+                at their own peak where operands are taken apart) / peak;
                 `traffic` is read from the committed rocprofv3 summary named
                 in `traffic_source`.  The memory-bound half of the metric is
                 there as plain numbers: `hbm_<layer>_gbs` / `_frac` (of the
@@ -88,6 +89,10 @@ def frac(value, peak, executed_share=1.0):
 
 
 WINOGRAD_SHARE = 4.0 / 9.0
+# The kernel that takes fp32 operands apart into two binary16 values each executes
+# three binary16 products per product; a share of the fp32 instruction's time for one.
+PEAK_F16_MFMA_TFLOPS = 2500.0
+HALVES_SHARE = 3 * PEAK_FP32_MFMA_TFLOPS / PEAK_F16_MFMA_TFLOPS
 
 RESNET = [(56, 64), (28, 128), (14, 256), (7, 512)]
 MOBILENET = [(112, 32, 1), (112, 64, 2), (56, 128, 1), (28, 256, 2),
@@ -231,7 +236,16 @@ def main():
     # reports for the same kernel.
     algo_names = {1: "direct", 2: "tiled", 3: "im2col", 4: "winograd",
                   6: "matmul"}
+
+    def kernel_of(w):
+        """The kernel that a layer's launch runs on, and what it really executes."""
+        if ops.halves_tile(w["p"], DIRECTION.FORWARD, w["algo"]) is not None:
+            return "binary16 parts", HALVES_SHARE
+        name = algo_names[w["algo"]]
+        return name, WINOGRAD_SHARE if name == "winograd" else 1.0
+
     per_layer = []
+    k3_executed = 0.0
     k3_flops = k3_kernel_ms = 0.0
     k3_kernels = 0
     executed_flops_per_step = 0.0
@@ -248,20 +262,19 @@ def main():
         per_layer.append({"layer": w["name"], "algorithm": algo_names[w["algo"]],
                           "ms": round(ms, 4), "kernel_ms": round(kernel_ms, 4),
                           "tflops": round(tf, 2),
+                          "kernel": kernel_of(w)[0],
                           "frac_mfma_peak": frac(
-                              tf, PEAK_FP32_MFMA_TFLOPS,
-                              WINOGRAD_SHARE
-                              if algo_names[w["algo"]] == "winograd" else 1.0)})
-        executed_flops_per_step += w["flops"] * (
-            WINOGRAD_SHARE if algo_names[w["algo"]] == "winograd" else 1.0)
+                              tf, PEAK_FP32_MFMA_TFLOPS, kernel_of(w)[1])})
+        executed_flops_per_step += w["flops"] * kernel_of(w)[1]
         if w["name"].startswith("3x3"):
             k3_flops += w["flops"] * kt.kernels
+            k3_executed += w["flops"] * kt.kernels * kernel_of(w)[1]
             k3_kernel_ms += kt.total_ms
             k3_kernels += kt.kernels
     achieved = k3_flops / k3_kernel_ms / 1e9
-    k3_algos = sorted({algo_names[w["algo"]] for w in work
+    k3_algos = sorted({kernel_of(w)[0] for w in work
                        if w["name"].startswith("3x3")})
-    k3_share = WINOGRAD_SHARE if k3_algos == ["winograd"] else 1.0
+    k3_share = k3_executed / k3_flops
     roofline = {
         "bound": "mfma",
         "kernel": "main kernel of the 3x3 s1 forward convolution (%s), the four "
@@ -271,7 +284,8 @@ def main():
         "achieved": round(achieved, 2), "peak": PEAK_FP32_MFMA_TFLOPS,
         "unit": "TFLOP/s",
         # the matrix pipe's own figure: the multiplications really executed
-        # (16/36 of the algorithmic count for Winograd F(2x2,3x3)) over the peak
+        # (16/36 of the algorithmic count for Winograd F(2x2,3x3); three binary16
+        # ones in place of one, at that instruction's peak) over the peak
         "frac": frac(achieved * k3_share, PEAK_FP32_MFMA_TFLOPS),
         # algorithmic flops over the peak; above 1 when the Winograd kernel
         # outruns what the matrix cores could do on the direct algorithm
@@ -279,8 +293,9 @@ def main():
         "achieved_executed": round(achieved * k3_share, 2),
         "avg_kernel_ms": round(k3_kernel_ms / k3_kernels, 5),
         "algorithmic_gflop_per_launch": round(k3_flops / k3_kernels / 1e9, 4),
-        # the whole step (Winograd layers at 16/36 of their flops, the 1x1
-        # GEMM layers at all of them) over the step time
+        # the whole step (Winograd layers at 16/36 of their flops, layers in
+        # binary16 parts at three of those, the 1x1 GEMM layers at all of them)
+        # over the step time
         "step_executed_tflops": round(
             executed_flops_per_step / ms_per_step / 1e9, 2),
         "step_executed_frac": frac(

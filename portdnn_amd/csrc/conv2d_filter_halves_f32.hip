@@ -554,7 +554,8 @@ __global__ void __launch_bounds__(512)
   auto store = [&](int exponent) {
     const int a = max(min(-exponent, 100), -100);
     const float s1 = pow2(a), s2 = pow2(max(min(-exponent - a, 100), -100));
-    float* const to = part + static_cast<size_t>(slice) * taps * g.channels * g.features;
+    float* const to =
+        part + static_cast<size_t>(slice) * taps * g.channels * g.features;
 #pragma unroll
     for (int t = 0; t < TR * TC; ++t)
 #pragma unroll
@@ -676,6 +677,7 @@ struct FilterHalvesPlan {
   Shape shape = kNone;
   FilterHalves g;
   int nx = 0;
+  bool wanted = false;  // against the kernels behind the same tags
   double us = 0;
 };
 
@@ -720,9 +722,9 @@ FilterHalvesPlan compute_plan(const snn_hip_conv2d_params& p, bool winograd) {
   // that of the kernel behind the same tags 0.56e-7 and 1.29e-8 per root of the pixels
   // of one of its waves (27 random layers, normal values, all within a tenth).  The
   // sums are stored in time for it to be no larger; reductions that are too short for
-  // that stay there, and so do those of fewer pixels than that kernel takes (0.6 ... 1.1e-7),
-  // unless one work-group holds all taps and channels (1.3 ... 1.7e-7).  (The Winograd
-  // kernel's is above either: 3.6e-7 at 5000 pixels, 2.0e-7 here.)
+  // that stay there, and so do those of fewer pixels than that kernel takes (0.5 ...
+  // 0.7e-7), unless one work-group holds all taps and channels (1.3 ... 1.7e-7).  (The
+  // Winograd kernel's is above either: 3.6e-7 at 5000 pixels, 2.0e-7 here.)
   const double pixels = static_cast<double>(p.batch) * p.out_rows * p.out_cols;
   const double chain = winograd || !conv2d_filter_backprop_direct_f32_wanted(p)
                            ? 0
@@ -730,8 +732,8 @@ FilterHalvesPlan compute_plan(const snn_hip_conv2d_params& p, bool winograd) {
   const double most_pixels = chain > 0 ? 3.36 * chain - 135 : pixels;
   const bool few_rows = p.channels < 32 && p.window_rows * p.window_cols *
                                                    p.channels <= 192;
-  if (most_pixels < 32 ||
-      (!winograd && !few_rows && !conv2d_filter_backprop_direct_f32_supports(p, true)))
+  if (most_pixels < 32 || (!winograd && !few_rows &&
+                           !conv2d_filter_backprop_direct_f32_supports(p, true)))
     return plan;
   double best = -1;
   FilterHalves chosen = g;
@@ -777,8 +779,8 @@ FilterHalvesPlan compute_plan(const snn_hip_conv2d_params& p, bool winograd) {
           const long least_sums = (per_split + most_tasks - 1) / most_tasks;
           const long per_sum = (per_split + least_sums - 1) / least_sums;
           const long sums = (per_split + per_sum - 1) / per_sum;
-          const long slices = (splits - 1) * sums +
-                              (tasks - (splits - 1) * per_split + per_sum - 1) / per_sum;
+          const long last = tasks - (splits - 1) * per_split;
+          const long slices = (splits - 1) * sums + (last + per_sum - 1) / per_sum;
           if (slices * filter_mb > 256) continue;
           const double rounds =
               std::ceil(static_cast<double>(splits) * n_units / kNumCus);
@@ -807,6 +809,10 @@ FilterHalvesPlan compute_plan(const snn_hip_conv2d_params& p, bool winograd) {
   g.by_bands = divisor(g.bands_per_image);
   plan.shape = five ? k5x5 : k3x3;
   plan.us = best;
+  if (p.channels >= 16 && p.features >= 16)
+    plan.wanted = winograd ? pixels >= 1024
+                           : !conv2d_filter_backprop_direct_f32_wanted(p) ||
+                                 1.05 * best < conv2d_filter_backprop_direct_f32_us(p);
   return plan;
 }
 
@@ -820,9 +826,11 @@ void launch_shape(const float* x, const float* dy, float* part,
                   const FilterHalvesPlan& plan, hipStream_t stream) {
   const FilterHalves& g = plan.g;
   auto kernel = filter_halves_kernel<TR, TC, CB, FB, NX>;
-  constexpr int kXSlots = NX * kLoaders / (8 * CB), kYSlots = kNY * kLoaders / (8 * FB);
-  constexpr size_t kLds = 128 + (kXSlots + kYSlots) * 4 +
-                          2 * (kXSlots * slot_bytes(32 * CB) + kYSlots * slot_bytes(32 * FB));
+  constexpr int kXSlots = NX * kLoaders / (8 * CB);
+  constexpr int kYSlots = kNY * kLoaders / (8 * FB);
+  constexpr size_t kLds =
+      128 + (kXSlots + kYSlots) * 4 +
+      2 * (kXSlots * slot_bytes(32 * CB) + kYSlots * slot_bytes(32 * FB));
   static_assert(kLds <= kMaxLdsBytes, "LDS");
   static const hipError_t attr = hipFuncSetAttribute(
       reinterpret_cast<const void*>(kernel),
@@ -842,17 +850,24 @@ void launch_shape(const float* x, const float* dy, float* part,
 
 }  // namespace
 
-double conv2d_filter_halves_f32_us(const snn_hip_conv2d_params& p, bool winograd) {
-  const FilterHalvesPlan& plan = make_plan(p, winograd);
-  return plan.shape != kNone ? plan.us : -1;
+// Behind the Winograd tag from 1024 output pixels on, where the default policy names
+// that tag (28x28x128 at batch 32: 38 us instead of 56, 64x64x256 at batch 8: 124
+// instead of 195); behind the others in place of the kernel that holds all taps and
+// channels (163x212x24 at batch 7 -> 32: 39 us instead of 150) and of the one for tiles
+// of 64 where its estimate is higher (17x27x27 96 -> 256, 5x5: 88 us instead of 180;
+// 9x9x144 -> 528 at batch 5, below the line: 18.3 here, 11.1 there).
+bool conv2d_filter_halves_f32_wanted(const snn_hip_conv2d_params& p, bool winograd) {
+  return make_plan(p, winograd).wanted;
 }
 
-int conv2d_filter_halves_f32_partials(const snn_hip_conv2d_params& p, bool winograd) {
+int conv2d_filter_halves_f32_partials(const snn_hip_conv2d_params& p,
+                                      bool winograd) {
   const FilterHalvesPlan& plan = make_plan(p, winograd);
   return plan.shape != kNone ? plan.g.n_slices : 0;
 }
 
-size_t conv2d_filter_halves_f32_partial_floats(const snn_hip_conv2d_params& p, bool winograd) {
+size_t conv2d_filter_halves_f32_partial_floats(const snn_hip_conv2d_params& p,
+                                               bool winograd) {
   const FilterHalvesPlan& plan = make_plan(p, winograd);
   if (plan.shape == kNone || plan.g.n_slices == 1) return 0;
   return static_cast<size_t>(plan.g.n_slices) * p.window_rows * p.window_cols *

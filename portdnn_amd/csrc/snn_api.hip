@@ -640,24 +640,9 @@ int launch_gemm_path_padded(int direction, const T* input, const T* filter,
   if (err != hipSuccess) return report_hip_error(err, "padded features");
   return SNN_HIP_OK;
 }
-// Filter gradients on the binary16 instruction (conv2d_filter_halves_f32.hip): behind
-// the Winograd tag from 1024 output pixels on, where the default policy names that tag
-// (28x28x128 at batch 32: 37.6 us instead of 56.1, 64x64x256 at batch 8: 132 instead
-// of 195); behind the others in place of the kernel that holds all taps and channels
-// (163x212x24 at batch 7 -> 32: 39 us instead of 150) and of the one for tiles of 64
-// where its estimate is higher (17x27x27 96 -> 256, 5x5: 88 us instead of 180; 9x9x144
-// -> 528 at batch 5, below the line: 18.3 here, 11.1 there).
 bool filter_halves_wanted(const snn_hip_conv2d_params& p, bool winograd) {
-  const double us = conv2d_filter_halves_f32_us(p, winograd);
-  if (us < 0) return false;
-#ifdef SNN_HIP_TUNING
-  if (const char* s = std::getenv("SNN_HIP_FHALVES")) return std::atoi(s) != 0;
-#endif
-  if (p.channels < 16 || p.features < 16) return false;
-  if (winograd)
-    return static_cast<long long>(p.batch) * p.out_rows * p.out_cols >= 1024;
-  return !conv2d_filter_backprop_direct_f32_wanted(p) ||
-         1.05 * us < conv2d_filter_backprop_direct_f32_us(p);
+  const char* off = SNN_TUNING_ENV("SNN_HIP_FHALVES_OFF");
+  return off == nullptr && conv2d_filter_halves_f32_wanted(p, winograd);
 }
 
 // The filter gradient on the binary16 instruction behind the Tiled / Im2col tags.

@@ -53,10 +53,11 @@ int launch_conv2d_halves_f32(int direction, const float* input,
                              const LaunchOptions* options);
 
 // The same for the filter gradient of 3x3 and 5x5 windows at stride 1
-// (conv2d_filter_halves_f32.hip): estimated time (below zero: not for it), the
+// (conv2d_filter_halves_f32.hip): whether it should have the layer, the
 // number of partial filters, and the floats of `workspace` that these take.
-double conv2d_filter_halves_f32_us(const snn_hip_conv2d_params& p, bool winograd);
-int conv2d_filter_halves_f32_partials(const snn_hip_conv2d_params& p, bool winograd);
+bool conv2d_filter_halves_f32_wanted(const snn_hip_conv2d_params& p, bool winograd);
+int conv2d_filter_halves_f32_partials(const snn_hip_conv2d_params& p,
+                                      bool winograd);
 size_t conv2d_filter_halves_f32_partial_floats(const snn_hip_conv2d_params& p,
                                                bool winograd);
 int launch_conv2d_filter_halves_f32(const float* x, const float* dy, float* dw,
