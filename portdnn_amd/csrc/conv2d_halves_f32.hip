@@ -28,8 +28,9 @@
 // would lose bits: such values are left out of a block's operands, and the block
 // is taken once more with these alone, scaled up by 2^26.  Where that is not enough
 // (values below 2^-52 of the block's largest, exponents that differ by more than
-// 2^30 between blocks, infinities, NaNs in the filter) the tile is summed on the fp32
-// instruction instead, from the same LDS tile.
+// 2^30 between blocks, small values in both operands beside sums whose exponent has
+// to rise so far that they would overflow, infinities, NaNs in the filter) the tile is
+// summed on the fp32 instruction instead, from the same LDS tile.
 //
 //   * A work-group owns a run of output pixels (images, strips of columns, rows and
 //     columns flattened) and up to 128 features.  The input rows the run needs, halo
@@ -82,6 +83,7 @@ struct Halves {
   int n_slots;
   int n_fslices, n_fblocks, n_cblocks;
   int part;        // channel blocks whose sums are taken together
+  int headroom;    // powers of two that sums can be scaled up by
   int transposed;  // w[taps - 1 - tap][feature][channel]
   int relu;
   Divisor by_padded_rows, by_halo_cols, by_strip_cols, by_out_rows, by_strips;
@@ -302,6 +304,7 @@ __global__ void __launch_bounds__(128 * WF * WP)
     int head_fb = 0;
     bool mine = false;            // whether there is one
     bool plain = false;  // a tile's filter, or one of its blocks, cannot be taken apart
+    int spread = 0;      // of the exponents of a tile's filter
     auto load_pieces = [&](int cb) {
       head_now = head[cb * g.n_fblocks + head_fb];
       const unsigned c = static_cast<unsigned>(cb) * (kKC * 4) + piece_at;
@@ -335,7 +338,8 @@ __global__ void __launch_bounds__(128 * WF * WP)
       if (!plain) {
         const unsigned up = wave_max(static_cast<unsigned>(highest + 1024));
         const unsigned down = wave_max(static_cast<unsigned>(1024 - lowest));
-        plain = static_cast<int>(up) + static_cast<int>(down) - 2048 > 30;
+        spread = max(static_cast<int>(up) + static_cast<int>(down) - 2048, 0);
+        plain = spread > 30;
       }
     };
     auto put = [&](int buf, float scale, float scale2048) {
@@ -388,6 +392,8 @@ __global__ void __launch_bounds__(128 * WF * WP)
           stop = true;
         } else {
           int flags = 0;
+          const int small = static_cast<int>(__builtin_amdgcn_ballot_w64(
+              mine && ((head_now >> 16) & kSmall) != 0));
           if (band == 0) {
 #pragma unroll
             for (int k = 0; k < NW; ++k) {
@@ -406,6 +412,10 @@ __global__ void __launch_bounds__(128 * WF * WP)
               flags = loses(r, ex);
               plain |= (flags & kBeyond) != 0 || ex_high - ex_low > 30;
             }
+            // (sums of larger blocks may lie above this block's by both exponents, and
+            // are scaled up for the small values of either operand)
+            plain |= ex - ex_low + spread + ((flags & kSmall) != 0 ? kBand : 0) +
+                         (small != 0 ? kBand : 0) > g.headroom;
           }
           const bool again = band == 0 && (flags & kSmall) != 0;
           const bool last = !again && cb + 1 >= g.n_cblocks;
@@ -416,8 +426,6 @@ __global__ void __launch_bounds__(128 * WF * WP)
           const int by = (first ? 0 : to - acc_exp) + (band != 0 ? kBand : 0);
           const bool rescales =
               __builtin_amdgcn_ballot_w64(mine && by != 0) != 0;
-          const int small = static_cast<int>(__builtin_amdgcn_ballot_w64(
-              mine && ((head_now >> 16) & kSmall) != 0));
           acc_exp = to;
           if (wave == NW) {
             if (lane < kMaxBlocks) {
@@ -1053,6 +1061,10 @@ HalvesPlan compute_plan(int direction, const snn_hip_conv2d_params& p,
   const int taps = g.win_rows * g.win_cols;
   const int parts = parts_wanted(direction, p, g, winograd);
   if (parts == 0) return best;
+  // (n products below 2^15 * 2^15 each, and fp32 ends at 2^128)
+  g.headroom = 97;
+  for (long n = static_cast<long>(taps) * g.channels; n > 1; n = (n + 1) / 2)
+    --g.headroom;
   g.part = ceil_div(g.n_cblocks, parts);
   const int only = tuned(SNN_TUNING_ENV("SNN_HIP_HALVES_FORM"), -1);
   for (int strips = 1; strips <= 8; ++strips) {

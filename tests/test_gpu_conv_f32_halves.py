@@ -167,6 +167,38 @@ def test_exponents_that_change(direction, operand):
     compare(p, direction, TILED, a, b, 2 * np.sqrt(16 * depth) * 2.0**-24)
 
 
+# Three blocks of 32 channels, sixteen and nine taps.
+DROPS = [(F, TILED, (8, 28, 28, 96, 96, 4, 1, True)),
+         (I, TILED, (8, 28, 28, 96, 96, 4, 1, True)),
+         (F, WINO, (16, 28, 28, 96, 128, 3, 1, True)),
+         (I, WINO, (16, 28, 28, 128, 96, 3, 1, True))]
+
+
+@pytest.mark.parametrize("direction,tag,shape", DROPS)
+@pytest.mark.parametrize("drops", [(5, 5), (14, 14), (20, 20), (30, 30),
+                                   (30, 15), (15, 30)])
+def test_sums_that_follow_both_operands_down(direction, tag, shape, drops):
+    """The blocks of channels behind the first are smaller in both operands and hold
+    values too small for their own exponents in both: the first one's sums are scaled
+    up by all four powers of two together."""
+    p, a, b, _ = operands(shape, direction, 5410)
+    assert ops.halves_tile(p, direction, tag) is not None
+    depth = p.channels if direction == F else p.features
+    taps = p.window_rows * p.window_cols
+    block = np.minimum(np.arange(depth) // 32, 1)
+    # (the sums of the first block as large as they can be)
+    va = np.where(block == 0, 0.99, a.reshape(-1, depth)) * np.exp2(-drops[0] * block)
+    va[:, 40] *= 2.0**-28
+    vb = np.moveaxis(b.reshape(taps, p.channels, p.features), 1 if direction == F else 2,
+                     2)
+    vb = np.where(block == 0, 0.99, vb) * np.exp2(-drops[1] * block)
+    vb[..., 50] *= 2.0**-28
+    vb = np.moveaxis(vb, 2, 1 if direction == F else 2)
+    compare(p, direction, tag, va.astype(np.float32).reshape(-1),
+            np.ascontiguousarray(vb, np.float32).reshape(-1),
+            2 * np.sqrt(taps * depth) * 2.0**-24)
+
+
 @pytest.mark.parametrize("direction", [F, I])
 @pytest.mark.parametrize("operand", [0, 1])
 @pytest.mark.parametrize("value", [np.inf, np.nan, np.finfo(np.float32).max])
