@@ -358,7 +358,7 @@ __global__ void __launch_bounds__(128 * WF * WP)
     while (id < n_groups) {
       start_tile();
       bool have = false;  // a block that is not zero has set `ex`
-      bool first = true;  // block of the tile
+      bool empty = true;  // the sums of feature block lane % 4 are zeros
       int ex = 0, ex_low = 0, ex_high = 0, acc_exp = 0;
       int buf = 0, cb = 0, band = 0;
       bool stop = false;
@@ -423,7 +423,8 @@ __global__ void __launch_bounds__(128 * WF * WP)
           // (a feature block per lane)
           const int to = mine && ((head_now >> 16) & kZero) == 0
                              ? ex + static_cast<short>(head_now) : acc_exp;
-          const int by = (first ? 0 : to - acc_exp) + (band != 0 ? kBand : 0);
+          // (zeros keep their value at any exponent, by however much it changes)
+          const int by = (empty ? 0 : to - acc_exp) + (band != 0 ? kBand : 0);
           const bool rescales =
               __builtin_amdgcn_ballot_w64(mine && by != 0) != 0;
           acc_exp = to;
@@ -442,7 +443,8 @@ __global__ void __launch_bounds__(128 * WF * WP)
                                   small * kSmallFilter;
             }
           }
-          first = false;
+          empty &= !(band == 0 && r.big != 0 &&
+                     ((head_now >> 16) & kZero) == 0);
           if (plain) {
             stop = true;
           } else {
@@ -480,7 +482,7 @@ __global__ void __launch_bounds__(128 * WF * WP)
               } else {
                 cb = 0;
                 have = false;
-                first = true;
+                empty = true;
                 acc_exp = 0;
                 id += gridDim.x;
                 now = next;

@@ -199,6 +199,36 @@ def test_sums_that_follow_both_operands_down(direction, tag, shape, drops):
             2 * np.sqrt(taps * depth) * 2.0**-24)
 
 
+@pytest.mark.parametrize("direction,tag,shape", DROPS)
+@pytest.mark.parametrize("zero", ["filter", "pixels"])
+def test_exponents_behind_zeros(direction, tag, shape, zero):
+    """The first block of one operand is zeros, so that the sums are zeros too where
+    their exponent first changes, by up to 2^100 and more: magnitudes on both sides of
+    where that power of two is none of fp32's."""
+    p, a, b, _ = operands(shape, direction, 5420)
+    assert ops.halves_tile(p, direction, tag) is not None
+    depth = p.channels if direction == F else p.features
+    taps = p.window_rows * p.window_cols
+    va = a.reshape(-1, depth)
+    vb = b.reshape(taps, p.channels, p.features)
+    first = (slice(None), slice(0, 32)) if direction == F else \
+        (slice(None), slice(None), slice(0, 32))
+    if zero == "filter":
+        vb[first] = 0
+    else:
+        va[:, :32] = 0
+    for e in range(-54, -46):
+        if zero == "filter":
+            sa, sb = 2.0**-50, np.float64(2.0**e)
+        else:
+            # (the filter falls behind the zeros by what is missing to 2^128)
+            sa, sb = 2.0**-85, np.full(vb.shape, 2.0**(e + 22))
+            sb[first] = 1
+        compare(p, direction, tag, (va * sa).astype(np.float32).reshape(-1),
+                (vb * sb).astype(np.float32).reshape(-1),
+                2 * np.sqrt(taps * depth) * 2.0**-24)
+
+
 @pytest.mark.parametrize("direction", [F, I])
 @pytest.mark.parametrize("operand", [0, 1])
 @pytest.mark.parametrize("value", [np.inf, np.nan, np.finfo(np.float32).max])
