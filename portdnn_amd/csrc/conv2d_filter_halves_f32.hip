@@ -553,7 +553,8 @@ __global__ void __launch_bounds__(512)
   int slice = split * g.sums;
   auto store = [&](int exponent) {
     const int a = max(min(-exponent, 100), -100);
-    const float s1 = pow2(a), s2 = pow2(max(min(-exponent - a, 100), -100));
+    // (in two steps: up to 2^228)
+    const float s1 = pow2(a), s2 = pow2(max(min(-exponent - a, 127), -126));
     float* const to =
         part + static_cast<size_t>(slice) * taps * g.channels * g.features;
 #pragma unroll

@@ -800,7 +800,8 @@ __global__ void __launch_bounds__(128 * WF * WP)
         for (int i = 0; i < FA; ++i) {
           const int by = -__builtin_amdgcn_readfirstlane(
               blocks[buf].acc_exp[(wf * FA + i) / 2]);
-          // (results that are no normal numbers are rounded by a second step)
+          // (in two steps: up to 2^226; what is no normal number is rounded by the
+          // second)
           const float s = pow2(max(min(by, 100), -100));
 #pragma unroll
           for (int j = 0; j < PB; ++j)
@@ -809,7 +810,7 @@ __global__ void __launch_bounds__(128 * WF * WP)
               acc[i][j][v] =
                   __builtin_fmaf(low[i][j][v], 0x1p-11f, acc[i][j][v]) * s;
           if (by > 100 || by < -100) {
-            const float t = pow2(max(min(by - (by > 0 ? 100 : -100), 100), -100));
+            const float t = pow2(max(min(by - (by > 0 ? 100 : -100), 126), -126));
 #pragma unroll
             for (int j = 0; j < PB; ++j) acc[i][j] *= t;
           }

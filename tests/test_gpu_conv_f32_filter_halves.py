@@ -151,6 +151,18 @@ def test_not_finite(value, at):
     assert torch.allclose(got[rest].double(), ref[rest], rtol=1e-4, atol=1e-3)
 
 
+def test_results_beyond_fp32():
+    """Every element is one product of values far below the largest of their task,
+    which are close to fp32's own: it overflows, and the sum is scaled by more than
+    2^200 at the end."""
+    p, x, dy = operands((16, 28, 28, 64, 64, 3, True), 8)
+    x[:], dy[:] = 2.0 ** 76, 0
+    x[..., 0] = 2.0 ** 127
+    dy[0, 13, 13] = 2.0 ** 76
+    dy[0, 13, 13, 0] = 2.0 ** 127
+    assert torch.all(launch(p, WINO, x, dy) == float("inf"))
+
+
 def test_short_workspace():
     """Without room for the partial filters: a temporary behind the Im2col tag, the
     Winograd kernel behind its own."""

@@ -230,6 +230,26 @@ def test_exponents_behind_zeros(direction, tag, shape, zero):
 
 
 @pytest.mark.parametrize("direction", [F, I])
+def test_results_beyond_fp32(direction):
+    """Every output is one product of values far below the largest of their blocks,
+    which are close to fp32's own: it overflows, and the sum is scaled by more than
+    2^200 at the end."""
+    p, a, b, _ = operands(SHAPE, direction, 5430)
+    depth = p.channels if direction == F else p.features
+    va = np.full((a.size // depth, depth), 2.0**127)
+    va[:, 1::2] = 2.0**75
+    # the tap that meets the output's own pixel
+    vb = np.zeros((16, p.channels, p.features))
+    if direction == F:
+        vb[5, 33], vb[5, 33, ::32] = 2.0**75, 2.0**127
+    else:
+        vb[5, :, 33], vb[5, ::32, 33] = 2.0**75, 2.0**127
+    got = launch(p, direction, TILED, va.astype(np.float32).reshape(-1),
+                 vb.astype(np.float32).reshape(-1))
+    assert torch.all(got == float("inf"))
+
+
+@pytest.mark.parametrize("direction", [F, I])
 @pytest.mark.parametrize("operand", [0, 1])
 @pytest.mark.parametrize("value", [np.inf, np.nan, np.finfo(np.float32).max])
 def test_infinities_stay_with_their_outputs(direction, operand, value):
