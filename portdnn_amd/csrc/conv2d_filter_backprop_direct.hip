@@ -303,16 +303,20 @@ __global__ void __launch_bounds__(64 * kWaves)
 
   float4v xa[kDepth], yb[kDepth];
   auto issue = [&](int d) {
+    unsigned vy_now = vy;
     if constexpr (WINDOW) {
       const int iy = px_y * g.stride_rows + tap_y;
       const int ix = px_x * g.stride_cols + tap_x;
       // all ones where the tap falls outside the image (mask arithmetic: a
-      // per-lane condition around the load would become a branch)
-      const unsigned bad =
-          x_dead |
-          (0u - static_cast<unsigned>(
-                    (static_cast<unsigned>(iy) >= static_cast<unsigned>(g.in_rows)) |
-                    (static_cast<unsigned>(ix) >= static_cast<unsigned>(g.in_cols))));
+      // per-lane condition around the load would become a branch).  There is no
+      // such product: both operands are zeros, for an infinite dY times X's
+      // alone is a NaN.
+      const unsigned outside =
+          0u - static_cast<unsigned>(
+                   (static_cast<unsigned>(iy) >= static_cast<unsigned>(g.in_rows)) |
+                   (static_cast<unsigned>(ix) >= static_cast<unsigned>(g.in_cols)));
+      const unsigned bad = x_dead | outside;
+      vy_now = (vy & ~outside) | (kOob & outside);
       const unsigned off =
           static_cast<unsigned>((px_n * g.in_rows + iy) * g.in_cols + ix) * x_row +
           x_col;
@@ -327,7 +331,7 @@ __global__ void __launch_bounds__(64 * kWaves)
       }
     }
     xa[d] = load_four<T, VEC>(x_rsrc, vx, x_dead_e);
-    yb[d] = load_four<T, VEC>(y_rsrc, vy, y_dead_e);
+    yb[d] = load_four<T, VEC>(y_rsrc, vy_now, y_dead_e);
     if constexpr (!WINDOW) vx += x_step;
     vy += y_step;
   };

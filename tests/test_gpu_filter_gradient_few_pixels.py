@@ -47,3 +47,34 @@ def test_few_pixels(shape):
     assert np.all(error <= (pixels + 4) * 2.0 ** -24 * norm)
     again = ops.conv2d(dev(x), dev(dy), p, W, algorithm)
     assert torch.equal(got.view(torch.int32), again.view(torch.int32))
+
+
+@pytest.mark.parametrize("shape", [
+    (1, 8, 12, 37, 53, 3, 1, True),
+    (1, 5, 7, 64, 132, 3, 1, True),
+    (5, 3, 17, 128, 4, 5, 1, True),
+    (2, 9, 9, 36, 52, 3, 2, True),
+    (2, 14, 13, 64, 64, 3, 2, True),    # 98 pixels; and larger layers
+    (4, 14, 14, 64, 128, 5, 2, True),
+])
+@pytest.mark.parametrize("value", [np.inf, -np.inf, np.nan])
+def test_borders_of_not_finite_gradients(shape, value):
+    """A gradient in the corner belongs to the taps that meet the image there, not to
+    those that meet its padding."""
+    p = ops.conv_params(*shape)
+    rng = np.random.default_rng(23 + shape[1])
+    n_x, n_dy, _ = ops.conv_sizes(p, W)
+    x, dy = uniform(rng, n_x), uniform(rng, n_dy)
+    dy[1] = value
+    dy[-2] = value
+    ref = oracle.conv2d_filter_backprop(x, dy, oracle_params(p, p.features),
+                                        acc64=True).reshape(-1)
+    algorithm = ops.default_algorithm(p, W, DTYPE.F32)
+    got = ops.conv2d(dev(x), dev(dy), p, W, algorithm).cpu().numpy().reshape(-1)
+    finite = np.isfinite(ref)
+    assert finite.any() and not finite.all()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    pixels = p.batch * p.out_rows * p.out_cols
+    assert np.all(np.abs(got[finite] - ref[finite]) <=
+                  2 * pixels * 2.0 ** -24 * np.sqrt(pixels))
