@@ -1790,12 +1790,17 @@ bool conv2d_filter_backprop_direct_f32_wanted(const snn_hip_conv2d_params& p,
   // measured faster: 112x112x32 -> 64, 1x1, at batch 32 89.6 us there; with
   // at most eight channels they are so empty that the one-work-group kernel
   // in parts wins -- 11x11x3 -> 96 stride 4 at batch 16: 1000 us here -- but
-  // it sums through atomics, so a reproducible launch stays here)
+  // it sums through atomics, so a reproducible launch stays here, and so do
+  // those of fewer than 256 pixels, which it hardly shares out and whose dY it
+  // multiplies by padding's zeros, infinities included -- 14x14x8 -> 64, 5x5
+  // stride 2, at batch 4: 31.6 us there, 6.8 here)
   const int q = p.window_rows * p.window_cols * p.channels;
+  const bool few_pixels =
+      static_cast<long>(p.batch) * p.out_rows * p.out_cols < 256;
   const bool small_q =
       p.features % 4 == 0 &&
       ((p.channels < 32 && q <= kSmallQMax) ||
-       (!reproducible && p.channels <= kSmallQPartsMaxChannels &&
+       (!reproducible && !few_pixels && p.channels <= kSmallQPartsMaxChannels &&
         q <= kSmallQParts * kSmallQMax));
   if (small_q || !conv2d_filter_backprop_direct_f32_supports(p, true))
     return false;

@@ -54,6 +54,8 @@ def test_few_pixels(shape):
     (1, 5, 7, 64, 132, 3, 1, True),
     (5, 3, 17, 128, 4, 5, 1, True),
     (2, 9, 9, 36, 52, 3, 2, True),
+    (8, 7, 7, 5, 100, 7, 2, True),      # few channels, many taps
+    (8, 7, 7, 5, 98, 7, 2, True),
     (2, 14, 13, 64, 64, 3, 2, True),    # 98 pixels; and larger layers
     (4, 14, 14, 64, 128, 5, 2, True),
 ])
