@@ -287,9 +287,10 @@ SNN_HIP_API int snn_hip_conv2d_deterministic_f32(
  *
  * snn_hip_conv2d_prepare_filter_f32 writes into `workspace` whatever a launch
  * with these parameters, direction and algorithm derives from the filter
- * alone -- today the transformed filter of the fused Winograd forward /
- * input-gradient kernels; for every other path it does nothing and returns
- * SNN_HIP_OK.  snn_hip_conv2d_prepared_f32 is then the same operation as the
+ * alone -- today, for forward convolutions and input gradients behind the
+ * Winograd tags, the fused kernels' transformed filter or the filter as two
+ * binary16 values per weight, whichever kernel the sizes choose; for every other
+ * path it does nothing and returns SNN_HIP_OK.  snn_hip_conv2d_prepared_f32 is then the same operation as the
  * three fp32 entry points, except that it trusts those contents instead of
  * recomputing them: the caller guarantees that `workspace` (same pointer,
  * same size) still holds what a prepare call with the same filter values,

@@ -1197,8 +1197,9 @@ double conv2d_halves_f32_us(int direction, const snn_hip_conv2d_params& p,
 }
 
 size_t conv2d_halves_f32_workspace_floats(int direction,
-                                          const snn_hip_conv2d_params& p) {
-  const HalvesPlan& plan = make_plan(direction, p, false);
+                                          const snn_hip_conv2d_params& p,
+                                          bool winograd) {
+  const HalvesPlan& plan = make_plan(direction, p, winograd);
   return plan.form >= 0 ? plan.workspace_bytes() / 4 : 0;
 }
 

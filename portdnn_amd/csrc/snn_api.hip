@@ -501,7 +501,8 @@ int workspace_size(const snn_hip_conv2d_params& p, int direction,
                             conv2d_gather_f32_workspace_floats(direction, p));
     if (halves_wanted(direction, p))
       *recommended = std::max(*recommended,
-                              conv2d_halves_f32_workspace_floats(direction, p));
+                              conv2d_halves_f32_workspace_floats(direction, p,
+                                                                 false));
   }
   return SNN_HIP_OK;
 }
@@ -961,7 +962,7 @@ int launch_gemm_path<float>(int direction, const float* input,
   // records a graph gives none.)
   if (workspace != nullptr && aligned16(workspace) && aligned16(input) &&
       aligned16(output) && halves_wanted(direction, p) &&
-      workspace_elems >= conv2d_halves_f32_workspace_floats(direction, p))
+      workspace_elems >= conv2d_halves_f32_workspace_floats(direction, p, false))
     return launch_conv2d_halves_f32(direction, input, filter, output, p,
                                     workspace, false, false, s, epilogue);
   if (direction == SNN_HIP_FILTER_BACKPROP && aligned16(input) &&
@@ -1042,9 +1043,10 @@ bool winograd_loses(int direction, const snn_hip_conv2d_params& p,
 }
 
 // Whether an aligned fused Winograd launch runs on the kernel that takes its operands
-// apart into binary16 values.  By sizes alone (the filter taken apart fits the
-// workspace that every such launch has to bring): a filter is prepared for the
-// kernel that its launches then take.
+// apart into binary16 values.  By sizes alone (the filter taken apart fits where
+// Winograd's transformed one lies, 16 C K floats that every such launch has to bring
+// and a prepared one keeps; one of 16 channels, rounded up to 32, does not): a
+// filter is prepared for the kernel that its launches then take.
 // Winograd's units (32 tiles x 32 features) go round 512 work-groups, two to a
 // compute unit; what a chunk of 16 channels takes was fitted to 40 random layers,
 // within 15 % (an odd number of chunks goes to its slower kernel).  28x28x128 at
@@ -1053,9 +1055,8 @@ bool winograd_loses(int direction, const snn_hip_conv2d_params& p,
 // is level, 87x87 96 -> 32 at batch 82 155 / 162.
 bool winograd_halves(int direction, const snn_hip_conv2d_params& p) {
   const double us = conv2d_halves_f32_us(direction, p, true);
-  size_t required = 0, recommended = 0;
-  winograd_workspace(p, direction, 2, 2, 3, 3, &required, &recommended);
-  if (us < 0 || conv2d_halves_f32_workspace_floats(direction, p) > required)
+  if (us < 0 || conv2d_halves_f32_workspace_floats(direction, p, true) >
+                    size_t{16} * p.channels * p.features)
     return false;
   if (const char* const env = SNN_TUNING_ENV("SNN_HIP_HALVES"))
     return std::atoi(env) != 0;

@@ -43,7 +43,8 @@ struct LaunchOptions {
 double conv2d_halves_f32_us(int direction, const snn_hip_conv2d_params& p,
                             bool winograd);
 size_t conv2d_halves_f32_workspace_floats(int direction,
-                                          const snn_hip_conv2d_params& p);
+                                          const snn_hip_conv2d_params& p,
+                                          bool winograd);
 void conv2d_halves_f32_tile(int direction, const snn_hip_conv2d_params& p,
                             bool winograd, int* pixels, int* features);
 int launch_conv2d_halves_f32(int direction, const float* input,

@@ -107,3 +107,30 @@ def test_prepared_workspace_is_only_read(shape, direction):
         two = ops.conv2d_prepared(da, db, p, direction, ALGO.WINOGRAD, ws)
         one = ops.conv2d(da, db, p, direction, ALGO.WINOGRAD, workspace=ws)
         assert torch.equal(one.view(torch.int32), two.view(torch.int32))
+
+
+@pytest.mark.parametrize("shape,direction", [
+    ((32, 36, 9, 16, 640), DIRECTION.FORWARD),
+    ((32, 23, 77, 16, 128), DIRECTION.FORWARD),
+    ((32, 9, 54, 16, 768), DIRECTION.INPUT_BACKPROP),
+    ((16, 28, 28, 32, 128), DIRECTION.INPUT_BACKPROP),
+    ((12, 33, 31, 48, 96), DIRECTION.FORWARD)],
+    ids=lambda s: "x".join(map(str, s)) if isinstance(s, tuple) else str(s))
+def test_prepared_filter_takes_sixteen_values(shape, direction):
+    """A prepared launch reads the first 16 * C * K elements of its workspace and no
+    others; whatever the filter was turned to fits there."""
+    batch, rows, cols, channels, features = shape
+    p = ops.conv_params(batch, rows, cols, *(
+        (channels, features) if direction == DIRECTION.FORWARD else
+        (features, channels)), 3, 1, True)
+    rng = np.random.default_rng(8300 + rows)
+    n_a, n_b, _ = ops.conv_sizes(p, direction)
+    a, b = uniform(rng, n_a), uniform(rng, n_b)
+    ref = np.asarray(ORACLE_FN[direction](
+        a, b, oracle_params(p, p.features), acc64=True)).reshape(-1)
+    _, rec = ops.workspace_size(p, direction, ALGO.WINOGRAD)
+    ws = torch.empty(rec, device="cuda")
+    ops.conv2d_prepare_filter(dev(b), p, direction, ALGO.WINOGRAD, ws)
+    ws[16 * channels * features:] = float("nan")
+    got = ops.conv2d_prepared(dev(a), dev(b), p, direction, ALGO.WINOGRAD, ws)
+    assert_close(got.cpu().numpy(), ref, (shape, direction))
