@@ -817,13 +817,26 @@ __global__ void __launch_bounds__(128 * WF * WP)
         }
         buf ^= 1;
       } else {
-        // The fp32 instruction sums.
+        // The fp32 instruction sums, a block's channels of one tap at a time (in `low`):
+        // what it makes of an infinity or NaN in the filter and the zeros of padding is
+        // left out, there are no such products.
         restart = true;
         clear();
+        int row0[PB], col0[PB];  // of the first tap's pixel
+#pragma unroll
+        for (int j = 0; j < PB; ++j) {
+          const Place place = place_of(j);
+          row0[j] = place.y * g.step_rows - g.pad_rows;
+          col0[j] = place.x * g.step_cols - g.pad_cols;
+        }
         for (int cb = 0; cb < g.n_cblocks; ++cb) {
           __syncthreads();
           at = col = 0;
-          for (int tap = 0; tap < taps; ++tap) {
+          for (int tap = 0, row = 0; tap < taps; ++tap) {
+#pragma unroll
+            for (int i = 0; i < FA; ++i)
+#pragma unroll
+              for (int j = 0; j < PB; ++j) low[i][j] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
               float4v y[PB];
@@ -841,53 +854,27 @@ __global__ void __launch_bounds__(128 * WF * WP)
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
                   for (int j = 0; j < PB; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                        x[e], y[j][e], acc[i][j], 0, 0, 0);
+                    low[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                        x[e], y[j][e], low[i][j], 0, 0, 0);
               }
             }
+#pragma unroll
+            for (int j = 0; j < PB; ++j) {
+              const bool there =
+                  static_cast<unsigned>(row0[j] + row) <
+                      static_cast<unsigned>(g.in_rows) &&
+                  static_cast<unsigned>(col0[j] + col) <
+                      static_cast<unsigned>(g.in_cols);
+#pragma unroll
+              for (int i = 0; i < FA; ++i)
+#pragma unroll
+                for (int v = 0; v < 4; ++v)
+                  acc[i][j][v] += there ? low[i][j][v] : 0.f;
+            }
             next_tap();
+            row += col == 0 ? 1 : 0;
           }
           __syncthreads();
-        }
-        // A sum that is a NaN and holds products of padding pixels: the taps that
-        // exist, one by one.
-#pragma unroll
-        for (int j = 0; j < PB; ++j) {
-          const Place place = place_of(j);
-          const int iy = place.y * g.step_rows - g.pad_rows;
-          const int ix = place.x * g.step_cols - g.pad_cols;
-          if (place.n < 0 ||
-              (iy >= 0 && iy + g.win_rows <= g.in_rows && ix >= 0 &&
-               ix + g.win_cols <= g.in_cols))
-            continue;
-#pragma nounroll
-          for (int u = 0; u < 4 * FA; ++u) {
-            float value = 0.f;
-#pragma unroll
-            for (int t = 0; t < 4 * FA; ++t)
-              value = t == u ? acc[t / 4][j][t % 4] : value;
-            const int f = (fb0 + u / 4) * 16 + 4 * q + u % 4;
-            if (value == value || f >= g.features) continue;
-            float sum = 0.f;
-            for (int tap = 0; tap < taps; ++tap) {
-              const int y = iy + tap / g.win_cols, x = ix + tap % g.win_cols;
-              if (y < 0 || y >= g.in_rows || x < 0 || x >= g.in_cols) continue;
-              const float* const from =
-                  src + (static_cast<size_t>(place.n * g.in_rows + y) * g.in_cols +
-                         x) * g.channels;
-              const float* const by =
-                  g.transposed != 0
-                      ? w + (static_cast<size_t>(taps - 1 - tap) * g.features + f) *
-                                g.channels
-                      : w + static_cast<size_t>(tap) * g.channels * g.features + f;
-              const size_t stride = g.transposed != 0 ? 1 : g.features;
-              for (int c = 0; c < g.channels && sum == sum; ++c)
-                sum += from[c] * by[c * stride];
-            }
-#pragma unroll
-            for (int t = 0; t < 4 * FA; ++t)
-              acc[t / 4][j][t % 4] = t == u ? sum : acc[t / 4][j][t % 4];
-          }
         }
         start_filter(a_slice_next);
       }

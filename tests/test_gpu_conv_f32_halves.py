@@ -271,6 +271,32 @@ def test_infinities_stay_with_their_outputs(direction, operand, value):
     assert error.max() <= 2 * n * 2.0**-24 * np.abs(ref[part]).max()
 
 
+@pytest.mark.parametrize("direction,tag,shape", DROPS + [
+    (F, TILED, (12, 37, 39, 128, 256, 3, 2, True)),     # stride 2
+    (F, TILED, (6, 57, 61, 40, 36, 7, 1, True))])       # most windows at a border
+@pytest.mark.parametrize("operand", [0, 1])
+def test_many_infinities(direction, tag, shape, operand):
+    """So many that every tile holds some; outputs whose windows lie partly in the
+    padding are sums of the products that exist."""
+    p, a, b, _ = operands(shape, direction, 5510)
+    assert ops.halves_tile(p, direction, tag) is not None
+    if operand == 0:
+        a[::997] = np.inf
+    else:
+        # in the corner taps, of a few features' filters
+        v = b.reshape(-1, p.channels, p.features)
+        v[0, 3, ::9], v[-1, 1, ::7] = np.inf, np.nan
+    ref = reference(p, direction, a, b)
+    got = launch(p, direction, tag, a, b).cpu().numpy().reshape(-1)
+    finite = np.isfinite(ref)
+    assert finite.any() and not finite.all()
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert np.array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    n = products(p, direction)
+    error = np.abs(got[finite].astype(np.float64) - ref[finite])
+    assert error.max() <= 2 * np.sqrt(n) * n * 2.0**-24
+
+
 def test_prepared_filter_without_a_pack():
     """A prepared launch behind another tag than Winograd packs for itself."""
     p, a, b, _ = operands(SHAPE, F, 5600)
