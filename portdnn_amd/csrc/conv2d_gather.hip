@@ -2008,6 +2008,26 @@ bool conv2d_gather_f32_wanted(int direction, const snn_hip_conv2d_params& p,
   return gather_f32_wanted(direction, p, fused, true);
 }
 
+namespace {
+
+// Into how many a launch of the implicit-GEMM kernel divides its reductions.
+double igemm_splits(const Products& r) {
+  const double tiles = std::ceil(r.pixels / 64) * std::ceil(r.columns / 64);
+  const double chunks = std::ceil(r.reduced / 32);
+  return tiles < 640 ? std::max(1.0, std::min(std::ceil(2048 / tiles),
+                                              std::floor(chunks / 8)))
+                     : 1.0;
+}
+
+// Whether an input gradient that is not for the kernels before it multiplies dY by the
+// whole filter per output pixel and folds the taps (the launch's own rule).
+bool folds_taps(int direction, const snn_hip_conv2d_params& p) {
+  return direction == SNN_HIP_INPUT_BACKPROP && p.channels < 16 &&
+         p.features % 32 == 0 && !conv2d_stem_input_backprop_supports(p);
+}
+
+}  // namespace
+
 double conv2d_gemm_f32_shares(int direction, const snn_hip_conv2d_params& p) {
   if (conv2d_gather_f32_wanted(direction, p, false)) {
     const GatherPlan& plan = make_plan<float>(direction, p);
@@ -2018,13 +2038,8 @@ double conv2d_gemm_f32_shares(int direction, const snn_hip_conv2d_params& p) {
   if ((direction == SNN_HIP_FORWARD || as_forward_of_dy(p, &q)) &&
       (conv2d_rowtile_supports(q) || conv2d_rowsplit_supports(q)))
     return 0.25;
-  // (the launch's own rule; the estimate's is what a split is worth)
-  const Products r = products_of(direction, p);
-  const double tiles = std::ceil(r.pixels / 64) * std::ceil(r.columns / 64);
-  const double chunks = std::ceil(r.reduced / 32);
-  const double splits =
-      tiles < 640 ? std::min(std::ceil(2048 / tiles), std::floor(chunks / 8)) : 1.0;
-  return 0.25 * std::max(1.0, splits);
+  if (folds_taps(direction, p)) return 0.25 * p.window_rows * p.window_cols;
+  return 0.25 * igemm_splits(products_of(direction, p));
 }
 
 double conv2d_gemm_f32_us(int direction, const snn_hip_conv2d_params& p) {
@@ -2037,7 +2052,29 @@ double conv2d_gemm_f32_us(int direction, const snn_hip_conv2d_params& p) {
   if ((direction == SNN_HIP_FORWARD || as_forward_of_dy(p, &q)) &&
       (conv2d_rowtile_supports(q) || conv2d_rowsplit_supports(q)))
     return 6 + r.macs / 55e6;
-  return igemm_f32_us(r);
+  // Both fitted to random layers with windows of 2x2 to 9x9, by the tiles, chunks and
+  // splits of the launch: nine of ten within a tenth (412 layers), within a sixth
+  // (237 layers of 4 to 12 channels).
+  const auto tiles_of = [](double pixels, double columns) {
+    return std::ceil(pixels / 64) * std::ceil(columns / 64);
+  };
+  if (folds_taps(direction, p)) {
+    const double taps = static_cast<double>(p.window_rows) * p.window_cols;
+    const double pixels = static_cast<double>(p.batch) * p.out_rows * p.out_cols;
+    const double columns = taps * p.channels, chunks = p.features / 32;
+    const double tiles = tiles_of(pixels, columns);
+    // (products beyond what the cache between them and the fold holds)
+    const double beyond = std::max(0.0, pixels * columns - double(1 << 24));
+    return 9.7 + 0.4 * tiles * chunks / kNumCus +
+           0.4 * chunks * std::ceil(tiles / 1024) + 0.22 * taps +
+           1.5e-6 * r.pixels * columns + 0.7e-6 * beyond;
+  }
+  const double tiles = tiles_of(r.pixels, r.columns);
+  const double chunks = std::ceil(r.reduced / 32), splits = igemm_splits(r);
+  return 3.8 + 0.5 * tiles * chunks / kNumCus +
+         0.29 * std::ceil(chunks / splits) * std::ceil(tiles * splits / 1024) +
+         (splits > 1 ? 4.3 : 0.0) +
+         0.75e-6 * r.pixels * r.columns * (splits > 1 ? 2 : 1);
 }
 
 bool conv2d_gather_tile_f32(int direction, const snn_hip_conv2d_params& p,

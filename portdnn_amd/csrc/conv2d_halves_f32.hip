@@ -1115,7 +1115,9 @@ HalvesPlan compute_plan(int direction, const snn_hip_conv2d_params& p,
                 f.features() * 4 / 14.5;
         double rounds = static_cast<double>(groups) / kNumCus;
         rounds = rounds < 4 ? std::ceil(rounds) : rounds + 0.5;
+        // (the launch that takes the filter apart holds 32 taps in registers)
         const double us = 7.9 + 3.5e-3 * taps * g.n_fblocks * g.n_cblocks +
+                          0.17 * std::max(0, taps - 25) +
                           rounds * tile_cycles / 2100;
         if (best.form >= 0 && us >= best.us) continue;
         best.form = form;

@@ -917,14 +917,17 @@ int launch_gemm_path<_Float16>(int direction, const _Float16* input,
   return launch_conv2d_direct<_Float16>(direction, input, filter, output, p, s);
 }
 // Whether a launch behind the Tiled, Im2col or Matmul tag goes to the kernel that
-// takes its operands apart into binary16 values, by the estimates of both.  Of 220 random layers with windows of 3x3 and
-// 5x5 120 run there, in 0.58 of the time in the geometric mean, none slower by more
-// than 6 % (17x27x27 96 -> 256, 5x5: 114 -> 54 us, its gradient 160 -> 77; 64x16x16
-// 256 -> 120, 3x3: 85 -> 40); small ones stay, whose reductions the others share
-// among work-groups (4x10x10 896 -> 192, 3x3: 25 -> 89).  A strided window reads
-// four times the pixels for a tile, and the estimate has missed that by a third.  1x1
-// windows have no taps to take an operand apart for, and 3x3 layers of whole chunks
-// come here behind the Winograd tag, which brings room for the filter.
+// takes its operands apart into binary16 values, by the estimates of both.  Of 1700
+// random layers with windows of 2x2 to 9x9 and 4 to 900 channels 335 run there, in
+// 0.61 of the time in the geometric mean, nine of them slower by more than 3 %, one by
+// 15 (17x27x27 96 -> 256, 5x5: 113 -> 62 us, its gradient 159 -> 76; 64x16x16
+// 256 -> 120, 3x3: 84 -> 35); small ones stay, whose reductions the others share
+// among work-groups (4x10x10 896 -> 192, 3x3: 23 -> 89), and gradients of a few
+// channels, whose taps are multiplied at once and folded (60x10x10 4 <- 544, 5x5:
+// 29 -> 103).  A strided window reads four times the pixels for a tile, which the
+// estimate meets less well.  1x1 windows have no taps to take an operand apart for,
+// and 3x3 layers of whole chunks come here behind the Winograd tag, which brings room
+// for the filter.
 bool halves_wanted(int direction, const snn_hip_conv2d_params& p) {
   if (direction == SNN_HIP_FILTER_BACKPROP || p.input_format != 0 ||
       p.window_rows * p.window_cols == 1 ||
@@ -935,7 +938,7 @@ bool halves_wanted(int direction, const snn_hip_conv2d_params& p) {
   if (const char* const env = SNN_TUNING_ENV("SNN_HIP_HALVES"))
     return std::atoi(env) != 0;
   const bool strided = p.stride_rows > 1 || p.stride_cols > 1;
-  return (strided ? 1.3 : 1.0) * us < conv2d_gemm_f32_us(direction, p);
+  return (strided ? 1.1 : 1.0) * us < conv2d_gemm_f32_us(direction, p);
 }
 
 template <>

@@ -11,7 +11,7 @@ import torch
 
 from golden_cases import GOLDEN_DIR
 from portdnn_amd import capi, ops
-from portdnn_amd.capi import ALGO, DIRECTION, STATUS
+from portdnn_amd.capi import ALGO, DIRECTION, DTYPE, STATUS
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 FAKE = ctypes.c_void_p(0x1000)  # never dereferenced: every call returns early
@@ -439,3 +439,20 @@ def test_lds_form_refuses_bad_arguments():
     p.batch = 0
     assert fn(ctypes.byref(p), DIRECTION.FORWARD, ref) == \
         STATUS.INVALID_PARAMETER
+
+
+@pytest.mark.parametrize("shape", [
+    # gradients of a few channels, whose taps are multiplied at once and folded
+    (60, 10, 10, 4, 544, 5, 1, True),
+    (9, 62, 46, 4, 480, 9, 1, True),
+    (104, 35, 35, 4, 480, 5, 1, False),
+    (35, 44, 44, 4, 800, 3, 1, False),
+    (1, 113, 146, 8, 320, 7, 1, False),
+    (19, 45, 13, 4, 736, 4, 1, True),
+])
+def test_gradients_of_few_channels_stay(shape):
+    """Those are several times as fast on the kernel that they had."""
+    p = ops.conv_params(*shape)
+    direction = DIRECTION.INPUT_BACKPROP
+    algorithm = ops.default_algorithm(p, direction, DTYPE.F32)
+    assert ops.halves_tile(p, direction, algorithm) is None
