@@ -25,6 +25,8 @@
 //
 // The multiplications done on the matrix cores are 16/36 of the direct
 // algorithm's.
+#include <algorithm>
+#include <cmath>
 #include <cstdlib>
 
 #include "gemm_tile.h"
@@ -837,6 +839,77 @@ bool conv2d_winograd_fused_supports(int direction,
          biggest * sizeof(float) <= kMaxBufferBytes;
 }
 
+namespace {
+
+// Each XCD has its own L2: with the XCDs arranged xcd_m x xcd_f over (tile
+// blocks, feature blocks), U is fetched from memory xcd_m times and the
+// input xcd_f times.  Take the arrangement with the least traffic that
+// still gives every XCD work.
+UnitGrid unit_grid(int n_tiles, int out_ch, size_t u_elems, size_t in_elems) {
+  UnitGrid ug;
+  ug.n_mblocks = ceil_div(n_tiles, kTiles);
+  ug.n_fblocks = out_ch / kFeat;
+  ug.xcd_m = 8;
+  ug.xcd_f = 1;
+  double best = -1.0;
+  for (int xf = 1; xf <= 8; xf *= 2) {
+    const int xm = 8 / xf;
+    if (xf > ug.n_fblocks || (xm > ug.n_mblocks && xm > 1)) continue;
+    const double traffic = static_cast<double>(u_elems) * xm +
+                           static_cast<double>(in_elems) * xf;
+    if (best < 0.0 || traffic < best) {
+      best = traffic;
+      ug.xcd_m = xm;
+      ug.xcd_f = xf;
+    }
+  }
+  if (const char* tune = SNN_TUNING_ENV("SNN_HIP_WINO_XCDF")) {
+    const int xf = std::atoi(tune);
+    if (xf == 1 || xf == 2 || xf == 4 || xf == 8) {
+      ug.xcd_f = xf;
+      ug.xcd_m = 8 / xf;
+    }
+  }
+  return ug;
+}
+
+// Units with those that fill the XCDs up to the one that has the most.
+unsigned groups_of(const UnitGrid& ug) {
+  return 8u * static_cast<unsigned>(ceil_div(ug.n_mblocks, ug.xcd_m)) *
+         static_cast<unsigned>(ceil_div(ug.n_fblocks, ug.xcd_f));
+}
+
+}  // namespace
+
+// Estimated time of a launch: the work-groups go round 512 places, two to a compute
+// unit, and half a round takes 0.6 of one; what a chunk of 16 channels takes in each,
+// and the filter's transform where it is large.  An odd number of chunks goes to a
+// kernel with a work-group of its own per unit, which is slower by the chunk but meets
+// its last round better.  Fitted to 700 random layers of 128 units and more: nine of
+// ten within a twelfth.
+double conv2d_winograd_fused_us(int direction, const snn_hip_conv2d_params& p) {
+  const bool backprop = direction == SNN_HIP_INPUT_BACKPROP;
+  const int in_ch = backprop ? p.features : p.channels;
+  const int out_ch = backprop ? p.channels : p.features;
+  const size_t in_pixels =
+      static_cast<size_t>(p.batch) * (backprop ? p.out_rows : p.in_rows) *
+      (backprop ? p.out_cols : p.in_cols);
+  const int tiles = p.batch * ceil_div(backprop ? p.in_rows : p.out_rows, 2) *
+                    ceil_div(backprop ? p.in_cols : p.out_cols, 2);
+  const double filter = static_cast<double>(in_ch) * out_ch;
+  const double most = groups_of(unit_grid(tiles, out_ch,
+                                          size_t{16} * in_ch * out_ch,
+                                          in_pixels * in_ch)) / 512.0;
+  double rounds = most <= 0.5 ? 0.6
+                  : most < 4  ? std::max(1.0, std::ceil(2 * most) / 2)
+                              : most;
+  const int chunks = in_ch / kChunk;
+  const bool odd = chunks % 2 != 0;
+  if (odd) rounds *= most <= 1 ? 0.82 : most <= 2 ? 0.9 : most < 4 ? 0.94 : 1.0;
+  return 7 + 2e-5 * std::max(0.0, filter - 2e4) +
+         rounds * (odd ? 1.5 + 3.3 * chunks : 1.9 + 2.2 * chunks);
+}
+
 int launch_conv2d_winograd_fused_f32(int direction, const float* input,
                                      const float* filter, float* output,
                                      const snn_hip_conv2d_params& p,
@@ -872,40 +945,9 @@ int launch_conv2d_winograd_fused_f32(int direction, const float* input,
   const size_t out_elems = static_cast<size_t>(p.batch) * g.out_rows *
                            g.out_cols * g.out_ch;
 
-  UnitGrid ug;
-  ug.n_mblocks = ceil_div(g.n_tiles, kTiles);
-  ug.n_fblocks = g.out_ch / kFeat;
+  const UnitGrid ug = unit_grid(g.n_tiles, g.out_ch, u_elems, in_elems);
   const unsigned n_units = static_cast<unsigned>(ug.n_mblocks) * ug.n_fblocks;
-  // Each XCD has its own L2: with the XCDs arranged xcd_m x xcd_f over (tile
-  // blocks, feature blocks), U is fetched from memory xcd_m times and the
-  // input xcd_f times.  Take the arrangement with the least traffic that
-  // still gives every XCD work.
-  ug.xcd_m = 8;
-  ug.xcd_f = 1;
-  {
-    double best = -1.0;
-    for (int xf = 1; xf <= 8; xf *= 2) {
-      const int xm = 8 / xf;
-      if (xf > ug.n_fblocks || (xm > ug.n_mblocks && xm > 1)) continue;
-      const double traffic = static_cast<double>(u_elems) * xm +
-                             static_cast<double>(in_elems) * xf;
-      if (best < 0.0 || traffic < best) {
-        best = traffic;
-        ug.xcd_m = xm;
-        ug.xcd_f = xf;
-      }
-    }
-  }
-  if (const char* tune = SNN_TUNING_ENV("SNN_HIP_WINO_XCDF")) {
-    const int xf = std::atoi(tune);
-    if (xf == 1 || xf == 2 || xf == 4 || xf == 8) {
-      ug.xcd_f = xf;
-      ug.xcd_m = 8 / xf;
-    }
-  }
-  const unsigned grid_x =
-      8u * static_cast<unsigned>(ceil_div(ug.n_mblocks, ug.xcd_m)) *
-      static_cast<unsigned>(ceil_div(ug.n_fblocks, ug.xcd_f));
+  const unsigned grid_x = groups_of(ug);
   const int n_chunks = g.in_ch / kChunk;
   // Splitting the channel range across work-groups costs a zero fill and
   // float atomics on every output (measured: slower than leaving CUs idle as

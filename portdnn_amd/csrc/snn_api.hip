@@ -1050,12 +1050,11 @@ bool winograd_loses(int direction, const snn_hip_conv2d_params& p,
 // Winograd's transformed one lies, 16 C K floats that every such launch has to bring
 // and a prepared one keeps; one of 16 channels, rounded up to 32, does not): a
 // filter is prepared for the kernel that its launches then take.
-// Winograd's units (32 tiles x 32 features) go round 512 work-groups, two to a
-// compute unit; what a chunk of 16 channels takes was fitted to 40 random layers,
-// within 15 % (an odd number of chunks goes to its slower kernel).  28x28x128 at
-// batch 32: 50 -> 37 us with the filter's launch, 14x14x256 50 -> 37, 13x13
-// 512 -> 64 at batch 116 81 -> 63, 80x104 624 -> 224 170 -> 94; 56x56x64 at batch 32
-// is level, 87x87 96 -> 32 at batch 82 155 / 162.
+// By the estimates of both: of 700 random layers of 128 of Winograd's units (32 tiles x
+// 32 features) and more 477 run here, in 0.80 of the time in the geometric mean, ten of
+// them slower by more than 3 %, one by 11 (28x28x128 at batch 32: 50 -> 40 us with
+// the filter's launch, 80x104 624 -> 224 170 -> 94, gradient of 44x14x14 704 <- 32,
+// VALID, 27.8 -> 29.1).
 bool winograd_halves(int direction, const snn_hip_conv2d_params& p) {
   const double us = conv2d_halves_f32_us(direction, p, true);
   if (us < 0 || conv2d_halves_f32_workspace_floats(direction, p, true) >
@@ -1064,21 +1063,13 @@ bool winograd_halves(int direction, const snn_hip_conv2d_params& p) {
   if (const char* const env = SNN_TUNING_ENV("SNN_HIP_HALVES"))
     return std::atoi(env) != 0;
   const bool backprop = direction == SNN_HIP_INPUT_BACKPROP;
-  const int chunks = (backprop ? p.features : p.channels) / 16;
   const size_t tiles =
       static_cast<size_t>(p.batch) *
       ceil_div(backprop ? p.in_rows : p.out_rows, 2) *
       ceil_div(backprop ? p.in_cols : p.out_cols, 2);
   const size_t units = ceil_div(tiles, size_t{32}) *
                        ((backprop ? p.channels : p.features) / 32);
-  if (units < 128) return false;
-  double rounds = units / 512.0;
-  rounds = rounds <= 0.5 ? 0.6
-           : rounds < 4  ? std::max(1.0, std::ceil(2 * rounds) / 2)
-                         : rounds;
-  const double winograd_us =
-      7 + rounds * (chunks % 2 == 0 ? 1.9 + 2.2 * chunks : 1.5 + 3.3 * chunks);
-  return us < winograd_us;
+  return units >= 128 && us < conv2d_winograd_fused_us(direction, p);
 }
 
 // Winograd / WinogradLarge: F(2x2,3x3) for forward and input backprop of 3x3

@@ -117,6 +117,7 @@ int launch_conv2d_winograd_1d_f32(int direction, const float* input,
 // aligned pointers and only the transformed-filter part of the workspace.
 bool conv2d_winograd_fused_supports(int direction,
                                     const snn_hip_conv2d_params& p);
+double conv2d_winograd_fused_us(int direction, const snn_hip_conv2d_params& p);
 int launch_conv2d_winograd_fused_f32(int direction, const float* input,
                                      const float* filter, float* output,
                                      const snn_hip_conv2d_params& p,

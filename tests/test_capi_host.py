@@ -456,3 +456,16 @@ def test_gradients_of_few_channels_stay(shape):
     direction = DIRECTION.INPUT_BACKPROP
     algorithm = ops.default_algorithm(p, direction, DTYPE.F32)
     assert ops.halves_tile(p, direction, algorithm) is None
+
+
+@pytest.mark.parametrize("shape,direction", [
+    ((8, 61, 61, 528, 32), DIRECTION.FORWARD),
+    ((10, 41, 41, 656, 32), DIRECTION.FORWARD),
+    ((27, 29, 29, 752, 32), DIRECTION.FORWARD),
+    ((83, 14, 14, 80, 32), DIRECTION.FORWARD),
+])
+def test_winograd_layers_of_an_odd_number_of_chunks_stay(shape, direction):
+    """Those are up to a fifth faster on Winograd's kernel, which goes round the compute
+    units in fractions of a round."""
+    p = ops.conv_params(*shape, 3, 1, True)
+    assert ops.halves_tile(p, direction, ALGO.WINOGRAD) is None
