@@ -15,11 +15,9 @@
 // (2^-24.7 in the root mean square, of either sign): three instructions for what takes
 // eight of the fp32 one.  The two small products have accumulators of their own.
 // Against 64 bits the sums are closer than those of the fp32 instruction, which rounds
-// at every second product (this one at every sixteenth) and than Winograd's; where a
-// launch would otherwise run on tiles of three bfloat16 parts, or divide its
-// reductions, this one sums in parts too (parts_wanted).  On 40 random layers of 250
-// to 8200 products no result is further off by more than 3 % in the 2-norm, 0.6 of
-// the error before in the middle of those that run here.
+// more often, and than Winograd's; where a launch would otherwise run on tiles of
+// three bfloat16 parts, or divide its reductions, this one sums in parts too
+// (choose_parts).
 //
 // Nothing is lost of small values beside large ones.  The exponents are chosen for
 // every 32 channels of a tile's pixels, and of 32 features' filter, from their
@@ -83,6 +81,8 @@ struct Halves {
   int n_slots;
   int n_fslices, n_fblocks, n_cblocks;
   int part;        // channel blocks whose sums are taken together
+  int pause;       // taps of one block that are, or all it has
+  int least;       // ... where so many follow
   int headroom;    // powers of two that sums can be scaled up by
   int transposed;  // w[taps - 1 - tap][feature][channel]
   int relu;
@@ -616,7 +616,7 @@ __global__ void __launch_bounds__(128 * WF * WP)
   };
   // A tap: units `u` ... of a group of three taps.  `rem` units are left at its start,
   // at `a_at`; after the last ones come the first ones at `a_next`.
-  int rem = 0;
+  int rem = 0, exchange = 0, pause = 0;
   unsigned a_at = 0, a_next = 0;
   auto one_tap = [&](auto first) {
     constexpr int U = decltype(first)::value;
@@ -720,18 +720,27 @@ __global__ void __launch_bounds__(128 * WF * WP)
       barrier();  // the first block is there
       restart = false;
     }
-    int flags;
+    int flags = 0;
     a_at = a_slice;
     // Parts of the reduction: the sums of all but the last lie in `dst` meanwhile.
+    bool inside = false;  // a block goes on behind its part
     for (bool first = true;; first = false) {
       clear();
       for (;; buf ^= 1) {
-        cur = tile_lds + buf * tile_bytes;
-        at = col = 0;
+        if (!inside) {
+          cur = tile_lds + buf * tile_bytes;
+          at = col = 0;
+          flags = __builtin_amdgcn_readfirstlane(blocks[buf].flags);
+          rem = taps * FA;
+          // (the loading waves exchange their ranges in the middle)
+          exchange = rem - taps / 3 / 2 * (3 * FA);
+          pause = (flags & kBand1) != 0 ? 0 : rem;
+        }
+        pause -= g.pause * FA;
+        if (pause < g.least * FA) pause = 0;
 #pragma unroll
-        for (int j = 0; j < PB; ++j) read_b(j, 0);
-        flags = __builtin_amdgcn_readfirstlane(blocks[buf].flags);
-        if ((flags & kRare) != 0) {
+        for (int j = 0; j < PB; ++j) read_b(j, at);
+        if ((flags & kRare) != 0 && !inside) {
           if ((flags & kPlain) != 0) break;
           if ((flags & kAgain) != 0) {
             a_at -= block_bytes;
@@ -744,11 +753,9 @@ __global__ void __launch_bounds__(128 * WF * WP)
                              blocks[buf].by[(wf * FA + i) / 2]));
           }
         }
-        rem = taps * FA;
         // (of the block after this one: the tile's next, or the next tile's first)
-        a_next = (flags & kLast) != 0 ? a_slice_next : a_at + block_bytes;
-        // (the loading waves exchange their ranges in the middle)
-        const int exchange = rem - taps / 3 / 2 * (3 * FA);
+        if (!inside)
+          a_next = (flags & kLast) != 0 ? a_slice_next : a_at + block_bytes;
         while (rem >= 3 * FA) {
           if (rem == exchange) barrier();
           one_tap(std::integral_constant<int, 0>{});
@@ -756,7 +763,10 @@ __global__ void __launch_bounds__(128 * WF * WP)
           one_tap(std::integral_constant<int, 2 * FA>{});
           rem -= 3 * FA;
           a_at += 3 * tap_bytes;
+          if (rem == pause) break;
         }
+        inside = rem > 0 && rem == pause;
+        if (inside) break;
         if (taps < 3) barrier();
         if (rem >= FA) {
           one_tap(std::integral_constant<int, 0>{});
@@ -815,7 +825,7 @@ __global__ void __launch_bounds__(128 * WF * WP)
             for (int j = 0; j < PB; ++j) acc[i][j] *= t;
           }
         }
-        buf ^= 1;
+        if (!inside) buf ^= 1;
       } else {
         // The fp32 instruction sums, a block's channels of one tap at a time (in `low`):
         // what it makes of an infinity or NaN in the filter and the zeros of padding is
@@ -882,7 +892,7 @@ __global__ void __launch_bounds__(128 * WF * WP)
       // (a lane holds four features of a pixel, four lanes 16: runs of 64 bytes)
       const __amdgpu_buffer_rsrc_t bias_rsrc =
           make_rsrc(bias, bias != nullptr ? g.features * 4u : 0u);
-      const bool complete = (flags & (kLast | kPlain)) != 0;
+      const bool complete = (flags & (kLast | kPlain)) != 0 && !inside;
       const bool act = complete && (bias != nullptr || g.relu != 0);
       unsigned to[PB];
 #pragma unroll
@@ -1018,25 +1028,57 @@ int rows_spanned(const Halves& g, int pixels) {
          strips_in * (g.win_rows - g.step_rows > 0 ? g.win_rows - g.step_rows : 0);
 }
 
+// What the result is off by against 64 bits, squared and relative in the 2-norm: by the
+// operands, by the sums (a root law: parts count by the squares of their products) and
+// by adding up the parts.  Fitted to 700 random layers, within a tenth.
+double error2(const Halves& g, int* parts) {
+  const int taps = g.win_rows * g.win_cols;
+  double squares = 0, part = 0;
+  *parts = 0;
+  for (int cb = 0; cb < g.n_cblocks; ++cb) {
+    const int channels = std::min(kKC, g.channels - cb * kKC);
+    for (int left = taps; left > 0;) {
+      const bool pauses = left - g.pause >= g.least;
+      const int now = pauses ? g.pause : left;
+      left -= now;
+      part += now * channels;
+      if (pauses || (left == 0 && ((cb + 1) % g.part == 0 ||
+                                   cb + 1 == g.n_cblocks))) {
+        squares += part * part;
+        part = 0;
+        ++*parts;
+      }
+    }
+  }
+  return 0.78e-14 + 38.4e-18 * squares / (taps * g.channels) + 0.02e-14 * *parts;
+}
+
 // Parts of the reduction whose sums are added up by themselves, so that the result is
-// no further from 64 bits than that of the kernel the launch would run on otherwise;
-// 0: none are enough.  What the sum of n products in order is off by, in the 2-norm,
-// is 6.1e-9 sqrt(n) here (17x27x27 96 -> 256, 5x5, 2400 products: 3.1e-7), and less by
-// the root of the number of parts; the operands' own error is 0.9e-7.  The gathering
-// kernel's tiles of three bfloat16 parts have that of the sums alone, with the shares
-// of a reduction as parts (the same layer in two: 2.3e-7), the fp32 instruction twice
-// as much, Winograd more (28x28x128: 3e-7 and 2.3e-7 here).
-int parts_wanted(int direction, const snn_hip_conv2d_params& p, const Halves& g,
-                 bool winograd) {
+// no further from 64 bits than that of the kernel the launch would run on otherwise:
+// their number, 0 if that cannot be had.  (17x27x27 96 -> 256, 5x5, 2400 products,
+// 1.56e-7 on tiles of three bfloat16 parts with the reduction in two: 3.1e-7 whole,
+// 1.98e-7 in three, 1.58e-7 in six.  Winograd's kernel is off by more: 28x28x128
+// 3.1e-7, here 2.3e-7 whole.)
+int choose_parts(int direction, const snn_hip_conv2d_params& p, bool winograd,
+                 Halves* g) {
+  const int taps = g->win_rows * g->win_cols;
+  int parts = 0;
+  g->part = g->n_cblocks;
+  g->pause = g->least = taps;
   if (winograd) return 1;
-  const double shares = conv2d_gemm_f32_shares(direction, p);
-  const double n = static_cast<double>(g.win_rows) * g.win_cols * g.channels;
-  const double own = 0.9e-7 / 6.1e-9;
-  // (a tenth of the square is nothing)
-  const double left = 1.1 / shares - own * own / n;
-  if (left * g.n_cblocks < 0.9) return 0;
-  return std::max(1, std::min(g.n_cblocks,
-                              static_cast<int>(std::ceil(1 / left))));
+  // (a hundredth is nothing)
+  const double most = 1.02 * conv2d_gemm_f32_error2(direction, p);
+  for (int n = 1; n <= g->n_cblocks; ++n) {
+    const int part = ceil_div(g->n_cblocks, n);
+    if (n > 1 && part == g->part) continue;
+    g->part = part;
+    if (error2(*g, &parts) <= most) return parts;
+  }
+  for (g->pause = taps / 6 * 3; g->pause > 0; g->pause -= 3) {
+    g->least = std::min(g->pause, 6);
+    if (error2(*g, &parts) <= most) return parts;
+  }
+  return 0;
 }
 
 int tuned(const char* value, int otherwise) {
@@ -1049,13 +1091,12 @@ HalvesPlan compute_plan(int direction, const snn_hip_conv2d_params& p,
   Halves g;
   if (!geometry(direction, p, &g)) return best;
   const int taps = g.win_rows * g.win_cols;
-  const int parts = parts_wanted(direction, p, g, winograd);
+  const int parts = choose_parts(direction, p, winograd, &g);
   if (parts == 0) return best;
   // (n products below 2^15 * 2^15 each, and fp32 ends at 2^128)
   g.headroom = 97;
   for (long n = static_cast<long>(taps) * g.channels; n > 1; n = (n + 1) / 2)
     --g.headroom;
-  g.part = ceil_div(g.n_cblocks, parts);
   const int only = tuned(SNN_TUNING_ENV("SNN_HIP_HALVES_FORM"), -1);
   for (int strips = 1; strips <= 8; ++strips) {
     g.strip_cols = ceil_div(g.out_cols, strips);
@@ -1111,8 +1152,7 @@ HalvesPlan compute_plan(int direction, const snn_hip_conv2d_params& p,
         const double fill = 900 + 510.0 * pieces;
         const double tile_cycles =
             fill + g.n_cblocks * std::max(products, fill) +
-            (2.0 * ceil_div(g.n_cblocks, g.part) - 1) * f.pixels() *
-                f.features() * 4 / 14.5;
+            (2.0 * parts - 1) * f.pixels() * f.features() * 4 / 14.5;
         double rounds = static_cast<double>(groups) / kNumCus;
         rounds = rounds < 4 ? std::ceil(rounds) : rounds + 0.5;
         // (the launch that takes the filter apart holds 32 taps in registers)

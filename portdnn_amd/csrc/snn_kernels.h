@@ -310,10 +310,8 @@ int launch_conv2d_general_f16(int direction, const _Float16* src,
 // implicit-GEMM kernels, whichever it takes.
 double conv2d_gemm_f32_us(int direction, const snn_hip_conv2d_params& p);
 
-// Into how many sums of their own such a launch divides its reductions, counted as a
-// quarter each where the fp32 instruction adds them, whose sums are twice as far from
-// 64 bits as those of operands in parts.
-double conv2d_gemm_f32_shares(int direction, const snn_hip_conv2d_params& p);
+// The square of its relative error against 64 bits, in the 2-norm, at least.
+double conv2d_gemm_f32_error2(int direction, const snn_hip_conv2d_params& p);
 
 // Forward convolution (with bias and activation, if asked for) and input
 // gradient in fp32 on the same gathering kernel: every window, stride, channel

@@ -84,6 +84,61 @@ def test_taken_apart(shape, direction, tag, tile):
                        got.view(torch.int32).reshape(-1))
 
 
+@pytest.mark.parametrize("shape,direction,before", [
+    ((17, 27, 27, 96, 256, 5, 1, True), F, 1.56e-7),   # parts inside a block of channels
+    ((16, 16, 16, 192, 240, 5, 1, True), F, 1.58e-7),
+    ((24, 39, 39, 32, 48, 7, 1, True), F, 1.77e-7),    # one block
+    ((7, 36, 27, 128, 320, 4, 1, True), F, 1.43e-7),
+    ((51, 26, 26, 204, 324, 3, 2, False), F, 1.42e-7),
+    ((28, 18, 18, 176, 244, 3, 1, True), F, 1.25e-7),
+    ((17, 39, 50, 48, 300, 3, 1, True), F, 9.0e-8),    # a short reduction
+    ((13, 17, 22, 128, 480, 2, 1, True), F, 1.17e-7),  # eight waves' sums of their own
+    ((40, 8, 10, 192, 208, 4, 1, True), I, 1.65e-7),
+    ((16, 20, 26, 72, 512, 4, 1, True), I, 2.72e-7),
+])
+def test_error_is_that_of_the_kernel_before(shape, direction, before):
+    """Against 64 bits in the 2-norm, normal values: no more than on the kernel that the
+    layer has without room for the filter, whose error stands here (and a thirtieth:
+    what the estimate of the parts is good for)."""
+    p = ops.conv_params(*shape)
+    rng = torch.Generator().manual_seed(5150)
+    x_shape = (p.batch, p.in_rows, p.in_cols, p.channels)
+    y_shape = (p.batch, p.out_rows, p.out_cols, p.features)
+    k, s = p.window_rows, p.stride_rows
+    w = torch.randn(k, k, p.channels, p.features, generator=rng).cuda()
+    a = torch.randn(x_shape if direction == F else y_shape, generator=rng).cuda()
+    if direction == F:
+        a.relu_()
+    rows = (p.out_rows - 1) * s + k
+    cols = (p.out_cols - 1) * s + k
+    whole = torch.zeros(p.batch, max(rows, p.pad_rows + p.in_rows),
+                        max(cols, p.pad_cols + p.in_cols), p.channels,
+                        dtype=torch.float64, device="cuda")
+    inner = whole[:, p.pad_rows:p.pad_rows + p.in_rows,
+                  p.pad_cols:p.pad_cols + p.in_cols]
+    if direction == F:
+        inner.copy_(a)
+    y = torch.zeros(a.numel() // a.shape[-1] if direction == I else
+                    p.batch * p.out_rows * p.out_cols, p.features,
+                    dtype=torch.float64, device="cuda")
+    for r in range(k):
+        for c in range(k):
+            taps = whole[:, r:r + (p.out_rows - 1) * s + 1:s,
+                         c:c + (p.out_cols - 1) * s + 1:s]
+            if direction == F:
+                y += taps.reshape(-1, p.channels) @ w[r, c].double()
+            else:
+                taps += (a.double().reshape(-1, p.features) @
+                         w[r, c].double().t().contiguous()).reshape(taps.shape)
+    ref = (y if direction == F else inner).reshape(-1)
+    algorithm = ops.default_algorithm(p, direction, DTYPE.F32)
+    _, rec = ops.workspace_size(p, direction, algorithm, DTYPE.F32)
+    got = ops.conv2d(a.reshape(-1), w.reshape(-1), p, direction, algorithm,
+                     workspace=torch.empty(max(rec, 1), device="cuda"))
+    error = (got.reshape(-1).double() - ref).norm() / ref.norm()
+    assert error.item() <= 1.033 * before
+
+
 @pytest.mark.parametrize("tag,shape", [
     (TILED, (9, 41, 43, 100, 68, 4, 1, False)),
     (TILED, (16, 27, 27, 96, 256, 5, 1, True)),   # in parts
