@@ -718,19 +718,26 @@ FilterHalvesPlan compute_plan(const snn_hip_conv2d_params& p, bool winograd) {
   // instructions take turns with these, and a constant, in cycles of a 2.1 GHz clock;
   // a partial filter is written and read back: 0.6 us per MB.  Fitted to 110 random
   // layers of 1e5 ... 2e10 products: nine of ten within a tenth.
-  // Pixels whose products a sum adds one after another.  Its error against 64 bits,
-  // relative, is 1.0e-7 (the operands' low parts) and 7.0e-9 per root of these pixels;
-  // that of the kernel behind the same tags 0.56e-7 and 1.29e-8 per root of the pixels
-  // of one of its waves (27 random layers, normal values, all within a tenth).  The
-  // sums are stored in time for it to be no larger; reductions that are too short for
-  // that stay there, and so do those of fewer pixels than that kernel takes (0.5 ...
-  // 0.7e-7), unless one work-group holds all taps and channels (1.3 ... 1.7e-7).  (The
-  // Winograd kernel's is above either: 3.6e-7 at 5000 pixels, 2.0e-7 here.)
+  // The error against 64 bits, squared and relative in the 2-norm: of the operands' low
+  // parts, by the pixels whose products a sum adds one after another, and by the sums
+  // that are added up.  That of the kernel behind the same tags goes by the pixels of
+  // one of its waves and by the waves (400 and 870 random layers, normal values, within
+  // a tenth).  The sums are stored in time for it to be no larger; reductions that are
+  // too short for that stay there, and so do those of fewer pixels than that kernel
+  // takes (0.5 ... 0.7e-7), unless one work-group holds all taps and channels (1.3 ...
+  // 1.7e-7).  (The Winograd kernel's is above either: 3.6e-7 at 5000 pixels, 2.0e-7
+  // here.)
   const double pixels = static_cast<double>(p.batch) * p.out_rows * p.out_cols;
   const double chain = winograd || !conv2d_filter_backprop_direct_f32_wanted(p)
                            ? 0
                            : conv2d_filter_backprop_direct_f32_chain(p);
-  const double most_pixels = chain > 0 ? 3.36 * chain - 135 : pixels;
+  const double operands2 = 0.93e-14, pixel2 = 41.5e-18, sum2 = 0.87e-16;
+  // (what either is off by more or less than that)
+  const double most_error2 =
+      chain > 0 ? 0.91 * (0.28e-14 + 151e-18 * chain + 0.435e-16 * pixels / chain)
+                : 1.0;
+  const double most_pixels =
+      std::min(pixels, (most_error2 - operands2) / pixel2);
   const bool few_rows = p.channels < 32 && p.window_rows * p.window_cols *
                                                    p.channels <= 192;
   if (most_pixels < 32 || (!winograd && !few_rows &&
@@ -771,18 +778,25 @@ FilterHalvesPlan compute_plan(const snn_hip_conv2d_params& p, bool winograd) {
         const long most = std::max<long>(1, std::min<long>(tasks, kNumCus / n_units));
         const long fewer = std::lround(std::sqrt(tasks * task_us / (filter_mb * 0.6)));
         const long task_pixels = std::max(1l, std::lround(pixels / tasks));
-        const long most_tasks = static_cast<long>(1.05 * most_pixels) / task_pixels;
-        if (most_tasks < 1) continue;
+        if (most_pixels < task_pixels) continue;
         for (const long want : {most, std::max(1l, std::min(most, fewer))}) {
           const long per_split = (tasks + want - 1) / want;
           const long splits = (tasks + per_split - 1) / per_split;
           // (as many tasks for each sum of a split as can be)
-          const long least_sums = (per_split + most_tasks - 1) / most_tasks;
-          const long per_sum = (per_split + least_sums - 1) / least_sums;
-          const long sums = (per_split + per_sum - 1) / per_sum;
           const long last = tasks - (splits - 1) * per_split;
-          const long slices = (splits - 1) * sums + (last + per_sum - 1) / per_sum;
-          if (slices * filter_mb > 256) continue;
+          long per_sum = std::min(
+              per_split, std::max(1l, std::lround(most_pixels / task_pixels)));
+          long sums = 0, slices = 0;
+          bool close = false;
+          for (;;) {
+            sums = (per_split + per_sum - 1) / per_sum;
+            slices = (splits - 1) * sums + (last + per_sum - 1) / per_sum;
+            const double added2 = operands2 + sum2 * slices;
+            close = added2 + pixel2 * per_sum * task_pixels <= most_error2;
+            if (close || per_sum == 1 || added2 > most_error2) break;
+            per_sum = std::min(per_sum - 1, (per_split + sums) / (sums + 1));
+          }
+          if (!close || slices * filter_mb > 256) continue;
           const double rounds =
               std::ceil(static_cast<double>(splits) * n_units / kNumCus);
           const double cost = rounds * per_split * task_us + 7.9 +
