@@ -924,8 +924,8 @@ int launch_gemm_path<_Float16>(int direction, const _Float16* input,
 // 256 -> 120, 3x3: 84 -> 35); small ones stay, whose reductions the others share
 // among work-groups (4x10x10 896 -> 192, 3x3: 23 -> 89), and gradients of a few
 // channels, whose taps are multiplied at once and folded (60x10x10 4 <- 544, 5x5:
-// 29 -> 103).  A strided window reads four times the pixels for a tile, which the
-// estimate meets less well.  1x1 windows have no taps to take an operand apart for,
+// 29 -> 103).  A strided window reads four times the pixels for a tile and a small one
+// has few products for them, which the estimate meets less well.  1x1 windows have no taps to take an operand apart for,
 // and 3x3 layers of whole chunks come here behind the Winograd tag, which brings room
 // for the filter.
 bool halves_wanted(int direction, const snn_hip_conv2d_params& p) {
@@ -937,8 +937,9 @@ bool halves_wanted(int direction, const snn_hip_conv2d_params& p) {
   if (us < 0) return false;
   if (const char* const env = SNN_TUNING_ENV("SNN_HIP_HALVES"))
     return std::atoi(env) != 0;
-  const bool strided = p.stride_rows > 1 || p.stride_cols > 1;
-  return (strided ? 1.1 : 1.0) * us < conv2d_gemm_f32_us(direction, p);
+  const bool rough = p.stride_rows > 1 || p.stride_cols > 1 ||
+                     p.window_rows * p.window_cols < 9;
+  return (rough ? 1.1 : 1.0) * us < conv2d_gemm_f32_us(direction, p);
 }
 
 template <>

@@ -29,8 +29,8 @@ CASES = [
     ((8, 30, 29, 160, 132, 3, 1, True), I, TILED, (60, 128)),   # ragged channels
     ((9, 41, 43, 100, 64, 3, 1, True), F, WINO, (64, 64)),
     ((40, 8, 8, 256, 132, 3, 1, True), I, TILED, (64, 64)),     # whole images
-    ((3, 50, 60, 128, 160, 2, 1, True), F, TILED, (120, 64)),   # four taps
-    ((3, 50, 60, 128, 160, 2, 1, True), I, TILED, (40, 128)),   # strips
+    ((3, 50, 60, 256, 160, 2, 1, True), F, TILED, (120, 64)),   # four taps
+    ((3, 50, 60, 256, 160, 2, 1, True), I, TILED, (75, 128)),   # strips
     ((9, 41, 43, 100, 68, 4, 1, False), F, TILED, (60, 128)),   # sixteen taps
     ((1, 80, 104, 112, 224, 3, 1, True), F, WINO, (240, 32)),
     ((6, 57, 61, 40, 36, 7, 1, True), F, TILED, (93, 64)),      # 49 taps
