@@ -1155,7 +1155,8 @@ HalvesPlan compute_plan(int direction, const snn_hip_conv2d_params& p,
         const double fill = 900 + 510.0 * pieces;
         const double tile_cycles =
             fill + g.n_cblocks * std::max(products, fill) +
-            (2.0 * parts - 1) * f.pixels() * f.features() * 4 / 14.5;
+            (2.0 * parts - 1) * f.pixels() * f.features() * 4 / 14.5 +
+            1500.0 * (parts - ceil_div(g.n_cblocks, g.part));  // ends inside blocks
         double rounds = static_cast<double>(groups) / kNumCus;
         rounds = rounds < 4 ? std::ceil(rounds) : rounds + 0.5;
         // (the launch that takes the filter apart holds 32 taps in registers)
