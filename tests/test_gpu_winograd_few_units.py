@@ -71,6 +71,7 @@ def test_winograd_few_units(shape, direction):
     (2, 14, 14, 160, 96, True),   # ... and a split channel range
     (3, 14, 14, 64, 64, True),
     (9, 20, 42, 16, 736, True),
+    (16, 28, 28, 96, 128, True),  # its filter is taken apart into binary16 values
 ], ids=lambda s: "x".join(map(str, s)))
 def test_prepared_workspace_is_only_read(shape, direction):
     """What a filter was transformed to survives every prepared launch, aligned or
@@ -80,6 +81,7 @@ def test_prepared_workspace_is_only_read(shape, direction):
     p = ops.conv_params(batch, rows, cols, *(
         (channels, features) if direction == DIRECTION.FORWARD else
         (features, channels)), 3, 1, same)
+    assert (ops.halves_tile(p, direction, ALGO.WINOGRAD) is not None) == (batch == 16)
     rng = np.random.default_rng(8200 + rows)
     n_a, n_b, n_out = ops.conv_sizes(p, direction)
     a, b = uniform(rng, n_a), uniform(rng, n_b)
