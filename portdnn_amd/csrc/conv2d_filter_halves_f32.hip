@@ -90,9 +90,9 @@ __device__ __forceinline__ unsigned between(const uint4v& before, const uint4v& 
                                    16);
 }
 
-// 17x27x27 96 -> 256, 5x5: 88 us with the launch that adds (180 on the fp32
-// instruction); 28x28x128 at batch 32, 3x3: 37.6 (56.1 by Winograd's transform),
-// 64x64x256 at batch 8: 132 (195).  A chunk's 54 (60) matrix instructions of a wave
+// 17x27x27 96 -> 256, 5x5: 81 us with the launch that adds (179 on the fp32
+// instruction); 28x28x128 at batch 32, 3x3: 34 (51 by Winograd's transform),
+// 64x64x256 at batch 8: 126 (196).  A chunk's 54 (60) matrix instructions of a wave
 // are 864 (960) cycles, half the time: the vector instructions of the SIMD's other
 // wave, 22 per piece of 16 bytes for scaling, taking apart and noting the range, take
 // turns with them.  So the range of a task is looked at while its values are taken
@@ -679,7 +679,6 @@ struct FilterHalvesPlan {
   FilterHalves g;
   int nx = 0;
   bool wanted = false;  // against the kernels behind the same tags
-  double us = 0;
 };
 
 int round_up(int a, int b) { return ceil_div(a, b) * b; }
@@ -823,7 +822,6 @@ FilterHalvesPlan compute_plan(const snn_hip_conv2d_params& p, bool winograd) {
   g.by_segs = divisor(g.segs);
   g.by_bands = divisor(g.bands_per_image);
   plan.shape = five ? k5x5 : k3x3;
-  plan.us = best;
   if (p.channels >= 16 && p.features >= 16)
     plan.wanted = winograd ? pixels >= 1024
                            : !conv2d_filter_backprop_direct_f32_wanted(p) ||
@@ -866,10 +864,10 @@ void launch_shape(const float* x, const float* dy, float* part,
 }  // namespace
 
 // Behind the Winograd tag from 1024 output pixels on, where the default policy names
-// that tag (28x28x128 at batch 32: 38 us instead of 56, 64x64x256 at batch 8: 124
-// instead of 195); behind the others in place of the kernel that holds all taps and
+// that tag (28x28x128 at batch 32: 34 us instead of 51, 64x64x256 at batch 8: 126
+// instead of 196); behind the others in place of the kernel that holds all taps and
 // channels (163x212x24 at batch 7 -> 32: 39 us instead of 150) and of the one for tiles
-// of 64 where its estimate is higher (17x27x27 96 -> 256, 5x5: 88 us instead of 180;
+// of 64 where its estimate is higher (17x27x27 96 -> 256, 5x5: 81 us instead of 179;
 // 9x9x144 -> 528 at batch 5, below the line: 18.3 here, 11.1 there).
 bool conv2d_filter_halves_f32_wanted(const snn_hip_conv2d_params& p, bool winograd) {
   return make_plan(p, winograd).wanted;

@@ -2,7 +2,7 @@
 // instruction (gfx950): every operand as the sum of two binary16 values, fp32
 // accumulation.
 //
-// The fp32 matrix instruction does 64 multiply-adds per cycle and SIMD, the
+// The fp32 matrix instruction does 32 multiply-adds per cycle and SIMD, the
 // binary16 one 512, of values with 11 significant bits.  A value times a power of two
 // that brings it into binary16's range is
 //
@@ -12,14 +12,15 @@
 //
 //   v w = hi hi' + 2^-11 (hi lo' + lo hi') + what is left out, below 2^-22 |v w|
 //
-// (2^-24.7 in the root mean square, of either sign): three instructions for what takes
-// eight of the fp32 one.  The two small products have accumulators of their own.
-// Against 64 bits the sums are closer than those of the fp32 instruction, which rounds
+// (2^-24.7 in the root mean square, of either sign): three instructions' time for what
+// takes sixteen with the fp32 one.  The two small products have accumulators of their
+// own.  Against 64 bits the sums are closer than those of the fp32 instruction, which rounds
 // more often, and than Winograd's; where a launch would otherwise run on tiles of
 // three bfloat16 parts, or divide its reductions, this one sums in parts too
-// (choose_parts).
+// (choose_parts).  A sum of a few products that are not zero is further off than on the
+// fp32 instruction, by what the operands are.
 //
-// Nothing is lost of small values beside large ones.  The exponents are chosen for
+// Small values beside large ones keep as many bits as those.  The exponents are chosen for
 // every 32 channels of a tile's pixels, and of 32 features' filter, from their
 // largest value; accumulators follow by multiplying with powers of two.  What is
 // smaller than 2^-26 of the largest (one value in 2e7 of normally distributed ones)
@@ -39,8 +40,9 @@
 //     instruction's operand) and streams from L2 into registers.
 //
 // Whole calls with the filter's launch of 5 us, before / here: 28x28x128 at batch 32,
-// 3x3, 47 (Winograd) / 36 us, 64x64x256 at batch 8 162 / 99, 17x27x27 96 -> 256, 5x5,
-// 114 (three bfloat16 parts) / 64 and its gradient 160 (fp32 instruction) / 77.  Of the
+// 3x3, 44 (Winograd) / 34 us, 64x64x256 at batch 8 161 / 98, 17x27x27 96 -> 256, 5x5,
+// 112 (three bfloat16 parts) / 76 in six parts, 62 in three, and its gradient 159 (fp32
+// instruction) / 78.  Of the
 // 28 us of the first one's kernel the matrix units need 13; the rest is the first
 // pixels' way into LDS (6), the last stores (3), 0.85 of their rate in between, and
 // 32 compute units without a tile.

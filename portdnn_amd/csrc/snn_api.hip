@@ -918,10 +918,10 @@ int launch_gemm_path<_Float16>(int direction, const _Float16* input,
 }
 // Whether a launch behind the Tiled, Im2col or Matmul tag goes to the kernel that
 // takes its operands apart into binary16 values, by the estimates of both.  Of 1700
-// random layers with windows of 2x2 to 9x9 and 4 to 900 channels 335 run there, in
-// 0.61 of the time in the geometric mean, nine of them slower by more than 3 %, one by
-// 15 (17x27x27 96 -> 256, 5x5: 113 -> 62 us, its gradient 159 -> 76; 64x16x16
-// 256 -> 120, 3x3: 84 -> 35); small ones stay, whose reductions the others share
+// random layers with windows of 2x2 to 9x9 and 4 to 900 channels 315 run there, in
+// 0.60 of the time in the geometric mean, eleven of them slower by more than 3 %, one
+// by 11 (17x27x27 96 -> 256, 5x5: 112 -> 76 us, its gradient 159 -> 78; 64x16x16
+// 256 -> 120, 3x3: 84 -> 36); small ones stay, whose reductions the others share
 // among work-groups (4x10x10 896 -> 192, 3x3: 23 -> 89), and gradients of a few
 // channels, whose taps are multiplied at once and folded (60x10x10 4 <- 544, 5x5:
 // 29 -> 103).  A strided window reads four times the pixels for a tile and a small one
@@ -1053,8 +1053,8 @@ bool winograd_loses(int direction, const snn_hip_conv2d_params& p,
 // filter is prepared for the kernel that its launches then take.
 // By the estimates of both: of 700 random layers of 128 of Winograd's units (32 tiles x
 // 32 features) and more 477 run here, in 0.80 of the time in the geometric mean, ten of
-// them slower by more than 3 %, one by 11 (28x28x128 at batch 32: 50 -> 40 us with
-// the filter's launch, 80x104 624 -> 224 170 -> 94, gradient of 44x14x14 704 <- 32,
+// them slower by more than 3 %, one by 11 (28x28x128 at batch 32: 44 -> 34 us with
+// the filter's launch, 80x104 624 -> 224 169 -> 87, gradient of 44x14x14 704 <- 32,
 // VALID, 27.8 -> 29.1).
 bool winograd_halves(int direction, const snn_hip_conv2d_params& p) {
   const double us = conv2d_halves_f32_us(direction, p, true);

@@ -202,10 +202,10 @@ size_t conv2d_filter_backprop_direct_f32_partial_floats(
     const snn_hip_conv2d_params& p);
 size_t conv2d_filter_backprop_direct_f16_partial_floats(
     const snn_hip_conv2d_params& p);
-// estimated time of the f16 form with multiples of 4
 double conv2d_filter_backprop_direct_f32_us(const snn_hip_conv2d_params& p);
 // Pixels of a wave's sums; 0 where the kernel does not take the layer.
 double conv2d_filter_backprop_direct_f32_chain(const snn_hip_conv2d_params& p);
+// estimated time of the f16 form with multiples of 4
 double conv2d_filter_backprop_direct_f16_us(const snn_hip_conv2d_params& p);
 int launch_conv2d_filter_backprop_direct_f32(const float* input,
                                              const float* output_gradient,
