@@ -352,6 +352,70 @@ def test_many_infinities(direction, tag, shape, operand):
     assert error.max() <= 2 * np.sqrt(n) * n * 2.0**-24
 
 
+def forward64(p, x, w):
+    k = p.window_rows
+    whole = torch.zeros(p.batch, p.out_rows + k - 1, p.out_cols + k - 1, p.channels,
+                        dtype=torch.float64, device="cuda")
+    whole[:, p.pad_rows:p.pad_rows + p.in_rows,
+          p.pad_cols:p.pad_cols + p.in_cols] = x
+    y = torch.zeros(p.batch * p.out_rows * p.out_cols, p.features,
+                    dtype=torch.float64, device="cuda")
+    for r in range(k):
+        for c in range(k):
+            taps = whole[:, r:r + p.out_rows, c:c + p.out_cols]
+            y += taps.reshape(-1, p.channels) @ w[r, c].double()
+    return y
+
+
+@pytest.mark.parametrize("shape", [
+    (2, 49, 55, 32, 68, 7, 1, True),     # 24 and 25 taps of one block
+    (7, 29, 54, 64, 192, 4, 1, True),    # 6 and 10 of two
+    (8, 29, 47, 48, 192, 5, 1, True)])   # 12 and 13, a block of half the channels
+@pytest.mark.parametrize("kind", ["normal", "pixels", "filter", "both", "blocks",
+                                  "zeros", "late"])
+def test_parts_inside_blocks(shape, kind):
+    """Sums that are taken among a block's taps, beside small values that pass a second
+    time, exponents that change, zeros, and a block that ends on the fp32 instruction
+    after parts of the tile are stored; with bias and ReLU behind the last part."""
+    p = ops.conv_params(*shape)
+    tag = ops.default_algorithm(p, F, DTYPE.F32)
+    assert ops.halves_tile(p, F, tag) is not None
+    rng = torch.Generator().manual_seed(5700)
+    x = torch.randn(p.batch, p.in_rows, p.in_cols, p.channels, generator=rng)
+    w = torch.randn(p.window_rows, p.window_rows, p.channels, p.features,
+                    generator=rng) * 0.1
+
+    def few(t):
+        return torch.where(torch.rand(t.shape, generator=rng) < 1e-3, t * 2.0**-30, t)
+    if kind in ("pixels", "both"):
+        x = few(x)
+    if kind in ("filter", "both"):
+        w = few(w)
+    if kind == "blocks":
+        x[..., 32:] *= 2.0**-9
+        w[:, :, 32:] *= 2.0**5
+        x[0] *= 2.0**20
+    if kind == "zeros":
+        x[..., :32] = 0
+        w[:, :, :, 5] = 0
+    if kind == "late":
+        x[0, 3, 4, -1] = 2.0**-100     # of the last block: beyond both exponents
+        w[:, :, -1, 7] = 2.0**-90
+    bias = torch.randn(p.features, generator=rng)
+    x, w, bias = x.cuda(), w.cuda(), bias.cuda()
+    ref, size = forward64(p, x, w), forward64(p, x.abs(), w.abs())
+    _, rec = ops.workspace_size(p, F, tag, DTYPE.F32)
+    ws = torch.empty(rec, device="cuda")
+    n = products(p, F)
+    got = ops.conv2d(x.reshape(-1), w.reshape(-1), p, F, tag, workspace=ws)
+    error = (got.double().reshape(ref.shape) - ref).abs()
+    assert torch.all(error <= 2 * np.sqrt(n) * 2.0**-24 * size + 2.0**-149)
+    act = ops.conv2d_bias_act(x.reshape(-1), w.reshape(-1), bias, p, tag, relu=True,
+                              workspace=ws).double().reshape(ref.shape)
+    want = (got.double().reshape(ref.shape) + bias.double()).clamp_min(0)
+    assert torch.all((act - want).abs() <= 2.0**-23 * want.abs() + 2.0**-149)
+
+
 def test_prepared_filter_without_a_pack():
     """A prepared launch behind another tag than Winograd packs for itself."""
     p, a, b, _ = operands(SHAPE, F, 5600)
