@@ -58,7 +58,8 @@ TRAFFIC_PROFILE = os.path.join("profiles",
 
 def profiled_traffic_bytes(kernel_prefix):
     """Mean of the 'HBM MB / launch' column over the table rows whose kernel
-    name starts with `kernel_prefix`, in bytes; None if there is no such row."""
+    name starts with `kernel_prefix` (or one of them), in bytes; None if there is
+    no such row."""
     path = os.path.join(ROOT, TRAFFIC_PROFILE)
     if not os.path.exists(path):
         return None
@@ -308,8 +309,9 @@ def main():
             total_flops / prepared_ms / 1e9, 3),
         # not measured in this run: FETCH_SIZE / WRITE_SIZE of the same kernel
         # from the committed rocprofv3 summary
-        "traffic": (profiled_traffic_bytes("wino_direct_kernel")
-                    if k3_algos == ["winograd"] else None),
+        "traffic": (profiled_traffic_bytes(("conv_halves_kernel",
+                                            "wino_direct_kernel"))
+                    if k3_algos == ["binary16 parts", "winograd"] else None),
         "traffic_source": "committed profile, not this run: " + TRAFFIC_PROFILE}
 
     # ---- memory-bound half of the metric: depthwise and pooling against HBM ----
